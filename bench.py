@@ -40,15 +40,13 @@ KECCAK_OPS = 4163
 # a generic SHA-256 compression priced at 1450 VALU ops (F needs fewer); the
 # compression rate against 39.32 T / 1450 is reported as frac_at_1450_ops
 SHA256_OPS_UNFUSED = 1450
-# Issue rate of independent instruction blocks in the proportions of the unit's
-# loop body (wave-instructions per SIMD per ns, "mix" rows of profiles/valu_issue_rates.md):
-# SHA-256 F = 717 four-cycle (508 alignbit, 205 add3, 4 perm) : 506 two-cycle
-# (312 bitop3, 194 VOP2) ~ 7:5; Keccak-f round of a WOTS chain step (bit-interleaved)
-# = 52 alignbit : 122 bitop3/xor ~ 3:7.
-# Mixing the two classes issues slower than the sum of their separate rates,
-# so this measured rate, not a 4c/2c model, is the ceiling of a unit.
-MIX_RATE_SHA256 = 0.6235
-MIX_RATE_KECCAK = 0.7501
+# Issue rate of independent instructions in the proportions and the two-phase
+# order of the unit's rounds (wave-instructions per SIMD per ns; rotates and
+# v_add3 at raised wave priority, the rest beside other waves' rotates):
+# SHA-256 10 : 18 at 8 waves per SIMD, a wave instruction every 2.22 cycles;
+# Keccak-f 48 : 120 at 5 waves, every 2.33 cycles.
+MIX_RATE_SHA256 = 1.079
+MIX_RATE_KECCAK = 1.030
 
 
 def mix_ceiling_units(rate, ops_per_unit):
@@ -69,6 +67,11 @@ def kernel_work(p, batch):
         return leaves * (p.len * 16 + tlen) + nodes * hblk
     tlen = (p.n + 32 + p.len * p.n) // 136 + 1
     return leaves * (p.len * 16 + tlen) + nodes
+
+
+def chain_work(p, batch):
+    """The part of kernel_work that k_chains runs: PRF + 15 F per chain."""
+    return batch * p.d * (1 << (p.full_h // p.d)) * p.len * 16
 
 
 def fors_work(p, batch):
@@ -602,8 +605,8 @@ def main():
     sign_s = sum(sign_ms) / len(sign_ms) / 1e3
     ver_s = sum(ver_ms) / len(ver_ms) / 1e3
 
-    # the dominant kernel: the fused FORS + hypertree launch, or k_ht alone
-    kname = "k_sign_fused" if "k_sign_fused" in prof else "k_ht"
+    # the dominant kernel: the WOTS chains, with the FORS tiles in small batches
+    kname = "k_sign_fused" if "k_sign_fused" in prof else "k_chains"
     pmc = None
     try:
         tj = json.load(open(os.path.join(ROOT, "profiles", "pmc_counters.json")))
@@ -636,7 +639,7 @@ def main():
                             long_slots=args.serve_long_slots)
     kt, kn = prof.get(kname, (0.0, 0))
     k_avg = kt / max(kn, 1) / 1e3
-    work = kernel_work(p, B) + (fors_work(p, B) if kname == "k_sign_fused" else 0)
+    work = chain_work(p, B) + (fors_work(p, B) if kname == "k_sign_fused" else 0)
     # lane-instructions per unit: the launch's SQ_INSTS_VALU x 64 over its
     # units, as counted for this kernel and batch (profiles/pmc_counters.json)
     if pmc and pmc.get("sq_insts_valu"):

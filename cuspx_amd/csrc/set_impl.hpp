@@ -17,11 +17,11 @@ template <class P>
 struct Layout {
     static constexpr uint64_t al(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 
-    // lanes per WOTS leaf for a k_ht launch over `trees` subtrees: a tuned
-    // value when the tuning table has one, else double S while the launch
-    // would still fill less than half the chip (S = 1 for large batches).
-    // Subtrees too wide for one workgroup are split into parts, so every
-    // set takes S up to 8.
+    // The split of a sign / keygen batch over `trees` subtrees: a tuned value
+    // when the tuning table has one, else doubled while the launch would
+    // still fill less than half the chip.  k_ht runs a lane per WOTS leaf at
+    // 1 and a lane pair per leaf from 2 on (the chains take a lane each
+    // whatever the split); mixed batches go to the family kernel up to 2.
     static constexpr int max_split() { return 16; }
     static int split(int pid, int op, uint32_t trees) {
         const int t = tuned_split(pid, op, trees);
@@ -64,26 +64,22 @@ struct Layout {
         while (G < vmax() && (uint64_t)n * G * 8 <= kFillLanes) G *= 2;
         return G;
     }
-    // most parts any split gives one subtree (1 when no split subtree exists)
-    static constexpr int max_parts() { return HtShape<P, 16>::PARTS; }
+    static constexpr int L = 1 << P::th;
     template <int S>
     static uint32_t ht_blocks(uint32_t trees) {
         return HtShape<P, S>::PARTS > 1 ? trees * HtShape<P, S>::PARTS
                                         : cdiv(trees, HtShape<P, S>::TPW);
     }
-    template <int S>
+    // workspace room for split subtrees (k_ht uses up to 4 parts) and for the
+    // chain ends' columns, whole workgroups of leaves: the sizes that callers
+    // with a fixed scratch area have had for their batch limits
+    static constexpr int max_parts() { return L * 16 > 1024 ? L * 16 / 256 : 1; }
     static uint64_t tl_cols(uint32_t trees) {
-        return HtShape<P, S>::park ? (uint64_t)ht_blocks<S>(trees) * HtShape<P, S>::NL : 0;
+        constexpr uint64_t lanes = (uint64_t)L * (P::hash == kShake ? 1 : 2);
+        constexpr uint64_t tpw = lanes < 256 ? 256 / lanes : 1;
+        return (trees + tpw - 1) / tpw * tpw * L;
     }
-    static uint64_t tl_cols(uint32_t trees, int S) {
-        switch (S) {
-            case 1: return tl_cols<1>(trees);
-            case 2: return tl_cols<2>(trees);
-            case 4: return tl_cols<4>(trees);
-            case 8: return tl_cols<8>(trees);
-            default: return tl_cols<16>(trees);
-        }
-    }
+    static_assert(max_parts() >= HtShape<P, 2>::PARTS, "part roots fit");
     static uint64_t bytes(int pid, uint32_t n, int op) {
         uint64_t b = al((uint64_t)n * sizeof(Plan));
         b += al((uint64_t)n * P::k * P::n);   // fors roots
@@ -93,14 +89,11 @@ struct Layout {
         if (op == kOpSign) {
             b += al((uint64_t)n * P::d * P::n);                    // layer roots
             b += al((uint64_t)n * P::d * P::len * 16 * P::n);      // chain capture
-            b += al(4);                                            // fused-kernel tile counter
+            b += al(4);                                            // (spare)
         }
         if (op != kOpVerify) {
-            // sized for every split, so a workspace stays valid whichever S runs
             const uint32_t trees = op == kOpSign ? n * P::d : n;
-            uint64_t cols = 0;
-            for (int S = 1; S <= 16; S *= 2) cols = tl_cols(trees, S) > cols ? tl_cols(trees, S) : cols;
-            b += al(cols * P::len * P::nw * 4);
+            b += al(tl_cols(trees) * P::len * P::nw * 4);
             if (max_parts() > 1) {
                 b += al((uint64_t)trees * max_parts() * P::nw * 4);  // part roots
                 b += al((uint64_t)trees * 4);                       // part counters
@@ -109,7 +102,7 @@ struct Layout {
         (void)pid;
         return b + 256;
     }
-    static void carve(int pid, BatchArgs& A, uint8_t* ws, uint32_t n, int op, int S) {
+    static void carve(int pid, BatchArgs& A, uint8_t* ws, uint32_t n, int op) {
         uint8_t* p = (uint8_t*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
         A.plan = (Plan*)p;
         p += al((uint64_t)n * sizeof(Plan));
@@ -129,7 +122,6 @@ struct Layout {
         A.tl_lanes = 0;
         A.ht_parts = nullptr;
         A.ht_count = nullptr;
-        A.tile_ctr = nullptr;
         if (op == kOpVerify) {
             A.cap = p;
             p += al(spec_bytes(n));
@@ -139,16 +131,13 @@ struct Layout {
             p += al((uint64_t)n * P::d * P::n);
             A.cap = p;
             p += al((uint64_t)n * P::d * P::len * 16 * P::n);
-            A.tile_ctr = (uint32_t*)p;
             p += al(4);
         }
         if (op != kOpVerify) {
             const uint32_t trees = op == kOpSign ? n * P::d : n;
             A.tl_buf = (uint32_t*)p;
-            A.tl_lanes = (uint32_t)tl_cols(trees, S);
-            uint64_t cols = 0;
-            for (int s2 = 1; s2 <= 16; s2 *= 2) cols = tl_cols(trees, s2) > cols ? tl_cols(trees, s2) : cols;
-            p += al(cols * P::len * P::nw * 4);
+            A.tl_lanes = leaf_count<P>(trees);
+            p += al(tl_cols(trees) * P::len * P::nw * 4);
             if (max_parts() > 1) {
                 A.ht_parts = (uint32_t*)p;
                 p += al((uint64_t)trees * max_parts() * P::nw * 4);
@@ -160,74 +149,37 @@ struct Layout {
     }
 };
 
-// J: FORS leaves per lane (2^(a-J) lanes per tree) in the tiles of split
-// S >= 4 (small batches: short tiles keep FORS off the critical path; one
-// SHA2-192f request signs in 0.41 ms at J against 0.70 at JB) and in the
-// unfused k_fors; JB: the same in the fused launch at S = 1 and 2 (larger
-// batches, where longer tiles spend less on tile set-up and barriers:
-// SHA2-192f at 1024 requests, S = 2, 7.07 -> 6.63 ms)
+// Chain waves up to which FORS and chains share a launch (k_sign_fused): as
+// many as the chip holds at once, so the batch is a matter of latency and
+// FORS should not run before the chains.  Larger batches launch k_fors and
+// k_chains one after the other: the fused kernel takes the FORS tile's
+// registers (88-144 VGPRs) for the chains too, and k_chains alone needs 64
+// or fewer for SHA-256 and so issues from 8 waves per SIMD instead of 3-5.
+static constexpr uint32_t kFuseWaves = 8192;
+
+// J: FORS leaves per lane (2^(a-J) lanes per tree) in the tiles of the fused
+// launch (short tiles keep FORS off the critical path); JB: the same in
+// k_fors, where longer tiles spend less on tile set-up and barriers
 template <class P, int J, int JB>
 struct SetImpl {
     using Lay = Layout<P>;
-    template <int S>
-    static constexpr int fors_j() { return S <= 2 ? JB : J; }
 
     static int pid_;
     static const char* set_name_;
     static size_t workspace(uint32_t n, int op) { return (size_t)Lay::bytes(pid_, n, op); }
 
-    template <int MODE, int S>
-    static void launch_ht(const BatchArgs& A, uint32_t trees, hipStream_t s) {
-        if constexpr (HtShape<P, S>::WG <= 1024) {
-            hipLaunchKernelGGL((k_ht<P, MODE, S>), dim3(Lay::template ht_blocks<S>(trees)),
-                               dim3(HtShape<P, S>::WG), 0, s, A);
-        }
-    }
-    // FORS and hypertree tiles in one persistent launch (when the split's
-    // hypertree tiles are 256-lane workgroups); false = not applicable
-    template <int S>
-    static bool launch_fused(const BatchArgs& A, uint32_t n, hipStream_t s) {
-        if constexpr (HtShape<P, S>::WG == 256) {
-            constexpr int FJ = fors_j<S>();
-            static const uint32_t resident = [] {
-                int per_cu = 0, cus = 0, dev = 0;
-                if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                        &per_cu, reinterpret_cast<const void*>(&k_sign_fused<P, FJ, S>), 256, 0) !=
-                        hipSuccess ||
-                    hipGetDevice(&dev) != hipSuccess ||
-                    hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-                        hipSuccess)
-                    return 256u;
-                return (uint32_t)((per_cu > 0 ? per_cu : 1) * (cus > 0 ? cus : 1));
-            }();
-            constexpr uint32_t fors_tpw = 256u >> (P::a - FJ);
-            const uint32_t n_ht = Lay::template ht_blocks<S>(n * P::d);
-            const uint32_t n_fors = cdiv((uint64_t)n * P::k, fors_tpw);
-            const uint32_t grid = n_ht + n_fors < resident ? n_ht + n_fors : resident;
-            hipLaunchKernelGGL((k_sign_fused<P, FJ, S>), dim3(grid), dim3(256), 0, s, A, n_ht, n_fors);
-            return true;
-        }
-        return false;
-    }
-    static bool launch_fused(const BatchArgs& A, uint32_t n, int S, hipStream_t s) {
-        switch (S) {
-            case 1: return launch_fused<1>(A, n, s);
-            case 2: return launch_fused<2>(A, n, s);
-            case 4: return launch_fused<4>(A, n, s);
-            case 8: return launch_fused<8>(A, n, s);
-            default: return launch_fused<16>(A, n, s);
-        }
-    }
-
     template <int MODE>
     static void launch_ht(const BatchArgs& A, uint32_t trees, int S, hipStream_t s) {
-        switch (S) {
-            case 1: launch_ht<MODE, 1>(A, trees, s); break;
-            case 2: launch_ht<MODE, 2>(A, trees, s); break;
-            case 4: launch_ht<MODE, 4>(A, trees, s); break;
-            case 8: launch_ht<MODE, 8>(A, trees, s); break;
-            default: launch_ht<MODE, 16>(A, trees, s); break;
-        }
+        if (S == 1)
+            hipLaunchKernelGGL((k_ht<P, MODE, 1>), dim3(Lay::template ht_blocks<1>(trees)),
+                               dim3(256), 0, s, A);
+        else
+            hipLaunchKernelGGL((k_ht<P, MODE, 2>), dim3(Lay::template ht_blocks<2>(trees)),
+                               dim3(256), 0, s, A);
+    }
+    template <int FJ>
+    static uint32_t fors_tiles(uint32_t n) {
+        return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ));
     }
 
     template <int G>
@@ -249,34 +201,33 @@ struct SetImpl {
         A.n_req = b.n;
         const uint32_t n = b.n;
         const int S = Lay::split(pid_, kOpSign, n * P::d);
-        Lay::carve(pid_, A, (uint8_t*)b.ws, b.n, kOpSign, S);
-        constexpr uint32_t fors_tpw = 256u >> (P::a - J);
+        Lay::carve(pid_, A, (uint8_t*)b.ws, b.n, kOpSign);
         (void)hipGetLastError();  // report only errors of these launches
         prof_begin(s, set_name_);
         const uint32_t prep_grid_wgs = prep_grid<P>(A, n, b.mlen_bound);  // sets fields of A
         hipLaunchKernelGGL((k_prep<P>), dim3(prep_grid_wgs), dim3(kPrepWg), 0, s, A);
         prof_mark(s, "k_prep");
-        // one persistent launch for FORS + hypertree tiles: FORS then overlaps
-        // the hypertree instead of running before it
-        // (small batches: T_k runs on the lane that stores a request's last
-        // FORS root, inside the FORS tiles)
-        if (launch_fused(A, n, S, s)) {
+        // (up to kForsPkInline requests T_k runs on the lane that stores a
+        // request's last FORS root, inside the FORS tiles)
+        const uint32_t nwaves = chain_waves<P>(n * P::d);
+        if (nwaves <= kFuseWaves) {
+            const uint32_t nf = fors_tiles<J>(n);
+            hipLaunchKernelGGL((k_sign_fused<P, J>), dim3(nf + cdiv(nwaves, 4)), dim3(256), 0, s,
+                               A, nf, nwaves);
             prof_mark(s, "k_sign_fused");
-            if (!A.fors_count) {
-                hipLaunchKernelGGL((k_fors_pk<P>), dim3(cdiv(2ull * n, 64)), dim3(64), 0, s, A);
-                prof_mark(s, "k_fors_pk");
-            }
         } else {
-            hipLaunchKernelGGL((k_fors<P, J>), dim3(cdiv((uint64_t)n * P::k, fors_tpw)), dim3(256),
-                               0, s, A);
+            hipLaunchKernelGGL((k_fors<P, JB>), dim3(fors_tiles<JB>(n)), dim3(256), 0, s, A);
             prof_mark(s, "k_fors");
-            if (!A.fors_count) {
-                hipLaunchKernelGGL((k_fors_pk<P>), dim3(cdiv(2ull * n, 64)), dim3(64), 0, s, A);
-                prof_mark(s, "k_fors_pk");
-            }
-            launch_ht<0>(A, n * P::d, S, s);
-            prof_mark(s, "k_ht");
+            hipLaunchKernelGGL((k_chains<P, 0>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
+                               nwaves);
+            prof_mark(s, "k_chains");
         }
+        if (!A.fors_count) {
+            hipLaunchKernelGGL((k_fors_pk<P>), dim3(cdiv(2ull * n, 64)), dim3(64), 0, s, A);
+            prof_mark(s, "k_fors_pk");
+        }
+        launch_ht<0>(A, n * P::d, S, s);
+        prof_mark(s, "k_ht");
         hipLaunchKernelGGL((k_wots_gather<P>), dim3(cdiv((uint64_t)n * P::d * P::len, 256)),
                            dim3(256), 0, s, A);
         prof_mark(s, "k_wots_gather");
@@ -296,7 +247,7 @@ struct SetImpl {
         A.sig_stride = b.sig_stride;
         A.status = b.status;
         A.n_req = b.n;
-        Lay::carve(pid_, A, (uint8_t*)b.ws, b.n, kOpVerify, 1);
+        Lay::carve(pid_, A, (uint8_t*)b.ws, b.n, kOpVerify);
         const uint32_t n = b.n;
         const int G = Lay::vsplit(pid_, n);
         (void)hipGetLastError();  // report only errors of these launches
@@ -330,11 +281,14 @@ struct SetImpl {
         A.n_req = b.n;
         const uint32_t n = b.n;
         const int S = Lay::split(pid_, kOpKeygen, n);
-        Lay::carve(pid_, A, (uint8_t*)b.ws, b.n, kOpKeygen, S);
+        Lay::carve(pid_, A, (uint8_t*)b.ws, b.n, kOpKeygen);
         (void)hipGetLastError();  // report only errors of these launches
         prof_begin(s, set_name_);
         hipLaunchKernelGGL((k_kprep<P>), dim3(cdiv(n, 64)), dim3(64), 0, s, A);
         prof_mark(s, "k_kprep");
+        const uint32_t nwaves = chain_waves<P>(n);
+        hipLaunchKernelGGL((k_chains<P, 1>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A, nwaves);
+        prof_mark(s, "k_chains_keygen");
         launch_ht<1>(A, n, S, s);
         prof_mark(s, "k_ht_keygen");
         return hipGetLastError() == hipSuccess ? 0 : kErrHip;

@@ -110,6 +110,228 @@ __device__ __forceinline__ void sha256_rounds(uint32_t v[8], uint32_t w[16]) {
     v[7] = h;
 }
 
+// ------------------------------------------------------ two-phase rounds
+//
+// A SIMD issues two VALU instructions at a time, from two waves, if the
+// first one picked is any instruction and the second is a simple one (xor,
+// add, shift, v_bitop3): rotates (v_alignbit) and v_add3 only go in the first
+// place.  Picked in age order the simple ones mostly take both places or the
+// first, and a mix of the two kinds issues every 4.1-4.2 cycles whatever its
+// order.  With s_setprio 3 before a run of rotates and s_setprio 0 after it
+// a wave in its rotates is picked first and the other waves' simple
+// instructions ride along: 8 rotates + 8 v_bitop3 in turn issue every 2.86 /
+// 2.45 / 2.27 cycles at 2 / 4 / 8 waves per SIMD (one wave: 4.7, as before).
+// A round is therefore one asm block in two phases: first the rotates of
+// this round and of the schedule with two v_add3 (h + K + W[t] and the
+// schedule word), then Sigma / Ch / Maj / sigma and two-operand adds (26
+// instructions, 12 : 14; all v_add3 would be 24 but 14 : 10, and the
+// rotate-class place would be the bound).  The F step of a chain, G/s at
+// 1 / 2 / 4 / 8 waves per SIMD: n = 16 25.3 / 28.1 / 31.0 / 32.6 -> 23.3 /
+// 38.2 / 39.7 / 46.1, n = 32 27.9 / 30.1 / 31.1 / 31.6 -> 21.8 / 35.2 / 37.8
+// / 43.5; where one wave runs alone on its SIMD sha256_compress stays ahead.
+
+#define SPX_R_ROT                                                                        \
+    "v_alignbit_b32 %[r1], %[e], %[e], 6\n\tv_alignbit_b32 %[r2], %[e], %[e], 11\n\t"    \
+    "v_alignbit_b32 %[r3], %[e], %[e], 25\n\tv_alignbit_b32 %[q1], %[a], %[a], 2\n\t"    \
+    "v_alignbit_b32 %[q2], %[a], %[a], 13\n\tv_alignbit_b32 %[q3], %[a], %[a], 22\n\t"
+#define SPX_R_KW "v_add3_u32 %[h], %[h], %[K], %[wt]\n\t"
+#define SPX_R_KL "v_add_u32 %[h], %[K], %[h]\n\t"
+#define SPX_R_X "v_alignbit_b32 %[x1], %[wx], %[wx], 7\n\tv_alignbit_b32 %[x2], %[wx], %[wx], 18\n\t"
+#define SPX_R_Y "v_alignbit_b32 %[y1], %[wy], %[wy], 17\n\tv_alignbit_b32 %[y2], %[wy], %[wy], 19\n\t"
+#define SPX_R_SUM "v_add3_u32 %[wn], %[wn], %[p1], %[ss]\n\t"
+#define SPX_R_BIT                                                                        \
+    "v_bitop3_b32 %[r1], %[r1], %[r2], %[r3] bitop3:0x96\n\t"                            \
+    "v_bitop3_b32 %[r2], %[e], %[f], %[g] bitop3:0xca\n\t"                               \
+    "v_bitop3_b32 %[q1], %[q1], %[q2], %[q3] bitop3:0x96\n\t"                            \
+    "v_bitop3_b32 %[q2], %[a], %[b], %[c] bitop3:0xe8\n\t"
+#define SPX_R_X3 "v_lshrrev_b32 %[r3], 3, %[wx]\n\t"
+#define SPX_R_Y3 "v_lshrrev_b32 %[q3], 10, %[wy]\n\t"
+#define SPX_R_A1 "v_add_u32 %[r1], %[r1], %[r2]\n\tv_add_u32 %[q1], %[q1], %[q2]\n\t"
+#define SPX_R_XX "v_bitop3_b32 %[x1], %[x1], %[x2], %[r3] bitop3:0x96\n\t"
+#define SPX_R_A2 "v_add_u32 %[h], %[h], %[r1]\n\t"
+#define SPX_R_YY "v_bitop3_b32 %[y1], %[y1], %[y2], %[q3] bitop3:0x96\n\t"
+#define SPX_R_A3 "v_add_u32 %[d], %[d], %[h]\n\t"
+#define SPX_R_SS "v_add_u32 %[ss], %[x1], %[y1]\n\t"
+#define SPX_R_A4 "v_add_u32 %[h], %[h], %[q1]\n\t"
+#define SPX_O_ST                                                                         \
+    [d] "+&v"(d), [h] "+&v"(h), [r1] "=&v"(r1), [r2] "=&v"(r2), [r3] "=&v"(r3),          \
+        [q1] "=&v"(q1), [q2] "=&v"(q2), [q3] "=&v"(q3)
+#define SPX_O_X [x1] "=&v"(x1), [x2] "=&v"(x2)
+#define SPX_O_Y [y1] "=&v"(y1), [y2] "=&v"(y2)
+#define SPX_I_ST [a] "v"(a), [b] "v"(b), [c] "v"(c), [e] "v"(e), [f] "v"(f), [g] "v"(g)
+
+// One round.  X / Y: it also makes ss, the sigma0(wx) / sigma1(wy) part of
+// the next schedule word; SUM (with X and Y, or neither): wn += p1 + the old
+// ss, the schedule word of this round; WV: W[t] varies (else K + W[t] is a
+// literal, and SUM is not taken).
+template <bool X, bool Y, bool SUM, bool WV>
+__device__ __forceinline__ void sha256_round_ph(uint32_t a, uint32_t b, uint32_t c, uint32_t& d,
+                                                uint32_t e, uint32_t f, uint32_t g, uint32_t& h,
+                                                const uint32_t K, uint32_t wt, uint32_t wx,
+                                                uint32_t wy, uint32_t p1, uint32_t& ss,
+                                                uint32_t& wn) {
+    static_assert(!SUM || (WV && X == Y), "no such round");
+    uint32_t r1, r2, r3, q1, q2, q3, x1, x2, y1, y2;
+    if constexpr (!WV) {
+        const uint32_t kw = K + wt;
+        if constexpr (X && Y)
+            asm volatile(SPX_HI SPX_R_ROT SPX_R_X SPX_R_Y SPX_LO SPX_R_KL SPX_R_BIT SPX_R_X3
+                             SPX_R_Y3 SPX_R_A1 SPX_R_XX SPX_R_A2 SPX_R_YY SPX_R_A3 SPX_R_SS SPX_R_A4
+                         : SPX_O_ST, [ss] "=&v"(ss), SPX_O_X, SPX_O_Y
+                         : SPX_I_ST, [wx] "v"(wx), [wy] "v"(wy), [K] "i"((int)kw));
+        else if constexpr (X)
+            asm volatile(SPX_HI SPX_R_ROT SPX_R_X SPX_LO SPX_R_KL SPX_R_BIT SPX_R_X3 SPX_R_A1
+                             SPX_R_XX SPX_R_A2 SPX_R_A3 SPX_R_A4
+                         : SPX_O_ST, SPX_O_X
+                         : SPX_I_ST, [wx] "v"(wx), [K] "i"((int)kw));
+        else if constexpr (Y)
+            asm volatile(SPX_HI SPX_R_ROT SPX_R_Y SPX_LO SPX_R_KL SPX_R_BIT SPX_R_Y3 SPX_R_A1
+                             SPX_R_A2 SPX_R_YY SPX_R_A3 SPX_R_A4
+                         : SPX_O_ST, SPX_O_Y
+                         : SPX_I_ST, [wy] "v"(wy), [K] "i"((int)kw));
+        else
+            asm volatile(SPX_HI SPX_R_ROT SPX_LO SPX_R_KL SPX_R_BIT SPX_R_A1 SPX_R_A2 SPX_R_A3
+                             SPX_R_A4
+                         : SPX_O_ST
+                         : SPX_I_ST, [K] "i"((int)kw));
+    } else if constexpr (X && Y && SUM) {
+        asm volatile(SPX_HI SPX_R_ROT SPX_R_KW SPX_R_X SPX_R_Y SPX_R_SUM SPX_LO SPX_R_BIT SPX_R_X3
+                         SPX_R_Y3 SPX_R_A1 SPX_R_XX SPX_R_A2 SPX_R_YY SPX_R_A3 SPX_R_SS SPX_R_A4
+                     : SPX_O_ST, [ss] "+&v"(ss), [wn] "+&v"(wn), SPX_O_X, SPX_O_Y
+                     : SPX_I_ST, [wt] "v"(wt), [wx] "v"(wx), [wy] "v"(wy), [p1] "v"(p1),
+                       [K] "s"(K));
+    } else if constexpr (X && Y) {
+        asm volatile(SPX_HI SPX_R_ROT SPX_R_KW SPX_R_X SPX_R_Y SPX_LO SPX_R_BIT SPX_R_X3 SPX_R_Y3
+                         SPX_R_A1 SPX_R_XX SPX_R_A2 SPX_R_YY SPX_R_A3 SPX_R_SS SPX_R_A4
+                     : SPX_O_ST, [ss] "=&v"(ss), SPX_O_X, SPX_O_Y
+                     : SPX_I_ST, [wt] "v"(wt), [wx] "v"(wx), [wy] "v"(wy), [K] "s"(K));
+    } else if constexpr (X) {
+        asm volatile(SPX_HI SPX_R_ROT SPX_R_KW SPX_R_X SPX_LO SPX_R_BIT SPX_R_X3 SPX_R_A1 SPX_R_XX
+                         SPX_R_A2 SPX_R_A3 SPX_R_A4
+                     : SPX_O_ST, SPX_O_X
+                     : SPX_I_ST, [wt] "v"(wt), [wx] "v"(wx), [K] "s"(K));
+    } else if constexpr (Y) {
+        asm volatile(SPX_HI SPX_R_ROT SPX_R_KW SPX_R_Y SPX_LO SPX_R_BIT SPX_R_Y3 SPX_R_A1 SPX_R_A2
+                         SPX_R_YY SPX_R_A3 SPX_R_A4
+                     : SPX_O_ST, SPX_O_Y
+                     : SPX_I_ST, [wt] "v"(wt), [wy] "v"(wy), [K] "s"(K));
+    } else if constexpr (SUM) {
+        asm volatile(SPX_HI SPX_R_ROT SPX_R_KW SPX_R_SUM SPX_LO SPX_R_BIT SPX_R_A1 SPX_R_A2
+                         SPX_R_A3 SPX_R_A4
+                     : SPX_O_ST, [wn] "+&v"(wn)
+                     : SPX_I_ST, [wt] "v"(wt), [p1] "v"(p1), [ss] "v"(ss), [K] "s"(K));
+    } else {
+        asm volatile(SPX_HI SPX_R_ROT SPX_R_KW SPX_LO SPX_R_BIT SPX_R_A1 SPX_R_A2 SPX_R_A3 SPX_R_A4
+                     : SPX_O_ST
+                     : SPX_I_ST, [wt] "v"(wt), [K] "s"(K));
+    }
+    if constexpr (X && !Y) ss = x1;
+    if constexpr (Y && !X) ss = y1;
+}
+
+__device__ __forceinline__ uint32_t sha256_s0(uint32_t x) {
+    return xor3(rotr32(x, 7), rotr32(x, 18), x >> 3);
+}
+__device__ __forceinline__ uint32_t sha256_s1(uint32_t y) {
+    return xor3(rotr32(y, 17), rotr32(y, 19), y >> 10);
+}
+
+// What is known about the schedule words of a block: 0 a compile-time
+// constant, 1 fixed along a chain (held in registers), 2 varies.
+enum : int { kWordConst = 0, kWordChain = 1, kWordVar = 2 };
+struct Sha2Kinds {
+    int k[64];
+    // words with a bit in `known` are constants, those in `chain` fixed
+    constexpr Sha2Kinds(uint32_t known, uint32_t chain) : k{} {
+        for (int t = 0; t < 64; t++) {
+            if (t < 16) {
+                k[t] = (known >> t) & 1 ? kWordConst : (chain >> t) & 1 ? kWordChain : kWordVar;
+            } else {
+                const int q[4] = {t - 2, t - 7, t - 15, t - 16};
+                int m = 0;
+                for (int i = 0; i < 4; i++) m = k[q[i]] > m ? k[q[i]] : m;
+                // a word of constants only is treated as a register value
+                k[t] = m == kWordConst ? kWordVar : m;
+            }
+        }
+    }
+    // the parts of W[u] that do not vary include a chain word / any word
+    constexpr bool has_chain(int u) const {
+        return k[u - 2] == kWordChain || k[u - 7] == kWordChain || k[u - 15] == kWordChain ||
+               k[u - 16] == kWordChain;
+    }
+    constexpr bool all_var(int u) const {
+        return k[u - 2] == kWordVar && k[u - 7] == kWordVar && k[u - 15] == kWordVar &&
+               k[u - 16] == kWordVar;
+    }
+};
+
+// Rounds T..63 on the working variables v (before round T0 = the first one
+// run: a..h in v[0..7]); schedule word U = T + LA is made in round T (LA =
+// 16 - T0, so that round T0 makes W[16]).  w is the ring W[t & 15]; fix[u -
+// 16]: the sum of W[u]'s parts that do not vary, where one is a chain word.
+template <uint32_t KNOWN, uint32_t CHAIN, int T0, int T>
+__device__ __forceinline__ void sha256_rounds_ph(uint32_t v[8], uint32_t w[16],
+                                                 const uint32_t* fix, uint32_t& ss) {
+    if constexpr (T < 64) {
+        constexpr Sha2Kinds kd(KNOWN, CHAIN);
+        constexpr int LA = 16 - T0, U = T + LA, R = 64 + T0 - T;
+        uint32_t &d = v[(R + 3) & 7], &h = v[(R + 7) & 7];
+        const uint32_t a = v[R & 7], b = v[(R + 1) & 7], c = v[(R + 2) & 7], e = v[(R + 4) & 7],
+                       f = v[(R + 5) & 7], g = v[(R + 6) & 7];
+        const uint32_t wt = w[T & 15];
+        constexpr bool wv = kd.k[T] != kWordConst;
+        uint32_t none = 0;
+        if constexpr (U < 64) {
+            constexpr bool x = U + 1 < 64 && kd.k[U - 14] == kWordVar;
+            constexpr bool y = U + 1 < 64 && kd.k[U - 1] == kWordVar;
+            if constexpr (kd.all_var(U) && wv && x == y) {
+                sha256_round_ph<x, y, true, wv>(a, b, c, d, e, f, g, h, kSha256K[T], wt,
+                                                w[(U - 14) & 15], w[(U - 1) & 15], w[(U - 7) & 15],
+                                                ss, w[U & 15]);
+            } else {
+                constexpr bool v0 = kd.k[U - 16] == kWordVar, v7 = kd.k[U - 7] == kWordVar,
+                               g0 = kd.k[U - 15] == kWordVar, g1 = kd.k[U - 2] == kWordVar;
+                uint32_t wn = 0;
+                if constexpr (kd.has_chain(U)) {
+                    wn = fix[U - 16];
+                } else {
+                    if constexpr (!v0) wn += w[U & 15];
+                    if constexpr (!v7) wn += w[(U - 7) & 15];
+                    if constexpr (!g0) wn += sha256_s0(w[(U - 15) & 15]);
+                    if constexpr (!g1) wn += sha256_s1(w[(U - 2) & 15]);
+                }
+                if constexpr (v0) wn += w[U & 15];
+                if constexpr (v7) wn += w[(U - 7) & 15];
+                if constexpr (g0 || g1) wn += ss;
+                sha256_round_ph<x, y, false, wv>(a, b, c, d, e, f, g, h, kSha256K[T], wt,
+                                                 w[(U - 14) & 15], w[(U - 1) & 15], 0u, ss, none);
+                w[U & 15] = wn;
+            }
+        } else {
+            sha256_round_ph<false, false, false, wv>(a, b, c, d, e, f, g, h, kSha256K[T], wt, 0u, 0u,
+                                                     0u, ss, none);
+        }
+        sha256_rounds_ph<KNOWN, CHAIN, T0, T + 1>(v, w, fix, ss);
+    }
+}
+
+// One compression in two-phase rounds; bit t of KNOWN: W[t] is a
+// compile-time constant at the call
+template <uint32_t KNOWN>
+__device__ __forceinline__ void sha256_compress_ph(uint32_t st[8], uint32_t w[16]) {
+    constexpr Sha2Kinds kd(KNOWN, 0);
+    uint32_t v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = st[i];
+    uint32_t ss = 0;  // the varying sigma parts of W[16]
+    if constexpr (kd.k[1] == kWordVar) ss += sha256_s0(w[1]);
+    if constexpr (kd.k[14] == kWordVar) ss += sha256_s1(w[14]);
+    sha256_rounds_ph<KNOWN, 0, 0, 0>(v, w, nullptr, ss);
+#pragma unroll
+    for (int i = 0; i < 8; i++) st[i] += v[i];
+}
+
 // ------------------------------------------------------------ lane pairs
 //
 // One compression on a lane pair (lanes 2i and 2i+1 of a wave, both active,
@@ -321,6 +543,16 @@ __device__ __forceinline__ void put16(uint32_t b[16], int q, uint32_t x) {
     for (int i = 0; i < 16; i++) b[i] = (q == i) ? x : b[i];
 }
 
+// words of block blk of T over M payload words that are known: the zeros
+// after the 0x80 byte and the length
+template <int M>
+constexpr uint32_t sha2_known_words(int blk) {
+    uint32_t m = 0;
+    for (int i = 0; i < 16; i++)
+        if (16 * blk + i > 5 + M) m |= 1u << i;
+    return m;
+}
+
 template <int N>
 struct Sha2 {
     static constexpr int hash = kSha2;
@@ -362,15 +594,17 @@ struct Sha2 {
     __device__ static __forceinline__ void thash_words(const Key& k, const Adr& a,
                                                        const uint32_t d[M], uint32_t out[NW]) {
         constexpr int B = (6 + M + 2 + 15) / 16;
-        uint32_t st[8];
+        static_assert(B <= 2, "F and H");
+        uint32_t st[8], w[16];
 #pragma unroll
         for (int i = 0; i < 8; i++) st[i] = k.mid[i];
 #pragma unroll
-        for (int blk = 0; blk < B; blk++) {
-            uint32_t w[16];
+        for (int i = 0; i < 16; i++) w[i] = block_word<M>(a, d, 0, i);
+        sha256_compress_ph<sha2_known_words<M>(0)>(st, w);
+        if constexpr (B == 2) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) w[i] = block_word<M>(a, d, blk, i);
-            sha256_compress(st, w);
+            for (int i = 0; i < 16; i++) w[i] = block_word<M>(a, d, 1, i);
+            sha256_compress_ph<sha2_known_words<M>(1)>(st, w);
         }
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = st[i];
@@ -408,6 +642,56 @@ struct Sha2 {
         for (int i = 0; i < NW; i++) out[i] = k.mid[i] + v[i];
     }
 
+    // F along one chain in two-phase rounds.  The address words W[0..4] are
+    // fixed along the chain, so are rounds 0-4 and, of the schedule words,
+    // W[17] and W[19] (n = 16) and parts of W[16..21], W[24], W[26] and
+    // W[32..35]: all made once per chain (chain_begin).
+    static constexpr uint32_t kFKnown = sha2_known_words<NW>(0);
+    static constexpr int kFix = 20;  // W[16 .. 35]
+    struct Chain {
+        uint32_t st[8];      // working variables after round 4
+        uint32_t fix[kFix];  // parts of W[16 + i] fixed along the chain
+    };
+    __device__ static __forceinline__ void chain_begin(const Key& k, const Adr& a, Chain& c) {
+        constexpr Sha2Kinds kd(kFKnown, 0x1Fu);
+        uint32_t w[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            w[i] = i < 5 ? a.w[i] : i == 15 ? (uint32_t)(64 + 22 + N) * 8u : 0u;
+        uint32_t x[16 + kFix];
+#pragma unroll
+        for (int i = 0; i < 16; i++) x[i] = w[i];
+#pragma unroll
+        for (int t = 16; t < 16 + kFix; t++) {
+            uint32_t f = 0;
+            if (kd.k[t - 2] != kWordVar) f += sha256_s1(x[t - 2]);
+            if (kd.k[t - 7] != kWordVar) f += x[t - 7];
+            if (kd.k[t - 15] != kWordVar) f += sha256_s0(x[t - 15]);
+            if (kd.k[t - 16] != kWordVar) f += x[t - 16];
+            c.fix[t - 16] = f;
+            x[t] = f;  // the word itself where no part varies
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) c.st[i] = k.mid[i];
+        sha256_rounds<0, 5>(c.st, w);
+    }
+    // one step at hash address s; in and out may be the same array
+    __device__ static __forceinline__ void chain_step(const Key& k, const Chain& c, uint32_t s,
+                                                      const uint32_t in[NW], uint32_t out[NW]) {
+        static_assert((6 + NW + 2 + 15) / 16 == 1, "F is one block");
+        Adr a{};
+        adr_hash(a, s);
+        uint32_t w[16], v[8];
+#pragma unroll
+        for (int i = 0; i < 16; i++) w[i] = block_word<NW>(a, in, 0, i);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = c.st[i];
+        uint32_t ss = 0;
+        sha256_rounds_ph<kFKnown, 0x1Fu, 5, 5>(v, w, c.fix, ss);
+#pragma unroll
+        for (int i = 0; i < NW; i++) out[i] = k.mid[i] + v[(i + 5) & 7];
+    }
+
     // H: two input values (Merkle node)
     __device__ static __forceinline__ void H(const Key& k, const Adr& a, const uint32_t l[NW],
                                              const uint32_t r[NW], uint32_t out[NW]) {
@@ -435,59 +719,10 @@ struct Sha2 {
         }
 #pragma unroll
         for (int i = 0; i < 8; i++) st[i] = kSha256IV[i];
-        sha256_compress(st, w);
+        sha256_compress_ph<sha2_known_words<NW>(0)>(st, w);  // sk_seed in the place of a value
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = st[i];
     }
-
-    // Streaming T_l: items of NW words appended one word at a time with a
-    // wave-uniform position; used for T_len (leaf) and T_k (FORS pk).
-    struct Stream {
-        uint32_t st[8];
-        uint32_t b[16];
-        int q;
-        uint32_t carry;
-
-        __device__ __forceinline__ void begin(const Key& k, const Adr& a) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) st[i] = k.mid[i];
-#pragma unroll
-            for (int i = 0; i < 16; i++) b[i] = i < 5 ? a.w[i] : 0u;
-            q = 5;
-            carry = a.w[5] >> 16;
-        }
-        // append one payload word (must be called from a single site in a loop)
-        __device__ __forceinline__ void word(uint32_t dw) {
-            put16(b, q, __builtin_amdgcn_alignbit(carry, dw, 16));
-            carry = dw;
-            q++;
-            if (q == 16) {
-                sha256_compress(st, b);
-                q = 0;
-            }
-        }
-        // D = total payload words appended; finishes with compile-time layout
-        template <int D>
-        __device__ __forceinline__ void finish(uint32_t out[NW]) {
-            constexpr int qe = (5 + D) % 16;
-            constexpr uint32_t bits = (64u + 22u + 4u * D) * 8u;
-            b[qe] = (carry << 16) | 0x8000u;
-#pragma unroll
-            for (int i = qe + 1; i < 16; i++) b[i] = 0;
-            if (qe <= 13) {
-                b[15] = bits;
-                sha256_compress(st, b);
-            } else {
-                sha256_compress(st, b);
-#pragma unroll
-                for (int i = 0; i < 15; i++) b[i] = 0;
-                b[15] = bits;
-                sha256_compress(st, b);
-            }
-#pragma unroll
-            for (int i = 0; i < NW; i++) out[i] = st[i];
-        }
-    };
 
     // ------------------------------------------------ per-request hashing
 

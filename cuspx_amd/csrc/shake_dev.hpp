@@ -113,12 +113,121 @@ __device__ __forceinline__ void keccak_round(uint32_t s[50], uint32_t rc_lo, uin
     s[1] ^= rc_hi;
 }
 
-// Keccak-f[1600]: round 0 unrolled (so constant state words fold after an
-// absorb), rounds 1..23 in a loop with the constants from constant memory.
+// ------------------------------------------------------- two-phase rounds
+//
+// Rotates (v_alignbit) and simple instructions of different waves issue
+// together when a wave in its rotates is picked first (sha2_dev.hpp says
+// how): theta's rotates by one and rho are asm blocks between s_setprio 3 and
+// s_setprio 0, the xors and chi run at priority 0 beside other waves'
+// rotates.  The empty asm blocks keep theta's xors before rho's run.  The F
+// step of a chain, G permutations/s at 1 / 2 / 4 / 5 waves per SIMD:
+// interleaved 7.4 / 9.0 / 10.4 / 10.5 -> 8.4 / 13.1 / 14.4 / 14.6.
+
+#define SPX_AL(d, h, l, n) "v_alignbit_b32 %" #d ", %" #h ", %" #l ", %" #n "\n\t"
+#define SPX_AL1(d, h, l) "v_alignbit_b32 %" #d ", %" #h ", %" #l ", 31\n\t"
+#define SPX_PIN10(v, i)                                                                  \
+    asm volatile(""                                                                      \
+                 : "+v"(v[i]), "+v"(v[i + 1]), "+v"(v[i + 2]), "+v"(v[i + 3]),           \
+                   "+v"(v[i + 4]), "+v"(v[i + 5]), "+v"(v[i + 6]), "+v"(v[i + 7]),       \
+                   "+v"(v[i + 8]), "+v"(v[i + 9]))
+
+// theta's column parities
+__device__ __forceinline__ void keccak_parity(const uint32_t s[50], uint32_t C[10]) {
+#pragma unroll
+    for (int i = 0; i < 10; i++)
+        C[i] = xor3(xor3(s[i], s[i + 10], s[i + 20]), s[i + 30], s[i + 40]);
+}
+// chi and iota on the rotated lanes B
+__device__ __forceinline__ void keccak_chi(uint32_t s[50], const uint32_t B[50], uint32_t rc0,
+                                           uint32_t rc1) {
+#pragma unroll
+    for (int y = 0; y < 5; y++)
+#pragma unroll
+        for (int x = 0; x < 5; x++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                s[2 * (x + 5 * y) + h] = bit_chi(B[2 * (x + 5 * y) + h],
+                                                 B[2 * ((x + 1) % 5 + 5 * y) + h],
+                                                 B[2 * ((x + 2) % 5 + 5 * y) + h]);
+    s[0] ^= rc0;
+    s[1] ^= rc1;
+}
+
+// v_alignbit count and half order of rho's rotate of lane l: out = (lo, hi)
+// by alignbit(hi, lo, n) and alignbit(lo, hi, n), swapped for rotates over 32
+constexpr int keccak_rho_count(int l) { return (64 - kRho[l]) & 31; }
+constexpr bool keccak_rho_swap(int l) { return kRho[l] > 32; }
+
+// one round on s[50] (low, high words)
+__device__ __forceinline__ void keccak_round_ph(uint32_t s[50], uint32_t rc_lo, uint32_t rc_hi) {
+    uint32_t C[10], R[10];  // R = C rotated by one
+    keccak_parity(s, C);
+    asm volatile(SPX_HI SPX_AL1(0, 10, 11) SPX_AL1(1, 11, 10) SPX_AL1(2, 12, 13)
+                     SPX_AL1(3, 13, 12) SPX_AL1(4, 14, 15) SPX_AL1(5, 15, 14)
+                         SPX_AL1(6, 16, 17) SPX_AL1(7, 17, 16) SPX_AL1(8, 18, 19)
+                             SPX_AL1(9, 19, 18) SPX_LO
+                 : "=&v"(R[0]), "=&v"(R[1]), "=&v"(R[2]), "=&v"(R[3]), "=&v"(R[4]), "=&v"(R[5]),
+                   "=&v"(R[6]), "=&v"(R[7]), "=&v"(R[8]), "=&v"(R[9])
+                 : "v"(C[0]), "v"(C[1]), "v"(C[2]), "v"(C[3]), "v"(C[4]), "v"(C[5]), "v"(C[6]),
+                   "v"(C[7]), "v"(C[8]), "v"(C[9]));
+#pragma unroll
+    for (int i = 0; i < 50; i++) {
+        const int x = (i % 10) / 2, h = i & 1;
+        s[i] = xor3(s[i], C[2 * ((x + 4) % 5) + h], R[2 * ((x + 1) % 5) + h]);
+    }
+    SPX_PIN10(s, 0);
+    SPX_PIN10(s, 10);
+    SPX_PIN10(s, 20);
+    SPX_PIN10(s, 30);
+    SPX_PIN10(s, 40);
+    uint32_t B[50];
+    // rho of lanes l .. l + 3 into q, then pi
+#define SPX_RHO4(pre, post, l)                                                           \
+    do {                                                                                 \
+        uint32_t q[8];                                                                   \
+        asm volatile(pre SPX_AL(0, 9, 8, 16) SPX_AL(1, 8, 9, 16) SPX_AL(2, 11, 10, 17)   \
+                         SPX_AL(3, 10, 11, 17) SPX_AL(4, 13, 12, 18) SPX_AL(5, 12, 13, 18) \
+                             SPX_AL(6, 15, 14, 19) SPX_AL(7, 14, 15, 19) post            \
+                     : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3]), "=&v"(q[4]),  \
+                       "=&v"(q[5]), "=&v"(q[6]), "=&v"(q[7])                             \
+                     : "v"(s[2 * (l)]), "v"(s[2 * (l) + 1]), "v"(s[2 * (l) + 2]),        \
+                       "v"(s[2 * (l) + 3]), "v"(s[2 * (l) + 4]), "v"(s[2 * (l) + 5]),    \
+                       "v"(s[2 * (l) + 6]), "v"(s[2 * (l) + 7]),                         \
+                       "i"(keccak_rho_count(l)), "i"(keccak_rho_count((l) + 1)),         \
+                       "i"(keccak_rho_count((l) + 2)), "i"(keccak_rho_count((l) + 3)));  \
+        _Pragma("unroll") for (int i = 0; i < 4; i++) {                                  \
+            const int src = (l) + i, x = src % 5, y = src / 5;                           \
+            const int dst = y + 5 * ((2 * x + 3 * y) % 5);                               \
+            const int w = keccak_rho_swap(src) ? 0 : 1;                                  \
+            B[2 * dst] = q[2 * i + w];                                                   \
+            B[2 * dst + 1] = q[2 * i + 1 - w];                                           \
+        }                                                                                \
+    } while (0)
+    B[0] = s[0];
+    B[1] = s[1];
+    SPX_RHO4(SPX_HI, "", 1);
+    SPX_RHO4("", "", 5);
+    SPX_RHO4("", "", 9);
+    SPX_RHO4("", "", 13);
+    SPX_RHO4("", "", 17);
+    SPX_RHO4("", SPX_LO, 21);
+#undef SPX_RHO4
+    keccak_chi(s, B, rc_lo, rc_hi);
+}
+
+// Keccak-f[1600].  HEAD: only the first words of the result are used, so the
+// last round is left to the compiler, which drops what those do not need
+// (about 50 of its 180 instructions stay for a 16-byte output)
+template <bool HEAD>
 __device__ __forceinline__ void keccak_f(uint32_t s[50]) {
-    keccak_round(s, 0x00000001u, 0x00000000u);
+    keccak_round_ph(s, 0x00000001u, 0x00000000u);
 #pragma unroll 1
-    for (int r = 1; r < 24; r++) keccak_round(s, kKeccakRC[2 * r], kKeccakRC[2 * r + 1]);
+    for (int r = 1; r < 23; r += 2) {
+        keccak_round_ph(s, kKeccakRC[2 * r], kKeccakRC[2 * r + 1]);
+        keccak_round_ph(s, kKeccakRC[2 * r + 2], kKeccakRC[2 * r + 3]);
+    }
+    if constexpr (HEAD) keccak_round(s, 0x80008008u, 0x80000000u);
+    else keccak_round_ph(s, 0x80008008u, 0x80000000u);
 }
 
 // ---------------------------------------------------- bit-interleaved form
@@ -265,12 +374,86 @@ __device__ __forceinline__ void keccak_round_il(uint32_t s[50], uint32_t rc_e, u
     s[1] ^= rc_o;
 }
 
-// Keccak-f[1600] on the interleaved state; round 0 unrolled as in keccak_f
+// the same round in two phases (keccak_round_ph): 52 rotates, all in place.
+// Word j (half j & 1 of lane j / 2) is rotated left by keccak_il_rot(j); odd
+// rotations swap the halves, which pi's renaming does.
+constexpr int keccak_il_rot(int j) {
+    const int r = kRho[j >> 1];
+    return (r & 1) == 0 ? r / 2 : (j & 1) ? (r + 1) / 2 : (r - 1) / 2;
+}
+constexpr int keccak_il_count(int j) { return (32 - keccak_il_rot(j)) & 31; }
+static_assert(keccak_il_rot(0) == 0 && keccak_il_rot(1) == 0 && keccak_il_rot(2) == 0,
+              "words 3..49 rotate");
+
+__device__ __forceinline__ void keccak_round_il_ph(uint32_t s[50], uint32_t rc_e, uint32_t rc_o) {
+    uint32_t C[10], R[5];  // R[x] = odd half of column x rotated by one
+    keccak_parity(s, C);
+    asm volatile(SPX_HI SPX_AL1(0, 5, 5) SPX_AL1(1, 6, 6) SPX_AL1(2, 7, 7)
+                     SPX_AL1(3, 8, 8) SPX_AL1(4, 9, 9) SPX_LO
+                 : "=&v"(R[0]), "=&v"(R[1]), "=&v"(R[2]), "=&v"(R[3]), "=&v"(R[4])
+                 : "v"(C[1]), "v"(C[3]), "v"(C[5]), "v"(C[7]), "v"(C[9]));
+#pragma unroll
+    for (int l = 0; l < 25; l++) {
+        const int x = l % 5, xp = (x + 1) % 5, xm = (x + 4) % 5;
+        s[2 * l] = xor3(s[2 * l], C[2 * xm], R[xp]);
+        s[2 * l + 1] = xor3(s[2 * l + 1], C[2 * xm + 1], C[2 * xp]);
+    }
+    SPX_PIN10(s, 0);
+    SPX_PIN10(s, 10);
+    SPX_PIN10(s, 20);
+    SPX_PIN10(s, 30);
+    SPX_PIN10(s, 40);
+#define SPX_SV(i) "+v"(s[i])
+#define SPX_SN(i) "i"(keccak_il_count(i))
+#define SPX_RHO10(pre, i)                                                                \
+    asm volatile(pre SPX_AL(0, 0, 0, 10) SPX_AL(1, 1, 1, 11) SPX_AL(2, 2, 2, 12)         \
+                     SPX_AL(3, 3, 3, 13) SPX_AL(4, 4, 4, 14) SPX_AL(5, 5, 5, 15)         \
+                         SPX_AL(6, 6, 6, 16) SPX_AL(7, 7, 7, 17) SPX_AL(8, 8, 8, 18)     \
+                             SPX_AL(9, 9, 9, 19)                                         \
+                 : SPX_SV(i), SPX_SV(i + 1), SPX_SV(i + 2), SPX_SV(i + 3), SPX_SV(i + 4), \
+                   SPX_SV(i + 5), SPX_SV(i + 6), SPX_SV(i + 7), SPX_SV(i + 8), SPX_SV(i + 9) \
+                 : SPX_SN(i), SPX_SN(i + 1), SPX_SN(i + 2), SPX_SN(i + 3), SPX_SN(i + 4), \
+                   SPX_SN(i + 5), SPX_SN(i + 6), SPX_SN(i + 7), SPX_SN(i + 8), SPX_SN(i + 9))
+    SPX_RHO10(SPX_HI, 3);
+    SPX_RHO10("", 13);
+    SPX_RHO10("", 23);
+    SPX_RHO10("", 33);
+    asm volatile(SPX_AL(0, 0, 0, 7) SPX_AL(1, 1, 1, 8) SPX_AL(2, 2, 2, 9) SPX_AL(3, 3, 3, 10)
+                     SPX_AL(4, 4, 4, 11) SPX_AL(5, 5, 5, 12) SPX_AL(6, 6, 6, 13) SPX_LO
+                 : SPX_SV(43), SPX_SV(44), SPX_SV(45), SPX_SV(46), SPX_SV(47), SPX_SV(48), SPX_SV(49)
+                 : SPX_SN(43), SPX_SN(44), SPX_SN(45), SPX_SN(46), SPX_SN(47), SPX_SN(48), SPX_SN(49));
+#undef SPX_RHO10
+#undef SPX_SV
+#undef SPX_SN
+    SPX_PIN10(s, 0);
+    SPX_PIN10(s, 10);
+    SPX_PIN10(s, 20);
+    SPX_PIN10(s, 30);
+    SPX_PIN10(s, 40);
+    uint32_t B[50];
+#pragma unroll
+    for (int l = 0; l < 25; l++) {
+        const int x = l % 5, y = l / 5, dst = y + 5 * ((2 * x + 3 * y) % 5);
+        const int w = kRho[l] & 1;
+        B[2 * dst] = s[2 * l + w];
+        B[2 * dst + 1] = s[2 * l + 1 - w];
+    }
+    keccak_chi(s, B, rc_e, rc_o);
+}
+
+// Keccak-f[1600] on the interleaved state.  HEAD: only the first words of
+// the result are used, so the last round is left to the compiler, which drops
+// the rest of it (see keccak_f); else all of it is.
+template <bool HEAD>
 __device__ __forceinline__ void keccak_f_il(uint32_t s[50]) {
-    keccak_round_il(s, 1u, 0u);  // RC[0] = 1: bit 0 is even
+    keccak_round_il_ph(s, 1u, 0u);  // RC[0] = 1: bit 0 is even
 #pragma unroll 1
-    for (int r = 1; r < 24; r++)
-        keccak_round_il(s, kKeccakRcIl.w[2 * r], kKeccakRcIl.w[2 * r + 1]);
+    for (int r = 1; r < 23; r += 2) {
+        keccak_round_il_ph(s, kKeccakRcIl.w[2 * r], kKeccakRcIl.w[2 * r + 1]);
+        keccak_round_il_ph(s, kKeccakRcIl.w[2 * r + 2], kKeccakRcIl.w[2 * r + 3]);
+    }
+    if constexpr (HEAD) keccak_round_il(s, kKeccakRcIl.w[46], kKeccakRcIl.w[47]);
+    else keccak_round_il_ph(s, kKeccakRcIl.w[46], kKeccakRcIl.w[47]);
 }
 
 // Keccak-f[1600] on a lane pair in the interleaved form: the even lane holds
@@ -371,7 +554,7 @@ struct Shake {
             if (i == 33) x ^= 0x80000000u;
             s[i] = x;
         }
-        keccak_f(s);
+        keccak_f<true>(s);
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = s[i];
     }
@@ -415,9 +598,18 @@ struct Shake {
         }
         s[2 * kHashLane] ^= ((h & 1u) << 20) | (((h >> 2) & 1u) << 21);
         s[2 * kHashLane + 1] ^= (((h >> 1) & 1u) << 20) | (((h >> 3) & 1u) << 21);
-        keccak_f_il(s);
+        keccak_f_il<true>(s);
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = s[i];
+    }
+    // the chain form shared with Sha2 (values interleaved)
+    using Chain = ChainIl;
+    __device__ static __forceinline__ void chain_begin(const Key& k, const Adr& a, Chain& c) {
+        chain_il_begin(k, a, c);
+    }
+    __device__ static __forceinline__ void chain_step(const Key&, const Chain& c, uint32_t h,
+                                                      const uint32_t in[NW], uint32_t out[NW]) {
+        F_il(c, h, in, out);
     }
     // NW plain words (NW / 2 lanes) <-> interleaved
     __device__ static __forceinline__ void to_il(const uint32_t in[NW], uint32_t out[NW]) {

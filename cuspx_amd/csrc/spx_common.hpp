@@ -101,6 +101,11 @@ __device__ __forceinline__ uint32_t lane_sel(uint32_t m, uint32_t a, uint32_t b)
     return __builtin_amdgcn_bitop3_b32(m, a, b, 0xCA);
 }
 
+// wave priority around the rotate runs of the two-phase hash rounds
+// (sha2_dev.hpp), as text for asm blocks
+#define SPX_HI "s_setprio 3\n\t"
+#define SPX_LO "s_setprio 0\n\t"
+
 // ------------------------------------------------------------- addresses
 //
 // The 32-byte address as 8 big-endian words: word i holds bytes 4i..4i+3.

@@ -7,17 +7,19 @@
 //           k_fors       L lanes per FORS tree (2^J leaves per lane), LDS reduce
 //           k_fors_pk    lane pair per request: T_k over the k roots (small
 //                        batches: run by the lane storing the last root)
-//           k_ht         lane per WOTS leaf of every hypertree layer (all d
-//                        layers at once: every layer's tree/leaf comes from
-//                        H_msg alone), LDS reduce, auth path, layer root;
-//                        the signing leaf's chain values are captured
+//           k_chains     lane per WOTS chain of every leaf of every hypertree
+//                        layer (all d layers at once: every layer's tree/leaf
+//                        comes from H_msg alone); the signing leaf's chain
+//                        values are captured.  k_sign_fused: k_fors and
+//                        k_chains in one launch
+//           k_ht         T_len per leaf, LDS reduce, auth path, layer root
 //           k_wots_gather lane per (request, layer, chain): picks the
 //                        captured chain value for the layer's message
 //   verify: k_vprep, k_vfors, k_fors_pk, k_vht (the chains of a workgroup's
 //           requests dealt over its lanes, layers in sequence); small
 //           batches: k_vspec (every chain from every start) + k_vht_spec
 //           (T_len and the climb per layer)
-//   keygen: k_kprep, k_ht in keygen mode (top layer only)
+//   keygen: k_kprep, k_chains and k_ht in keygen mode (top layer only)
 //
 // Semantics follow sign.cu:1924-1994 (sign), sign.cu:3048-3121 (verify),
 // sign.cu:154-182 (keygen), utils.cu:94-241 (compute_root / treehash),
@@ -61,11 +63,10 @@ struct BatchArgs {
     uint8_t* fors_pk;         // [N][n]
     uint8_t* roots;           // [N][d][n]
     uint8_t* cap;             // [N][d][len][16][n]
-    uint32_t* tl_buf;         // SHAKE T_len parking: [len*nw][lanes]
+    uint32_t* tl_buf;         // chain ends: [len*nw][leaves]
     uint32_t tl_lanes;
     uint32_t* ht_parts;       // split subtrees: part roots [tree][part][nw]
     uint32_t* ht_count;       // split subtrees: parts finished per tree (zeroed by the prep kernel)
-    uint32_t* tile_ctr;       // fused signing: next tile (zeroed by the prep kernel)
     uint32_t* fors_count;     // FORS roots finished per request (zeroed by the prep kernels)
     uint32_t n_req;
     // prep kernels: workgroups of the lane-pair part; messages of long_min
@@ -206,7 +207,6 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
         for (int layer = 0; layer < P::d; layer++)
             if (threadIdx.x % kPrepLanes == 0) A.ht_count[(size_t)i * P::d + layer] = 0;
     }
-    if (A.tile_ctr && i == 0 && threadIdx.x == 0) *A.tile_ctr = 0;
     if (A.fors_count && threadIdx.x % kPrepLanes == 0) A.fors_count[i] = 0;
     if (prep_is_long(A, i)) return;
     prep_sign_one<P, false>(A, i, (threadIdx.x & 1u) == 0, nullptr, false);
@@ -355,10 +355,8 @@ constexpr int fors_lds_words() {
 }
 
 // sign: FORS trees, L = 2^(a-J) lanes per tree, 2^J leaves per lane; `blk`
-// is the workgroup's tile (TPW trees), so the same body serves k_fors and the
-// fused persistent signing kernels.  smem: fors_lds_words<P>() words of LDS
-// owned by the kernel (shared with the hypertree tiles of a persistent
-// kernel, which never run at the same time in one workgroup)
+// is the workgroup's tile (TPW trees), so the same body serves the fused
+// signing kernels.  smem: fors_lds_words<P>() words of LDS owned by the kernel
 template <class P, int J>
 __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint32_t* smem) {
     using Hh = HashT<P>;
@@ -526,7 +524,7 @@ __device__ __forceinline__ void thash_sha2_rd(const uint32_t mid[8], const Adr& 
                 }
             }
         }
-        sha256_compress(st, w);
+        sha256_compress_ph<0>(st, w);
     }
 #pragma unroll
     for (int i = 0; i < NW; i++) out[i] = st[i];
@@ -702,8 +700,8 @@ __device__ __forceinline__ void thash_shake_rd(const typename Shake<P::n>::Key& 
             }
             s[33] ^= 0x80000000u;  // 0x80 at byte 135 (lane 16, bit 63: odd, so the same word)
         }
-        if constexpr (IL) keccak_f_il(s);
-        else keccak_f(s);
+        if constexpr (IL) keccak_f_il<false>(s);
+        else keccak_f<false>(s);
     }
     if constexpr (IL) Hh::from_il(s, out);
     else {
@@ -907,6 +905,24 @@ __device__ __forceinline__ uint64_t layer_tree(uint64_t tree, uint32_t layer) {
     return sh >= 64 ? 0ull : (tree >> sh);
 }
 
+// a chain value into the capture, as signature bytes for SHA-256 and
+// bit-interleaved for SHAKE256, in 16-byte (n = 24: 8-byte) stores
+template <class P>
+__device__ __forceinline__ void store_raw(uint8_t* p, const uint32_t v[P::nw]) {
+    if constexpr (P::nw % 4 == 0) {
+#pragma unroll
+        for (int k = 0; k < P::nw / 4; k++)
+            reinterpret_cast<uint4*>(p)[k] =
+                make_uint4(to_native<P::hash>(v[4 * k]), to_native<P::hash>(v[4 * k + 1]),
+                           to_native<P::hash>(v[4 * k + 2]), to_native<P::hash>(v[4 * k + 3]));
+    } else {
+#pragma unroll
+        for (int k = 0; k < P::nw / 2; k++)
+            reinterpret_cast<uint2*>(p)[k] =
+                make_uint2(to_native<P::hash>(v[2 * k]), to_native<P::hash>(v[2 * k + 1]));
+    }
+}
+
 // One Merkle node of a hypertree subtree (treehash, utils.cu:189-241): node x
 // of level l = H(left, right) under the subtree's HASHTREE address; writes the
 // node into the signature's auth path when it is the sibling of the signing
@@ -945,142 +961,167 @@ __device__ __forceinline__ void ht_node(const BatchArgs& A, uint32_t g, uint32_t
     }
 }
 
-// Hypertree leaves.  MODE 0 = sign: every (request, layer) subtree, auth
-// path into the signature, layer root into roots[], chain values of the
-// signing leaf captured.  MODE 1 = keygen: the top subtree only, root into
-// the key outputs.
+// WOTS chains of the hypertree leaves.  MODE 0 = sign: every (request, layer)
+// subtree, the chain values of the signing leaf captured.  MODE 1 = keygen:
+// the top subtree only.
 //
-// S lanes share one WOTS leaf (lane q takes chains q, q+S, ...): S = 1 gives
-// the most work per lane (throughput), larger S shortens the per-lane chain
-// of dependent compressions (latency of small batches); the launcher picks S.
-// With S > 1 (and always for SHAKE) the chain outputs are parked in tl_buf
-// ([word][leaf], coalesced) and absorbed into T_len by the lane pair q = 0, 1
-// (sha256_compress_pair / keccak_f_il_pair; SHAKE256 at S = 1: lane q = 0).
-//
-// A subtree whose 2^h' x S lanes exceed one 1024-lane workgroup (the s sets
-// at S >= 4) is split over PARTS workgroups of 256 lanes.  Each part reduces
-// its leaves to a part root in LDS; the part that finishes last (device-scope
-// counter, release/acquire fences, no waiting) climbs the remaining log2(PARTS)
-// levels from the part roots.
-template <class P, int S>
-struct HtShape {
-    static constexpr int L = 1 << P::th;              // leaves per subtree
-    static constexpr int LT = L * S;                  // lanes per subtree
-    static constexpr int PARTS = LT > 1024 ? LT / 256 : 1;
-    static constexpr int LP = L / PARTS;              // leaves per part
-    static constexpr int LOGP = P::th - ilog2(PARTS); // levels reduced inside a part
-    static constexpr int WG = PARTS > 1 ? 256 : (LT > 256 ? LT : 256);
-    static constexpr int TPW = PARTS > 1 ? 1 : WG / LT;  // subtrees per workgroup
-    static constexpr int NL = WG / S;                 // leaves per workgroup
-    static constexpr bool park = S > 1 || P::hash == kShake;
-    static constexpr int NLDS = NL > PARTS ? NL : PARTS;  // the last part climbs from PARTS roots
-    static constexpr int lds_words = 2 * NLDS * P::nw;    // two levels of nodes
-};
+// One lane per chain: wave `wave` runs chain j = wave % len of the 64 leaves
+// of block wave / len, PRF and 15 F, and parks the chain's end in tl_buf
+// ([word][leaf], coalesced; SHAKE256 values bit-interleaved).  Bound by VALU
+// issue.  A lane holds one chain and no T_len state, so SHA-256 runs 8 waves
+// per SIMD (64 VGPRs), where the two-phase rounds issue best; and a batch of
+// any size splits into len x as many equal items as it has leaves.  (Before:
+// S = 1..16 lanes per leaf, each walking len / S chains, T_len streamed in
+// registers at S = 1.)
+template <class P>
+__host__ __device__ constexpr uint32_t leaf_count(uint32_t trees) {
+    return trees << P::th;
+}
+template <class P>
+__host__ __device__ constexpr uint32_t chain_waves(uint32_t trees) {
+    return (leaf_count<P>(trees) + 63) / 64 * P::len;
+}
 
-// smem: HtShape<P, S>::lds_words words of LDS owned by the kernel
-template <class P, int MODE, int S>
-__device__ __forceinline__ void ht_tile(const BatchArgs& A, uint32_t blk, uint32_t* smem) {
+template <class P, int MODE>
+__device__ __forceinline__ void chain_wave(const BatchArgs& A, uint32_t wave) {
     using Hh = HashT<P>;
-    using Key = typename Hh::Key;
-    using Sh = HtShape<P, S>;
     constexpr int NW = P::nw;
-    constexpr int LOGL = P::th;
-    constexpr int L = Sh::L, TPW = Sh::TPW, NL = Sh::NL;
-    constexpr int PARTS = Sh::PARTS, LP = Sh::LP, LOGP = Sh::LOGP;
-    constexpr int LPT = PARTS > 1 ? LP * S : Sh::LT;  // lanes per subtree in this workgroup
-    constexpr int NLDS = Sh::NLDS;
-    auto& lds = *reinterpret_cast<uint32_t (*)[2][NLDS][NW]>(smem);
-
-    const int tid = threadIdx.x;
-    const int tau = tid / LPT;
-    const uint32_t part = PARTS > 1 ? blk % PARTS : 0;
-    const uint32_t u = part * LP + (tid % LPT) / S;  // leaf index = keypair address
-    const int q = tid % S;                            // chain phase of this lane
-    const int slot = tid / S;                         // leaf slot in the workgroup
-    const uint32_t g = (blk / PARTS) * TPW + tau;
+    constexpr int L = 1 << P::th;
     const uint32_t ntrees = MODE == 0 ? A.n_req * P::d : A.n_req;
-    const bool active = g < ntrees;
-    const uint32_t req = active ? (MODE == 0 ? g / P::d : g) : 0;
-    const uint32_t layer = MODE == 0 ? (active ? g % P::d : 0) : P::d - 1;
+    const uint32_t j = wave % P::len;
+    const uint32_t leaf_g = wave / P::len * 64 + (threadIdx.x & 63u);  // column in tl_buf
+    if (leaf_g >= leaf_count<P>(ntrees)) return;
+    const uint32_t g = leaf_g / L, u = leaf_g % L;  // subtree; leaf index = keypair address
+    const uint32_t req = MODE == 0 ? g / P::d : g;
+    const uint32_t layer = MODE == 0 ? g % P::d : P::d - 1;
     const Plan& pl = A.plan[req];
-    Key key;
+    typename Hh::Key key;
     Hh::load_key(pl, key);
     uint64_t tree = 0;
-    uint32_t target = 0;
+    uint32_t target = ~0u;
     if (MODE == 0) {
         tree = layer_tree<P>(pl.tree, layer);
         target = layer == 0 ? pl.leaf
                             : (uint32_t)((pl.tree >> ((layer - 1) * P::th)) & (L - 1));
     }
-    const bool capture = MODE == 0 && active && u == target;
-    uint8_t* cap = A.cap + ((size_t)req * P::d + layer) * P::len * 16 * P::n;
-    const uint32_t leaf_g = blk * NL + slot;  // leaf column in tl_buf
-
-    // ---- WOTS public key of leaf u (wots_gen_leaf, sign.cu:87-104)
+    const bool capture = MODE == 0 && u == target;
+    uint8_t* cap = A.cap + (((size_t)req * P::d + layer) * P::len + j) * 16 * P::n;
     Adr wa = adr_make(layer, tree, kWots);
     adr_keypair<P::th>(wa, u);
-    Adr pa = adr_make(layer, tree, kWotsPk);
-    adr_keypair<P::th>(pa, u);
-    // SHA-256 at S = 1 streams T_len in registers; otherwise the chain ends
-    // are parked in tl_buf and absorbed afterwards (by the leaf's lane pair
-    // when S > 1)
-    typename Sha2<P::n>::Stream ts;
-    if constexpr (P::hash == kSha2 && !Sh::park) ts.begin(key, pa);
-    auto parked = [&](int w) { return A.tl_buf[(size_t)w * A.tl_lanes + leaf_g]; };
-#pragma unroll 1
-    for (int j = q; j < P::len; j += S) {
-        uint32_t v[NW];
-        adr_chain(wa, j);
-        adr_hash(wa, 0);
-        Hh::PRF(key, wa, v);  // wots_gen_sk, wots.cu:27-33
-        if constexpr (P::hash == kSha2) {
-            if (capture) store_val<P::hash, NW>(cap + (size_t)(j * 16) * P::n, v);
-#pragma unroll 1
-            for (int s = 0; s < P::w - 1; s++) {  // gen_chain(0, w-1), wots.cu:51-62
-                adr_hash(wa, s);
-                Hh::F(key, wa, v, v);
-                if (capture) store_val<P::hash, NW>(cap + (size_t)(j * 16 + s + 1) * P::n, v);
-            }
-        } else {
-            // SHAKE: the chain runs bit-interleaved; the capture keeps that
-            // form (k_wots_gather converts the values it picks)
-            typename Hh::ChainIl ch;
-            Hh::chain_il_begin(key, wa, ch);
-            uint32_t vi[NW];
-            Hh::to_il(v, vi);
-            if (capture) store_val<P::hash, NW>(cap + (size_t)(j * 16) * P::n, vi);
-#pragma unroll 1
-            for (int s = 0; s < P::w - 1; s++) {  // gen_chain(0, w-1), wots.cu:51-62
-                Hh::F_il(ch, s, vi, vi);
-                if (capture) store_val<P::hash, NW>(cap + (size_t)(j * 16 + s + 1) * P::n, vi);
-            }
+    adr_chain(wa, j);
+    uint32_t v[NW];
+    Hh::PRF(key, wa, v);  // wots_gen_sk, wots.cu:27-33
+    typename Hh::Chain ch;
+    Hh::chain_begin(key, wa, ch);
+    if constexpr (P::hash == kShake) {
+        // the chain runs bit-interleaved; the capture keeps that form
+        // (k_wots_gather converts the values it picks)
+        uint32_t t[NW];
+        Hh::to_il(v, t);
 #pragma unroll
-            for (int w = 0; w < NW; w++) v[w] = vi[w];  // parked interleaved
-        }
-        if constexpr (!Sh::park) {
-#pragma unroll 1
-            for (int i = 0; i < NW; i++) ts.word(pick<NW>(v, i));
-        } else {
-#pragma unroll
-            for (int i = 0; i < NW; i++) A.tl_buf[(size_t)(j * NW + i) * A.tl_lanes + leaf_g] = v[i];
-        }
+        for (int w = 0; w < NW; w++) v[w] = t[w];
     }
-    if constexpr (S > 1) __syncthreads();  // all chains of the leaf parked
-    uint32_t node[NW];
-    // T_len: with S > 1 on the lane pair q = 0, 1 of the leaf (S is even, so
-    // the pair is lanes 2i, 2i + 1), else on lane q = 0
-    constexpr bool pair = S > 1;
-    if (q < (pair ? 2 : 1)) {
+    if (capture) store_raw<P>(cap, v);
+#pragma unroll 1
+    for (int s = 0; s < P::w - 1; s++) {  // gen_chain(0, w-1), wots.cu:51-62
+        Hh::chain_step(key, ch, s, v, v);
+        if (capture) store_raw<P>(cap + (s + 1) * P::n, v);
+    }
+#pragma unroll
+    for (int i = 0; i < NW; i++) A.tl_buf[(size_t)(j * NW + i) * A.tl_lanes + leaf_g] = v[i];
+}
+
+template <class P, int MODE>
+__global__ void __launch_bounds__(256) k_chains(BatchArgs A, uint32_t nwaves) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + threadIdx.x / 64);
+    if (wave < nwaves) chain_wave<P, MODE>(A, wave);
+}
+
+// Signing: the FORS tiles of a batch (n_fors workgroups, first: a tile is
+// longer than a chain) and its WOTS chains in one launch, so that small
+// batches have both in flight together
+template <class P, int J>
+__global__ void __launch_bounds__(256) k_sign_fused(BatchArgs A, uint32_t n_fors, uint32_t nwaves) {
+    __shared__ uint32_t smem[fors_lds_words<P>()];
+    if (blockIdx.x < n_fors) {
+        fors_tile<P, J>(A, blockIdx.x, smem);
+        return;
+    }
+    const uint32_t wave =
+        __builtin_amdgcn_readfirstlane((blockIdx.x - n_fors) * 4 + threadIdx.x / 64);
+    if (wave < nwaves) chain_wave<P, 0>(A, wave);
+}
+
+// Hypertree subtrees from the parked chain ends: T_len of every leaf, then
+// the Merkle levels in LDS, auth paths and roots.  S lanes per leaf: S = 1
+// the most leaves per wave (large batches), S = 2 a lane pair per leaf, which
+// shares the serial T_len (sha256_compress_pair / keccak_f_il_pair).
+//
+// A subtree whose lanes exceed a 256-lane workgroup is split over PARTS
+// workgroups.  Each part reduces its leaves to a part root in LDS; the part
+// that finishes last (device-scope counter, release/acquire fences, no
+// waiting) climbs the remaining log2(PARTS) levels from the part roots.
+template <class P, int S>
+struct HtShape {
+    static constexpr int L = 1 << P::th;                 // leaves per subtree
+    static constexpr int LT = L * S;                     // lanes per subtree
+    static constexpr int PARTS = LT > 256 ? LT / 256 : 1;
+    static constexpr int LP = L / PARTS;                 // leaves per part
+    static constexpr int LOGP = P::th - ilog2(PARTS);    // levels reduced inside a part
+    static constexpr int TPW = PARTS > 1 ? 1 : 256 / LT; // subtrees per workgroup
+    static constexpr int NL = 256 / S;                   // leaves per workgroup
+    static constexpr int NLDS = NL > PARTS ? NL : PARTS; // the last part climbs from PARTS roots
+};
+
+template <class P, int MODE, int S>
+__global__ void __launch_bounds__(256) k_ht(BatchArgs A) {
+    using Hh = HashT<P>;
+    using Key = typename Hh::Key;
+    using Sh = HtShape<P, S>;
+    constexpr int NW = P::nw;
+    constexpr int L = Sh::L, TPW = Sh::TPW, NL = Sh::NL;
+    constexpr int PARTS = Sh::PARTS, LP = Sh::LP, LOGP = Sh::LOGP;
+    constexpr int LPT = LP * S;  // lanes per subtree in this workgroup
+    __shared__ uint32_t lds[2][Sh::NLDS][NW];  // two levels of nodes
+
+    const int tid = threadIdx.x;
+    const uint32_t blk = blockIdx.x;
+    const uint32_t part = PARTS > 1 ? blk % PARTS : 0;
+    const uint32_t u = part * LP + (tid % LPT) / S;  // leaf index = keypair address
+    const int q = tid % S;
+    const int slot = tid / S;                         // leaf slot in the workgroup
+    const uint32_t g = (blk / PARTS) * TPW + tid / LPT;
+    const uint32_t ntrees = MODE == 0 ? A.n_req * P::d : A.n_req;
+    const bool active = g < ntrees;
+    const uint32_t req = active ? (MODE == 0 ? g / P::d : g) : 0;
+    const uint32_t layer = MODE == 0 ? (active ? g % P::d : 0) : P::d - 1;
+    const uint32_t leaf_g = active ? g * L + u : 0;   // column in tl_buf
+    {
+        const Plan& pl = A.plan[req];
+        Key key;
+        Hh::load_key(pl, key);
+        uint64_t tree = 0;
+        uint32_t target = 0;
+        if (MODE == 0) {
+            tree = layer_tree<P>(pl.tree, layer);
+            target = layer == 0 ? pl.leaf
+                                : (uint32_t)((pl.tree >> ((layer - 1) * P::th)) & (L - 1));
+        }
+        // ---- T_len of leaf u (wots_gen_leaf, sign.cu:87-104)
+        Adr pa = adr_make(layer, tree, kWotsPk);
+        adr_keypair<P::th>(pa, u);
         constexpr int TLW = P::len * NW;
+        auto parked = [&](int w) { return A.tl_buf[(size_t)w * A.tl_lanes + leaf_g]; };
         auto parked2 = [&](int j) {
             const int i = j + q;
             return parked(i < 0 ? 0 : i < TLW ? i : TLW - 1);
         };
+        uint32_t node[NW];
         if constexpr (P::hash == kSha2) {
-            if constexpr (pair) thash_sha2_pair<NW, TLW>(key.mid, pa, parked2, node);
-            else ts.template finish<TLW>(node);
+            if constexpr (S == 2) thash_sha2_pair<NW, TLW>(key.mid, pa, parked2, node);
+            else thash_sha2_rd<NW, TLW>(key.mid, pa, parked, node);
         } else {
-            if constexpr (pair) thash_shake_pair<P, TLW>(key, pa, parked2, node);
+            if constexpr (S == 2) thash_shake_pair<P, TLW>(key, pa, parked2, node);
             else thash_shake_rd<P, TLW, true>(key, pa, parked, node);
         }
         if (q == 0) {
@@ -1115,6 +1156,7 @@ __device__ __forceinline__ void ht_tile(const BatchArgs& A, uint32_t blk, uint32
     if constexpr (PARTS > 1) {
         // part root -> ht_parts; the last part of the subtree climbs the rest
         __shared__ uint32_t last;
+        __syncthreads();
         if (tid == 0) {
             uint32_t* dst = A.ht_parts + ((size_t)g * PARTS + part) * NW;
 #pragma unroll
@@ -1132,7 +1174,7 @@ __device__ __forceinline__ void ht_tile(const BatchArgs& A, uint32_t blk, uint32
                     lds[LOGP & 1][tid][w] = __builtin_nontemporal_load(srcp + w);
             }
 #pragma unroll 1
-            for (int l = LOGP + 1; l <= LOGL; l++) {
+            for (int l = LOGP + 1; l <= P::th; l++) {
                 __syncthreads();
                 const int src = (l - 1) & 1, dst = l & 1;
                 if (tid < (L >> l)) {
@@ -1151,44 +1193,7 @@ __device__ __forceinline__ void ht_tile(const BatchArgs& A, uint32_t blk, uint32
     }
 }
 
-template <class P, int MODE, int S>
-__global__ void __launch_bounds__((HtShape<P, S>::WG)) k_ht(BatchArgs A) {
-    __shared__ uint32_t smem[HtShape<P, S>::lds_words];
-    ht_tile<P, MODE, S>(A, blockIdx.x, smem);
-}
-
 constexpr int max_int(int a, int b) { return a > b ? a : b; }
-
-// Signing as one persistent kernel: a grid of resident 256-lane workgroups
-// pulls tiles from a device counter (zeroed by k_prep) until the queue is
-// empty -- first the hypertree tiles (long), then the FORS tiles (short),
-// which fill the tail.  The tiles are independent given the plans, so no
-// workgroup ever waits on another; every workgroup exits once the counter
-// passes the last tile.
-// SHA-256: 4 waves per SIMD, as k_ht (5, at 96 VGPRs, keeps the F loop free
-// of spills but spills in T_len, and took 13.87-13.90 ms at SHA2-128f / 4096
-// against 13.73-13.81, both with 16 lanes per FORS tree); SHAKE256 (50-word
-// sponge): 3, as k_ht -- at 4 (128 VGPRs) every fast set signed slower, also
-// with the chain-step loop kept free of spills (SHAKE256-128f at 4096 40.4
-// against 39.95 ms)
-template <class P, int J, int S>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P::hash == kSha2 ? 4 : 3)))
-k_sign_fused(BatchArgs A, uint32_t n_ht, uint32_t n_fors) {
-    static_assert(HtShape<P, S>::WG == 256, "hypertree tiles of 256 lanes");
-    __shared__ uint32_t tile;
-    // one LDS buffer for both tile kinds (a workgroup runs one tile at a time)
-    __shared__ uint32_t smem[max_int(HtShape<P, S>::lds_words, fors_lds_words<P>())];
-#pragma unroll 1
-    while (true) {
-        if (threadIdx.x == 0) tile = atomicAdd(A.tile_ctr, 1u);
-        __syncthreads();
-        const uint32_t t = tile;
-        __syncthreads();  // every lane has the tile (and left the previous one)
-        if (t >= n_ht + n_fors) break;
-        if (t < n_ht) ht_tile<P, 0, S>(A, t, smem);
-        else fors_tile<P, J>(A, t - n_ht, smem);
-    }
-}
 
 // WOTS signatures: lane per (request, layer, chain); the layer signs the FORS
 // public key (layer 0) or the root of the layer below (sign.cu:1970-1989)
