@@ -397,11 +397,9 @@ typedef uint32_t __attribute__((address_space(3))) lds_u32;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 __attribute__((address_space(3))) lds_u32x4;
 
-// the 64 rounds of sha256_compress_pair with K[t] + W[t] precomputed (kw,
-// read by both lanes; the odd lane masks it out)
-// The 64 rounds of a lane pair with K[t] + W[t] precomputed (kw, read by both
-// lanes), with the odd (a-side) lane two rounds behind the even (e-side) one.
-// In sha256_compress_pair every round waits for its exchange: e' = d + T1
+// The 64 rounds of a lane pair with K[t] + W[t] precomputed, with the odd
+// (a-side) lane two rounds behind the even (e-side) one.  In
+// sha256_compress_pair every round waits for its exchange: e' = d + T1
 // needs the odd lane's d and a' = T1 + T2 the even lane's T1, so each round
 // is alignbit, xor3, add3, select, DPP swap and add in a row.  Here each
 // lane's own recurrence is alignbit, xor3, add3:
@@ -410,27 +408,31 @@ typedef u32x4 __attribute__((address_space(3))) lds_u32x4;
 //   odd,  iteration i:  A[i-1] = S0(A[i-2]) + Maj(A[i-2], A[i-3], A[i-4]) + T1[i-2],
 //                       T1[i-2] = E[i-1] - A[i-5]
 // and the swap of iteration i (each lane sends its new value) is first used
-// in iteration i + 1, to form pre[i+1] (even) and T1[i-1] (odd).  66
-// iterations; the odd lane's outputs of the first two are b and a, the even
-// lane's state is taken after iteration 63.  K + W is read about 16 rounds
-// ahead of its use (two groups of 16 registers).
+// in iteration i + 1, to form pre[i+1] (even) and T1[i-1] (odd).  Both are
+// (own ^ m) + (kw + swapped): kw points to the block's K + W on the even lane
+// and to kw_ones on the odd one, -A being ~A + 1, so they take a DPP add and
+// a v_xad (9 instructions per round).  66 iterations; the odd lane's outputs
+// of the first two are b and a, the even lane's state is taken after
+// iteration 63.  kw is read about 16 rounds ahead of its use (two groups of
+// 16 registers).
+constexpr int kKwOnes = 64;  // LDS words, all 1, that odd lanes read for K + W
 template <class KW>
 __device__ __forceinline__ void sha256_rounds_pair_kw(uint32_t s[4], KW kw) {
     const bool odd = threadIdx.x & 1u;
     const uint32_t m = odd ? ~0u : 0u;
     const uint32_t r1 = odd ? 2u : 6u, r2 = odd ? 13u : 11u, r3 = odd ? 22u : 25u;
-    uint32_t c0[16], c1[16];  // K + W [16g, 16g + 16) and the group after it
+    uint32_t c0[16], c1[16];  // kw [16g, 16g + 16) and the group after it
 #pragma unroll
     for (int j = 0; j < 16; j++) c0[j] = kw[j];
 #pragma unroll
     for (int j = 0; j < 16; j++) c1[j] = kw[16 + j];
     // even: e f g h; odd: a b c d.  The odd lane starts at c, d; the even
     // lane needs d (pre[0]) and c (A[-2], for pre[1]) from it.
-    const uint32_t d_ev = pair_swap(s[3]), c_ev = pair_swap(s[2]);
+    const uint32_t d_ev = pair_swap(s[3]);
     const uint32_t a_od = s[0], b_od = s[1];
     uint32_t q0 = lane_sel(m, s[2], s[0]), q1 = lane_sel(m, s[3], s[1]), q2 = s[2], q3 = s[3];
     uint32_t x = q3 + c0[0] + d_ev;  // even: pre[0]; odd: unused
-    uint32_t rp = c_ev;              // the previous iteration's swap
+    uint32_t nwp = s[2];             // the value each lane sent last
     uint32_t e0 = 0, e1 = 0, e2 = 0, e3 = 0;
 #pragma unroll
     for (int i = 0; i < 66; i++) {
@@ -449,14 +451,15 @@ __device__ __forceinline__ void sha256_rounds_pair_kw(uint32_t s[4], KW kw) {
         uint32_t nw = sg + fn + x;                                // E[i+1] | A[i-1]
         if (i == 0) nw = lane_sel(m, b_od, nw);
         if (i == 1) nw = lane_sel(m, a_od, nw);
-        const uint32_t r = pair_swap(nw);
-        const uint32_t kn = i + 1 < 64 ? c0[(i + 1) & 15] : 0u;
-        x = lane_sel(m, rp - q2, q2 + kn + rp);  // T1[i-1] | pre[i+1]
+        // pre[i+1] | T1[i-1]; past the even lane's last round only the odd
+        // lane's is used, whose kw is 1 throughout
+        const uint32_t y = c0[i + 1 < 64 ? (i + 1) & 15 : 15] + pair_swap(nwp);
+        x = (q2 ^ m) + y;
         q3 = q2;
         q2 = q1;
         q1 = q0;
         q0 = nw;
-        rp = r;
+        nwp = nw;
         if (i == 63) {
             e0 = q0;
             e1 = q1;
@@ -489,9 +492,9 @@ __device__ __forceinline__ void sha256_compress_dup(uint32_t st[8], const uint32
     }
 }
 
-// sha256_compress_dup with K[t] + W[t] precomputed (kw, LDS): the message
-// hashes' blocks made only of message words, whose schedules another wave
-// computed ahead
+// sha256_compress_dup with K[t] + W[t] precomputed (kw as for
+// sha256_rounds_pair_kw): the message hashes' blocks made only of message
+// words, whose schedules another wave computed ahead
 __device__ __forceinline__ void sha256_rounds_dup_kw(uint32_t st[8], const lds_u32* kw) {
     const uint32_t m = (threadIdx.x & 1u) ? ~0u : 0u;
     uint32_t s4[4];
@@ -856,7 +859,7 @@ struct Sha2 {
     // blocks go through stream_range.  Both waves call this with the same
     // arguments and pass the same 1 + stages barriers.
     static constexpr uint32_t kLongStage = 32;
-    static constexpr uint32_t kLongLdsWords = 2 * kLongStage * 64;
+    static constexpr uint32_t kLongLdsWords = 2 * kLongStage * 64 + kKwOnes;
 
     template <int NPRE>
     __device__ static void stream_msg_long(uint32_t st[8], const uint32_t pre[NPRE],
@@ -873,8 +876,12 @@ struct Sha2 {
             if (lane < kLongStage && blk < nfb)
                 sha256_kw_msg_block(mw + 16 * blk, kw_s + ((c & 1) * kLongStage + lane) * 64);
         };
-        if (prod) produce(0);
-        else if (nfb) stream_range<NPRE>(st, pre, m, mlen, before, 0, kk0);
+        lds_u32* ones = kw_s + 2 * kLongStage * 64;
+        const uint32_t odd = threadIdx.x & 1u;
+        if (prod) {
+            produce(0);
+            ones[lane] = 1u;
+        } else if (nfb) stream_range<NPRE>(st, pre, m, mlen, before, 0, kk0);
         __syncthreads();
         uint32_t sl[8];  // in registers across the stages
 #pragma unroll
@@ -888,7 +895,8 @@ struct Sha2 {
                                                                       : kLongStage;
                 const lds_u32* rows = kw_s + (c & 1) * kLongStage * 64;
 #pragma unroll 1
-                for (uint32_t b = 0; b < nb; b++) sha256_rounds_dup_kw(sl, rows + 64 * b);
+                for (uint32_t b = 0; b < nb; b++)
+                    sha256_rounds_dup_kw(sl, odd ? ones : rows + 64 * b);
             }
             __syncthreads();
         }

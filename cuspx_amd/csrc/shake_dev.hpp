@@ -261,6 +261,10 @@ __device__ __forceinline__ void il_to(uint32_t lo, uint32_t hi, uint32_t& e, uin
     e = il_even16(lo) | (il_even16(hi) << 16);
     o = il_even16(lo >> 1) | (il_even16(hi >> 1) << 16);
 }
+// E (h = 0) or O (h = 1) of (lo, hi)
+__device__ __forceinline__ uint32_t il_half(uint32_t lo, uint32_t hi, uint32_t h) {
+    return il_even16(lo >> h) | (il_even16(hi >> h) << 16);
+}
 // (E, O) -> (lo, hi)
 __device__ __forceinline__ void il_from(uint32_t e, uint32_t o, uint32_t& lo, uint32_t& hi) {
     lo = il_spread16(e) | (il_spread16(o) << 1);
@@ -514,6 +518,142 @@ __device__ __forceinline__ void keccak_f_il_pair(uint32_t s[25]) {
         keccak_round_il_pair(s, m, lane_sel(m, kKeccakRcIl.w[2 * r + 1], kKeccakRcIl.w[2 * r]));
 }
 
+// ---------------------------------------------------------- sixteen lanes
+//
+// One Keccak-f[1600] on a row of 16 lanes (all active), for serial sponges:
+// a wave alone on its SIMD issues an instruction every 4-5 cycles whatever it
+// holds, so a permutation costs what its instruction stream is long.  Lane p
+// < 7 holds the even-bit halves of one column, lane p + 8 the odd-bit halves:
+// s[y] = lane (x, y) with x = (p + 4) % 5.  Positions 0 and 6 repeat columns
+// 4 and 0 so that theta's two neighbours (x - 1, same half; x + 1, other half
+// rotated by one) are fixed DPP row moves; 7 and 15 idle.  After rho (a rotate
+// count per lane and row) every word goes through LDS to its place under pi,
+// and each lane reads its new column and the two after it, which chi needs.
+// About 34 instructions and one LDS round trip per round, against 128
+// instructions on a lane pair.
+struct Keccak16Tab {
+    uint8_t rot[16][5];   // v_alignbit count of row y
+    uint8_t wr[16][5];    // word written by row y
+    uint8_t rd[16][3];    // first word of columns x, x + 1, x + 2
+    constexpr Keccak16Tab() : rot{}, wr{}, rd{} {
+        for (int p = 0; p < 16; p++) {
+            const int h = p >> 3, q = p & 7, x = (q + 4) % 5;
+            const bool owner = q >= 1 && q <= 5;
+            for (int y = 0; y < 5; y++) {
+                const int r = kRho[x + 5 * y];
+                const int n = (r & 1) == 0 ? r / 2 : h ? (r + 1) / 2 : (r - 1) / 2;
+                const int h2 = h ^ (r & 1);  // odd rotations swap the halves
+                rot[p][y] = (uint8_t)((32 - n) & 31);
+                // column y, row 2x + 3y; the repeated columns write aside
+                wr[p][y] = (uint8_t)(owner ? (h2 * 5 + y) * 8 + (2 * x + 3 * y) % 5 : 80 + p);
+            }
+            for (int k = 0; k < 3; k++) rd[p][k] = (uint8_t)((h * 5 + (x + k) % 5) * 8);
+        }
+    }
+};
+__constant__ Keccak16Tab kKeccak16 = Keccak16Tab();
+
+struct Keccak16 {
+    static constexpr int kLdsWords = 96;  // per row of 16 lanes, 16-byte aligned
+    typedef uint32_t __attribute__((address_space(3))) lds_word;
+    typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+    typedef v4 __attribute__((address_space(3))) lds_v4;
+
+    uint32_t s[5];
+    uint32_t rot[5];
+    lds_word* wr[5];
+    lds_word* rd[3];
+    lds_word* base;
+    uint32_t me, mo;  // iota: all ones where column 0's even / odd half is held
+    uint32_t sh1;     // theta's rotate by one (even half)
+    uint32_t half;
+    int col;
+
+    __device__ __forceinline__ void init(lds_word* row) {
+        const int p = threadIdx.x & 15;
+        half = p >> 3;
+        col = ((p & 7) + 4) % 5;
+        base = row;
+#pragma unroll
+        for (int y = 0; y < 5; y++) {
+            rot[y] = kKeccak16.rot[p][y];
+            wr[y] = row + kKeccak16.wr[p][y];
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) rd[k] = row + kKeccak16.rd[p][k];
+        me = (col == 0 && !half) ? ~0u : 0u;
+        mo = (col == 0 && half) ? ~0u : 0u;
+        sh1 = half ? 0u : 31u;
+        clear();
+    }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int y = 0; y < 5; y++) s[y] = 0;
+    }
+    // LDS words written by other lanes of the row are read next: keep the order
+    __device__ static __forceinline__ void order() {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __device__ __forceinline__ void round(uint32_t rc_e, uint32_t rc_o) {
+        const uint32_t C = xor3(xor3(s[0], s[1], s[2]), s[3], s[4]);
+        // lane p - 1 (row_shr 1): column x - 1; lane p + 9 (row_ror 7): the
+        // other half of column x + 1
+        const uint32_t cm = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)C, 0x111, 0xF, 0xF, true);
+        const uint32_t t = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)C, 0x127, 0xF, 0xF, true);
+        const uint32_t cp = __builtin_amdgcn_alignbit(t, t, sh1);
+#pragma unroll
+        for (int y = 0; y < 5; y++) {
+            const uint32_t u = xor3(s[y], cm, cp);
+            *wr[y] = __builtin_amdgcn_alignbit(u, u, rot[y]);
+        }
+        order();
+        v4 b[3];
+        uint32_t b4[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            b[k] = *(const lds_v4*)rd[k];
+            b4[k] = rd[k][4];
+        }
+        order();
+        const uint32_t rc = (me & rc_e) | (mo & rc_o);
+#pragma unroll
+        for (int y = 0; y < 4; y++) s[y] = bit_chi(b[0][y], b[1][y], b[2][y]);
+        s[4] = bit_chi(b4[0], b4[1], b4[2]);
+        s[0] ^= rc;
+    }
+    __device__ __forceinline__ void permute() {
+        constexpr KeccakRcIl rc;  // as literals: no scalar load waits among the LDS reads
+#pragma unroll
+        for (int r = 0; r < 24; r++) round(rc.w[2 * r], rc.w[2 * r + 1]);
+    }
+    // this half of a 64-bit lane (lo, hi)
+    __device__ __forceinline__ uint32_t split(uint32_t lo, uint32_t hi) const {
+        return il_half(lo, hi, half);
+    }
+    // Keccak lane l of the state (l < 25), interleaved or plain, in every
+    // lane of the row
+    __device__ __forceinline__ void lane_il(int l, uint32_t& e, uint32_t& o) const {
+        const int at = (threadIdx.x & 48) + 1 + l % 5;
+        e = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * at, (int)s[l / 5]);
+        o = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (at + 8), (int)s[l / 5]);
+    }
+    __device__ __forceinline__ void lane(int l, uint32_t& lo, uint32_t& hi) const {
+        uint32_t e, o;
+        lane_il(l, e, o);
+        il_from(e, o, lo, hi);
+    }
+    // Absorb rate block b of a stream held in LDS as interleaved words (E, O
+    // of 64-bit lane i at buf[2 i], buf[2 i + 1]; whole blocks, padded)
+    __device__ __forceinline__ void absorb(const lds_word* buf, int b) {
+#pragma unroll
+        for (int y = 0; y < 4; y++) {
+            const int l = col + 5 * y;
+            if (l < 17) s[y] ^= buf[2 * (17 * b + l) + half];
+        }
+    }
+};
+
 template <int N>
 struct Shake {
     static constexpr int hash = kShake;
@@ -639,107 +779,74 @@ struct Shake {
 
     // ------------------------------------------------ per-request hashing
 
-    // SHAKE256(pre || m) squeezed to OUTB bytes (OUTB <= 136), on a lane pair
-    // (both lanes active with identical inputs; keccak_f_il_pair).  m is
-    // 4-byte aligned; the word holding the last message byte is the last one
-    // read.  The state is held interleaved, this lane's half of every Keccak
-    // lane; each absorbed plain word is split into its even or odd bits on
-    // the way in.  Whole 136-byte blocks of message words are absorbed
-    // directly, the head after the prefix and the tail word by word.  The
-    // output is in both lanes.
+    // SHAKE256(pre || m) squeezed to OUTB bytes (OUTB <= 136), on 16 lanes
+    // holding identical inputs (Keccak16).  m is 4-byte aligned; the word
+    // holding the last message byte is the last one read.  Lane p of the row
+    // loads words p, p + 16 and p + 32 of a block (the next block's while
+    // this one permutes) into LDS, from where every lane takes its halves.
+    // The output is in every lane.
+    static constexpr int kStage = 36;  // LDS words of one staged block
+    static constexpr int kRowWords = Keccak16::kLdsWords + kStage;
     template <int NPRE, int OUTB>
-    __device__ static void stream_msg_pair(const uint32_t pre[NPRE], const uint8_t* m,
-                                           uint32_t mlen, uint8_t out[OUTB]) {
+    __device__ static __forceinline__ void stream_msg(Keccak16& k, const uint32_t pre[NPRE], const uint8_t* m,
+                                      uint32_t mlen, uint8_t out[OUTB]) {
         static_assert(NPRE < 34 && OUTB <= 136, "prefix within one block");
-        const uint32_t h = threadIdx.x & 1u;
-        const uint32_t msk = h ? ~0u : 0u;
-        // this lane's interleaved half of plain word x at stream word q
-        auto half = [&](uint32_t x, int q) { return il_even16(x >> h) << (16 * (q & 1)); };
-        const uint32_t* mw = reinterpret_cast<const uint32_t*>(m);
-        uint32_t s[25];
-#pragma unroll
-        for (int i = 0; i < 25; i++) s[i] = 0;
-#pragma unroll
-        for (int q = 0; q < NPRE; q++) s[q >> 1] ^= half(pre[q], q);
-        int q = NPRE;
-        const uint32_t full = mlen / 4, rem = mlen & 3;
-        uint32_t i = 0;
-        // xor this lane's half of word x at a wave-uniform runtime q
-        auto put = [&](int qq, uint32_t x) {
-            const uint32_t c = il_even16(x >> h) << (16 * (qq & 1));
-#pragma unroll
-            for (int l = 0; l < 17; l++) s[l] ^= (qq >> 1) == l ? c : 0u;
+        const gbl_u32* mg = (gbl_u32*)reinterpret_cast<const uint32_t*>(m);  // address-space cast
+        Keccak16::lds_word* stage = k.base + Keccak16::kLdsWords;
+        const int p = threadIdx.x & 15;
+        const uint32_t nb = (uint32_t)((4ull * NPRE + mlen) / 136u) + 1;
+        // stream word g (behind the prefix): message bytes, then 0x1F
+        auto word = [&](uint32_t g) -> uint32_t {
+            const int64_t valid = (int64_t)mlen - 4 * ((int64_t)g - NPRE);
+            if (g < (uint32_t)NPRE || valid < 0) return 0u;
+            uint32_t x = valid > 0 ? mg[g - NPRE] : 0u;
+            if (valid < 4) {
+                const uint32_t sh = 8 * (uint32_t)valid;
+                x = (x & ((1u << sh) - 1u)) | (0x1Fu << sh);
+            }
+            return x;
         };
-        // the message words up to the first block boundary (stream positions
-        // NPRE .. 33, fixed at compile time), then the blocks made only of
-        // message words (block b + 1 loads while block b permutes), then the
-        // words left over (positions 0 .. 32 of the last block); the head's
-        // and the tail's words are each loaded together (one word per step
-        // had put a load on the serial path for every word)
-        const gbl_u32* mg = (gbl_u32*)mw;  // address-space cast
-        constexpr int HEAD = NPRE == 0 ? 0 : 34 - NPRE;
-        if constexpr (HEAD > 0) {
-            const uint32_t nh = (uint32_t)HEAD < full ? (uint32_t)HEAD : full;
-            uint32_t x[HEAD];
-#pragma unroll
-            for (int k = 0; k < HEAD; k++) x[k] = (uint32_t)k < nh ? mg[k] : 0u;
-#pragma unroll
-            for (int k = 0; k < HEAD; k++) s[(NPRE + k) >> 1] ^= half(x[k], NPRE + k);
-            i = nh;
-            q = NPRE + (int)nh;
-            if (q == 34) {
-                keccak_f_il_pair(s);
-                q = 0;
-            }
-        }
-        const uint32_t nfb = q == 0 ? (full - i) / 34 : 0u;
-        if (nfb) {
-            const gbl_u32* g = (gbl_u32*)mw + i;  // address-space cast
-            uint32_t cur[34];
-#pragma unroll
-            for (int l = 0; l < 34; l++) cur[l] = g[l];
+        auto fetch = [&](uint32_t b, uint32_t x[3]) {
+            x[0] = word(34 * b + p);
+            x[1] = word(34 * b + p + 16);
+            x[2] = p < 2 ? word(34 * b + p + 32) : 0u;
+        };
+        uint32_t x[3];
+        fetch(0, x);
+        k.clear();
 #pragma unroll 1
-            for (uint32_t b = 0; b < nfb; b++) {
+        for (uint32_t b = 0; b < nb; b++) {
+            stage[p] = x[0];
+            stage[p + 16] = x[1];
+            if (p < 2) stage[p + 32] = b + 1 == nb && p == 1 ? x[2] ^ 0x80000000u : x[2];
+            Keccak16::order();
+            if (b == 0) {  // the same values from every lane
 #pragma unroll
-                for (int l = 0; l < 17; l++)
-                    s[l] ^= il_even16(cur[2 * l] >> h) | (il_even16(cur[2 * l + 1] >> h) << 16);
-                if (b + 1 < nfb) {
-#pragma unroll
-                    for (int l = 0; l < 34; l++) cur[l] = g[34 * (b + 1) + l];
-                }
-                keccak_f_il_pair(s);
+                for (int q = 0; q < NPRE; q++) stage[q] = pre[q];
+                Keccak16::order();
             }
-            i += 34 * nfb;
-        }
-        if (q == 0) {  // else the message ended inside the first block: i == full
-            const uint32_t r = full - i;  // < 34
-            uint32_t x[34];
 #pragma unroll
-            for (int k = 0; k < 34; k++) x[k] = (uint32_t)k < r ? mg[i + k] : 0u;
-#pragma unroll
-            for (int k = 0; k < 34; k++) s[k >> 1] ^= half(x[k], k);
-            q = (int)r;
-            i = full;
+            for (int y = 0; y < 4; y++) {
+                const int l = k.col + 5 * y;
+                if (l < 17) k.s[y] ^= k.split(stage[2 * l], stage[2 * l + 1]);
+            }
+            Keccak16::order();
+            if (b + 1 < nb) fetch(b + 1, x);
+            k.permute();
         }
-        uint32_t last = rem ? (mw[full] & (0xFFFFFFFFu >> (8 * (4 - rem)))) : 0u;
-        last |= 0x1Fu << (8 * rem);
-        put(q, last);
-        s[16] ^= half(0x80000000u, 33);
-        keccak_f_il_pair(s);
 #pragma unroll
         for (int l = 0; l < (OUTB + 7) / 8; l++) {
-            const uint32_t other = pair_swap(s[l]);
             uint32_t lo, hi;
-            il_from(lane_sel(msk, other, s[l]), lane_sel(msk, s[l], other), lo, hi);
+            k.lane(l, lo, hi);
 #pragma unroll
             for (int o = 0; o < 8; o++)
                 if (8 * l + o < OUTB) out[8 * l + o] = (uint8_t)((o < 4 ? lo : hi) >> (8 * (o & 3)));
         }
     }
 
-    // R = SHAKE256(sk_prf || optrand || m, n) (hash_shake256.cu:64-75), on a
-    // lane pair holding identical inputs
-    __device__ static void prf_msg(const uint32_t skprf[NW], const uint32_t opt[NW],
+    // R = SHAKE256(sk_prf || optrand || m, n) (hash_shake256.cu:64-75), on 16
+    // lanes holding identical inputs
+    __device__ static __forceinline__ void prf_msg(Keccak16& k, const uint32_t skprf[NW], const uint32_t opt[NW],
                                    const uint8_t* m, uint32_t mlen, uint32_t R[NW]) {
         uint32_t pre[2 * NW];
         uint8_t o[N];
@@ -748,24 +855,24 @@ struct Shake {
             pre[i] = skprf[i];
             pre[NW + i] = opt[i];
         }
-        stream_msg_pair<2 * NW, N>(pre, m, mlen, o);
+        stream_msg<2 * NW, N>(k, pre, m, mlen, o);
 #pragma unroll
         for (int i = 0; i < NW; i++)
             R[i] = (uint32_t)o[4 * i] | (uint32_t)o[4 * i + 1] << 8 |
                    (uint32_t)o[4 * i + 2] << 16 | (uint32_t)o[4 * i + 3] << 24;
     }
 
-    // digest = SHAKE256(R || pk || m, DG) (hash_shake256.cu:96-130), on a
-    // lane pair holding identical inputs
+    // digest = SHAKE256(R || pk || m, DG) (hash_shake256.cu:96-130), on 16
+    // lanes holding identical inputs
     template <int DG>
-    __device__ static void h_msg(const uint32_t R[NW], const uint32_t pk[2 * NW],
+    __device__ static __forceinline__ void h_msg(Keccak16& k, const uint32_t R[NW], const uint32_t pk[2 * NW],
                                  const uint8_t* m, uint32_t mlen, uint8_t dg[DG]) {
         uint32_t pre[3 * NW];
 #pragma unroll
         for (int i = 0; i < NW; i++) pre[i] = R[i];
 #pragma unroll
         for (int i = 0; i < 2 * NW; i++) pre[NW + i] = pk[i];
-        stream_msg_pair<3 * NW, DG>(pre, m, mlen, dg);
+        stream_msg<3 * NW, DG>(k, pre, m, mlen, dg);
     }
 
     // no midstate for SHAKE256 (zeros); PAIR as for Sha2::midstate

@@ -3,9 +3,9 @@
 // One signature is split across many lanes (MI355X needs >> 256 workgroups
 // and prefers uniform control flow inside a wave):
 //
-//   sign:   k_prep       lane pair per request: midstate, PRF_msg, H_msg, plan
+//   sign:   k_prep       lane group per request: midstate, PRF_msg, H_msg, plan
 //           k_fors       L lanes per FORS tree (2^J leaves per lane), LDS reduce
-//           k_fors_pk    lane pair per request: T_k over the k roots (small
+//           k_fors_pk    lane group per request: T_k over the k roots (small
 //                        batches: run by the lane storing the last root)
 //           k_chains     lane per WOTS chain of every leaf of every hypertree
 //                        layer (all d layers at once: every layer's tree/leaf
@@ -106,14 +106,15 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
 }
 
 // The prep kernels (128-lane workgroups).  Workgroups [0, prep_wgs): every
-// request hashes its message on a lane pair (sha256_compress_dup /
-// Shake::stream_msg_pair; both lanes compute everything, the even lane
-// stores), 64 requests per workgroup.  SHA-256 messages of at least
-// long_min bytes are left to the workgroups after those: each takes long
-// requests in turn and runs one with both waves (Sha2::stream_msg_long), the
-// schedules of its message-only blocks computed by wave 1 ahead of wave 0's
-// rounds.
-constexpr uint32_t kPrepLanes = 2;
+// request hashes its message on a lane group (SHA-256: a pair,
+// sha256_compress_dup, 64 requests per workgroup; SHAKE256: 16 lanes,
+// Keccak16, 8 requests); all its lanes compute everything, the first one
+// stores.  SHA-256 messages of at least long_min bytes are left to the
+// workgroups after those: each takes long requests in turn and runs one with
+// both waves (Sha2::stream_msg_long), the schedules of its message-only blocks
+// computed by wave 1 ahead of wave 0's rounds.
+template <class P>
+__host__ __device__ constexpr uint32_t prep_lanes() { return P::hash == kSha2 ? 2 : 16; }
 constexpr uint32_t kPrepWg = 128;
 // the two-wave path from this length: a single SHA2-128f / 256f request of
 // 512 B signs in 0.329 / 0.624 ms against 0.336 / 0.634 on the lane pair,
@@ -141,10 +142,11 @@ __device__ __forceinline__ void prep_plan_init(const BatchArgs& A, uint32_t row,
 }
 
 // sign, one request: midstate, R = PRF_msg, digest = H_msg, plan; LONG: the
-// two-wave form over kw_s (prod: wave 1), else a lane pair
+// two-wave form over kw_s (prod: wave 1), else a lane group (SHAKE256: with
+// its row's sponge k)
 template <class P, bool LONG>
 __device__ __forceinline__ void prep_sign_one(const BatchArgs& A, uint32_t i, bool store,
-                                              lds_u32* kw_s, bool prod) {
+                                              lds_u32* kw_s, bool prod, Keccak16* k) {
     using Hh = HashT<P>;
     constexpr int NW = P::nw;
     const uint32_t row = A.key_idx ? A.key_idx[i] : i;
@@ -169,12 +171,16 @@ __device__ __forceinline__ void prep_sign_one(const BatchArgs& A, uint32_t i, bo
     if constexpr (LONG) {
         Hh::template prf_msg<true>(skprf, opt, m, ml, R, kw_s, prod);
         Hh::template h_msg<P::dgst_bytes, true>(R, pk, m, ml, dg, kw_s, prod);
+    } else if constexpr (P::hash == kShake) {
+        Hh::prf_msg(*k, skprf, opt, m, ml, R);
+        Hh::template h_msg<P::dgst_bytes>(*k, R, pk, m, ml, dg);
     } else {
-        (void)kw_s;
-        (void)prod;
         Hh::prf_msg(skprf, opt, m, ml, R);
         Hh::template h_msg<P::dgst_bytes>(R, pk, m, ml, dg);
     }
+    (void)kw_s;
+    (void)prod;
+    (void)k;
     if (!store) return;
     uint8_t* sig = A.sig + (size_t)i * A.sig_stride;
     store_val<P::hash, NW>(sig, R);
@@ -196,27 +202,36 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
 #pragma unroll 1
             for (uint32_t i = blockIdx.x - A.prep_wgs; i < A.n_req; i += gridDim.x - A.prep_wgs)
                 if (prep_is_long(A, i))
-                    prep_sign_one<P, true>(A, i, threadIdx.x == 0, (lds_u32*)kw_s, prod);
+                    prep_sign_one<P, true>(A, i, threadIdx.x == 0, (lds_u32*)kw_s, prod, nullptr);
         }
         return;
     }
-    const uint32_t i = (blockIdx.x * kPrepWg + threadIdx.x) / kPrepLanes;
+    constexpr uint32_t PL = prep_lanes<P>();
+    const uint32_t i = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
     if (i >= A.n_req) return;
-    if (A.ht_count) {
+    const bool first = threadIdx.x % PL == 0;
+    if (A.ht_count && first) {
 #pragma unroll 1
-        for (int layer = 0; layer < P::d; layer++)
-            if (threadIdx.x % kPrepLanes == 0) A.ht_count[(size_t)i * P::d + layer] = 0;
+        for (int layer = 0; layer < P::d; layer++) A.ht_count[(size_t)i * P::d + layer] = 0;
     }
-    if (A.fors_count && threadIdx.x % kPrepLanes == 0) A.fors_count[i] = 0;
+    if (A.fors_count && first) A.fors_count[i] = 0;
     if (prep_is_long(A, i)) return;
-    prep_sign_one<P, false>(A, i, (threadIdx.x & 1u) == 0, nullptr, false);
+    if constexpr (P::hash == kShake) {
+        constexpr int RW = HashT<P>::kRowWords;
+        __shared__ __align__(16) uint32_t row_s[kPrepWg / PL * RW];
+        Keccak16 k;
+        k.init((lds_u32*)row_s + threadIdx.x / PL * RW);
+        prep_sign_one<P, false>(A, i, first, nullptr, false, &k);
+    } else {
+        prep_sign_one<P, false>(A, i, first, nullptr, false, nullptr);
+    }
 }
 
 // verify, one request: midstate, digest = H_msg(R from the signature), plan
 // (LONG as for prep_sign_one)
 template <class P, bool LONG>
 __device__ __forceinline__ void prep_verify_one(const BatchArgs& A, uint32_t i, bool store,
-                                                lds_u32* kw_s, bool prod) {
+                                                lds_u32* kw_s, bool prod, Keccak16* k) {
     using Hh = HashT<P>;
     constexpr int NW = P::nw;
     const uint32_t row = A.key_idx ? A.key_idx[i] : i;
@@ -238,11 +253,14 @@ __device__ __forceinline__ void prep_verify_one(const BatchArgs& A, uint32_t i, 
     if constexpr (LONG) {
         Hh::template h_msg<P::dgst_bytes, true>(R, pk, A.msg + A.moff[i], A.mlen[i], dg, kw_s,
                                                 prod);
+    } else if constexpr (P::hash == kShake) {
+        Hh::template h_msg<P::dgst_bytes>(*k, R, pk, A.msg + A.moff[i], A.mlen[i], dg);
     } else {
-        (void)kw_s;
-        (void)prod;
         Hh::template h_msg<P::dgst_bytes>(R, pk, A.msg + A.moff[i], A.mlen[i], dg);
     }
+    (void)kw_s;
+    (void)prod;
+    (void)k;
     if (!store) return;
     plan_from_digest<P>(pl, dg);
     pl.status = 0;
@@ -260,20 +278,30 @@ __global__ void __launch_bounds__(kPrepWg) k_vprep(BatchArgs A) {
 #pragma unroll 1
             for (uint32_t i = blockIdx.x - A.prep_wgs; i < A.n_req; i += gridDim.x - A.prep_wgs)
                 if (prep_is_long(A, i))
-                    prep_verify_one<P, true>(A, i, threadIdx.x == 0, (lds_u32*)kw_s, prod);
+                    prep_verify_one<P, true>(A, i, threadIdx.x == 0, (lds_u32*)kw_s, prod, nullptr);
         }
         return;
     }
-    const uint32_t i = (blockIdx.x * kPrepWg + threadIdx.x) / kPrepLanes;
+    constexpr uint32_t PL = prep_lanes<P>();
+    const uint32_t i = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
     if (i >= A.n_req || prep_is_long(A, i)) return;
-    prep_verify_one<P, false>(A, i, (threadIdx.x & 1u) == 0, nullptr, false);
+    const bool first = threadIdx.x % PL == 0;
+    if constexpr (P::hash == kShake) {
+        constexpr int RW = HashT<P>::kRowWords;
+        __shared__ __align__(16) uint32_t row_s[kPrepWg / PL * RW];
+        Keccak16 k;
+        k.init((lds_u32*)row_s + threadIdx.x / PL * RW);
+        prep_verify_one<P, false>(A, i, first, nullptr, false, &k);
+    } else {
+        prep_verify_one<P, false>(A, i, first, nullptr, false, nullptr);
+    }
 }
 
 // grid of the prep kernels for n requests whose messages are at most
 // mlen_bound bytes (0: not known); sets A.prep_wgs / A.long_min
 template <class P>
 inline uint32_t prep_grid(BatchArgs& A, uint32_t n, uint32_t mlen_bound) {
-    A.prep_wgs = (uint32_t)(((uint64_t)n * kPrepLanes + kPrepWg - 1) / kPrepWg);
+    A.prep_wgs = (uint32_t)(((uint64_t)n * prep_lanes<P>() + kPrepWg - 1) / kPrepWg);
     const bool lng = prep_has_long<P>() && (mlen_bound == 0 || mlen_bound >= kLongMsgBytes);
     A.long_min = lng ? kLongMsgBytes : 0;
     return A.prep_wgs + (lng ? (n < kLongWgs ? n : kLongWgs) : 0);
@@ -328,8 +356,8 @@ __global__ void __launch_bounds__(64) k_kprep(BatchArgs A) {
 
 // ------------------------------------------------------------------ FORS
 
-template <class P, bool PAIR>
-__device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i);
+template <class P, bool GROUP>
+__device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i, lds_u32* row);
 
 // a FORS root of request req is stored.  Small sign batches (fors_count
 // set): count it, and the lane that stores the request's last root computes
@@ -344,7 +372,7 @@ __device__ __forceinline__ void fors_root_done(const BatchArgs& A, uint32_t req)
     __threadfence();  // release this root before counting it
     if (atomicAdd(&A.fors_count[req], 1u) == (uint32_t)P::k - 1) {
         __threadfence();  // acquire: every root of the request is visible
-        fors_pk_of<P, false>(A, req);
+        fors_pk_of<P, false>(A, req, nullptr);
     }
 }
 
@@ -620,23 +648,46 @@ __device__ __forceinline__ void thash_sha2_pair(const uint32_t mid[8], const Adr
     SP::output(st, out);
 }
 
-// K[t] + W[t] (t = 0..63) of payload-only block b of a thash_sha2_pair
-// payload held in LDS as native words (pk), on one lane: the message
-// schedule of a block does not depend on the chaining value, so idle lanes
-// can run it ahead of the pair that compresses (sha256_rounds_pair_kw)
-__device__ __forceinline__ void sha2_kw_block(const uint32_t* pk, int b, uint32_t kw[64]) {
-    uint32_t w[16];
+// K[t] + W[t] (t = 0..63) of compression block b (any of Sha2Pair's, b may
+// differ from lane to lane) on one lane: a block's message schedule does not
+// depend on the chaining value, so lanes that would idle run it ahead of the
+// pair that compresses (sha256_rounds_pair_kw).  rd(i): payload word i.
+// kw: 16-byte aligned LDS.
+template <int NW, int M, class Rd>
+__device__ __forceinline__ void sha2_kw_block(const Adr& a, const Rd& rd, int b, uint32_t* kw) {
+    using SP = Sha2Pair<NW, M>;
+    uint32_t w[16], x[17];
     const int base = 16 * b - 6;
 #pragma unroll
-    for (int i = 0; i < 16; i++) w[i] = __builtin_amdgcn_alignbit(pk[base + i], pk[base + i + 1], 16);
+    for (int j = 0; j < 17; j++) {
+        const int i = base + j;
+        x[j] = rd(i < 0 ? 0 : i < M ? i : M - 1);
+    }
 #pragma unroll
-    for (int t = 0; t < 64; t++) {
-        if (t >= 16) {
-            const uint32_t x = w[(t - 15) & 15], y = w[(t - 2) & 15];
-            w[t & 15] = xor3(rotr32(y, 17), rotr32(y, 19), y >> 10) + w[(t - 7) & 15] +
-                        xor3(rotr32(x, 7), rotr32(x, 18), x >> 3) + w[t & 15];
+    for (int i = 0; i < 16; i++) {
+        uint32_t y = __builtin_amdgcn_alignbit(x[i], x[i + 1], 16);
+        if (i < 5) y = b == 0 ? a.w[i < 5 ? i : 0] : y;
+        if (i == 5) y = b == 0 ? (a.w[5] | (x[6] >> 16)) : y;
+        if (b >= SP::FT) {
+            const int g = 16 * b + i;
+            y = g < 5 + M ? y : g == 5 + M ? ((x[i] << 16) | 0x8000u) : 0u;
+            if (i == 15) y = b == SP::B - 1 ? SP::bits : y;
         }
-        kw[t] = kSha256K[t] + w[t & 15];
+        w[i] = y;
+    }
+    u32x4* out = reinterpret_cast<u32x4*>(kw);
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        uint32_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int t = 4 * q + j;
+            if (t >= 16)
+                w[t & 15] = sha256_s1(w[(t - 2) & 15]) + w[(t - 7) & 15] +
+                            sha256_s0(w[(t - 15) & 15]) + w[t & 15];
+            o[j] = kSha256K[t] + w[t & 15];
+        }
+        out[q] = u32x4{o[0], o[1], o[2], o[3]};
     }
 }
 
@@ -783,11 +834,58 @@ __device__ __forceinline__ void thash_shake_pair(const typename Shake<P::n>::Key
     Hh::from_il(il, out);
 }
 
+// SHAKE256 thash on 16 lanes (Keccak16) over a stream held in LDS as
+// interleaved words: pub_seed || address (PRE words) || M payload words ||
+// pad, in whole rate blocks.  The caller fills the payload; every lane of the
+// row calls these.
+template <class P, int M>
+struct Thash16 {
+    using Hh = Shake<P::n>;
+    static constexpr int NW = P::nw;
+    static constexpr int PRE = NW + 8;
+    static constexpr int T = PRE + M;
+    static constexpr int NB = T / 34 + 1;  // permutations (the pad always fits)
+    static constexpr int kWords = 34 * NB;
+    static_assert(PRE % 2 == 0 && M % 2 == 0, "whole 64-bit lanes");
+
+    // pub_seed and the pad, which stay for every hash of one key
+    __device__ static __forceinline__ void begin(const Keccak16& k, const uint32_t pub[NW],
+                                                 lds_u32* buf) {
+#pragma unroll
+        for (int l = 0; l < NW / 2; l++)
+            buf[2 * l + k.half] = k.split(pub[2 * l], pub[2 * l + 1]);
+        buf[PRE - 2 + k.half] = 0;  // address bytes 24..31
+        // 0x1F at the payload's end, 0x80 at the block's last byte
+        for (int i = T + (threadIdx.x & 15); i < kWords; i += 16)
+            buf[i] = (i == T ? 7u : i == T + 1 ? 3u : 0u) ^ (i == kWords - 1 ? 0x80000000u : 0u);
+    }
+    __device__ static __forceinline__ void address(const Keccak16& k, const Adr& a, lds_u32* buf) {
+#pragma unroll
+        for (int l = 0; l < 3; l++)
+            buf[NW + 2 * l + k.half] = k.split(Hh::aw(a, 2 * l), Hh::aw(a, 2 * l + 1));
+    }
+};
+// the sponge over nb blocks of such a stream
+__device__ __forceinline__ void sponge16(Keccak16& k, const lds_u32* buf, int nb) {
+    k.clear();
+    Keccak16::order();
+#pragma unroll 1
+    for (int b = 0; b < nb; b++) {
+        k.absorb(buf, b);
+        k.permute();
+    }
+}
+
 // FORS public key of request i: T_k over its k roots (fors.cu:142); the
 // roots are read past the caches, as another workgroup may have stored them.
-// PAIR: on a lane pair (both lanes active, the even lane stores).
-template <class P, bool PAIR>
-__device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i) {
+// GROUP: on a lane pair (SHA-256) or 16 lanes (SHAKE256; row: LDS of the row,
+// fors_pk_row words), all active, the first lane stores; else on one lane.
+template <class P>
+__host__ __device__ constexpr int fors_pk_row() {
+    return Keccak16::kLdsWords + Thash16<P, P::k * P::nw>::kWords;
+}
+template <class P, bool GROUP>
+__device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i, lds_u32* row) {
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
     constexpr int NW = P::nw;
@@ -800,9 +898,12 @@ __device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i) {
     const uint32_t* rw = reinterpret_cast<const uint32_t*>(A.fors_roots + (size_t)i * P::k * P::n);
     auto root = [&](int u) { return __builtin_nontemporal_load(rw + u); };
     const int h = threadIdx.x & 1;
+    bool first = true;
     uint32_t out[NW];
+    (void)row;
     if constexpr (P::hash == kSha2) {
-        if constexpr (PAIR) {
+        if constexpr (GROUP) {
+            first = h == 0;
             thash_sha2_pair<NW, KW>(key.mid, adr, [&](int j) {
                 const int u = j + h;
                 return bswap32(root(u < 0 ? 0 : u < KW ? u : KW - 1));
@@ -811,27 +912,41 @@ __device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i) {
             thash_sha2_rd<NW, KW>(key.mid, adr, [&](int u) { return bswap32(root(u)); }, out);
         }
     } else {
-        if constexpr (PAIR) {
-            thash_shake_pair<P, KW>(key, adr, [&](int j) {  // this lane's half of root lane j / 2
-                int l = j >> 1;
-                l = l < 0 ? 0 : l < KW / 2 ? l : KW / 2 - 1;
+        if constexpr (GROUP) {
+            using T16 = Thash16<P, KW>;
+            Keccak16 k;
+            k.init(row);
+            lds_u32* buf = row + Keccak16::kLdsWords;
+            const int p = threadIdx.x & 15;
+            first = p == 0;
+            T16::begin(k, key.pub, buf);
+            T16::address(k, adr, buf);
+            for (int l = p; l < KW / 2; l += 16) {
                 uint32_t e, o;
                 il_to(root(2 * l), root(2 * l + 1), e, o);
-                return h ? o : e;
-            }, out);
+                buf[T16::PRE + 2 * l] = e;
+                buf[T16::PRE + 2 * l + 1] = o;
+            }
+            sponge16(k, buf, T16::NB);
+#pragma unroll
+            for (int l = 0; l < NW / 2; l++) k.lane(l, out[2 * l], out[2 * l + 1]);
         } else {
             thash_shake_rd<P, KW, false>(key, adr, root, out);
         }
     }
-    if (!PAIR || h == 0) store_val<P::hash, NW>(A.fors_pk + (size_t)i * P::n, out);
+    if (first) store_val<P::hash, NW>(A.fors_pk + (size_t)i * P::n, out);
 }
 
-// FORS public keys of a whole batch, a lane pair per request (large sign
+// FORS public keys of a whole batch, a lane group per request (large sign
 // batches and verify)
 template <class P>
+__host__ __device__ constexpr uint32_t fors_pk_lanes() { return P::hash == kSha2 ? 2 : 16; }
+template <class P>
 __global__ void __launch_bounds__(64) k_fors_pk(BatchArgs A) {
-    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 1;
-    if (i < A.n_req) fors_pk_of<P, true>(A, i);
+    constexpr int RW = P::hash == kSha2 ? 0 : fors_pk_row<P>();
+    __shared__ __align__(16) uint32_t row_s[RW ? 4 * RW : 1];
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / fors_pk_lanes<P>();
+    if (i < A.n_req) fors_pk_of<P, true>(A, i, (lds_u32*)row_s + threadIdx.x / 16 * RW);
 }
 
 // verify: one FORS tree per lane: leaf from the revealed sk, climb with the
@@ -1245,7 +1360,7 @@ __global__ void __launch_bounds__(256) k_wots_gather(BatchArgs A) {
     for (int w = 0; w < NW; w++) reinterpret_cast<uint32_t*>(dst)[w] = v[w];
 }
 
-// The climb of one layer's subtree on a lane pair (compute_root,
+// The climb of one layer's subtree on a lane pair (SHA-256; compute_root,
 // utils.cu:94-135): node (in both lanes) is the WOTS public key's T_len on
 // entry and the layer root on exit; the auth path is in LDS (raw words) and
 // nd is NW words of LDS for the node.
@@ -1254,7 +1369,6 @@ __device__ __forceinline__ void climb_pair(const typename HashT<P>::Key& key, ui
                                            uint64_t tree, uint32_t leaf, const uint32_t* auth,
                                            uint32_t* nd, uint32_t node[P::nw]) {
     constexpr int NW = P::nw;
-    constexpr bool SHA2 = P::hash == kSha2;
     const int half = threadIdx.x & 1;
     uint32_t li = leaf;
     Adr ha = adr_make(layer, tree, kHashTree);
@@ -1266,28 +1380,17 @@ __device__ __forceinline__ void climb_pair(const typename HashT<P>::Key& key, ui
         // payload node || auth or auth || node from LDS (nd: the node as raw
         // words, like the auth path)
 #pragma unroll
-        for (int w = 0; w < NW; w++) nd[w] = SHA2 ? bswap32(node[w]) : node[w];
+        for (int w = 0; w < NW; w++) nd[w] = bswap32(node[w]);
         const uint32_t* ap = auth + h * NW;
         auto word = [&](int i) {  // payload word i (raw)
             const uint32_t* src = (i < NW) == right ? ap : nd;
             return src[i < NW ? i : i - NW];
         };
-        if constexpr (SHA2) {
-            thash_sha2_pair<NW, 2 * NW>(key.mid, ha, [&](int j) {
-                int i = j + half;
-                i = i < 0 ? 0 : i < 2 * NW ? i : 2 * NW - 1;
-                return bswap32(word(i));
-            }, node);
-        } else {
-            // this lane's interleaved half of payload lane j / 2
-            thash_shake_pair<P, 2 * NW>(key, ha, [&](int j) {
-                int l = j >> 1;
-                l = l < 0 ? 0 : l < NW ? l : NW - 1;
-                uint32_t e, o;
-                il_to(word(2 * l), word(2 * l + 1), e, o);
-                return half ? o : e;
-            }, node);
-        }
+        thash_sha2_pair<NW, 2 * NW>(key.mid, ha, [&](int j) {
+            int i = j + half;
+            i = i < 0 ? 0 : i < 2 * NW ? i : 2 * NW - 1;
+            return bswap32(word(i));
+        }, node);
     }
 }
 
@@ -1303,10 +1406,9 @@ struct PkPair {
     }
 };
 
-// Verification of one layer's subtree on a lane pair (both lanes active):
-// T_len over the WOTS public key in LDS (pk: native words for SHA-256,
-// interleaved for SHAKE256), then climb_pair.  node is the layer root, in
-// both lanes.
+// Verification of one layer's subtree on a lane pair (SHA-256, both lanes
+// active): T_len over the WOTS public key in LDS (pk, native words), then
+// climb_pair.  node is the layer root, in both lanes.
 template <class P>
 __device__ __forceinline__ void tlen_climb_pair(const typename HashT<P>::Key& key,
                                                 uint32_t layer, uint64_t tree, uint32_t leaf,
@@ -1317,9 +1419,55 @@ __device__ __forceinline__ void tlen_climb_pair(const typename HashT<P>::Key& ke
     Adr pa = adr_make(layer, tree, kWotsPk);
     adr_keypair<P::th>(pa, leaf);
     const PkPair<P> rpk{pk, (int)(threadIdx.x & 1)};
-    if constexpr (P::hash == kSha2) thash_sha2_pair<NW, TLW>(key.mid, pa, rpk, node);
-    else thash_shake_pair<P, TLW>(key, pa, rpk, node);
+    thash_sha2_pair<NW, TLW>(key.mid, pa, rpk, node);
     climb_pair<P>(key, layer, tree, leaf, auth, nd, node);
+}
+
+// The same for SHAKE256 on a row of 16 lanes (Keccak16), one loop over T_len
+// and the th nodes.  pk: the T_len stream (Thash16<P, len * nw>) with the
+// chain ends as payload; nd: the stream of one node; begin() of both has run.
+// auth: the auth path, interleaved words.  node is the layer root, plain, in
+// every lane.
+template <class P>
+struct Layer16 {
+    using TL = Thash16<P, P::len * P::nw>;
+    using TH = Thash16<P, 2 * P::nw>;
+    static constexpr int NW = P::nw;
+    static_assert(TH::NB == 1 && NW <= 8, "a node is one block");
+
+    __device__ static __forceinline__ void run(Keccak16& k, uint32_t layer, uint64_t tree,
+                                               uint32_t leaf, lds_u32* pk, const lds_u32* auth,
+                                               lds_u32* nd, uint32_t node[NW]) {
+        const int p = threadIdx.x & 15;
+        Adr a = adr_make(layer, tree, kWotsPk);
+        adr_keypair<P::th>(a, leaf);
+        TL::address(k, a, pk);
+        Adr ha = adr_make(layer, tree, kHashTree);
+        uint32_t li = leaf;
+#pragma unroll 1
+        for (int h = 0; h <= P::th; h++) {
+            if (h > 0) {
+                const bool right = li & 1u;  // node is the right child
+                li >>= 1;
+                adr_node(ha, h, li);
+                TH::address(k, ha, nd);
+                lds_u32* own = nd + TH::PRE + (right ? NW : 0);
+                lds_u32* sib = nd + TH::PRE + (right ? 0 : NW);
+                // the node is in row 0 of the columns' owners (p & 7 in 1..5)
+                if (k.col < NW / 2 && (p & 7) >= 1 && (p & 7) <= 5) own[2 * k.col + k.half] = k.s[0];
+                if (p < NW) sib[p] = auth[(h - 1) * NW + p];
+            }
+            sponge16(k, h == 0 ? pk : nd, h == 0 ? TL::NB : 1);
+        }
+#pragma unroll
+        for (int l = 0; l < NW / 2; l++) k.lane(l, node[2 * l], node[2 * l + 1]);
+    }
+};
+
+// words of a WOTS public key in LDS: native, or the whole T_len stream
+template <class P>
+__host__ __device__ constexpr int tlen_words() {
+    return P::hash == kSha2 ? P::len * P::nw : Thash16<P, P::len * P::nw>::kWords;
 }
 
 // verify: the d layers of R = 256 / G requests per workgroup in order
@@ -1332,8 +1480,7 @@ __device__ __forceinline__ void tlen_climb_pair(const typename HashT<P>::Key& ke
 // SHAKE256 chains run bit-interleaved).  The lane pair 2r, 2r + 1 then
 // computes T_len of request r block by block from LDS and climbs its subtree
 // (compute_root, utils.cu:94-135; tlen_climb_pair, or for SHA-256 with n <=
-// 24 the rounds of T_len's payload-only blocks on K + W that waves 1-3
-// computed meanwhile).  The next layer's WOTS signature words and this
+// 24 the rounds of T_len's blocks on K + W that all waves computed before); SHAKE256 does so on 16 lanes per request (Layer16).  The next layer's WOTS signature words and this
 // layer's auth path are fetched into registers while the chains run, so the
 // layer loop waits on no global load.
 template <class P, int G>
@@ -1352,9 +1499,9 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
     constexpr int AW = TH * NW;                  // auth path words per request
     constexpr int MAXA = (R * AW + 255) / 256;   // prefetched auth words per lane
     static_assert(NCH < 4096, "chain ids take 12 bits of an order entry");
-    // SHA-256 with n <= 24: T_len's payload-only blocks take their message
-    // schedules from waves 1-3 (the LDS for n = 32 would not fit)
-    constexpr int MB = (TLW + 5) / 16 - 1;  // payload-only blocks of T_len
+    // SHA-256 with n <= 24: T_len's blocks take their message schedules from
+    // all waves (the LDS for n = 32 would not fit)
+    constexpr int MB = Sha2Pair<NW, TLW>::B;  // blocks of T_len
     constexpr bool PRE = SHA2 && NW <= 6;
     __builtin_amdgcn_s_setprio(2);  // d dependent layers per request: latency-bound
     __shared__ uint32_t key_s[R][8];    // SHA-256 midstate / SHAKE256 pub_seed
@@ -1362,13 +1509,21 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
     __shared__ uint64_t tree_s[R];
     __shared__ uint32_t leaf_s[R];
     __shared__ uint32_t sig_s[R][TLW];  // WOTS signature of the layer, raw words
-    __shared__ uint32_t pk_s[R][TLW];   // chain ends (SHAKE256: interleaved)
-    __shared__ uint32_t auth_s[R][AW];  // auth path of the layer, raw words
-    __shared__ uint32_t node_s[R][NW];  // climb: the node, raw words
-    // K + W of T_len's payload-only blocks: 64-word rows, row (r, b) skewed
-    // by 4 words per request so the pairs' 16-byte reads of one t (one row
-    // per request) fall into distinct bank groups
+    // chain ends: native words, for SHAKE256 the payload of a T_len stream
+    // (Layer16), interleaved
+    constexpr int PKW = tlen_words<P>(), PKO = SHA2 ? 0 : NW + 8;
+    __shared__ uint32_t pk_s[R][PKW];
+    __shared__ uint32_t auth_s[R][AW];  // auth path of the layer, raw / interleaved words
+    // climb: the node, raw words (SHAKE256: the stream of one node)
+    __shared__ uint32_t node_s[R][SHA2 ? NW : 34];
+    // SHAKE256: the rows' sponges
+    __shared__ __align__(16) uint32_t row_s[SHA2 ? 1 : R][Keccak16::kLdsWords];
+    // K + W of T_len's blocks: 64-word rows, row (r, b) skewed by 4 words per
+    // request so the pairs' 16-byte reads of one t (one row per request) fall
+    // into distinct bank groups
     __shared__ __align__(16) uint32_t kw_s[PRE ? R * MB * 64 + 64 : 1];
+    __shared__ __align__(16) uint32_t ones_s[PRE ? kKwOnes : 1];
+    if (PRE && threadIdx.x < kKwOnes) ones_s[threadIdx.x] = 1u;
     auto kw_row = [&](int r, int b) { return &kw_s[(r * MB + b) * 64 + 4 * (r & 15)]; };
     __shared__ uint16_t order_s[NCH];   // rank -> chain id | remaining steps << 12
     __shared__ uint32_t hist_s[16];     // chains per remaining-step count
@@ -1399,6 +1554,18 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
     for (int k = 0; k < MAXW; k++) {
         const int u = tid + 256 * k;
         if (u < nact * TLW) sig_s[u / TLW][u % TLW] = wots_of(u / TLW, 0)[u % TLW];
+    }
+    Keccak16 sponge;
+    if constexpr (!SHA2) {
+        const int r16 = tid >> 4;
+        if (r16 < nact) {
+            const Plan& pl = A.plan[req0 + r16];
+            Key k2;
+            Hh::load_key(pl, k2);
+            sponge.init((lds_u32*)row_s[r16]);
+            Layer16<P>::TL::begin(sponge, k2.pub, (lds_u32*)pk_s[r16]);
+            Layer16<P>::TH::begin(sponge, k2.pub, (lds_u32*)node_s[r16]);
+        }
     }
 
 #pragma unroll 1
@@ -1497,7 +1664,7 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
         while (c < nm) {
             if (s >= (uint32_t)P::w - 1) {  // chain done: park its end, take the next
 #pragma unroll
-                for (int w = 0; w < NW; w++) pk_s[r][j * NW + w] = v[w];
+                for (int w = 0; w < NW; w++) pk_s[r][PKO + j * NW + w] = v[w];
                 c++;
                 if (c < nm) take(c);
                 continue;
@@ -1513,8 +1680,14 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
 #pragma unroll
         for (int k = 0; k < MAXA; k++) {
             const int u = tid + 256 * k;
+            if constexpr (!SHA2) {  // adjacent threads hold the words of one 64-bit lane
+                const uint32_t other = pair_swap(au[k]);
+                const bool odd = tid & 1;
+                au[k] = il_half(odd ? other : au[k], odd ? au[k] : other, tid & 1);
+            }
             if (u < nact * AW) auth_s[u / AW][u % AW] = au[k];
         }
+        __builtin_amdgcn_s_setprio(2);  // the SHAKE256 rounds leave 0
         __syncthreads();  // every chain end parked; this layer's sig_s reads done
 #pragma unroll
         for (int k = 0; k < MAXW; k++) {
@@ -1526,39 +1699,31 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
         // 2 rq + 1 (sha256_compress_pair / keccak_f_il_pair)
         const int rq = tid >> 1;
         if constexpr (PRE) {
-            // SHA-256: waves 1-3 run the message schedules of T_len's
-            // payload-only blocks (they depend on the chain ends only) while
-            // the pairs of wave 0 compress block 0; the pairs then take
-            // K + W of those blocks from LDS
+            // SHA-256: every wave runs message schedules of T_len's blocks
+            // (they depend on the chain ends only); the pairs then take K + W
+            // from LDS.  Consecutive lanes take consecutive requests.
             using SP = Sha2Pair<NW, TLW>;
-            uint32_t st[4];
-            Key k2;
-            uint64_t tree = 0;
-            uint32_t leaf = 0;
-            Adr pa{};
-            const PkPair<P> rpk{&pk_s[rq < R ? rq : 0][0], tid & 1};
+            for (int it = tid; it < nact * MB; it += 256) {
+                const int r = it % nact, b = it / nact;
+                Adr pa = adr_make(layer, tree_s[r], kWotsPk);
+                adr_keypair<TH>(pa, leaf_s[r]);
+                const uint32_t* pk = &pk_s[r][0];
+                sha2_kw_block<NW, TLW>(pa, [&](int i) { return pk[i]; }, b, kw_row(r, b));
+            }
+            __syncthreads();  // K + W of every block in LDS
             if (tid < 2 * nact) {
-                tree = tree_s[rq];
-                leaf = leaf_s[rq];
+                const uint64_t tree = tree_s[rq];
+                const uint32_t leaf = leaf_s[rq];
+                Key k2;
 #pragma unroll
                 for (int i = 0; i < NW; i++) k2.sk[i] = 0;
 #pragma unroll
                 for (int i = 0; i < 8; i++) k2.mid[i] = key_s[rq][i];
-                pa = adr_make(layer, tree, kWotsPk);
-                adr_keypair<TH>(pa, leaf);
+                uint32_t st[4], node[NW];
                 SP::init(k2.mid, st);
-                SP::absorb(st, 0, 1, pa, rpk);
-            }
-            if (tid >= 64) {  // consecutive lanes take consecutive requests
-                for (int it = tid - 64; it < nact * MB; it += 192)
-                    sha2_kw_block(&pk_s[it % nact][0], 1 + it / nact, kw_row(it % nact, it / nact));
-            }
-            __syncthreads();  // K + W of every payload-only block in LDS
-            if (tid < 2 * nact) {
 #pragma unroll 1
-                for (int b = 0; b < MB; b++) sha256_rounds_pair_kw(st, kw_row(rq, b));
-                SP::absorb(st, SP::FT, SP::B, pa, rpk);
-                uint32_t node[NW];
+                for (int b = 0; b < MB; b++)
+                    sha256_rounds_pair_kw(st, (tid & 1) ? &ones_s[0] : kw_row(rq, b));
                 SP::output(st, node);
                 climb_pair<P>(k2, layer, tree, leaf, &auth_s[rq][0], &node_s[rq][0], node);
                 if ((tid & 1) == 0) {
@@ -1568,19 +1733,29 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
                     tree_s[rq] = tree >> TH;
                 }
             }
+        } else if constexpr (!SHA2) {
+            const int r16 = tid >> 4;
+            if (r16 < nact) {
+                const uint64_t tree = tree_s[r16];
+                const uint32_t leaf = leaf_s[r16];
+                uint32_t node[NW];
+                Layer16<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s[r16],
+                                (lds_u32*)auth_s[r16], (lds_u32*)node_s[r16], node);
+                if ((tid & 15) == 0) {
+#pragma unroll
+                    for (int w = 0; w < NW; w++) root_s[r16][w] = node[w];
+                    leaf_s[r16] = (uint32_t)(tree & ((1u << TH) - 1));
+                    tree_s[r16] = tree >> TH;
+                }
+            }
         } else if (tid < 2 * nact) {
             const uint64_t tree = tree_s[rq];
             const uint32_t leaf = leaf_s[rq];
             Key k2;
 #pragma unroll
             for (int i = 0; i < NW; i++) k2.sk[i] = 0;
-            if constexpr (SHA2) {
 #pragma unroll
-                for (int i = 0; i < 8; i++) k2.mid[i] = key_s[rq][i];
-            } else {
-#pragma unroll
-                for (int i = 0; i < NW; i++) k2.pub[i] = key_s[rq][i];
-            }
+            for (int i = 0; i < 8; i++) k2.mid[i] = key_s[rq][i];
             uint32_t node[NW];
             tlen_climb_pair<P>(k2, layer, tree, leaf, &pk_s[rq][0], &auth_s[rq][0], &node_s[rq][0],
                                node);
@@ -1679,7 +1854,8 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A) {
 // (sign.cu:3077-3113): lanes pick each chain's end for the layer's message
 // from the candidates of k_vspec and load the auth path, then lanes 0 and 1
 // run T_len and compute_root (utils.cu:94-135) as a lane pair (SHA-256: with
-// the message schedules of T_len's payload-only blocks from lanes 2..).  The serial
+// the message schedules of T_len's blocks from all lanes; SHAKE256: lanes
+// 0-15, Layer16).  The serial
 // work per layer is T_len + h' nodes instead of the longest chain + T_len +
 // h' nodes.
 template <class P>
@@ -1691,14 +1867,21 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
     constexpr int TH = P::th;
     constexpr int TLW = LEN * NW;
     constexpr int AW = TH * NW;
-    __shared__ uint32_t pk_s[TLW];    // chain ends (SHAKE256: interleaved)
-    __shared__ uint32_t auth_s[AW];   // auth path, raw words
+    constexpr bool SHA2 = P::hash == kSha2;
+    // as in k_vht
+    constexpr int PKO = SHA2 ? 0 : NW + 8;
+    __shared__ uint32_t pk_s[tlen_words<P>()];
+    __shared__ uint32_t auth_s[AW];
     __shared__ uint32_t root_s[NW];
-    __shared__ uint32_t node_s[NW];   // climb: the node, raw words
-    // SHA-256: K + W of T_len's payload-only blocks
-    constexpr int MB = P::hash == kSha2 ? (TLW + 5) / 16 - 1 : 1;
-    static_assert(MB <= 62, "one lane per block");
-    __shared__ uint32_t kw_s[MB][64];
+    __shared__ uint32_t node_s[SHA2 ? NW : 34];
+    __shared__ __align__(16) uint32_t row_s[SHA2 ? 1 : Keccak16::kLdsWords];
+    // SHA-256: K + W of T_len's blocks, 68-word rows (the lanes' 16-byte
+    // writes fall into distinct banks)
+    constexpr int MB = SHA2 ? Sha2Pair<NW, TLW>::B : 1;
+    static_assert(MB <= 64, "one lane per block");
+    __shared__ __align__(16) uint32_t kw_s[SHA2 ? MB : 1][68];
+    __shared__ __align__(16) uint32_t ones_s[SHA2 ? kKwOnes : 1];
+    if (SHA2) ones_s[threadIdx.x] = 1u;
     const int tid = threadIdx.x;
     const uint32_t req = blockIdx.x;  // grid = n_req
     const Plan& pl = A.plan[req];
@@ -1709,6 +1892,16 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
         load_val<P::hash, NW>(A.fors_pk + (size_t)req * P::n, fp);
 #pragma unroll
         for (int w = 0; w < NW; w++) root_s[w] = fp[w];
+    }
+    Keccak16 sponge;
+    if constexpr (!SHA2) {
+        if (tid < 16) {
+            Key key;
+            Hh::load_key(pl, key);
+            sponge.init((lds_u32*)row_s);
+            Layer16<P>::TL::begin(sponge, key.pub, (lds_u32*)pk_s);
+            Layer16<P>::TH::begin(sponge, key.pub, (lds_u32*)node_s);
+        }
     }
     uint64_t tree = pl.tree;
     uint32_t leaf = pl.leaf;
@@ -1723,38 +1916,37 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
         for (int j = tid; j < LEN; j += 64) {
             const uint32_t d = chain_len<P>(msg, j);
 #pragma unroll
-            for (int w = 0; w < NW; w++) pk_s[j * NW + w] = lc[((size_t)j * 16 + d) * NW + w];
+            for (int w = 0; w < NW; w++) pk_s[PKO + j * NW + w] = lc[((size_t)j * 16 + d) * NW + w];
         }
         const uint32_t* auth = reinterpret_cast<const uint32_t*>(
             sig + P::n + P::fors_bytes + (size_t)layer * P::layer_bytes + P::wots_bytes);
-        for (int u = tid; u < AW; u += 64) auth_s[u] = auth[u];
+        for (int u = tid; u < AW; u += 64)
+            auth_s[u] = SHA2 ? auth[u] : il_half(auth[u & ~1], auth[u | 1], u & 1);
         __syncthreads();
         uint32_t node[NW];
         if constexpr (P::hash == kSha2) {
-            // lanes 2.. compute K + W of T_len's payload-only blocks (one
-            // pass for all of them), then the pair runs only their rounds
-            if (tid >= 2 && tid < 2 + MB) sha2_kw_block(pk_s, tid - 1, kw_s[tid - 2]);
+            // every lane computes K + W of one of T_len's blocks, then the
+            // pair 0, 1 runs only their rounds
+            Adr pa = adr_make(layer, tree, kWotsPk);
+            adr_keypair<TH>(pa, leaf);
+            if (tid < MB)
+                sha2_kw_block<NW, TLW>(pa, [&](int i) { return pk_s[i]; }, tid, kw_s[tid]);
             __syncthreads();
             if (tid < 2) {  // T_len and the climb on the lane pair 0, 1
                 using SP = Sha2Pair<NW, TLW>;
                 Key key;
                 Hh::load_key(pl, key);
-                Adr pa = adr_make(layer, tree, kWotsPk);
-                adr_keypair<TH>(pa, leaf);
-                const PkPair<P> rpk{pk_s, tid};
                 uint32_t st[4];
                 SP::init(key.mid, st);
-                SP::absorb(st, 0, 1, pa, rpk);
 #pragma unroll 1
-                for (int b = 0; b < MB; b++) sha256_rounds_pair_kw(st, kw_s[b]);
-                SP::absorb(st, SP::FT, SP::B, pa, rpk);
+                for (int b = 0; b < MB; b++)
+                    sha256_rounds_pair_kw(st, tid ? &ones_s[0] : &kw_s[b][0]);
                 SP::output(st, node);
                 climb_pair<P>(key, layer, tree, leaf, auth_s, node_s, node);
             }
-        } else if (tid < 2) {  // T_len and the climb on the lane pair 0, 1
-            Key key;
-            Hh::load_key(pl, key);
-            tlen_climb_pair<P>(key, layer, tree, leaf, pk_s, auth_s, node_s, node);
+        } else if (tid < 16) {  // T_len and the climb on lanes 0-15
+            Layer16<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s, (lds_u32*)auth_s,
+                            (lds_u32*)node_s, node);
         }
         if (tid == 0) {
 #pragma unroll
