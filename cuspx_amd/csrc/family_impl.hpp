@@ -68,7 +68,7 @@ struct FamilyImpl {
                            dim3(256), 0, s, A);
         prof_mark(s, "k_ht");
         if (!A.fors_count) {
-            hipLaunchKernelGGL((k_fors_pk<P>), dim3(cdiv((uint64_t)fors_pk_lanes<P>() * n, 64)), dim3(64), 0, s, A);
+            launch_fors_pk<P>(A, n, s);
             prof_mark(s, "k_fors_pk");
         }
         hipLaunchKernelGGL((k_wots_gather<P>), dim3(cdiv((uint64_t)n * P::d * P::len, 256)),

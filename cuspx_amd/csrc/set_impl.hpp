@@ -20,8 +20,9 @@ struct Layout {
     // The split of a sign / keygen batch over `trees` subtrees: a tuned value
     // when the tuning table has one, else doubled while the launch would
     // still fill less than half the chip.  k_ht runs a lane per WOTS leaf at
-    // 1 and a lane pair per leaf from 2 on (the chains take a lane each
-    // whatever the split); mixed batches go to the family kernel up to 2.
+    // 1, a lane pair at 2 and 4 and 16 lanes at 8 and 16 (the chains take a
+    // lane each whatever the split); mixed batches go to the family kernel up
+    // to 2.
     static constexpr int max_split() { return 16; }
     static int split(int pid, int op, uint32_t trees) {
         const int t = tuned_split(pid, op, trees);
@@ -70,7 +71,7 @@ struct Layout {
         return HtShape<P, S>::PARTS > 1 ? trees * HtShape<P, S>::PARTS
                                         : cdiv(trees, HtShape<P, S>::TPW);
     }
-    // workspace room for split subtrees (k_ht uses up to 4 parts) and for the
+    // workspace room for split subtrees (part roots) and for the
     // chain ends' columns, whole workgroups of leaves: the sizes that callers
     // with a fixed scratch area have had for their batch limits
     static constexpr int max_parts() { return L * 16 > 1024 ? L * 16 / 256 : 1; }
@@ -79,7 +80,7 @@ struct Layout {
         constexpr uint64_t tpw = lanes < 256 ? 256 / lanes : 1;
         return (trees + tpw - 1) / tpw * tpw * L;
     }
-    static_assert(max_parts() >= HtShape<P, 2>::PARTS, "part roots fit");
+    static_assert(max_parts() >= HtShape<P, 16>::PARTS, "part roots fit");
     static uint64_t bytes(int pid, uint32_t n, int op) {
         uint64_t b = al((uint64_t)n * sizeof(Plan));
         b += al((uint64_t)n * P::k * P::n);   // fors roots
@@ -173,8 +174,11 @@ struct SetImpl {
         if (S == 1)
             hipLaunchKernelGGL((k_ht<P, MODE, 1>), dim3(Lay::template ht_blocks<1>(trees)),
                                dim3(256), 0, s, A);
-        else
+        else if (S <= 4)
             hipLaunchKernelGGL((k_ht<P, MODE, 2>), dim3(Lay::template ht_blocks<2>(trees)),
+                               dim3(256), 0, s, A);
+        else
+            hipLaunchKernelGGL((k_ht<P, MODE, 16>), dim3(Lay::template ht_blocks<16>(trees)),
                                dim3(256), 0, s, A);
     }
     template <int FJ>
@@ -182,9 +186,18 @@ struct SetImpl {
         return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ));
     }
 
+    // workgroups of k_vht up to which each has a CU to itself
+    static constexpr uint32_t kVhtAlone = 256;
     template <int G>
     static void launch_vht(const BatchArgs& A, uint32_t n, hipStream_t s) {
-        hipLaunchKernelGGL((k_vht<P, G>), dim3(cdiv(n, 256 / G)), dim3(256), 0, s, A);
+        const uint32_t wgs = cdiv(n, 256 / G);
+        if constexpr (P::hash == kSha2 && G <= 32) {  // wider groups only serve small batches
+            if (wgs > kVhtAlone) {
+                hipLaunchKernelGGL((k_vht<P, G, true>), dim3(wgs), dim3(256), 0, s, A);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_vht<P, G, false>), dim3(wgs), dim3(256), 0, s, A);
     }
     static int sign(const DevBatch& b, hipStream_t s) {
         BatchArgs A{};
@@ -223,7 +236,7 @@ struct SetImpl {
             prof_mark(s, "k_chains");
         }
         if (!A.fors_count) {
-            hipLaunchKernelGGL((k_fors_pk<P>), dim3(cdiv((uint64_t)fors_pk_lanes<P>() * n, 64)), dim3(64), 0, s, A);
+            launch_fors_pk<P>(A, n, s);
             prof_mark(s, "k_fors_pk");
         }
         launch_ht<0>(A, n * P::d, S, s);
@@ -257,7 +270,7 @@ struct SetImpl {
         prof_mark(s, "k_vprep");
         hipLaunchKernelGGL((k_vfors<P>), dim3(cdiv((uint64_t)n * P::k, 64)), dim3(64), 0, s, A);
         prof_mark(s, "k_vfors");
-        hipLaunchKernelGGL((k_fors_pk<P>), dim3(cdiv((uint64_t)fors_pk_lanes<P>() * n, 64)), dim3(64), 0, s, A);
+        launch_fors_pk<P>(A, n, s);
         prof_mark(s, "k_fors_pk");
         if (G == 1) {
             hipLaunchKernelGGL((k_vspec<P>), dim3(cdiv((uint64_t)n * P::d * P::len * 8, 256)),

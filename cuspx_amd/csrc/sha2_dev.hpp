@@ -453,7 +453,8 @@ __device__ __forceinline__ void sha256_rounds_pair_kw(uint32_t s[4], KW kw) {
         if (i == 1) nw = lane_sel(m, a_od, nw);
         // pre[i+1] | T1[i-1]; past the even lane's last round only the odd
         // lane's is used, whose kw is 1 throughout
-        const uint32_t y = c0[i + 1 < 64 ? (i + 1) & 15 : 15] + pair_swap(nwp);
+        uint32_t y = c0[i + 1 < 64 ? (i + 1) & 15 : 15] + pair_swap(nwp);
+        asm("" : "+v"(y));  // else (q2 ^ m), mov_dpp and v_add3 come out: one more
         x = (q2 ^ m) + y;
         q3 = q2;
         q2 = q1;

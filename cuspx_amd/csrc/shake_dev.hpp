@@ -545,16 +545,20 @@ struct Keccak16Tab {
                 const int h2 = h ^ (r & 1);  // odd rotations swap the halves
                 rot[p][y] = (uint8_t)((32 - n) & 31);
                 // column y, row 2x + 3y; the repeated columns write aside
-                wr[p][y] = (uint8_t)(owner ? (h2 * 5 + y) * 8 + (2 * x + 3 * y) % 5 : 80 + p);
+                wr[p][y] = (uint8_t)(owner ? (h2 * 5 + y) * 8 + 4 * h2 + (2 * x + 3 * y) % 5 : 84 + p);
             }
-            for (int k = 0; k < 3; k++) rd[p][k] = (uint8_t)((h * 5 + (x + k) % 5) * 8);
+            for (int k = 0; k < 3; k++) rd[p][k] = (uint8_t)((h * 5 + (x + k) % 5) * 8 + 4 * h);
         }
     }
 };
 __constant__ Keccak16Tab kKeccak16 = Keccak16Tab();
 
 struct Keccak16 {
-    static constexpr int kLdsWords = 96;  // per row of 16 lanes, 16-byte aligned
+    // per row of 16 lanes, 16-byte aligned.  Columns are 8 words apart, the odd
+    // halves 4 words further, and rows an odd multiple of 16 words, so that
+    // the four rows of a wave touch different banks.
+    static constexpr int kLdsWords = 112;
+    static constexpr int row_words(int w) { return ((w + 15) / 16 | 1) * 16; }
     typedef uint32_t __attribute__((address_space(3))) lds_word;
     typedef uint32_t v4 __attribute__((ext_vector_type(4)));
     typedef v4 __attribute__((address_space(3))) lds_v4;
@@ -786,7 +790,7 @@ struct Shake {
     // this one permutes) into LDS, from where every lane takes its halves.
     // The output is in every lane.
     static constexpr int kStage = 36;  // LDS words of one staged block
-    static constexpr int kRowWords = Keccak16::kLdsWords + kStage;
+    static constexpr int kRowWords = Keccak16::row_words(Keccak16::kLdsWords + kStage);
     template <int NPRE, int OUTB>
     __device__ static __forceinline__ void stream_msg(Keccak16& k, const uint32_t pre[NPRE], const uint8_t* m,
                                       uint32_t mlen, uint8_t out[OUTB]) {

@@ -32,6 +32,8 @@
 
 namespace spx {
 
+__host__ __device__ constexpr int max_int(int a, int b) { return a > b ? a : b; }
+
 template <class P>
 using HashT = typename std::conditional<P::hash == kSha2, Sha2<P::n>, Shake<P::n>>::type;
 
@@ -113,6 +115,12 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
 // workgroups after those: each takes long requests in turn and runs one with
 // both waves (Sha2::stream_msg_long), the schedules of its message-only blocks
 // computed by wave 1 ahead of wave 0's rounds.
+//
+// Lanes past the last request repeat it and store nothing, here and in the
+// other kernels whose time is one wave's: a wave with less than all its
+// lanes active has been slower by up to a third, and four such waves on one CU
+// by up to 3.5 times, changing from launch to launch (T_len's rounds on a
+// pair: 2.9k cycles a block with all lanes active, 2.9-10k with two of 16).
 template <class P>
 __host__ __device__ constexpr uint32_t prep_lanes() { return P::hash == kSha2 ? 2 : 16; }
 constexpr uint32_t kPrepWg = 128;
@@ -207,9 +215,10 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
         return;
     }
     constexpr uint32_t PL = prep_lanes<P>();
-    const uint32_t i = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
-    if (i >= A.n_req) return;
-    const bool first = threadIdx.x % PL == 0;
+    const uint32_t i0 = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
+    if ((blockIdx.x * kPrepWg + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
+    const uint32_t i = i0 < A.n_req ? i0 : A.n_req - 1;
+    const bool first = i0 < A.n_req && threadIdx.x % PL == 0;
     if (A.ht_count && first) {
 #pragma unroll 1
         for (int layer = 0; layer < P::d; layer++) A.ht_count[(size_t)i * P::d + layer] = 0;
@@ -283,9 +292,11 @@ __global__ void __launch_bounds__(kPrepWg) k_vprep(BatchArgs A) {
         return;
     }
     constexpr uint32_t PL = prep_lanes<P>();
-    const uint32_t i = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
-    if (i >= A.n_req || prep_is_long(A, i)) return;
-    const bool first = threadIdx.x % PL == 0;
+    const uint32_t i0 = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
+    if ((blockIdx.x * kPrepWg + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
+    const uint32_t i = i0 < A.n_req ? i0 : A.n_req - 1;
+    const bool first = i0 < A.n_req && threadIdx.x % PL == 0;
+    if (prep_is_long(A, i)) return;
     if constexpr (P::hash == kShake) {
         constexpr int RW = HashT<P>::kRowWords;
         __shared__ __align__(16) uint32_t row_s[kPrepWg / PL * RW];
@@ -356,24 +367,25 @@ __global__ void __launch_bounds__(64) k_kprep(BatchArgs A) {
 
 // ------------------------------------------------------------------ FORS
 
-template <class P, bool GROUP>
-__device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i, lds_u32* row);
+template <class P>
+__device__ __forceinline__ void fors_pk_wave(const BatchArgs& A, uint32_t i, lds_u32* lds);
+template <class P>
+__host__ __device__ constexpr int fors_pk_wave_words();
 
 // a FORS root of request req is stored.  Small sign batches (fors_count
-// set): count it, and the lane that stores the request's last root computes
-// the FORS public key, so T_k overlaps the hypertree tiles instead of taking
-// a launch of its own (the k roots of one request come from several
-// workgroups; every counter was zeroed by the prep kernel).  Large batches
-// launch k_fors_pk instead: there the per-tile release fences (an L2
-// write-back each) cost more than the launch.
+// set): count it; true for the request's last root.  The wave that stored it
+// then computes the FORS public key (fors_pk_wave), so T_k overlaps the
+// hypertree chains instead of taking a launch of its own (the k roots of one
+// request come from several workgroups; every counter was zeroed by the prep
+// kernel).  Large batches launch k_fors_pk instead: there the per-tile
+// release fences (an L2 write-back each) cost more than the launch.
 template <class P>
-__device__ __forceinline__ void fors_root_done(const BatchArgs& A, uint32_t req) {
-    if (!A.fors_count) return;
+__device__ __forceinline__ bool fors_root_done(const BatchArgs& A, uint32_t req) {
+    if (!A.fors_count) return false;
     __threadfence();  // release this root before counting it
-    if (atomicAdd(&A.fors_count[req], 1u) == (uint32_t)P::k - 1) {
-        __threadfence();  // acquire: every root of the request is visible
-        fors_pk_of<P, false>(A, req, nullptr);
-    }
+    const bool last = atomicAdd(&A.fors_count[req], 1u) == (uint32_t)P::k - 1;
+    if (last) __threadfence();  // acquire: every root of the request is visible
+    return last;
 }
 
 // LDS words a FORS tile of set P uses (two levels of 256 nodes)
@@ -456,10 +468,13 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
     for (int l = 1; l <= LOGL; l++) {
         __syncthreads();
         const int src = (l - 1) & 1, dst = l & 1;
-        if (tid < (WG >> l)) {
-            const uint32_t tau = tid >> (LOGL - l);
-            const uint32_t x = tid & ((L >> l) - 1);
+        // whole waves: lanes past the level's nodes repeat them
+        if (tid < max_int(WG >> l, 64)) {
+            const int i = tid & ((WG >> l) - 1);
+            const uint32_t tau = i >> (LOGL - l);
+            const uint32_t x = i & ((L >> l) - 1);
             const uint32_t g2 = blk * TPW + tau;
+            bool last = false;  // this lane stored its request's last root
             const bool act2 = g2 < A.n_req * P::k;
             const uint32_t req2 = act2 ? g2 / P::k : 0, t2 = act2 ? g2 % P::k : 0;
             const Plan& p2 = A.plan[req2];
@@ -468,17 +483,17 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
             uint32_t lft[NW], rgt[NW], out[NW];
 #pragma unroll
             for (int w = 0; w < NW; w++) {
-                lft[w] = lds[src][2 * tid][w];
-                rgt[w] = lds[src][2 * tid + 1][w];
+                lft[w] = lds[src][2 * i][w];
+                rgt[w] = lds[src][2 * i + 1][w];
             }
             const uint32_t hgt = J + l;
             Adr a2 = adr_make(0, p2.tree, kForsTree);
             adr_keypair<P::th>(a2, p2.leaf);
             adr_node(a2, hgt, ((t2 << P::a) >> hgt) + x);
             Hh::H(k2, a2, lft, rgt, out);
+            if (act2 && tid == i) {
 #pragma unroll
-            for (int w = 0; w < NW; w++) lds[dst][tid][w] = out[w];
-            if (act2) {
+                for (int w = 0; w < NW; w++) lds[dst][i][w] = out[w];
                 uint8_t* rec2 =
                     A.sig + (size_t)req2 * A.sig_stride + P::n + (size_t)t2 * (P::a + 1) * P::n;
                 const uint32_t tg = p2.fors_idx[t2];
@@ -486,8 +501,16 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
                     store_val<P::hash, NW>(rec2 + P::n + (size_t)hgt * P::n, out);
                 if (hgt == (uint32_t)P::a) {
                     store_val<P::hash, NW>(A.fors_roots + ((size_t)req2 * P::k + t2) * P::n, out);
-                    fors_root_done<P>(A, req2);
+                    last = fors_root_done<P>(A, req2);
                 }
+            }
+            if (l == LOGL) {
+                // wave 0 alone is here (TPW <= 64): the tile's LDS is free
+                static_assert(TPW <= 64 && fors_pk_wave_words<P>() <= fors_lds_words<P>(), "");
+#pragma unroll 1
+                for (uint64_t m = __ballot(last); m; m &= m - 1)
+                    fors_pk_wave<P>(A, __shfl((int)req2, __ffsll((unsigned long long)m) - 1),
+                                    (lds_u32*)smem);
             }
         }
     }
@@ -495,7 +518,7 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
 
 template <class P, int J>
 __global__ void __launch_bounds__(256) k_fors(BatchArgs A) {
-    __shared__ uint32_t smem[fors_lds_words<P>()];
+    __shared__ __align__(16) uint32_t smem[fors_lds_words<P>()];
     fors_tile<P, J>(A, blockIdx.x, smem);
 }
 
@@ -654,7 +677,7 @@ __device__ __forceinline__ void thash_sha2_pair(const uint32_t mid[8], const Adr
 // pair that compresses (sha256_rounds_pair_kw).  rd(i): payload word i.
 // kw: 16-byte aligned LDS.
 template <int NW, int M, class Rd>
-__device__ __forceinline__ void sha2_kw_block(const Adr& a, const Rd& rd, int b, uint32_t* kw) {
+__device__ __forceinline__ void sha2_kw_block(const Adr& a, const Rd& rd, int b, lds_u32* kw) {
     using SP = Sha2Pair<NW, M>;
     uint32_t w[16], x[17];
     const int base = 16 * b - 6;
@@ -675,7 +698,7 @@ __device__ __forceinline__ void sha2_kw_block(const Adr& a, const Rd& rd, int b,
         }
         w[i] = y;
     }
-    u32x4* out = reinterpret_cast<u32x4*>(kw);
+    lds_u32x4* out = (lds_u32x4*)kw;
 #pragma unroll
     for (int q = 0; q < 16; q++) {
         uint32_t o[4];
@@ -876,77 +899,133 @@ __device__ __forceinline__ void sponge16(Keccak16& k, const lds_u32* buf, int nb
     }
 }
 
-// FORS public key of request i: T_k over its k roots (fors.cu:142); the
-// roots are read past the caches, as another workgroup may have stored them.
-// GROUP: on a lane pair (SHA-256) or 16 lanes (SHAKE256; row: LDS of the row,
-// fors_pk_row words), all active, the first lane stores; else on one lane.
+// words of a WOTS public key in LDS: native, or the whole T_len stream
 template <class P>
-__host__ __device__ constexpr int fors_pk_row() {
-    return Keccak16::kLdsWords + Thash16<P, P::k * P::nw>::kWords;
-}
-template <class P, bool GROUP>
-__device__ __forceinline__ void fors_pk_of(const BatchArgs& A, uint32_t i, lds_u32* row) {
-    using Hh = HashT<P>;
-    using Key = typename Hh::Key;
-    constexpr int NW = P::nw;
-    constexpr int KW = P::k * NW;
-    const Plan& pl = A.plan[i];
-    Key key;
-    Hh::load_key(pl, key);
-    Adr adr = adr_make(0, pl.tree, kForsPk);
-    adr_keypair<P::th>(adr, pl.leaf);
-    const uint32_t* rw = reinterpret_cast<const uint32_t*>(A.fors_roots + (size_t)i * P::k * P::n);
-    auto root = [&](int u) { return __builtin_nontemporal_load(rw + u); };
-    const int h = threadIdx.x & 1;
-    bool first = true;
-    uint32_t out[NW];
-    (void)row;
-    if constexpr (P::hash == kSha2) {
-        if constexpr (GROUP) {
-            first = h == 0;
-            thash_sha2_pair<NW, KW>(key.mid, adr, [&](int j) {
-                const int u = j + h;
-                return bswap32(root(u < 0 ? 0 : u < KW ? u : KW - 1));
-            }, out);
-        } else {
-            thash_sha2_rd<NW, KW>(key.mid, adr, [&](int u) { return bswap32(root(u)); }, out);
-        }
-    } else {
-        if constexpr (GROUP) {
-            using T16 = Thash16<P, KW>;
-            Keccak16 k;
-            k.init(row);
-            lds_u32* buf = row + Keccak16::kLdsWords;
-            const int p = threadIdx.x & 15;
-            first = p == 0;
-            T16::begin(k, key.pub, buf);
-            T16::address(k, adr, buf);
-            for (int l = p; l < KW / 2; l += 16) {
-                uint32_t e, o;
-                il_to(root(2 * l), root(2 * l + 1), e, o);
-                buf[T16::PRE + 2 * l] = e;
-                buf[T16::PRE + 2 * l + 1] = o;
-            }
-            sponge16(k, buf, T16::NB);
-#pragma unroll
-            for (int l = 0; l < NW / 2; l++) k.lane(l, out[2 * l], out[2 * l + 1]);
-        } else {
-            thash_shake_rd<P, KW, false>(key, adr, root, out);
-        }
-    }
-    if (first) store_val<P::hash, NW>(A.fors_pk + (size_t)i * P::n, out);
+__host__ __device__ constexpr int tlen_words() {
+    return P::hash == kSha2 ? P::len * P::nw : Thash16<P, P::len * P::nw>::kWords;
 }
 
-// FORS public keys of a whole batch, a lane group per request (large sign
-// batches and verify)
+// FORS public key of request i: T_k over its k roots (fors.cu:142); the
+// roots are read past the caches, as another workgroup may have stored them.
+template <class P>
+__device__ __forceinline__ uint32_t fors_root_word(const BatchArgs& A, uint32_t i, int u) {
+    return __builtin_nontemporal_load(
+        reinterpret_cast<const uint32_t*>(A.fors_roots + (size_t)i * P::k * P::n) + u);
+}
+template <class P>
+__device__ __forceinline__ Adr fors_pk_adr(const Plan& pl) {
+    Adr adr = adr_make(0, pl.tree, kForsPk);
+    adr_keypair<P::th>(adr, pl.leaf);
+    return adr;
+}
+// SHAKE256 on 16 lanes; row: fors_pk_row words of LDS
+template <class P>
+__host__ __device__ constexpr int fors_pk_row() {
+    return Keccak16::row_words(Keccak16::kLdsWords + Thash16<P, P::k * P::nw>::kWords);
+}
+template <class P>
+__device__ __forceinline__ void fors_pk_16(const BatchArgs& A, uint32_t i, lds_u32* row,
+                                           uint32_t out[P::nw]) {
+    constexpr int NW = P::nw, KW = P::k * NW;
+    using T16 = Thash16<P, KW>;
+    const Plan& pl = A.plan[i];
+    typename HashT<P>::Key key;
+    HashT<P>::load_key(pl, key);
+    Keccak16 k;
+    k.init(row);
+    lds_u32* buf = row + Keccak16::kLdsWords;
+    T16::begin(k, key.pub, buf);
+    T16::address(k, fors_pk_adr<P>(pl), buf);
+    for (int l = threadIdx.x & 15; l < KW / 2; l += 16) {
+        uint32_t e, o;
+        il_to(fors_root_word<P>(A, i, 2 * l), fors_root_word<P>(A, i, 2 * l + 1), e, o);
+        buf[T16::PRE + 2 * l] = e;
+        buf[T16::PRE + 2 * l + 1] = o;
+    }
+    sponge16(k, buf, T16::NB);
+#pragma unroll
+    for (int l = 0; l < NW / 2; l++) k.lane(l, out[2 * l], out[2 * l + 1]);
+}
+// a whole wave on one request, for latency: SHA-256 with the schedules of
+// T_k's blocks on one lane each, then their rounds on the pairs (all alike);
+// SHAKE256 on the rows of 16 lanes (all alike).  lds: fors_pk_wave_words
+// words of the wave's own.
+template <class P>
+__host__ __device__ constexpr int fors_pk_wave_words() {
+    return P::hash == kSha2 ? Sha2Pair<P::nw, P::k * P::nw>::B * 68 + kKwOnes : fors_pk_row<P>();
+}
+template <class P>
+__device__ __forceinline__ void fors_pk_wave(const BatchArgs& A, uint32_t i, lds_u32* lds) {
+    using Hh = HashT<P>;
+    constexpr int NW = P::nw, KW = P::k * NW;
+    const int lane = threadIdx.x & 63;
+    uint32_t out[NW];
+    if constexpr (P::hash == kSha2) {
+        using SP = Sha2Pair<NW, KW>;
+        const Plan& pl = A.plan[i];
+        typename Hh::Key key;
+        Hh::load_key(pl, key);
+        lds_u32* ones = lds + SP::B * 68;
+        ones[lane] = 1u;
+        if (lane < SP::B)
+            sha2_kw_block<NW, KW>(fors_pk_adr<P>(pl),
+                                  [&](int u) { return bswap32(fors_root_word<P>(A, i, u)); }, lane,
+                                  lds + 68 * lane);
+        Keccak16::order();
+        uint32_t st[4];
+        SP::init(key.mid, st);
+#pragma unroll 1
+        for (int b = 0; b < SP::B; b++)
+            sha256_rounds_pair_kw(st, (lane & 1) ? ones : lds + 68 * b);
+        Keccak16::order();
+        SP::output(st, out);
+    } else {
+        fors_pk_16<P>(A, i, lds, out);
+    }
+    if (lane == 0) store_val<P::hash, NW>(A.fors_pk + (size_t)i * P::n, out);
+}
+
+// FORS public keys of a whole batch (large sign batches and verify): a wave
+// per request up to kForsPkWaves requests, else a lane group (SHA-256: a
+// pair, SHAKE256: 16 lanes).
+constexpr uint32_t kForsPkWaves = 1024;  // a wave per SIMD
 template <class P>
 __host__ __device__ constexpr uint32_t fors_pk_lanes() { return P::hash == kSha2 ? 2 : 16; }
-template <class P>
+template <class P, bool WAVE>
 __global__ void __launch_bounds__(64) k_fors_pk(BatchArgs A) {
-    constexpr int RW = P::hash == kSha2 ? 0 : fors_pk_row<P>();
-    __shared__ __align__(16) uint32_t row_s[RW ? 4 * RW : 1];
-    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / fors_pk_lanes<P>();
-    if (i < A.n_req) fors_pk_of<P, true>(A, i, (lds_u32*)row_s + threadIdx.x / 16 * RW);
+    constexpr int NW = P::nw, KW = P::k * NW;
+    if constexpr (WAVE) {
+        __shared__ __align__(16) uint32_t lds[fors_pk_wave_words<P>()];
+        fors_pk_wave<P>(A, blockIdx.x, (lds_u32*)lds);
+    } else {
+        const uint32_t i0 = (blockIdx.x * blockDim.x + threadIdx.x) / fors_pk_lanes<P>();
+        const uint32_t i = i0 < A.n_req ? i0 : A.n_req - 1;
+        uint32_t out[NW];
+        if constexpr (P::hash == kSha2) {
+            const Plan& pl = A.plan[i];
+            typename HashT<P>::Key key;
+            HashT<P>::load_key(pl, key);
+            const int h = threadIdx.x & 1;
+            thash_sha2_pair<NW, KW>(key.mid, fors_pk_adr<P>(pl), [&](int j) {
+                const int u = j + h;
+                return bswap32(fors_root_word<P>(A, i, u < 0 ? 0 : u < KW ? u : KW - 1));
+            }, out);
+        } else {
+            __shared__ __align__(16) uint32_t row_s[4 * fors_pk_row<P>()];
+            fors_pk_16<P>(A, i, (lds_u32*)row_s + threadIdx.x / 16 * fors_pk_row<P>(), out);
+        }
+        if (i0 == i && threadIdx.x % fors_pk_lanes<P>() == 0)
+            store_val<P::hash, NW>(A.fors_pk + (size_t)i * P::n, out);
+    }
+}
+template <class P>
+inline void launch_fors_pk(const BatchArgs& A, uint32_t n, hipStream_t s) {
+    if (n <= kForsPkWaves)
+        hipLaunchKernelGGL((k_fors_pk<P, true>), dim3(n), dim3(64), 0, s, A);
+    else
+        hipLaunchKernelGGL((k_fors_pk<P, false>),
+                           dim3((uint32_t)(((uint64_t)fors_pk_lanes<P>() * n + 63) / 64)),
+                           dim3(64), 0, s, A);
 }
 
 // verify: one FORS tree per lane: leaf from the revealed sk, climb with the
@@ -956,8 +1035,8 @@ __global__ void __launch_bounds__(64) k_vfors(BatchArgs A) {
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
     constexpr int NW = P::nw;
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= A.n_req * P::k) return;
+    const uint32_t g0 = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t g = g0 < A.n_req * P::k ? g0 : A.n_req * P::k - 1;  // repeated past the end
     const uint32_t req = g / P::k, t = g % P::k;
     const Plan& pl = A.plan[req];
     Key key;
@@ -1045,7 +1124,8 @@ __device__ __forceinline__ void store_raw(uint8_t* p, const uint32_t v[P::nw]) {
 template <class P, int MODE>
 __device__ __forceinline__ void ht_node(const BatchArgs& A, uint32_t g, uint32_t ntrees, int l,
                                         uint32_t x, const uint32_t lft[P::nw],
-                                        const uint32_t rgt[P::nw], uint32_t out[P::nw]) {
+                                        const uint32_t rgt[P::nw], uint32_t out[P::nw],
+                                        bool store) {
     using Hh = HashT<P>;
     constexpr int NW = P::nw;
     constexpr int L = 1 << P::th;
@@ -1064,7 +1144,7 @@ __device__ __forceinline__ void ht_node(const BatchArgs& A, uint32_t g, uint32_t
     Adr ha = adr_make(lay, tree, kHashTree);
     adr_node(ha, l, x);
     Hh::H(key, ha, lft, rgt, out);
-    if (!act) return;
+    if (!act || !store) return;
     if (MODE == 0) {
         uint8_t* a2 = A.sig + (size_t)req * A.sig_stride + P::n + P::fors_bytes +
                       (size_t)lay * P::layer_bytes + P::wots_bytes;
@@ -1104,8 +1184,10 @@ __device__ __forceinline__ void chain_wave(const BatchArgs& A, uint32_t wave) {
     constexpr int L = 1 << P::th;
     const uint32_t ntrees = MODE == 0 ? A.n_req * P::d : A.n_req;
     const uint32_t j = wave % P::len;
-    const uint32_t leaf_g = wave / P::len * 64 + (threadIdx.x & 63u);  // column in tl_buf
-    if (leaf_g >= leaf_count<P>(ntrees)) return;
+    const uint32_t leaf_0 = wave / P::len * 64 + (threadIdx.x & 63u);
+    const uint32_t nleaf = leaf_count<P>(ntrees);
+    const bool own = leaf_0 < nleaf;
+    const uint32_t leaf_g = own ? leaf_0 : nleaf - 1;  // column in tl_buf
     const uint32_t g = leaf_g / L, u = leaf_g % L;  // subtree; leaf index = keypair address
     const uint32_t req = MODE == 0 ? g / P::d : g;
     const uint32_t layer = MODE == 0 ? g % P::d : P::d - 1;
@@ -1119,7 +1201,7 @@ __device__ __forceinline__ void chain_wave(const BatchArgs& A, uint32_t wave) {
         target = layer == 0 ? pl.leaf
                             : (uint32_t)((pl.tree >> ((layer - 1) * P::th)) & (L - 1));
     }
-    const bool capture = MODE == 0 && u == target;
+    const bool capture = MODE == 0 && own && u == target;
     uint8_t* cap = A.cap + (((size_t)req * P::d + layer) * P::len + j) * 16 * P::n;
     Adr wa = adr_make(layer, tree, kWots);
     adr_keypair<P::th>(wa, u);
@@ -1142,8 +1224,10 @@ __device__ __forceinline__ void chain_wave(const BatchArgs& A, uint32_t wave) {
         Hh::chain_step(key, ch, s, v, v);
         if (capture) store_raw<P>(cap + (s + 1) * P::n, v);
     }
+    if (own) {
 #pragma unroll
-    for (int i = 0; i < NW; i++) A.tl_buf[(size_t)(j * NW + i) * A.tl_lanes + leaf_g] = v[i];
+        for (int i = 0; i < NW; i++) A.tl_buf[(size_t)(j * NW + i) * A.tl_lanes + leaf_g] = v[i];
+    }
 }
 
 template <class P, int MODE>
@@ -1157,7 +1241,7 @@ __global__ void __launch_bounds__(256) k_chains(BatchArgs A, uint32_t nwaves) {
 // batches have both in flight together
 template <class P, int J>
 __global__ void __launch_bounds__(256) k_sign_fused(BatchArgs A, uint32_t n_fors, uint32_t nwaves) {
-    __shared__ uint32_t smem[fors_lds_words<P>()];
+    __shared__ __align__(16) uint32_t smem[fors_lds_words<P>()];
     if (blockIdx.x < n_fors) {
         fors_tile<P, J>(A, blockIdx.x, smem);
         return;
@@ -1169,8 +1253,11 @@ __global__ void __launch_bounds__(256) k_sign_fused(BatchArgs A, uint32_t n_fors
 
 // Hypertree subtrees from the parked chain ends: T_len of every leaf, then
 // the Merkle levels in LDS, auth paths and roots.  S lanes per leaf: S = 1
-// the most leaves per wave (large batches), S = 2 a lane pair per leaf, which
-// shares the serial T_len (sha256_compress_pair / keccak_f_il_pair).
+// the most leaves per wave (large batches); S = 2 a lane pair per leaf, which
+// shares the serial T_len (sha256_compress_pair / keccak_f_il_pair); S = 16
+// the shortest T_len (small batches: SHAKE256 on the 16 lanes, Keccak16;
+// SHA-256 with the schedules of 16 blocks at a time on the 16 lanes, then
+// their rounds on the first two).
 //
 // A subtree whose lanes exceed a 256-lane workgroup is split over PARTS
 // workgroups.  Each part reduces its leaves to a part root in LDS; the part
@@ -1197,9 +1284,19 @@ __global__ void __launch_bounds__(256) k_ht(BatchArgs A) {
     constexpr int L = Sh::L, TPW = Sh::TPW, NL = Sh::NL;
     constexpr int PARTS = Sh::PARTS, LP = Sh::LP, LOGP = Sh::LOGP;
     constexpr int LPT = LP * S;  // lanes per subtree in this workgroup
+    constexpr int TLW = P::len * NW;
     __shared__ uint32_t lds[2][Sh::NLDS][NW];  // two levels of nodes
+    // S = 16, per leaf: SHA-256 16 rows of K + W (68 words each and 16 more
+    // per leaf: distinct banks for the lanes' writes and the leaves' reads),
+    // SHAKE256 the row's sponge and T_len stream
+    constexpr int XW = S < 16            ? 0
+                       : P::hash == kSha2 ? 16 * 68 + 16
+                                          : Keccak16::row_words(Keccak16::kLdsWords + tlen_words<P>());
+    __shared__ __align__(16) uint32_t x_s[XW ? NL * XW : 1];
+    __shared__ __align__(16) uint32_t ones_s[XW && P::hash == kSha2 ? kKwOnes : 1];
 
     const int tid = threadIdx.x;
+    if (XW && P::hash == kSha2 && tid < kKwOnes) ones_s[tid] = 1u;
     const uint32_t blk = blockIdx.x;
     const uint32_t part = PARTS > 1 ? blk % PARTS : 0;
     const uint32_t u = part * LP + (tid % LPT) / S;  // leaf index = keypair address
@@ -1225,14 +1322,48 @@ __global__ void __launch_bounds__(256) k_ht(BatchArgs A) {
         // ---- T_len of leaf u (wots_gen_leaf, sign.cu:87-104)
         Adr pa = adr_make(layer, tree, kWotsPk);
         adr_keypair<P::th>(pa, u);
-        constexpr int TLW = P::len * NW;
         auto parked = [&](int w) { return A.tl_buf[(size_t)w * A.tl_lanes + leaf_g]; };
         auto parked2 = [&](int j) {
             const int i = j + q;
             return parked(i < 0 ? 0 : i < TLW ? i : TLW - 1);
         };
         uint32_t node[NW];
-        if constexpr (P::hash == kSha2) {
+        if constexpr (S == 16 && P::hash == kSha2) {
+            using SP = Sha2Pair<NW, TLW>;
+            uint32_t* kw = x_s + slot * XW;
+            uint32_t st[4];
+            SP::init(key.mid, st);
+#pragma unroll 1
+            for (int b0 = 0; b0 < SP::B; b0 += 16) {
+                const int nb = SP::B - b0 < 16 ? SP::B - b0 : 16;
+                if (q < nb) sha2_kw_block<NW, TLW>(pa, parked, b0 + q, (lds_u32*)kw + 68 * q);
+                __syncthreads();
+                // every pair of the leaf's lanes, all alike: with two lanes
+                // of 16 active the same rounds took 1-3.5 times as long from
+                // launch to launch
+#pragma unroll 1
+                for (int b = 0; b < nb; b++)
+                    sha256_rounds_pair_kw(st, (q & 1) ? &ones_s[0] : kw + 68 * b);
+                if (b0 + 16 < SP::B) __syncthreads();
+            }
+            SP::output(st, node);
+        } else if constexpr (S == 16) {
+            using TL = Thash16<P, TLW>;
+            Keccak16 k;
+            k.init((lds_u32*)x_s + slot * XW);
+            lds_u32* buf = (lds_u32*)x_s + slot * XW + Keccak16::kLdsWords;
+            TL::begin(k, key.pub, buf);
+            TL::address(k, pa, buf);
+            uint32_t x[(TLW + 15) / 16];  // one load latency for all
+#pragma unroll
+            for (int i = 0; i < (TLW + 15) / 16; i++) x[i] = parked(16 * i + q < TLW ? 16 * i + q : 0);
+#pragma unroll
+            for (int i = 0; i < (TLW + 15) / 16; i++)
+                if (16 * i + q < TLW) buf[TL::PRE + 16 * i + q] = x[i];
+            sponge16(k, buf, TL::NB);
+#pragma unroll
+            for (int l = 0; l < NW / 2; l++) k.lane(l, node[2 * l], node[2 * l + 1]);
+        } else if constexpr (P::hash == kSha2) {
             if constexpr (S == 2) thash_sha2_pair<NW, TLW>(key.mid, pa, parked2, node);
             else thash_sha2_rd<NW, TLW>(key.mid, pa, parked, node);
         } else {
@@ -1253,19 +1384,23 @@ __global__ void __launch_bounds__(256) k_ht(BatchArgs A) {
     for (int l = 1; l <= LOGP; l++) {
         __syncthreads();
         const int src = (l - 1) & 1, dst = l & 1;
-        if (tid < (NL >> l)) {
-            const uint32_t t2 = tid >> (LOGP - l);
-            const uint32_t x = part * (LP >> l) + (tid & ((LP >> l) - 1));
+        // whole waves: lanes past the level's nodes repeat them
+        if (tid < max_int(NL >> l, 64)) {
+            const int i = tid & ((NL >> l) - 1);
+            const uint32_t t2 = i >> (LOGP - l);
+            const uint32_t x = part * (LP >> l) + (i & ((LP >> l) - 1));
             uint32_t lft[NW], rgt[NW];
 #pragma unroll
             for (int w = 0; w < NW; w++) {
-                lft[w] = lds[src][2 * tid][w];
-                rgt[w] = lds[src][2 * tid + 1][w];
+                lft[w] = lds[src][2 * i][w];
+                rgt[w] = lds[src][2 * i + 1][w];
             }
             uint32_t out[NW];
-            ht_node<P, MODE>(A, (blk / PARTS) * TPW + t2, ntrees, l, x, lft, rgt, out);
+            ht_node<P, MODE>(A, (blk / PARTS) * TPW + t2, ntrees, l, x, lft, rgt, out, tid == i);
+            if (tid == i) {
 #pragma unroll
-            for (int w = 0; w < NW; w++) lds[dst][tid][w] = out[w];
+                for (int w = 0; w < NW; w++) lds[dst][i][w] = out[w];
+            }
         }
     }
     if constexpr (PARTS > 1) {
@@ -1292,23 +1427,24 @@ __global__ void __launch_bounds__(256) k_ht(BatchArgs A) {
             for (int l = LOGP + 1; l <= P::th; l++) {
                 __syncthreads();
                 const int src = (l - 1) & 1, dst = l & 1;
-                if (tid < (L >> l)) {
+                if (tid < 64) {  // at most PARTS / 2 = 16 nodes
+                    const int i = tid & ((L >> l) - 1);
                     uint32_t lft[NW], rgt[NW], out[NW];
 #pragma unroll
                     for (int w = 0; w < NW; w++) {
-                        lft[w] = lds[src][2 * tid][w];
-                        rgt[w] = lds[src][2 * tid + 1][w];
+                        lft[w] = lds[src][2 * i][w];
+                        rgt[w] = lds[src][2 * i + 1][w];
                     }
-                    ht_node<P, MODE>(A, g, ntrees, l, tid, lft, rgt, out);
+                    ht_node<P, MODE>(A, g, ntrees, l, i, lft, rgt, out, tid == i);
+                    if (tid == i) {
 #pragma unroll
-                    for (int w = 0; w < NW; w++) lds[dst][tid][w] = out[w];
+                        for (int w = 0; w < NW; w++) lds[dst][i][w] = out[w];
+                    }
                 }
             }
         }
     }
 }
-
-constexpr int max_int(int a, int b) { return a > b ? a : b; }
 
 // WOTS signatures: lane per (request, layer, chain); the layer signs the FORS
 // public key (layer 0) or the root of the layer below (sign.cu:1970-1989)
@@ -1464,12 +1600,6 @@ struct Layer16 {
     }
 };
 
-// words of a WOTS public key in LDS: native, or the whole T_len stream
-template <class P>
-__host__ __device__ constexpr int tlen_words() {
-    return P::hash == kSha2 ? P::len * P::nw : Thash16<P, P::len * P::nw>::kWords;
-}
-
 // verify: the d layers of R = 256 / G requests per workgroup in order
 // (sign.cu:3077-3113), so G is the mean number of lanes per request.  Per
 // layer the R * len WOTS chains of the workgroup (15 - len_j steps each,
@@ -1483,7 +1613,11 @@ __host__ __device__ constexpr int tlen_words() {
 // 24 the rounds of T_len's blocks on K + W that all waves computed before); SHAKE256 does so on 16 lanes per request (Layer16).  The next layer's WOTS signature words and this
 // layer's auth path are fetched into registers while the chains run, so the
 // layer loop waits on no global load.
-template <class P, int G>
+// PH (SHA-256): chain steps in two-phase rounds, for launches that put two or
+// more workgroups on a CU (SHA2-128f, G = 16: 8192 requests 2.70 -> 2.10 ms,
+// 16384 5.19 -> 4.15); with one wave per SIMD the compiler's order stays
+// ahead (4096 requests 1.51 against 1.77 ms).
+template <class P, int G, bool PH>
 __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
@@ -1555,10 +1689,13 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
         const int u = tid + 256 * k;
         if (u < nact * TLW) sig_s[u / TLW][u % TLW] = wots_of(u / TLW, 0)[u % TLW];
     }
+    // SHAKE256: request of this row of 16 lanes; rows past the last request
+    // repeat their wave's first one (in step with it, on its LDS)
+    const int row0 = tid / 64 * 4;
+    const int r16 = (tid >> 4) < nact ? tid >> 4 : row0;
     Keccak16 sponge;
     if constexpr (!SHA2) {
-        const int r16 = tid >> 4;
-        if (r16 < nact) {
+        if (row0 < nact) {
             const Plan& pl = A.plan[req0 + r16];
             Key k2;
             Hh::load_key(pl, k2);
@@ -1624,11 +1761,12 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
         // walk the chains: one flattened loop, one F site
         int c = 0, r = 0, j = 0;
         uint32_t s = P::w - 1;
-        Key key;
-        Adr wa;
+        Key key{};
+        Adr wa{};
         uint32_t v[NW];
         typename std::conditional<SHA2, int, typename Shake<P::n>::ChainIl>::type ch{};
-        uint32_t pre[SHA2 ? 8 : 1];  // SHA-256: the chain's rounds 0-4 (Sha2::F_prefix)
+        uint32_t pre[SHA2 ? 8 : 1] = {};  // SHA-256: the chain's rounds 0-4 (Sha2::F_prefix)
+        typename Hh::Chain chn{};         // the same for two-phase rounds
 #pragma unroll
         for (int w = 0; w < NW; w++) v[w] = 0;
 #pragma unroll
@@ -1648,7 +1786,8 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
             if constexpr (SHA2) {
 #pragma unroll
                 for (int i = 0; i < 8; i++) key.mid[i] = key_s[r][i];
-                Hh::F_prefix(key, wa, pre);
+                if constexpr (PH) Hh::chain_begin(key, wa, chn);
+                else Hh::F_prefix(key, wa, pre);
             } else {
 #pragma unroll
                 for (int i = 0; i < NW; i++) key.pub[i] = key_s[r][i];
@@ -1659,19 +1798,27 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
                 for (int w = 0; w < NW; w++) v[w] = t[w];
             }
         };
-        if (nm > 0) take(0);
+        bool run = nm > 0;
+        if (run) take(0);
+        // all lanes step until every chain of the wave is done (full waves run
+        // fastest); a lane without one steps on a value that nothing reads
 #pragma unroll 1
-        while (c < nm) {
-            if (s >= (uint32_t)P::w - 1) {  // chain done: park its end, take the next
+        while (true) {
+            while (run && s >= (uint32_t)P::w - 1) {  // chain done: park its end, take the next
 #pragma unroll
                 for (int w = 0; w < NW; w++) pk_s[r][PKO + j * NW + w] = v[w];
                 c++;
-                if (c < nm) take(c);
-                continue;
+                run = c < nm;
+                if (run) take(c);
             }
+            if (!__any(run)) break;
             if constexpr (SHA2) {
-                adr_hash(wa, s);
-                Hh::F_step(key, pre, wa, v, v);
+                if constexpr (PH) {
+                    Hh::chain_step(key, chn, s, v, v);
+                } else {
+                    adr_hash(wa, s);
+                    Hh::F_step(key, pre, wa, v, v);
+                }
             } else {
                 Hh::F_il(ch, s, v, v);
             }
@@ -1687,7 +1834,7 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
             }
             if (u < nact * AW) auth_s[u / AW][u % AW] = au[k];
         }
-        __builtin_amdgcn_s_setprio(2);  // the SHAKE256 rounds leave 0
+        __builtin_amdgcn_s_setprio(2);  // two-phase rounds leave 0
         __syncthreads();  // every chain end parked; this layer's sig_s reads done
 #pragma unroll
         for (int k = 0; k < MAXW; k++) {
@@ -1697,7 +1844,8 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
         if (tid < 16) hist_s[tid] = 0;
         // T_len and the subtree climb of request rq on the lane pair 2 rq,
         // 2 rq + 1 (sha256_compress_pair / keccak_f_il_pair)
-        const int rq = tid >> 1;
+        // (the other pairs of wave 0 repeat a request)
+        const int rq = (tid >> 1) < nact ? tid >> 1 : 0;
         if constexpr (PRE) {
             // SHA-256: every wave runs message schedules of T_len's blocks
             // (they depend on the chain ends only); the pairs then take K + W
@@ -1708,10 +1856,11 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
                 Adr pa = adr_make(layer, tree_s[r], kWotsPk);
                 adr_keypair<TH>(pa, leaf_s[r]);
                 const uint32_t* pk = &pk_s[r][0];
-                sha2_kw_block<NW, TLW>(pa, [&](int i) { return pk[i]; }, b, kw_row(r, b));
+                sha2_kw_block<NW, TLW>(pa, [&](int i) { return pk[i]; }, b,
+                                      (lds_u32*)kw_row(r, b));
             }
             __syncthreads();  // K + W of every block in LDS
-            if (tid < 2 * nact) {
+            if (tid < 64) {
                 const uint64_t tree = tree_s[rq];
                 const uint32_t leaf = leaf_s[rq];
                 Key k2;
@@ -1726,7 +1875,7 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
                     sha256_rounds_pair_kw(st, (tid & 1) ? &ones_s[0] : kw_row(rq, b));
                 SP::output(st, node);
                 climb_pair<P>(k2, layer, tree, leaf, &auth_s[rq][0], &node_s[rq][0], node);
-                if ((tid & 1) == 0) {
+                if (tid < 2 * nact && (tid & 1) == 0) {
 #pragma unroll
                     for (int w = 0; w < NW; w++) root_s[rq][w] = node[w];
                     leaf_s[rq] = (uint32_t)(tree & ((1u << TH) - 1));
@@ -1734,21 +1883,20 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
                 }
             }
         } else if constexpr (!SHA2) {
-            const int r16 = tid >> 4;
-            if (r16 < nact) {
+            if (row0 < nact) {
                 const uint64_t tree = tree_s[r16];
                 const uint32_t leaf = leaf_s[r16];
                 uint32_t node[NW];
                 Layer16<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s[r16],
                                 (lds_u32*)auth_s[r16], (lds_u32*)node_s[r16], node);
-                if ((tid & 15) == 0) {
+                if (tid == 16 * r16) {
 #pragma unroll
                     for (int w = 0; w < NW; w++) root_s[r16][w] = node[w];
                     leaf_s[r16] = (uint32_t)(tree & ((1u << TH) - 1));
                     tree_s[r16] = tree >> TH;
                 }
             }
-        } else if (tid < 2 * nact) {
+        } else if (tid < 64) {
             const uint64_t tree = tree_s[rq];
             const uint32_t leaf = leaf_s[rq];
             Key k2;
@@ -1759,7 +1907,7 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
             uint32_t node[NW];
             tlen_climb_pair<P>(k2, layer, tree, leaf, &pk_s[rq][0], &auth_s[rq][0], &node_s[rq][0],
                                node);
-            if ((tid & 1) == 0) {
+            if (tid < 2 * nact && (tid & 1) == 0) {
 #pragma unroll
                 for (int w = 0; w < NW; w++) root_s[rq][w] = node[w];
                 leaf_s[rq] = (uint32_t)(tree & ((1u << TH) - 1));
@@ -1791,8 +1939,9 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A) {
     using Key = typename Hh::Key;
     constexpr bool SHA2 = P::hash == kSha2;
     constexpr int NW = P::nw;
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (uint64_t)A.n_req * P::d * P::len * 8) return;
+    const uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t ng = (uint64_t)A.n_req * P::d * P::len * 8;
+    const uint64_t g = g0 < ng ? g0 : ng - 1;  // repeated past the end
     const int p = (int)(g & 7);
     const uint64_t c = g >> 3;                       // (req * d + layer) * len + j
     const int j = (int)(c % P::len);
@@ -1812,9 +1961,9 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A) {
     load_val<P::hash, NW>(A.sig + (size_t)req * A.sig_stride + P::n + P::fors_bytes +
                               (size_t)layer * P::layer_bytes + (size_t)j * P::n,
                           sg);
-    typename std::conditional<SHA2, int, typename Shake<P::n>::ChainIl>::type ch{};
+    typename Hh::Chain ch;
+    Hh::chain_begin(key, wa, ch);
     if constexpr (!SHA2) {
-        Hh::chain_il_begin(key, wa, ch);
         uint32_t t[NW];
         Hh::to_il(sg, t);
 #pragma unroll
@@ -1831,12 +1980,7 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A) {
     bool second = false;
 #pragma unroll 1
     for (int it = 0; it < 15; it++) {
-        if constexpr (SHA2) {
-            adr_hash(wa, s);
-            Hh::F(key, wa, v, v);
-        } else {
-            Hh::F_il(ch, s, v, v);
-        }
+        Hh::chain_step(key, ch, s, v, v);
         s++;
         if (s == (uint32_t)P::w - 1) {
             const int d = second ? 15 - p : p;
@@ -1852,10 +1996,10 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A) {
 
 // Speculative verify, part 2: one wave per request walks the d layers
 // (sign.cu:3077-3113): lanes pick each chain's end for the layer's message
-// from the candidates of k_vspec and load the auth path, then lanes 0 and 1
-// run T_len and compute_root (utils.cu:94-135) as a lane pair (SHA-256: with
-// the message schedules of T_len's blocks from all lanes; SHAKE256: lanes
-// 0-15, Layer16).  The serial
+// from the candidates of k_vspec and load the auth path, then run T_len and
+// compute_root (utils.cu:94-135): SHA-256 on lane pairs with the message
+// schedules of T_len's blocks from one lane each, SHAKE256 on rows of 16
+// lanes (Layer16).  The serial
 // work per layer is T_len + h' nodes instead of the longest chain + T_len +
 // h' nodes.
 template <class P>
@@ -1893,15 +2037,13 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
 #pragma unroll
         for (int w = 0; w < NW; w++) root_s[w] = fp[w];
     }
-    Keccak16 sponge;
+    Keccak16 sponge;  // every row of 16 lanes runs the same one in step
     if constexpr (!SHA2) {
-        if (tid < 16) {
-            Key key;
-            Hh::load_key(pl, key);
-            sponge.init((lds_u32*)row_s);
-            Layer16<P>::TL::begin(sponge, key.pub, (lds_u32*)pk_s);
-            Layer16<P>::TH::begin(sponge, key.pub, (lds_u32*)node_s);
-        }
+        Key key;
+        Hh::load_key(pl, key);
+        sponge.init((lds_u32*)row_s);
+        Layer16<P>::TL::begin(sponge, key.pub, (lds_u32*)pk_s);
+        Layer16<P>::TH::begin(sponge, key.pub, (lds_u32*)node_s);
     }
     uint64_t tree = pl.tree;
     uint32_t leaf = pl.leaf;
@@ -1930,21 +2072,20 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
             Adr pa = adr_make(layer, tree, kWotsPk);
             adr_keypair<TH>(pa, leaf);
             if (tid < MB)
-                sha2_kw_block<NW, TLW>(pa, [&](int i) { return pk_s[i]; }, tid, kw_s[tid]);
+                sha2_kw_block<NW, TLW>(pa, [&](int i) { return pk_s[i]; }, tid, (lds_u32*)kw_s[tid]);
             __syncthreads();
-            if (tid < 2) {  // T_len and the climb on the lane pair 0, 1
-                using SP = Sha2Pair<NW, TLW>;
-                Key key;
-                Hh::load_key(pl, key);
-                uint32_t st[4];
-                SP::init(key.mid, st);
+            // T_len and the climb on lane pairs, all alike (k_ht says why)
+            using SP = Sha2Pair<NW, TLW>;
+            Key key;
+            Hh::load_key(pl, key);
+            uint32_t st[4];
+            SP::init(key.mid, st);
 #pragma unroll 1
-                for (int b = 0; b < MB; b++)
-                    sha256_rounds_pair_kw(st, tid ? &ones_s[0] : &kw_s[b][0]);
-                SP::output(st, node);
-                climb_pair<P>(key, layer, tree, leaf, auth_s, node_s, node);
-            }
-        } else if (tid < 16) {  // T_len and the climb on lanes 0-15
+            for (int b = 0; b < MB; b++)
+                sha256_rounds_pair_kw(st, (tid & 1) ? &ones_s[0] : &kw_s[b][0]);
+            SP::output(st, node);
+            climb_pair<P>(key, layer, tree, leaf, auth_s, node_s, node);
+        } else {
             Layer16<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s, (lds_u32*)auth_s,
                             (lds_u32*)node_s, node);
         }
