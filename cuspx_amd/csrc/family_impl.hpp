@@ -57,9 +57,7 @@ struct FamilyImpl {
     }
     template <class P, int J>
     static void fors(const BatchArgs& A, uint32_t n, hipStream_t s) {
-        if (!n) return;
-        hipLaunchKernelGGL((k_fors<P, J>), dim3(cdiv((uint64_t)n * P::k, 256u >> (P::a - J))),
-                           dim3(256), 0, s, A);
+        if (n) launch_fors<P, J>(A, n, s);
     }
     template <class P>
     static void tail(const BatchArgs& A, uint32_t n, hipStream_t s) {

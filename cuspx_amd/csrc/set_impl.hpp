@@ -1,5 +1,5 @@
 // set_impl.hpp -- host-side launch sequences for one parameter set.
-// Each set_<name>.hip instantiates SetImpl<P, J, JB> and registers its SetOps.
+// Each set_<name>.hip instantiates SetImpl<P, J> and registers its SetOps.
 #pragma once
 #include "engine.hpp"
 #include "profile.hpp"
@@ -158,10 +158,22 @@ struct Layout {
 // or fewer for SHA-256 and so issues from 8 waves per SIMD instead of 3-5.
 static constexpr uint32_t kFuseWaves = 8192;
 
-// J: FORS leaves per lane (2^(a-J) lanes per tree) in the tiles of the fused
-// launch (short tiles keep FORS off the critical path); JB: the same in
-// k_fors, where longer tiles spend less on tile set-up and barriers
-template <class P, int J, int JB>
+// J: FORS leaves per lane, 2^J (2^(a-J) lanes per tree).  Short tiles at every
+// size: a tile is a serial run of 3-4 x 2^J hashes, and with the two-phase
+// rounds the longer tiles of before (2^4 to 2^6 leaves) gained 0-4% of k_fors
+// at 4096 requests and cost it up to 2.9 times at 128 (SHA2-256f, 2^6 -> 2^3
+// leaves: 512 requests 1377 -> 982 us, 4096 7.28 -> 7.15 ms; SHA2-128f 128
+// requests, 2^4 -> 2^2: 203 -> 105 us).
+template <class P, int J>
+inline void launch_fors(const BatchArgs& A, uint32_t n, hipStream_t s) {
+    const uint32_t tiles = cdiv((uint64_t)n * P::k, 256u >> (P::a - J));
+    if (A.fors_count)
+        hipLaunchKernelGGL((k_fors<P, J, true>), dim3(tiles), dim3(256), 0, s, A);
+    else
+        hipLaunchKernelGGL((k_fors<P, J, false>), dim3(tiles), dim3(256), 0, s, A);
+}
+
+template <class P, int J>
 struct SetImpl {
     using Lay = Layout<P>;
 
@@ -181,10 +193,7 @@ struct SetImpl {
             hipLaunchKernelGGL((k_ht<P, MODE, 16>), dim3(Lay::template ht_blocks<16>(trees)),
                                dim3(256), 0, s, A);
     }
-    template <int FJ>
-    static uint32_t fors_tiles(uint32_t n) {
-        return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ));
-    }
+    static uint32_t fors_tiles(uint32_t n) { return cdiv((uint64_t)n * P::k, 256u >> (P::a - J)); }
 
     // workgroups of k_vht up to which each has a CU to itself
     static constexpr uint32_t kVhtAlone = 256;
@@ -224,12 +233,12 @@ struct SetImpl {
         // request's last FORS root, inside the FORS tiles)
         const uint32_t nwaves = chain_waves<P>(n * P::d);
         if (nwaves <= kFuseWaves) {
-            const uint32_t nf = fors_tiles<J>(n);
+            const uint32_t nf = fors_tiles(n);
             hipLaunchKernelGGL((k_sign_fused<P, J>), dim3(nf + cdiv(nwaves, 4)), dim3(256), 0, s,
                                A, nf, nwaves);
             prof_mark(s, "k_sign_fused");
         } else {
-            hipLaunchKernelGGL((k_fors<P, JB>), dim3(fors_tiles<JB>(n)), dim3(256), 0, s, A);
+            launch_fors<P, J>(A, n, s);
             prof_mark(s, "k_fors");
             hipLaunchKernelGGL((k_chains<P, 0>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
                                nwaves);
@@ -347,15 +356,15 @@ struct SetImpl {
     }
 };
 
-template <class P, int J, int JB>
-int SetImpl<P, J, JB>::pid_ = -1;
-template <class P, int J, int JB>
-const char* SetImpl<P, J, JB>::set_name_ = "";
+template <class P, int J>
+int SetImpl<P, J>::pid_ = -1;
+template <class P, int J>
+const char* SetImpl<P, J>::set_name_ = "";
 
 }  // namespace spx
 
-#define SPX_REGISTER_SET(SYM, NAME, PID, PARAMS, J, JB)                    \
+#define SPX_REGISTER_SET(SYM, NAME, PID, PARAMS, J)                        \
     extern "C" const spx::SetOps* SYM(void) {                              \
-        static const spx::SetOps o = spx::SetImpl<PARAMS, J, JB>::ops(NAME, PID); \
+        static const spx::SetOps o = spx::SetImpl<PARAMS, J>::ops(NAME, PID); \
         return &o;                                                         \
     }

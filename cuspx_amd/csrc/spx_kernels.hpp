@@ -372,8 +372,7 @@ __device__ __forceinline__ void fors_pk_wave(const BatchArgs& A, uint32_t i, lds
 template <class P>
 __host__ __device__ constexpr int fors_pk_wave_words();
 
-// a FORS root of request req is stored.  Small sign batches (fors_count
-// set): count it; true for the request's last root.  The wave that stored it
+// a FORS root of request req is stored: count it; true for the request's last root.  The wave that stored it
 // then computes the FORS public key (fors_pk_wave), so T_k overlaps the
 // hypertree chains instead of taking a launch of its own (the k roots of one
 // request come from several workgroups; every counter was zeroed by the prep
@@ -381,7 +380,6 @@ __host__ __device__ constexpr int fors_pk_wave_words();
 // release fences (an L2 write-back each) cost more than the launch.
 template <class P>
 __device__ __forceinline__ bool fors_root_done(const BatchArgs& A, uint32_t req) {
-    if (!A.fors_count) return false;
     __threadfence();  // release this root before counting it
     const bool last = atomicAdd(&A.fors_count[req], 1u) == (uint32_t)P::k - 1;
     if (last) __threadfence();  // acquire: every root of the request is visible
@@ -397,7 +395,8 @@ constexpr int fors_lds_words() {
 // sign: FORS trees, L = 2^(a-J) lanes per tree, 2^J leaves per lane; `blk`
 // is the workgroup's tile (TPW trees), so the same body serves the fused
 // signing kernels.  smem: fors_lds_words<P>() words of LDS owned by the kernel
-template <class P, int J>
+// PK: count the roots and run T_k here (fors_count set)
+template <class P, int J, bool PK>
 __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint32_t* smem) {
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
@@ -501,10 +500,10 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
                     store_val<P::hash, NW>(rec2 + P::n + (size_t)hgt * P::n, out);
                 if (hgt == (uint32_t)P::a) {
                     store_val<P::hash, NW>(A.fors_roots + ((size_t)req2 * P::k + t2) * P::n, out);
-                    last = fors_root_done<P>(A, req2);
+                    if constexpr (PK) last = fors_root_done<P>(A, req2);
                 }
             }
-            if (l == LOGL) {
+            if (PK && l == LOGL) {
                 // wave 0 alone is here (TPW <= 64): the tile's LDS is free
                 static_assert(TPW <= 64 && fors_pk_wave_words<P>() <= fors_lds_words<P>(), "");
 #pragma unroll 1
@@ -516,10 +515,10 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
     }
 }
 
-template <class P, int J>
+template <class P, int J, bool PK>
 __global__ void __launch_bounds__(256) k_fors(BatchArgs A) {
     __shared__ __align__(16) uint32_t smem[fors_lds_words<P>()];
-    fors_tile<P, J>(A, blockIdx.x, smem);
+    fors_tile<P, J, PK>(A, blockIdx.x, smem);
 }
 
 // thash (SHA-256) over M payload words after the 22-byte address,
@@ -1243,7 +1242,7 @@ template <class P, int J>
 __global__ void __launch_bounds__(256) k_sign_fused(BatchArgs A, uint32_t n_fors, uint32_t nwaves) {
     __shared__ __align__(16) uint32_t smem[fors_lds_words<P>()];
     if (blockIdx.x < n_fors) {
-        fors_tile<P, J>(A, blockIdx.x, smem);
+        fors_tile<P, J, true>(A, blockIdx.x, smem);
         return;
     }
     const uint32_t wave =
