@@ -157,6 +157,15 @@ struct Layout {
 // registers (88-144 VGPRs) for the chains too, and k_chains alone needs 64
 // or fewer for SHA-256 and so issues from 8 waves per SIMD instead of 3-5.
 static constexpr uint32_t kFuseWaves = 8192;
+// Chain waves of a fused launch up to which its FORS tiles are the narrowest
+// (JF leaves per lane): with 3.5 chain waves per SIMD or fewer there is room
+// for twice the FORS waves and the tile's serial run is what the launch waits
+// for; beyond, the extra waves only compete with the chains.  Measured,
+// k_sign_fused with J -> JF, us: SHA2-128f 1 request 67 -> 51, 16 93 -> 77,
+// 32 (3080 waves) 134 -> 125, 61 (5880) 201 -> 202, 85 260 -> 263;
+// SHAKE256-256f 1 278 -> 138, 7 321 -> 245, 14 (3987) 399 -> 436;
+// SHA2-256f 14 201 -> 194, 28 315 -> 332.
+static constexpr uint32_t kShortForsWaves = 3584;
 
 // J: FORS leaves per lane, 2^J (2^(a-J) lanes per tree).  Short tiles at every
 // size: a tile is a serial run of 3-4 x 2^J hashes, and with the two-phase
@@ -193,7 +202,11 @@ struct SetImpl {
             hipLaunchKernelGGL((k_ht<P, MODE, 16>), dim3(Lay::template ht_blocks<16>(trees)),
                                dim3(256), 0, s, A);
     }
-    static uint32_t fors_tiles(uint32_t n) { return cdiv((uint64_t)n * P::k, 256u >> (P::a - J)); }
+    // FORS leaves per lane in a fused launch of few waves: 2, or as many as 256
+    // lanes per tree leave
+    static constexpr int JF = P::a - 8 > 1 ? P::a - 8 : 1;
+    template <int FJ>
+    static uint32_t fors_tiles(uint32_t n) { return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ)); }
 
     // workgroups of k_vht up to which each has a CU to itself
     static constexpr uint32_t kVhtAlone = 256;
@@ -233,9 +246,15 @@ struct SetImpl {
         // request's last FORS root, inside the FORS tiles)
         const uint32_t nwaves = chain_waves<P>(n * P::d);
         if (nwaves <= kFuseWaves) {
-            const uint32_t nf = fors_tiles(n);
-            hipLaunchKernelGGL((k_sign_fused<P, J>), dim3(nf + cdiv(nwaves, 4)), dim3(256), 0, s,
-                               A, nf, nwaves);
+            if (nwaves <= kShortForsWaves) {
+                const uint32_t nf = fors_tiles<JF>(n);
+                hipLaunchKernelGGL((k_sign_fused<P, JF>), dim3(nf + cdiv(nwaves, 4)), dim3(256),
+                                   0, s, A, nf, nwaves);
+            } else {
+                const uint32_t nf = fors_tiles<J>(n);
+                hipLaunchKernelGGL((k_sign_fused<P, J>), dim3(nf + cdiv(nwaves, 4)), dim3(256),
+                                   0, s, A, nf, nwaves);
+            }
             prof_mark(s, "k_sign_fused");
         } else {
             launch_fors<P, J>(A, n, s);

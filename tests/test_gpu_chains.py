@@ -44,3 +44,25 @@ def test_both_sides_of_the_fused_launch(name):
         assert bytes(all_[i]) == O.signature_with_optrand(pid, msgs[i], bytes(sk[i]),
                                                           opt[i].tobytes()), i
     assert (C.batch_verify(pid, pk, all_, msgs) == 0).all()
+
+
+@pytest.mark.parametrize("name", sorted(FUSED))
+def test_both_sides_of_the_narrow_fors_tiles(name):
+    """The last batch whose FORS tiles are the narrowest (3584 chain waves) and
+    the first of the set's own width, inside the fused launch."""
+    pid = C.param_id(name)
+    p = C.params(pid)
+    leaves = p.d << (p.full_h // p.d)
+    n = 1
+    while -(-(n + 1) * leaves // 64) * p.len <= 3584:
+        n += 1
+    rng = random.Random(n + pid)
+    pk, sk = C.batch_keygen(pid, np.frombuffer(rng.randbytes(3 * p.n * (n + 1)), np.uint8))
+    msgs = [rng.randbytes(rng.choice((0, 32, 77))) for _ in range(n + 1)]
+    opt = np.frombuffer(rng.randbytes(p.n * (n + 1)), np.uint8).reshape(n + 1, p.n)
+    print("%s: %d and %d requests" % (name, n, n + 1), flush=True)
+    few = C.batch_sign(pid, sk[:n], msgs[:n], opt[:n])
+    all_ = C.batch_sign(pid, sk, msgs, opt)
+    assert (few == all_[:n]).all()
+    assert bytes(few[0]) == O.signature_with_optrand(pid, msgs[0], bytes(sk[0]), opt[0].tobytes())
+    assert (C.batch_verify(pid, pk, all_, msgs) == 0).all()
