@@ -208,18 +208,25 @@ struct SetImpl {
     template <int FJ>
     static uint32_t fors_tiles(uint32_t n) { return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ)); }
 
-    // workgroups of k_vht up to which each has a CU to itself
+    // workgroups of k_vht up to which each has a CU to itself: beyond, pairs
+    // double the instructions that the CU's workgroups compete with
     static constexpr uint32_t kVhtAlone = 256;
     template <int G>
     static void launch_vht(const BatchArgs& A, uint32_t n, hipStream_t s) {
         const uint32_t wgs = cdiv(n, 256 / G);
-        if constexpr (P::hash == kSha2 && G <= 32) {  // wider groups only serve small batches
-            if (wgs > kVhtAlone) {
-                hipLaunchKernelGGL((k_vht<P, G, true>), dim3(wgs), dim3(256), 0, s, A);
+        if constexpr (G >= 64) {
+            if (wgs <= kVhtAlone) {
+                hipLaunchKernelGGL((k_vht<P, G, kVhtPair>), dim3(wgs), dim3(256), 0, s, A);
                 return;
             }
         }
-        hipLaunchKernelGGL((k_vht<P, G, false>), dim3(wgs), dim3(256), 0, s, A);
+        if constexpr (P::hash == kSha2 && G <= 32) {  // wider groups only serve small batches
+            if (wgs > kVhtAlone) {
+                hipLaunchKernelGGL((k_vht<P, G, kVhtPhased>), dim3(wgs), dim3(256), 0, s, A);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_vht<P, G, kVhtLane>), dim3(wgs), dim3(256), 0, s, A);
     }
     static int sign(const DevBatch& b, hipStream_t s) {
         BatchArgs A{};

@@ -346,7 +346,10 @@ __device__ __forceinline__ void sha256_compress_ph(uint32_t st[8], uint32_t w[16
 // lane would otherwise run alone (T_len and Merkle climbs of verification,
 // the parked T_len of signing, the message hashes of the prep kernels).
 
-__device__ __forceinline__ void sha256_compress_pair(uint32_t s[4], const uint32_t vin[8]) {
+// Rounds T0 .. T1 - 1 on q (e f g h | a b c d) without the final addition;
+// rounds 0 .. T0 - 1 have run on q before
+template <int T0, int T1>
+__device__ __forceinline__ void sha256_rounds_pair(uint32_t q[4], const uint32_t vin[8]) {
     const bool odd = threadIdx.x & 1u;
     const uint32_t m = odd ? ~0u : 0u;
     const uint32_t r1 = odd ? 2u : 6u, r2 = odd ? 13u : 11u, r3 = odd ? 22u : 25u;
@@ -356,9 +359,9 @@ __device__ __forceinline__ void sha256_compress_pair(uint32_t s[4], const uint32
         v[k] = vin[k];
         z[k] = pair_swap(vin[k]);
     }
-    uint32_t q0 = s[0], q1 = s[1], q2 = s[2], q3 = s[3];
+    uint32_t q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
 #pragma unroll
-    for (int t = 0; t < 64; t++) {
+    for (int t = T0; t < T1; t++) {
         if (t >= 16 && (t & 1) == 0) {
             // W[2k] = s1(W[2k-2]) + W[2k-7] + s0(W[2k-15]) + W[2k-16] (even lane)
             // W[2k+1] = s1(W[2k-1]) + W[2k-6] + s0(W[2k-14]) + W[2k-15] (odd lane)
@@ -385,10 +388,19 @@ __device__ __forceinline__ void sha256_compress_pair(uint32_t s[4], const uint32
         q1 = q0;
         q0 = nw;
     }
-    s[0] += q0;
-    s[1] += q1;
-    s[2] += q2;
-    s[3] += q3;
+    q[0] = q0;
+    q[1] = q1;
+    q[2] = q2;
+    q[3] = q3;
+}
+
+__device__ __forceinline__ void sha256_compress_pair(uint32_t s[4], const uint32_t vin[8]) {
+    uint32_t q[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[i] = s[i];
+    sha256_rounds_pair<0, 64>(q, vin);
+#pragma unroll
+    for (int i = 0; i < 4; i++) s[i] += q[i];
 }
 
 // a word pointer into LDS (address space 3), so that code reached through a
@@ -644,6 +656,45 @@ struct Sha2 {
         sha256_rounds<5, 64>(v, w);
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = k.mid[i] + v[i];
+    }
+
+    // F along one chain on a lane pair (both lanes active, the same chain):
+    // rounds 0-4 once per chain as in F_prefix.  The value is in both lanes.
+    static constexpr int kPairWords = NW;
+    struct PairChain {
+        uint32_t mid[4], q[4];  // e f g h | a b c d: the midstate, after round 4
+    };
+    __device__ static __forceinline__ void pair_begin(const Key& k, const Adr& a, PairChain& c) {
+        const uint32_t m = (threadIdx.x & 1u) ? ~0u : 0u;
+        uint32_t w[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            w[i] = i < 2 ? lane_sel(m, a.w[2 * i + 1], a.w[2 * i]) : i == 2 ? a.w[4] : 0u;
+#pragma unroll
+        for (int i = 0; i < 4; i++) c.q[i] = c.mid[i] = lane_sel(m, k.mid[i], k.mid[4 + i]);
+        sha256_rounds_pair<0, 5>(c.q, w);
+    }
+    // the step at hash address h: block words W[2k] | W[2k + 1], of which k <
+    // 2 only feed the schedule
+    __device__ static __forceinline__ void pair_step(const PairChain& c, const Adr& a, uint32_t h,
+                                                     uint32_t v[NW]) {
+        const uint32_t m = (threadIdx.x & 1u) ? ~0u : 0u;
+        Adr ah = a;
+        adr_hash(ah, h);
+        uint32_t w[8], q[4];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            w[i] = lane_sel(m, block_word<NW>(ah, v, 0, 2 * i + 1), block_word<NW>(ah, v, 0, 2 * i));
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[i] = c.q[i];
+        sha256_rounds_pair<5, 64>(q, w);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            q[i] += c.mid[i];
+            const uint32_t other = pair_swap(q[i]);
+            if (i < NW) v[i] = lane_sel(m, q[i], other);
+            if (4 + i < NW) v[4 + i < NW ? 4 + i : 0] = lane_sel(m, other, q[i]);
+        }
     }
 
     // F along one chain in two-phase rounds.  The address words W[0..4] are

@@ -755,6 +755,39 @@ struct Shake {
                                                       const uint32_t in[NW], uint32_t out[NW]) {
         F_il(c, h, in, out);
     }
+    // The same on a lane pair (both lanes active, the same chain): this lane's
+    // half of every Keccak lane.
+    static constexpr int kPairWords = NW / 2;
+    struct PairChain {
+        uint32_t w[(NW + 8) / 2];  // pub_seed and address lanes
+    };
+    __device__ static __forceinline__ void pair_begin(const Key& k, const Adr& a, PairChain& c) {
+        const uint32_t h = threadIdx.x & 1u;
+#pragma unroll
+        for (int l = 0; l < (NW + 8) / 2; l++)
+            c.w[l] = il_half(2 * l < NW ? k.pub[2 * l < NW ? 2 * l : 0] : aw(a, 2 * l - NW),
+                             2 * l + 1 < NW ? k.pub[2 * l + 1 < NW ? 2 * l + 1 : 0]
+                                            : aw(a, 2 * l + 1 - NW), h);
+    }
+    __device__ static __forceinline__ void pair_step(const PairChain& c, const Adr&, uint32_t h,
+                                                     uint32_t v[NW / 2]) {
+        constexpr int PL = (NW + 8) / 2, VL = NW / 2;
+        const uint32_t half = threadIdx.x & 1u;
+        const uint32_t m = half ? ~0u : 0u;
+        uint32_t s[25];
+#pragma unroll
+        for (int l = 0; l < 25; l++) {  // as F_il
+            s[l] = l < PL ? c.w[l < PL ? l : 0]
+                 : l < PL + VL ? v[l < PL ? 0 : l - PL < VL ? l - PL : 0] : 0u;
+            if (l == kPadLane) s[l] ^= lane_sel(m, 3u, 7u);
+            if (l == 16) s[l] ^= m & 0x80000000u;
+        }
+        const uint32_t x = h >> half;
+        s[kHashLane] ^= ((x & 1u) << 20) | (((x >> 2) & 1u) << 21);
+        keccak_f_il_pair(s);
+#pragma unroll
+        for (int l = 0; l < VL; l++) v[l] = s[l];
+    }
     // NW plain words (NW / 2 lanes) <-> interleaved
     __device__ static __forceinline__ void to_il(const uint32_t in[NW], uint32_t out[NW]) {
 #pragma unroll

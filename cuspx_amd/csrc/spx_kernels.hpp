@@ -1612,12 +1612,22 @@ struct Layer16 {
 // 24 the rounds of T_len's blocks on K + W that all waves computed before); SHAKE256 does so on 16 lanes per request (Layer16).  The next layer's WOTS signature words and this
 // layer's auth path are fetched into registers while the chains run, so the
 // layer loop waits on no global load.
-// PH (SHA-256): chain steps in two-phase rounds, for launches that put two or
-// more workgroups on a CU (SHA2-128f, G = 16: 8192 requests 2.70 -> 2.10 ms,
-// 16384 5.19 -> 4.15); with one wave per SIMD the compiler's order stays
-// ahead (4096 requests 1.51 against 1.77 ms).
-template <class P, int G, bool PH>
+// CH: how a chain step runs.
+//  kVhtLane: on one lane.
+//  kVhtPhased (SHA-256): in two-phase rounds, for launches that put two or
+//    more workgroups on a CU (SHA2-128f, G = 16: 8192 requests 2.70 -> 2.10
+//    ms, 16384 5.19 -> 4.15); with one wave per SIMD the compiler's order
+//    stays ahead (4096 requests 1.51 against 1.77 ms).
+//  kVhtPair: on a lane pair, where every workgroup has a CU to itself and
+//    holds few requests (G >= 64): the chain phase lasts as long as its longest
+//    chain, 15 steps, and a step is 4.2k cycles on a pair against 5.6k on a
+//    lane (Keccak 12.9k, 19.7k).  300 requests, k_vht: SHA2-128f 1281 -> 1084
+//    us, SHA2-192f 1693 -> 1493, SHAKE256-128f 3067 -> 2338, SHAKE256-256f
+//    3109 -> 2403.
+enum { kVhtLane, kVhtPhased, kVhtPair };
+template <class P, int G, int CH>
 __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
+    constexpr bool PH = CH == kVhtPhased;
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
     constexpr bool SHA2 = P::hash == kSha2;
@@ -1628,6 +1638,7 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
     constexpr int TLW = LEN * NW;                // WOTS signature / public key words
     constexpr int NCH = R * LEN;                 // chains per workgroup and layer
     constexpr int MAXC = (NCH + 255) / 256;      // chains per lane
+    constexpr int MAXP = (NCH + 127) / 128;      // chains per lane pair (kVhtPair)
     constexpr int MAXW = (R * TLW + 255) / 256;  // prefetched WOTS words per lane
     constexpr int AW = TH * NW;                  // auth path words per request
     constexpr int MAXA = (R * AW + 255) / 256;   // prefetched auth words per lane
@@ -1739,11 +1750,6 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
             }
         }
         __syncthreads();
-        // my chains: ranks tid, 511 - tid, 512 + tid, ... (snake order; the
-        // ranks grow with c, so the valid ones are a prefix)
-        int nm = 0;
-#pragma unroll
-        for (int c = 0; c < MAXC; c++) nm += ((c & 1) ? (c + 1) * 256 - 1 - tid : c * 256 + tid) < nch;
         // fetch the next layer's WOTS signature and this layer's auth path
         const bool more = layer + 1 < P::d;
         uint32_t nx[MAXW], au[MAXA];
@@ -1757,71 +1763,141 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
             const int u = tid + 256 * k;
             au[k] = u < nact * AW ? wots_of(u / AW, layer)[TLW + u % AW] : 0u;
         }
-        // walk the chains: one flattened loop, one F site
-        int c = 0, r = 0, j = 0;
-        uint32_t s = P::w - 1;
-        Key key{};
-        Adr wa{};
-        uint32_t v[NW];
-        typename std::conditional<SHA2, int, typename Shake<P::n>::ChainIl>::type ch{};
-        uint32_t pre[SHA2 ? 8 : 1] = {};  // SHA-256: the chain's rounds 0-4 (Sha2::F_prefix)
-        typename Hh::Chain chn{};         // the same for two-phase rounds
+        if constexpr (CH == kVhtPair) {
+            // the same with pair tid / 2 in the place of lane tid
+            const int p = tid >> 1;
+            int nm = 0;
 #pragma unroll
-        for (int w = 0; w < NW; w++) v[w] = 0;
+            for (int c = 0; c < MAXP; c++) nm += ((c & 1) ? (c + 1) * 128 - 1 - p : c * 128 + p) < nch;
+            int c = 0, r = 0, j = 0;
+            uint32_t s = P::w - 1;
+            Adr wa{};
+            typename Hh::PairChain pc{};
+            constexpr int VW = Hh::kPairWords;
+            uint32_t v[VW];
 #pragma unroll
-        for (int i = 0; i < NW; i++) key.sk[i] = 0;
-        auto take = [&](int cc) {  // start chain cc of this lane (everything from LDS)
-            const int rank = (cc & 1) ? (cc + 1) * 256 - 1 - tid : cc * 256 + tid;
-            const uint32_t e = order_s[rank];
-            const int q = e & 0xFFF;
-            r = q / LEN;
-            j = q % LEN;
-            s = P::w - 1 - (e >> 12);
+            for (int w = 0; w < VW; w++) v[w] = 0;
+            auto take = [&](int cc) {
+                const uint32_t e = order_s[(cc & 1) ? (cc + 1) * 128 - 1 - p : cc * 128 + p];
+                const int q = e & 0xFFF;
+                r = q / LEN;
+                j = q % LEN;
+                s = P::w - 1 - (e >> 12);
+                wa = adr_make(layer, tree_s[r], kWots);
+                adr_keypair<TH>(wa, leaf_s[r]);
+                adr_chain(wa, j);
+                const uint32_t* sg = &sig_s[r][j * NW];
+                Key key;
 #pragma unroll
-            for (int w = 0; w < NW; w++) v[w] = to_native<P::hash>(sig_s[r][j * NW + w]);
-            wa = adr_make(layer, tree_s[r], kWots);
-            adr_keypair<TH>(wa, leaf_s[r]);
-            adr_chain(wa, j);
-            if constexpr (SHA2) {
+                for (int i = 0; i < NW; i++) key.sk[i] = 0;
+                if constexpr (SHA2) {
 #pragma unroll
-                for (int i = 0; i < 8; i++) key.mid[i] = key_s[r][i];
-                if constexpr (PH) Hh::chain_begin(key, wa, chn);
-                else Hh::F_prefix(key, wa, pre);
-            } else {
+                    for (int w = 0; w < NW; w++) v[w] = bswap32(sg[w]);
 #pragma unroll
-                for (int i = 0; i < NW; i++) key.pub[i] = key_s[r][i];
-                Hh::chain_il_begin(key, wa, ch);
-                uint32_t t[NW];
-                Hh::to_il(v, t);
-#pragma unroll
-                for (int w = 0; w < NW; w++) v[w] = t[w];
-            }
-        };
-        bool run = nm > 0;
-        if (run) take(0);
-        // all lanes step until every chain of the wave is done (full waves run
-        // fastest); a lane without one steps on a value that nothing reads
-#pragma unroll 1
-        while (true) {
-            while (run && s >= (uint32_t)P::w - 1) {  // chain done: park its end, take the next
-#pragma unroll
-                for (int w = 0; w < NW; w++) pk_s[r][PKO + j * NW + w] = v[w];
-                c++;
-                run = c < nm;
-                if (run) take(c);
-            }
-            if (!__any(run)) break;
-            if constexpr (SHA2) {
-                if constexpr (PH) {
-                    Hh::chain_step(key, chn, s, v, v);
+                    for (int i = 0; i < 8; i++) key.mid[i] = key_s[r][i];
                 } else {
-                    adr_hash(wa, s);
-                    Hh::F_step(key, pre, wa, v, v);
+#pragma unroll
+                    for (int l = 0; l < VW; l++) v[l] = il_half(sg[2 * l], sg[2 * l + 1], tid & 1);
+#pragma unroll
+                    for (int i = 0; i < NW; i++) key.pub[i] = key_s[r][i];
                 }
-            } else {
-                Hh::F_il(ch, s, v, v);
+                Hh::pair_begin(key, wa, pc);
+            };
+            bool run = nm > 0;
+            if (run) take(0);
+#pragma unroll 1
+            while (true) {
+                while (run && s >= (uint32_t)P::w - 1) {
+                    uint32_t* out = &pk_s[r][PKO + j * NW];
+                    if constexpr (SHA2) {
+                        if ((tid & 1) == 0) {
+#pragma unroll
+                            for (int w = 0; w < NW; w++) out[w] = v[w];
+                        }
+                    } else {
+#pragma unroll
+                        for (int l = 0; l < VW; l++) out[2 * l + (tid & 1)] = v[l];
+                    }
+                    c++;
+                    run = c < nm;
+                    if (run) take(c);
+                }
+                if (!__any(run)) break;
+                Hh::pair_step(pc, wa, s, v);
+                s++;
             }
-            s++;
+        } else {
+            // walk the chains: ranks tid, 511 - tid, 512 + tid, ... (snake order;
+            // the ranks grow with c, so the valid ones are a prefix) in one
+            // flattened loop, one F site
+            int nm = 0;
+#pragma unroll
+            for (int c = 0; c < MAXC; c++) nm += ((c & 1) ? (c + 1) * 256 - 1 - tid : c * 256 + tid) < nch;
+            int c = 0, r = 0, j = 0;
+            uint32_t s = P::w - 1;
+            Key key{};
+            Adr wa{};
+            uint32_t v[NW];
+            typename std::conditional<SHA2, int, typename Shake<P::n>::ChainIl>::type ch{};
+            uint32_t pre[SHA2 ? 8 : 1] = {};  // SHA-256: the chain's rounds 0-4 (Sha2::F_prefix)
+            typename Hh::Chain chn{};         // the same for two-phase rounds
+#pragma unroll
+            for (int w = 0; w < NW; w++) v[w] = 0;
+#pragma unroll
+            for (int i = 0; i < NW; i++) key.sk[i] = 0;
+            auto take = [&](int cc) {  // start chain cc of this lane (everything from LDS)
+                const int rank = (cc & 1) ? (cc + 1) * 256 - 1 - tid : cc * 256 + tid;
+                const uint32_t e = order_s[rank];
+                const int q = e & 0xFFF;
+                r = q / LEN;
+                j = q % LEN;
+                s = P::w - 1 - (e >> 12);
+#pragma unroll
+                for (int w = 0; w < NW; w++) v[w] = to_native<P::hash>(sig_s[r][j * NW + w]);
+                wa = adr_make(layer, tree_s[r], kWots);
+                adr_keypair<TH>(wa, leaf_s[r]);
+                adr_chain(wa, j);
+                if constexpr (SHA2) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++) key.mid[i] = key_s[r][i];
+                    if constexpr (PH) Hh::chain_begin(key, wa, chn);
+                    else Hh::F_prefix(key, wa, pre);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NW; i++) key.pub[i] = key_s[r][i];
+                    Hh::chain_il_begin(key, wa, ch);
+                    uint32_t t[NW];
+                    Hh::to_il(v, t);
+#pragma unroll
+                    for (int w = 0; w < NW; w++) v[w] = t[w];
+                }
+            };
+            bool run = nm > 0;
+            if (run) take(0);
+            // all lanes step until every chain of the wave is done (full waves run
+            // fastest); a lane without one steps on a value that nothing reads
+#pragma unroll 1
+            while (true) {
+                while (run && s >= (uint32_t)P::w - 1) {  // chain done: park its end, take the next
+#pragma unroll
+                    for (int w = 0; w < NW; w++) pk_s[r][PKO + j * NW + w] = v[w];
+                    c++;
+                    run = c < nm;
+                    if (run) take(c);
+                }
+                if (!__any(run)) break;
+                if constexpr (SHA2) {
+                    if constexpr (PH) {
+                        Hh::chain_step(key, chn, s, v, v);
+                    } else {
+                        adr_hash(wa, s);
+                        Hh::F_step(key, pre, wa, v, v);
+                    }
+                } else {
+                    Hh::F_il(ch, s, v, v);
+                }
+                s++;
+            }
         }
 #pragma unroll
         for (int k = 0; k < MAXA; k++) {
