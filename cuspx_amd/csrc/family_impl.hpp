@@ -63,7 +63,7 @@ struct FamilyImpl {
     static void tail(const BatchArgs& A, uint32_t n, hipStream_t s) {
         if (!n) return;
         hipLaunchKernelGGL((k_ht<P, 0, 1>), dim3(Layout<P>::template ht_blocks<1>(n * P::d)),
-                           dim3(256), 0, s, A);
+                           dim3(HtShape<P, 1>::WG), 0, s, A);
         prof_mark(s, "k_ht");
         if (!A.fors_count) {
             launch_fors_pk<P>(A, n, s);

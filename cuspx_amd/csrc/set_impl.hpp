@@ -18,19 +18,19 @@ struct Layout {
     static constexpr uint64_t al(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 
     // The split of a sign / keygen batch over `trees` subtrees: a tuned value
-    // when the tuning table has one, else doubled while the launch would
-    // still fill less than half the chip.  k_ht runs a lane per WOTS leaf at
-    // 1, a lane pair at 2 and 4 and 16 lanes at 8 and 16 (the chains take a
-    // lane each whatever the split); mixed batches go to the family kernel up
-    // to 2.
-    static constexpr int max_split() { return 16; }
+    // when the tuning table has one.  k_ht runs a lane per WOTS leaf at 1, a
+    // lane pair at 2 and 4 and 16 lanes at 8 and 16 (the chains take a lane
+    // each whatever the split); mixed batches go to the family kernel up to 2.
+    // Without a table: 16 lanes while their waves are 2 per SIMD or fewer, a
+    // pair up to 24576 leaves.  k_ht at 1 / 4 / 16, us: SHA2-128f, 8000 leaves
+    // 47 / 50 / 45, 11264 51 / 41 / 67, 35200 51 / 62 / 168; SHA2-128s, 7168
+    // 75 / 63 / 73, 57344 79 / 108 / 456; SHAKE256-128f, 11264 80 / 60 / 82,
+    // 88000 93 / 121 / 360.
     static int split(int pid, int op, uint32_t trees) {
         const int t = tuned_split(pid, op, trees);
         if (t == 1 || t == 2 || t == 4 || t == 8 || t == 16) return t;
         const uint64_t leaves = (uint64_t)trees << P::th;
-        int S = 1;
-        while (S < max_split() && leaves * S * 2 <= kFillLanes) S *= 2;
-        return S;
+        return leaves <= 8192 ? 16 : leaves <= 24576 ? 4 : 1;
     }
     // Verify kernel width: G lanes per request on average (k_vht runs
     // 256 / G requests per workgroup and deals all their chains over its 256
@@ -194,7 +194,7 @@ struct SetImpl {
     static void launch_ht(const BatchArgs& A, uint32_t trees, int S, hipStream_t s) {
         if (S == 1)
             hipLaunchKernelGGL((k_ht<P, MODE, 1>), dim3(Lay::template ht_blocks<1>(trees)),
-                               dim3(256), 0, s, A);
+                               dim3(HtShape<P, 1>::WG), 0, s, A);
         else if (S <= 4)
             hipLaunchKernelGGL((k_ht<P, MODE, 2>), dim3(Lay::template ht_blocks<2>(trees)),
                                dim3(256), 0, s, A);
@@ -208,25 +208,22 @@ struct SetImpl {
     template <int FJ>
     static uint32_t fors_tiles(uint32_t n) { return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ)); }
 
-    // workgroups of k_vht up to which each has a CU to itself: beyond, pairs
-    // double the instructions that the CU's workgroups compete with
+    // workgroups of k_vht up to which each has a CU to itself
     static constexpr uint32_t kVhtAlone = 256;
     template <int G>
     static void launch_vht(const BatchArgs& A, uint32_t n, hipStream_t s) {
         const uint32_t wgs = cdiv(n, 256 / G);
         if constexpr (G >= 64) {
-            if (wgs <= kVhtAlone) {
-                hipLaunchKernelGGL((k_vht<P, G, kVhtPair>), dim3(wgs), dim3(256), 0, s, A);
-                return;
+            hipLaunchKernelGGL((k_vht<P, G, kVhtPair>), dim3(wgs), dim3(256), 0, s, A);
+        } else {
+            if constexpr (P::hash == kSha2) {
+                if (wgs > kVhtAlone) {
+                    hipLaunchKernelGGL((k_vht<P, G, kVhtPhased>), dim3(wgs), dim3(256), 0, s, A);
+                    return;
+                }
             }
+            hipLaunchKernelGGL((k_vht<P, G, kVhtLane>), dim3(wgs), dim3(256), 0, s, A);
         }
-        if constexpr (P::hash == kSha2 && G <= 32) {  // wider groups only serve small batches
-            if (wgs > kVhtAlone) {
-                hipLaunchKernelGGL((k_vht<P, G, kVhtPhased>), dim3(wgs), dim3(256), 0, s, A);
-                return;
-            }
-        }
-        hipLaunchKernelGGL((k_vht<P, G, kVhtLane>), dim3(wgs), dim3(256), 0, s, A);
     }
     static int sign(const DevBatch& b, hipStream_t s) {
         BatchArgs A{};

@@ -1258,24 +1258,27 @@ __global__ void __launch_bounds__(256) k_sign_fused(BatchArgs A, uint32_t n_fors
 // SHA-256 with the schedules of 16 blocks at a time on the 16 lanes, then
 // their rounds on the first two).
 //
-// A subtree whose lanes exceed a 256-lane workgroup is split over PARTS
-// workgroups.  Each part reduces its leaves to a part root in LDS; the part
+// At S = 1 a subtree is one workgroup's (512 lanes for 512 leaves).  With
+// more lanes per leaf, a subtree whose lanes exceed 256 is split over PARTS
+// workgroups, which costs each of them a device-scope fence: at S = 1 that
+// took longer than the hashes (SHA2-128s, 256 requests, 819 -> 378 us).  Each part reduces its leaves to a part root in LDS; the part
 // that finishes last (device-scope counter, release/acquire fences, no
 // waiting) climbs the remaining log2(PARTS) levels from the part roots.
 template <class P, int S>
 struct HtShape {
     static constexpr int L = 1 << P::th;                 // leaves per subtree
     static constexpr int LT = L * S;                     // lanes per subtree
-    static constexpr int PARTS = LT > 256 ? LT / 256 : 1;
+    static constexpr int WG = S == 1 && L > 256 ? L : 256;  // lanes per workgroup
+    static constexpr int PARTS = LT > WG ? LT / WG : 1;
     static constexpr int LP = L / PARTS;                 // leaves per part
     static constexpr int LOGP = P::th - ilog2(PARTS);    // levels reduced inside a part
-    static constexpr int TPW = PARTS > 1 ? 1 : 256 / LT; // subtrees per workgroup
-    static constexpr int NL = 256 / S;                   // leaves per workgroup
+    static constexpr int TPW = PARTS > 1 ? 1 : WG / LT;  // subtrees per workgroup
+    static constexpr int NL = WG / S;                    // leaves per workgroup
     static constexpr int NLDS = NL > PARTS ? NL : PARTS; // the last part climbs from PARTS roots
 };
 
 template <class P, int MODE, int S>
-__global__ void __launch_bounds__(256) k_ht(BatchArgs A) {
+__global__ void __launch_bounds__((HtShape<P, S>::WG)) k_ht(BatchArgs A) {
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
     using Sh = HtShape<P, S>;
@@ -1618,12 +1621,13 @@ struct Layer16 {
 //    more workgroups on a CU (SHA2-128f, G = 16: 8192 requests 2.70 -> 2.10
 //    ms, 16384 5.19 -> 4.15); with one wave per SIMD the compiler's order
 //    stays ahead (4096 requests 1.51 against 1.77 ms).
-//  kVhtPair: on a lane pair, where every workgroup has a CU to itself and
-//    holds few requests (G >= 64): the chain phase lasts as long as its longest
-//    chain, 15 steps, and a step is 4.2k cycles on a pair against 5.6k on a
-//    lane (Keccak 12.9k, 19.7k).  300 requests, k_vht: SHA2-128f 1281 -> 1084
-//    us, SHA2-192f 1693 -> 1493, SHAKE256-128f 3067 -> 2338, SHAKE256-256f
-//    3109 -> 2403.
+//  kVhtPair: on a lane pair, where a workgroup holds few requests (G >= 64):
+//    the chain phase lasts as long as its longest chain, 15 steps, and a step
+//    is 4.2k cycles on a pair against 5.6k on a lane (Keccak 12.9k, 19.7k).
+//    300 requests, k_vht: SHA2-128f 1281 -> 1084 us, SHA2-192f 1693 -> 1493,
+//    SHAKE256-128f 3067 -> 2338, SHAKE256-256f 3109 -> 2403; two workgroups
+//    per CU (2000 requests, G = 64): SHA2-128f 1916 -> 1696, SHAKE256-128f
+//    3374 -> 3075.
 enum { kVhtLane, kVhtPhased, kVhtPair };
 template <class P, int G, int CH>
 __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
