@@ -300,16 +300,20 @@ struct SetImpl {
         const uint32_t prep_grid_wgs = prep_grid<P>(A, n, b.mlen_bound);  // sets fields of A
         hipLaunchKernelGGL((k_vprep<P>), dim3(prep_grid_wgs), dim3(kPrepWg), 0, s, A);
         prof_mark(s, "k_vprep");
+        if (G == 1) {
+            const uint32_t nf = cdiv((uint64_t)n * P::k, 256);
+            hipLaunchKernelGGL((k_vspec<P>), dim3(nf + cdiv((uint64_t)n * P::d * P::len * 8, 256)),
+                               dim3(256), 0, s, A, nf);
+            prof_mark(s, "k_vspec");
+            hipLaunchKernelGGL((k_vht_spec<P>), dim3(n), dim3(64), 0, s, A);
+            prof_mark(s, "k_vht");
+            return hipGetLastError() == hipSuccess ? 0 : kErrHip;
+        }
         hipLaunchKernelGGL((k_vfors<P>), dim3(cdiv((uint64_t)n * P::k, 64)), dim3(64), 0, s, A);
         prof_mark(s, "k_vfors");
         launch_fors_pk<P>(A, n, s);
         prof_mark(s, "k_fors_pk");
-        if (G == 1) {
-            hipLaunchKernelGGL((k_vspec<P>), dim3(cdiv((uint64_t)n * P::d * P::len * 8, 256)),
-                               dim3(256), 0, s, A);
-            prof_mark(s, "k_vspec");
-            hipLaunchKernelGGL((k_vht_spec<P>), dim3(n), dim3(64), 0, s, A);
-        } else if (G == 16) launch_vht<16>(A, n, s);
+        if (G == 16) launch_vht<16>(A, n, s);
         else if (G == 32) launch_vht<32>(A, n, s);
         else if (G == 64) launch_vht<64>(A, n, s);
         else if constexpr (Lay::vmax() >= 128) launch_vht<128>(A, n, s);

@@ -948,17 +948,17 @@ __device__ __forceinline__ void fors_pk_16(const BatchArgs& A, uint32_t i, lds_u
 // a whole wave on one request, for latency: SHA-256 with the schedules of
 // T_k's blocks on one lane each, then their rounds on the pairs (all alike);
 // SHAKE256 on the rows of 16 lanes (all alike).  lds: fors_pk_wave_words
-// words of the wave's own.
+// words of the wave's own.  The value is in every lane.
 template <class P>
 __host__ __device__ constexpr int fors_pk_wave_words() {
     return P::hash == kSha2 ? Sha2Pair<P::nw, P::k * P::nw>::B * 68 + kKwOnes : fors_pk_row<P>();
 }
 template <class P>
-__device__ __forceinline__ void fors_pk_wave(const BatchArgs& A, uint32_t i, lds_u32* lds) {
+__device__ __forceinline__ void fors_pk_value(const BatchArgs& A, uint32_t i, lds_u32* lds,
+                                              uint32_t out[P::nw]) {
     using Hh = HashT<P>;
     constexpr int NW = P::nw, KW = P::k * NW;
     const int lane = threadIdx.x & 63;
-    uint32_t out[NW];
     if constexpr (P::hash == kSha2) {
         using SP = Sha2Pair<NW, KW>;
         const Plan& pl = A.plan[i];
@@ -981,7 +981,13 @@ __device__ __forceinline__ void fors_pk_wave(const BatchArgs& A, uint32_t i, lds
     } else {
         fors_pk_16<P>(A, i, lds, out);
     }
-    if (lane == 0) store_val<P::hash, NW>(A.fors_pk + (size_t)i * P::n, out);
+}
+template <class P>
+__device__ __forceinline__ void fors_pk_wave(const BatchArgs& A, uint32_t i, lds_u32* lds) {
+    uint32_t out[P::nw];
+    fors_pk_value<P>(A, i, lds, out);
+    if ((threadIdx.x & 63) == 0)
+        store_val<P::hash, P::nw>(A.fors_pk + (size_t)i * P::n, out);
 }
 
 // FORS public keys of a whole batch (large sign batches and verify): a wave
@@ -1030,11 +1036,10 @@ inline void launch_fors_pk(const BatchArgs& A, uint32_t n, hipStream_t s) {
 // verify: one FORS tree per lane: leaf from the revealed sk, climb with the
 // auth path (fors_pk_from_sig, fors.cu:596-633; compute_root utils.cu:94-135)
 template <class P>
-__global__ void __launch_bounds__(64) k_vfors(BatchArgs A) {
+__device__ __forceinline__ void vfors_lane(const BatchArgs& A, uint32_t g0) {
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
     constexpr int NW = P::nw;
-    const uint32_t g0 = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t g = g0 < A.n_req * P::k ? g0 : A.n_req * P::k - 1;  // repeated past the end
     const uint32_t req = g / P::k, t = g % P::k;
     const Plan& pl = A.plan[req];
@@ -1066,6 +1071,10 @@ __global__ void __launch_bounds__(64) k_vfors(BatchArgs A) {
         Hh::H(key, adr, l, r, node);
     }
     store_val<P::hash, NW>(A.fors_roots + (size_t)g * P::n, node);
+}
+template <class P>
+__global__ void __launch_bounds__(64) k_vfors(BatchArgs A) {
+    vfors_lane<P>(A, blockIdx.x * 64 + threadIdx.x);
 }
 
 // ------------------------------------------------------------- hypertree
@@ -2012,13 +2021,20 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
 // itself).  Lane p of a chain walks the starts p and 15 - p, 15 F steps for
 // every lane.  The per-layer pass that remains (k_vht_spec) is T_len and the
 // climb only.  SHAKE256 values are stored bit-interleaved.
+// The first n_fors workgroups are the batch's FORS trees: neither waits for
+// the other, and both are serial runs that leave most of the chip idle (one
+// SHAKE256-256f signature: 95 us of trees, 123 us of chains).
 template <class P>
-__global__ void __launch_bounds__(256) k_vspec(BatchArgs A) {
+__global__ void __launch_bounds__(256) k_vspec(BatchArgs A, uint32_t n_fors) {
+    if (blockIdx.x < n_fors) {
+        vfors_lane<P>(A, blockIdx.x * 256 + threadIdx.x);
+        return;
+    }
     using Hh = HashT<P>;
     using Key = typename Hh::Key;
     constexpr bool SHA2 = P::hash == kSha2;
     constexpr int NW = P::nw;
-    const uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t g0 = (uint64_t)(blockIdx.x - n_fors) * 256 + threadIdx.x;
     const uint64_t ng = (uint64_t)A.n_req * P::d * P::len * 8;
     const uint64_t g = g0 < ng ? g0 : ng - 1;  // repeated past the end
     const int p = (int)(g & 7);
@@ -2073,8 +2089,8 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A) {
     }
 }
 
-// Speculative verify, part 2: one wave per request walks the d layers
-// (sign.cu:3077-3113): lanes pick each chain's end for the layer's message
+// Speculative verify, part 2: one wave per request computes T_k and walks the
+// d layers (sign.cu:3077-3113): lanes pick each chain's end for the layer's message
 // from the candidates of k_vspec and load the auth path, then run T_len and
 // compute_root (utils.cu:94-135): SHA-256 on lane pairs with the message
 // schedules of T_len's blocks from one lane each, SHAKE256 on rows of 16
@@ -2104,17 +2120,20 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
     static_assert(MB <= 64, "one lane per block");
     __shared__ __align__(16) uint32_t kw_s[SHA2 ? MB : 1][68];
     __shared__ __align__(16) uint32_t ones_s[SHA2 ? kKwOnes : 1];
+    __shared__ __align__(16) uint32_t fpk_s[fors_pk_wave_words<P>()];
     if (SHA2) ones_s[threadIdx.x] = 1u;
     const int tid = threadIdx.x;
     const uint32_t req = blockIdx.x;  // grid = n_req
     const Plan& pl = A.plan[req];
     const uint8_t* sig = A.sig + (size_t)req * A.sig_stride;
     const uint32_t* cand = reinterpret_cast<const uint32_t*>(A.cap) + (size_t)req * P::d * LEN * 16 * NW;
-    if (tid == 0) {
+    {
         uint32_t fp[NW];
-        load_val<P::hash, NW>(A.fors_pk + (size_t)req * P::n, fp);
+        fors_pk_value<P>(A, req, (lds_u32*)fpk_s, fp);
+        if (tid == 0) {
 #pragma unroll
-        for (int w = 0; w < NW; w++) root_s[w] = fp[w];
+            for (int w = 0; w < NW; w++) root_s[w] = fp[w];
+        }
     }
     Keccak16 sponge;  // every row of 16 lanes runs the same one in step
     if constexpr (!SHA2) {
