@@ -554,6 +554,7 @@ struct Keccak16Tab {
 __constant__ Keccak16Tab kKeccak16 = Keccak16Tab();
 
 struct Keccak16 {
+    static constexpr int kLanes = 16;
     // per row of 16 lanes, 16-byte aligned.  Columns are 8 words apart, the odd
     // halves 4 words further, and rows an odd multiple of 16 words, so that
     // the four rows of a wave touch different banks.
@@ -594,6 +595,8 @@ struct Keccak16 {
 #pragma unroll
         for (int y = 0; y < 5; y++) s[y] = 0;
     }
+    // s[0] is lane (col, 0) and not a repeated column
+    __device__ static __forceinline__ bool own0() { return (threadIdx.x & 7u) - 1u < 5u; }
     // LDS words written by other lanes of the row are read next: keep the order
     __device__ static __forceinline__ void order() {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -654,6 +657,127 @@ struct Keccak16 {
         for (int y = 0; y < 4; y++) {
             const int l = col + 5 * y;
             if (l < 17) s[y] ^= buf[2 * (17 * b + l) + half];
+        }
+    }
+};
+
+// The same on two such rows, 32 lanes: the first holds rows y = 0, 1, 2 of the
+// columns in s, the second rows 3 and 4 (and a zero), and the column parities
+// are put together by swapping the rows (v_permlane16_swap).  About 26
+// instructions per round.  A permutation alone on its SIMD: 5.5 us on a lane
+// pair, 2.50 on 16 lanes, 2.12 on 32; four waves per CU 2.86 and 2.47.
+struct Keccak32Tab {
+    uint8_t rot[32][3], wr[32][3], rd[32][3];  // as Keccak16Tab
+    // column (h, x): 8 words, rows 0-2 in one half and 3, 4 in the other
+    static constexpr int at(int h, int x, int y) {
+        return (h * 5 + x) * 8 + ((4 * h) ^ (y < 3 ? y : y + 1));
+    }
+    constexpr Keccak32Tab() : rot{}, wr{}, rd{} {
+        for (int p = 0; p < 32; p++) {
+            const int g = p >> 4, h = (p >> 3) & 1, q = p & 7, x = (q + 4) % 5;
+            const bool owner = q >= 1 && q <= 5;
+            for (int i = 0; i < 3; i++) {
+                const int y = i + 3 * g;
+                const int r = kRho[x + 5 * (y < 5 ? y : 0)];
+                const int n = (r & 1) == 0 ? r / 2 : h ? (r + 1) / 2 : (r - 1) / 2;
+                const int h2 = h ^ (r & 1);
+                rot[p][i] = (uint8_t)((32 - n) & 31);
+                wr[p][i] = (uint8_t)(owner && y < 5 ? at(h2, y, (2 * x + 3 * y) % 5) : 80 + p);
+            }
+            for (int k = 0; k < 3; k++) rd[p][k] = (uint8_t)((h * 5 + (x + k) % 5) * 8 + 4 * (g ^ h));
+        }
+    }
+};
+__constant__ Keccak32Tab kKeccak32 = Keccak32Tab();
+
+struct Keccak32 {
+    static constexpr int kLanes = 32;
+    static constexpr int kLdsWords = 112;  // per 32 lanes, 16-byte aligned; as Keccak16
+    static constexpr int row_words(int w) { return Keccak16::row_words(w); }
+    typedef Keccak16::lds_word lds_word;
+    typedef Keccak16::v4 v4;
+    typedef Keccak16::lds_v4 lds_v4;
+
+    uint32_t s[3];    // lanes (col, row + i)
+    uint32_t rot[3];
+    lds_word* wr[3];
+    lds_word* rd[3];
+    lds_word* base;
+    uint32_t me, mo;  // as Keccak16
+    uint32_t sh1, half;
+    int col, row;
+
+    __device__ __forceinline__ void init(lds_word* lds) {
+        const int p = threadIdx.x & 31;
+        half = (p >> 3) & 1;
+        col = ((p & 7) + 4) % 5;
+        row = 3 * (p >> 4);
+        base = lds;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            rot[i] = kKeccak32.rot[p][i];
+            wr[i] = lds + kKeccak32.wr[p][i];
+            rd[i] = lds + kKeccak32.rd[p][i];
+        }
+        me = (col == 0 && row == 0 && !half) ? ~0u : 0u;
+        mo = (col == 0 && row == 0 && half) ? ~0u : 0u;
+        sh1 = half ? 0u : 31u;
+        clear();
+        // the third words of rows 3, 4 are read, and stay zero
+#pragma unroll
+        for (int i = 0; i < kLdsWords; i += 16) lds[i + (p & 15)] = 0;
+        order();
+    }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int i = 0; i < 3; i++) s[i] = 0;
+    }
+    __device__ static __forceinline__ bool own0() {
+        return (threadIdx.x & 7u) - 1u < 5u && (threadIdx.x & 16u) == 0;
+    }
+    __device__ static __forceinline__ void order() { Keccak16::order(); }
+    __device__ __forceinline__ void round(uint32_t rc_e, uint32_t rc_o) {
+        const uint32_t part = xor3(s[0], s[1], s[2]);
+        const auto sw = __builtin_amdgcn_permlane16_swap(part, part, false, false);
+        const uint32_t C = sw[0] ^ sw[1];
+        const uint32_t cm = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)C, 0x111, 0xF, 0xF, true);
+        const uint32_t t = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)C, 0x127, 0xF, 0xF, true);
+        const uint32_t cp = __builtin_amdgcn_alignbit(t, t, sh1);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const uint32_t u = xor3(s[i], cm, cp);
+            *wr[i] = __builtin_amdgcn_alignbit(u, u, rot[i]);
+        }
+        order();
+        v4 b[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) b[k] = *(const lds_v4*)rd[k];
+        order();
+        const uint32_t rc = (me & rc_e) | (mo & rc_o);
+#pragma unroll
+        for (int i = 0; i < 3; i++) s[i] = bit_chi(b[0][i], b[1][i], b[2][i]);
+        s[0] ^= rc;
+    }
+    __device__ __forceinline__ void permute() {
+        constexpr KeccakRcIl rc;
+#pragma unroll
+        for (int r = 0; r < 24; r++) round(rc.w[2 * r], rc.w[2 * r + 1]);
+    }
+    __device__ __forceinline__ uint32_t split(uint32_t lo, uint32_t hi) const {
+        return il_half(lo, hi, half);
+    }
+    __device__ __forceinline__ void lane(int l, uint32_t& lo, uint32_t& hi) const {
+        const int g = l >= 15, i = l / 5 - 3 * g;
+        const int at = (threadIdx.x & 32) + 16 * g + 1 + l % 5;
+        const uint32_t e = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * at, (int)s[i]);
+        const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (at + 8), (int)s[i]);
+        il_from(e, o, lo, hi);
+    }
+    __device__ __forceinline__ void absorb(const lds_word* buf, int b) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int l = col + 5 * (row + i);
+            if (l < 17) s[i] ^= buf[2 * (17 * b + l) + half];
         }
     }
 };
@@ -816,21 +940,21 @@ struct Shake {
 
     // ------------------------------------------------ per-request hashing
 
-    // SHAKE256(pre || m) squeezed to OUTB bytes (OUTB <= 136), on 16 lanes
-    // holding identical inputs (Keccak16).  m is 4-byte aligned; the word
+    // SHAKE256(pre || m) squeezed to OUTB bytes (OUTB <= 136), on 32 lanes
+    // holding identical inputs (Keccak32).  m is 4-byte aligned; the word
     // holding the last message byte is the last one read.  Lane p of the row
-    // loads words p, p + 16 and p + 32 of a block (the next block's while
-    // this one permutes) into LDS, from where every lane takes its halves.
-    // The output is in every lane.
+    // loads words p and p + 32 of a block (the next block's while this one
+    // permutes) into LDS, from where every lane takes its halves.  The output
+    // is in every lane.
     static constexpr int kStage = 36;  // LDS words of one staged block
-    static constexpr int kRowWords = Keccak16::row_words(Keccak16::kLdsWords + kStage);
+    static constexpr int kRowWords = Keccak32::row_words(Keccak32::kLdsWords + kStage);
     template <int NPRE, int OUTB>
-    __device__ static __forceinline__ void stream_msg(Keccak16& k, const uint32_t pre[NPRE], const uint8_t* m,
+    __device__ static __forceinline__ void stream_msg(Keccak32& k, const uint32_t pre[NPRE], const uint8_t* m,
                                       uint32_t mlen, uint8_t out[OUTB]) {
         static_assert(NPRE < 34 && OUTB <= 136, "prefix within one block");
         const gbl_u32* mg = (gbl_u32*)reinterpret_cast<const uint32_t*>(m);  // address-space cast
-        Keccak16::lds_word* stage = k.base + Keccak16::kLdsWords;
-        const int p = threadIdx.x & 15;
+        Keccak32::lds_word* stage = k.base + Keccak32::kLdsWords;
+        const int p = threadIdx.x & 31;
         const uint32_t nb = (uint32_t)((4ull * NPRE + mlen) / 136u) + 1;
         // stream word g (behind the prefix): message bytes, then 0x1F
         auto word = [&](uint32_t g) -> uint32_t {
@@ -843,31 +967,29 @@ struct Shake {
             }
             return x;
         };
-        auto fetch = [&](uint32_t b, uint32_t x[3]) {
+        auto fetch = [&](uint32_t b, uint32_t x[2]) {
             x[0] = word(34 * b + p);
-            x[1] = word(34 * b + p + 16);
-            x[2] = p < 2 ? word(34 * b + p + 32) : 0u;
+            x[1] = p < 2 ? word(34 * b + p + 32) : 0u;
         };
-        uint32_t x[3];
+        uint32_t x[2];
         fetch(0, x);
         k.clear();
 #pragma unroll 1
         for (uint32_t b = 0; b < nb; b++) {
             stage[p] = x[0];
-            stage[p + 16] = x[1];
-            if (p < 2) stage[p + 32] = b + 1 == nb && p == 1 ? x[2] ^ 0x80000000u : x[2];
-            Keccak16::order();
+            if (p < 2) stage[p + 32] = b + 1 == nb && p == 1 ? x[1] ^ 0x80000000u : x[1];
+            Keccak32::order();
             if (b == 0) {  // the same values from every lane
 #pragma unroll
                 for (int q = 0; q < NPRE; q++) stage[q] = pre[q];
-                Keccak16::order();
+                Keccak32::order();
             }
 #pragma unroll
-            for (int y = 0; y < 4; y++) {
-                const int l = k.col + 5 * y;
-                if (l < 17) k.s[y] ^= k.split(stage[2 * l], stage[2 * l + 1]);
+            for (int i = 0; i < 3; i++) {
+                const int l = k.col + 5 * (k.row + i);
+                if (l < 17) k.s[i] ^= k.split(stage[2 * l], stage[2 * l + 1]);
             }
-            Keccak16::order();
+            Keccak32::order();
             if (b + 1 < nb) fetch(b + 1, x);
             k.permute();
         }
@@ -881,9 +1003,9 @@ struct Shake {
         }
     }
 
-    // R = SHAKE256(sk_prf || optrand || m, n) (hash_shake256.cu:64-75), on 16
+    // R = SHAKE256(sk_prf || optrand || m, n) (hash_shake256.cu:64-75), on 32
     // lanes holding identical inputs
-    __device__ static __forceinline__ void prf_msg(Keccak16& k, const uint32_t skprf[NW], const uint32_t opt[NW],
+    __device__ static __forceinline__ void prf_msg(Keccak32& k, const uint32_t skprf[NW], const uint32_t opt[NW],
                                    const uint8_t* m, uint32_t mlen, uint32_t R[NW]) {
         uint32_t pre[2 * NW];
         uint8_t o[N];
@@ -899,10 +1021,10 @@ struct Shake {
                    (uint32_t)o[4 * i + 2] << 16 | (uint32_t)o[4 * i + 3] << 24;
     }
 
-    // digest = SHAKE256(R || pk || m, DG) (hash_shake256.cu:96-130), on 16
+    // digest = SHAKE256(R || pk || m, DG) (hash_shake256.cu:96-130), on 32
     // lanes holding identical inputs
     template <int DG>
-    __device__ static __forceinline__ void h_msg(Keccak16& k, const uint32_t R[NW], const uint32_t pk[2 * NW],
+    __device__ static __forceinline__ void h_msg(Keccak32& k, const uint32_t R[NW], const uint32_t pk[2 * NW],
                                  const uint8_t* m, uint32_t mlen, uint8_t dg[DG]) {
         uint32_t pre[3 * NW];
 #pragma unroll

@@ -109,8 +109,8 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
 
 // The prep kernels (128-lane workgroups).  Workgroups [0, prep_wgs): every
 // request hashes its message on a lane group (SHA-256: a pair,
-// sha256_compress_dup, 64 requests per workgroup; SHAKE256: 16 lanes,
-// Keccak16, 8 requests); all its lanes compute everything, the first one
+// sha256_compress_dup, 64 requests per workgroup; SHAKE256: 32 lanes,
+// Keccak32, 4 requests); all its lanes compute everything, the first one
 // stores.  SHA-256 messages of at least long_min bytes are left to the
 // workgroups after those: each takes long requests in turn and runs one with
 // both waves (Sha2::stream_msg_long), the schedules of its message-only blocks
@@ -122,7 +122,7 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
 // by up to 3.5 times, changing from launch to launch (T_len's rounds on a
 // pair: 2.9k cycles a block with all lanes active, 2.9-10k with two of 16).
 template <class P>
-__host__ __device__ constexpr uint32_t prep_lanes() { return P::hash == kSha2 ? 2 : 16; }
+__host__ __device__ constexpr uint32_t prep_lanes() { return P::hash == kSha2 ? 2 : 32; }
 constexpr uint32_t kPrepWg = 128;
 // the two-wave path from this length: a single SHA2-128f / 256f request of
 // 512 B signs in 0.329 / 0.624 ms against 0.336 / 0.634 on the lane pair,
@@ -154,7 +154,7 @@ __device__ __forceinline__ void prep_plan_init(const BatchArgs& A, uint32_t row,
 // its row's sponge k)
 template <class P, bool LONG>
 __device__ __forceinline__ void prep_sign_one(const BatchArgs& A, uint32_t i, bool store,
-                                              lds_u32* kw_s, bool prod, Keccak16* k) {
+                                              lds_u32* kw_s, bool prod, Keccak32* k) {
     using Hh = HashT<P>;
     constexpr int NW = P::nw;
     const uint32_t row = A.key_idx ? A.key_idx[i] : i;
@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
     if constexpr (P::hash == kShake) {
         constexpr int RW = HashT<P>::kRowWords;
         __shared__ __align__(16) uint32_t row_s[kPrepWg / PL * RW];
-        Keccak16 k;
+        Keccak32 k;
         k.init((lds_u32*)row_s + threadIdx.x / PL * RW);
         prep_sign_one<P, false>(A, i, first, nullptr, false, &k);
     } else {
@@ -240,7 +240,7 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
 // (LONG as for prep_sign_one)
 template <class P, bool LONG>
 __device__ __forceinline__ void prep_verify_one(const BatchArgs& A, uint32_t i, bool store,
-                                                lds_u32* kw_s, bool prod, Keccak16* k) {
+                                                lds_u32* kw_s, bool prod, Keccak32* k) {
     using Hh = HashT<P>;
     constexpr int NW = P::nw;
     const uint32_t row = A.key_idx ? A.key_idx[i] : i;
@@ -300,7 +300,7 @@ __global__ void __launch_bounds__(kPrepWg) k_vprep(BatchArgs A) {
     if constexpr (P::hash == kShake) {
         constexpr int RW = HashT<P>::kRowWords;
         __shared__ __align__(16) uint32_t row_s[kPrepWg / PL * RW];
-        Keccak16 k;
+        Keccak32 k;
         k.init((lds_u32*)row_s + threadIdx.x / PL * RW);
         prep_verify_one<P, false>(A, i, first, nullptr, false, &k);
     } else {
@@ -856,12 +856,12 @@ __device__ __forceinline__ void thash_shake_pair(const typename Shake<P::n>::Key
     Hh::from_il(il, out);
 }
 
-// SHAKE256 thash on 16 lanes (Keccak16) over a stream held in LDS as
+// SHAKE256 thash on a row of lanes (K: Keccak16, Keccak32) over a stream held in LDS as
 // interleaved words: pub_seed || address (PRE words) || M payload words ||
 // pad, in whole rate blocks.  The caller fills the payload; every lane of the
 // row calls these.
 template <class P, int M>
-struct Thash16 {
+struct ThashRow {
     using Hh = Shake<P::n>;
     static constexpr int NW = P::nw;
     static constexpr int PRE = NW + 8;
@@ -871,26 +871,29 @@ struct Thash16 {
     static_assert(PRE % 2 == 0 && M % 2 == 0, "whole 64-bit lanes");
 
     // pub_seed and the pad, which stay for every hash of one key
-    __device__ static __forceinline__ void begin(const Keccak16& k, const uint32_t pub[NW],
+    template <class K>
+    __device__ static __forceinline__ void begin(const K& k, const uint32_t pub[NW],
                                                  lds_u32* buf) {
 #pragma unroll
         for (int l = 0; l < NW / 2; l++)
             buf[2 * l + k.half] = k.split(pub[2 * l], pub[2 * l + 1]);
         buf[PRE - 2 + k.half] = 0;  // address bytes 24..31
         // 0x1F at the payload's end, 0x80 at the block's last byte
-        for (int i = T + (threadIdx.x & 15); i < kWords; i += 16)
+        for (int i = T + (threadIdx.x & (K::kLanes - 1)); i < kWords; i += K::kLanes)
             buf[i] = (i == T ? 7u : i == T + 1 ? 3u : 0u) ^ (i == kWords - 1 ? 0x80000000u : 0u);
     }
-    __device__ static __forceinline__ void address(const Keccak16& k, const Adr& a, lds_u32* buf) {
+    template <class K>
+    __device__ static __forceinline__ void address(const K& k, const Adr& a, lds_u32* buf) {
 #pragma unroll
         for (int l = 0; l < 3; l++)
             buf[NW + 2 * l + k.half] = k.split(Hh::aw(a, 2 * l), Hh::aw(a, 2 * l + 1));
     }
 };
 // the sponge over nb blocks of such a stream
-__device__ __forceinline__ void sponge16(Keccak16& k, const lds_u32* buf, int nb) {
+template <class K>
+__device__ __forceinline__ void sponge_row(K& k, const lds_u32* buf, int nb) {
     k.clear();
-    Keccak16::order();
+    K::order();
 #pragma unroll 1
     for (int b = 0; b < nb; b++) {
         k.absorb(buf, b);
@@ -901,7 +904,7 @@ __device__ __forceinline__ void sponge16(Keccak16& k, const lds_u32* buf, int nb
 // words of a WOTS public key in LDS: native, or the whole T_len stream
 template <class P>
 __host__ __device__ constexpr int tlen_words() {
-    return P::hash == kSha2 ? P::len * P::nw : Thash16<P, P::len * P::nw>::kWords;
+    return P::hash == kSha2 ? P::len * P::nw : ThashRow<P, P::len * P::nw>::kWords;
 }
 
 // FORS public key of request i: T_k over its k roots (fors.cu:142); the
@@ -917,37 +920,37 @@ __device__ __forceinline__ Adr fors_pk_adr(const Plan& pl) {
     adr_keypair<P::th>(adr, pl.leaf);
     return adr;
 }
-// SHAKE256 on 16 lanes; row: fors_pk_row words of LDS
+// SHAKE256 on a row of lanes; row: fors_pk_row words of LDS
 template <class P>
 __host__ __device__ constexpr int fors_pk_row() {
-    return Keccak16::row_words(Keccak16::kLdsWords + Thash16<P, P::k * P::nw>::kWords);
+    return Keccak16::row_words(Keccak16::kLdsWords + ThashRow<P, P::k * P::nw>::kWords);
 }
-template <class P>
-__device__ __forceinline__ void fors_pk_16(const BatchArgs& A, uint32_t i, lds_u32* row,
+template <class P, class K>
+__device__ __forceinline__ void fors_pk_rows(const BatchArgs& A, uint32_t i, lds_u32* row,
                                            uint32_t out[P::nw]) {
     constexpr int NW = P::nw, KW = P::k * NW;
-    using T16 = Thash16<P, KW>;
+    using T16 = ThashRow<P, KW>;
     const Plan& pl = A.plan[i];
     typename HashT<P>::Key key;
     HashT<P>::load_key(pl, key);
-    Keccak16 k;
+    K k;
     k.init(row);
-    lds_u32* buf = row + Keccak16::kLdsWords;
+    lds_u32* buf = row + K::kLdsWords;
     T16::begin(k, key.pub, buf);
     T16::address(k, fors_pk_adr<P>(pl), buf);
-    for (int l = threadIdx.x & 15; l < KW / 2; l += 16) {
+    for (int l = threadIdx.x & (K::kLanes - 1); l < KW / 2; l += K::kLanes) {
         uint32_t e, o;
         il_to(fors_root_word<P>(A, i, 2 * l), fors_root_word<P>(A, i, 2 * l + 1), e, o);
         buf[T16::PRE + 2 * l] = e;
         buf[T16::PRE + 2 * l + 1] = o;
     }
-    sponge16(k, buf, T16::NB);
+    sponge_row(k, buf, T16::NB);
 #pragma unroll
     for (int l = 0; l < NW / 2; l++) k.lane(l, out[2 * l], out[2 * l + 1]);
 }
 // a whole wave on one request, for latency: SHA-256 with the schedules of
 // T_k's blocks on one lane each, then their rounds on the pairs (all alike);
-// SHAKE256 on the rows of 16 lanes (all alike).  lds: fors_pk_wave_words
+// SHAKE256 on the rows of 32 lanes (all alike).  lds: fors_pk_wave_words
 // words of the wave's own.  The value is in every lane.
 template <class P>
 __host__ __device__ constexpr int fors_pk_wave_words() {
@@ -979,7 +982,7 @@ __device__ __forceinline__ void fors_pk_value(const BatchArgs& A, uint32_t i, ld
         Keccak16::order();
         SP::output(st, out);
     } else {
-        fors_pk_16<P>(A, i, lds, out);
+        fors_pk_rows<P, Keccak32>(A, i, lds, out);
     }
 }
 template <class P>
@@ -1017,7 +1020,7 @@ __global__ void __launch_bounds__(64) k_fors_pk(BatchArgs A) {
             }, out);
         } else {
             __shared__ __align__(16) uint32_t row_s[4 * fors_pk_row<P>()];
-            fors_pk_16<P>(A, i, (lds_u32*)row_s + threadIdx.x / 16 * fors_pk_row<P>(), out);
+            fors_pk_rows<P, Keccak16>(A, i, (lds_u32*)row_s + threadIdx.x / 16 * fors_pk_row<P>(), out);
         }
         if (i0 == i && threadIdx.x % fors_pk_lanes<P>() == 0)
             store_val<P::hash, NW>(A.fors_pk + (size_t)i * P::n, out);
@@ -1359,7 +1362,7 @@ __global__ void __launch_bounds__((HtShape<P, S>::WG)) k_ht(BatchArgs A) {
             }
             SP::output(st, node);
         } else if constexpr (S == 16) {
-            using TL = Thash16<P, TLW>;
+            using TL = ThashRow<P, TLW>;
             Keccak16 k;
             k.init((lds_u32*)x_s + slot * XW);
             lds_u32* buf = (lds_u32*)x_s + slot * XW + Keccak16::kLdsWords;
@@ -1371,7 +1374,7 @@ __global__ void __launch_bounds__((HtShape<P, S>::WG)) k_ht(BatchArgs A) {
 #pragma unroll
             for (int i = 0; i < (TLW + 15) / 16; i++)
                 if (16 * i + q < TLW) buf[TL::PRE + 16 * i + q] = x[i];
-            sponge16(k, buf, TL::NB);
+            sponge_row(k, buf, TL::NB);
 #pragma unroll
             for (int l = 0; l < NW / 2; l++) k.lane(l, node[2 * l], node[2 * l + 1]);
         } else if constexpr (P::hash == kSha2) {
@@ -1570,22 +1573,23 @@ __device__ __forceinline__ void tlen_climb_pair(const typename HashT<P>::Key& ke
     climb_pair<P>(key, layer, tree, leaf, auth, nd, node);
 }
 
-// The same for SHAKE256 on a row of 16 lanes (Keccak16), one loop over T_len
-// and the th nodes.  pk: the T_len stream (Thash16<P, len * nw>) with the
+// The same for SHAKE256 on a row of lanes (K: Keccak16, Keccak32), one loop over T_len
+// and the th nodes.  pk: the T_len stream (ThashRow<P, len * nw>) with the
 // chain ends as payload; nd: the stream of one node; begin() of both has run.
 // auth: the auth path, interleaved words.  node is the layer root, plain, in
 // every lane.
 template <class P>
-struct Layer16 {
-    using TL = Thash16<P, P::len * P::nw>;
-    using TH = Thash16<P, 2 * P::nw>;
+struct LayerRow {
+    using TL = ThashRow<P, P::len * P::nw>;
+    using TH = ThashRow<P, 2 * P::nw>;
     static constexpr int NW = P::nw;
     static_assert(TH::NB == 1 && NW <= 8, "a node is one block");
 
-    __device__ static __forceinline__ void run(Keccak16& k, uint32_t layer, uint64_t tree,
+    template <class K>
+    __device__ static __forceinline__ void run(K& k, uint32_t layer, uint64_t tree,
                                                uint32_t leaf, lds_u32* pk, const lds_u32* auth,
                                                lds_u32* nd, uint32_t node[NW]) {
-        const int p = threadIdx.x & 15;
+        const int p = threadIdx.x & (K::kLanes - 1);
         Adr a = adr_make(layer, tree, kWotsPk);
         adr_keypair<P::th>(a, leaf);
         TL::address(k, a, pk);
@@ -1600,11 +1604,10 @@ struct Layer16 {
                 TH::address(k, ha, nd);
                 lds_u32* own = nd + TH::PRE + (right ? NW : 0);
                 lds_u32* sib = nd + TH::PRE + (right ? 0 : NW);
-                // the node is in row 0 of the columns' owners (p & 7 in 1..5)
-                if (k.col < NW / 2 && (p & 7) >= 1 && (p & 7) <= 5) own[2 * k.col + k.half] = k.s[0];
+                if (k.col < NW / 2 && K::own0()) own[2 * k.col + k.half] = k.s[0];
                 if (p < NW) sib[p] = auth[(h - 1) * NW + p];
             }
-            sponge16(k, h == 0 ? pk : nd, h == 0 ? TL::NB : 1);
+            sponge_row(k, h == 0 ? pk : nd, h == 0 ? TL::NB : 1);
         }
 #pragma unroll
         for (int l = 0; l < NW / 2; l++) k.lane(l, node[2 * l], node[2 * l + 1]);
@@ -1621,7 +1624,7 @@ struct Layer16 {
 // SHAKE256 chains run bit-interleaved).  The lane pair 2r, 2r + 1 then
 // computes T_len of request r block by block from LDS and climbs its subtree
 // (compute_root, utils.cu:94-135; tlen_climb_pair, or for SHA-256 with n <=
-// 24 the rounds of T_len's blocks on K + W that all waves computed before); SHAKE256 does so on 16 lanes per request (Layer16).  The next layer's WOTS signature words and this
+// 24 the rounds of T_len's blocks on K + W that all waves computed before); SHAKE256 does so on 16 lanes per request (LayerRow).  The next layer's WOTS signature words and this
 // layer's auth path are fetched into registers while the chains run, so the
 // layer loop waits on no global load.
 // CH: how a chain step runs.
@@ -1667,7 +1670,7 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
     __shared__ uint32_t leaf_s[R];
     __shared__ uint32_t sig_s[R][TLW];  // WOTS signature of the layer, raw words
     // chain ends: native words, for SHAKE256 the payload of a T_len stream
-    // (Layer16), interleaved
+    // (LayerRow), interleaved
     constexpr int PKW = tlen_words<P>(), PKO = SHA2 ? 0 : NW + 8;
     __shared__ uint32_t pk_s[R][PKW];
     __shared__ uint32_t auth_s[R][AW];  // auth path of the layer, raw / interleaved words
@@ -1715,16 +1718,16 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
     // SHAKE256: request of this row of 16 lanes; rows past the last request
     // repeat their wave's first one (in step with it, on its LDS)
     const int row0 = tid / 64 * 4;
-    const int r16 = (tid >> 4) < nact ? tid >> 4 : row0;
+    const int rr = (tid >> 4) < nact ? tid >> 4 : row0;
     Keccak16 sponge;
     if constexpr (!SHA2) {
         if (row0 < nact) {
-            const Plan& pl = A.plan[req0 + r16];
+            const Plan& pl = A.plan[req0 + rr];
             Key k2;
             Hh::load_key(pl, k2);
-            sponge.init((lds_u32*)row_s[r16]);
-            Layer16<P>::TL::begin(sponge, k2.pub, (lds_u32*)pk_s[r16]);
-            Layer16<P>::TH::begin(sponge, k2.pub, (lds_u32*)node_s[r16]);
+            sponge.init((lds_u32*)row_s[rr]);
+            LayerRow<P>::TL::begin(sponge, k2.pub, (lds_u32*)pk_s[rr]);
+            LayerRow<P>::TH::begin(sponge, k2.pub, (lds_u32*)node_s[rr]);
         }
     }
 
@@ -1972,16 +1975,16 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
             }
         } else if constexpr (!SHA2) {
             if (row0 < nact) {
-                const uint64_t tree = tree_s[r16];
-                const uint32_t leaf = leaf_s[r16];
+                const uint64_t tree = tree_s[rr];
+                const uint32_t leaf = leaf_s[rr];
                 uint32_t node[NW];
-                Layer16<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s[r16],
-                                (lds_u32*)auth_s[r16], (lds_u32*)node_s[r16], node);
-                if (tid == 16 * r16) {
+                LayerRow<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s[rr],
+                                (lds_u32*)auth_s[rr], (lds_u32*)node_s[rr], node);
+                if (tid == 16 * rr) {
 #pragma unroll
-                    for (int w = 0; w < NW; w++) root_s[r16][w] = node[w];
-                    leaf_s[r16] = (uint32_t)(tree & ((1u << TH) - 1));
-                    tree_s[r16] = tree >> TH;
+                    for (int w = 0; w < NW; w++) root_s[rr][w] = node[w];
+                    leaf_s[rr] = (uint32_t)(tree & ((1u << TH) - 1));
+                    tree_s[rr] = tree >> TH;
                 }
             }
         } else if (tid < 64) {
@@ -2093,8 +2096,8 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A, uint32_t n_fors) {
 // d layers (sign.cu:3077-3113): lanes pick each chain's end for the layer's message
 // from the candidates of k_vspec and load the auth path, then run T_len and
 // compute_root (utils.cu:94-135): SHA-256 on lane pairs with the message
-// schedules of T_len's blocks from one lane each, SHAKE256 on rows of 16
-// lanes (Layer16).  The serial
+// schedules of T_len's blocks from one lane each, SHAKE256 on rows of 32
+// lanes (LayerRow).  The serial
 // work per layer is T_len + h' nodes instead of the longest chain + T_len +
 // h' nodes.
 template <class P>
@@ -2113,7 +2116,7 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
     __shared__ uint32_t auth_s[AW];
     __shared__ uint32_t root_s[NW];
     __shared__ uint32_t node_s[SHA2 ? NW : 34];
-    __shared__ __align__(16) uint32_t row_s[SHA2 ? 1 : Keccak16::kLdsWords];
+    __shared__ __align__(16) uint32_t row_s[SHA2 ? 1 : Keccak32::kLdsWords];
     // SHA-256: K + W of T_len's blocks, 68-word rows (the lanes' 16-byte
     // writes fall into distinct banks)
     constexpr int MB = SHA2 ? Sha2Pair<NW, TLW>::B : 1;
@@ -2135,13 +2138,13 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
             for (int w = 0; w < NW; w++) root_s[w] = fp[w];
         }
     }
-    Keccak16 sponge;  // every row of 16 lanes runs the same one in step
+    Keccak32 sponge;  // both rows of 32 lanes run the same one in step
     if constexpr (!SHA2) {
         Key key;
         Hh::load_key(pl, key);
         sponge.init((lds_u32*)row_s);
-        Layer16<P>::TL::begin(sponge, key.pub, (lds_u32*)pk_s);
-        Layer16<P>::TH::begin(sponge, key.pub, (lds_u32*)node_s);
+        LayerRow<P>::TL::begin(sponge, key.pub, (lds_u32*)pk_s);
+        LayerRow<P>::TH::begin(sponge, key.pub, (lds_u32*)node_s);
     }
     uint64_t tree = pl.tree;
     uint32_t leaf = pl.leaf;
@@ -2184,7 +2187,7 @@ __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
             SP::output(st, node);
             climb_pair<P>(key, layer, tree, leaf, auth_s, node_s, node);
         } else {
-            Layer16<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s, (lds_u32*)auth_s,
+            LayerRow<P>::run(sponge, layer, tree, leaf, (lds_u32*)pk_s, (lds_u32*)auth_s,
                             (lds_u32*)node_s, node);
         }
         if (tid == 0) {
