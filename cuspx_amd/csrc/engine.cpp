@@ -342,8 +342,9 @@ struct Job {
     uint8_t* out = nullptr;  // sign: signatures; verify: statuses; keygen: pk
     uint64_t out_stride = 0;
     uint8_t* out2 = nullptr;  // keygen: sk
-    uint32_t pieces = 0, per = 0;  // sign: output copies, items per copy
+    uint32_t pieces = 0, per = 0;  // sign: output copies, items per copy (0: one, no event)
     hipEvent_t after = nullptr;    // chained slices: the previous slice's kernels
+    bool mark = false;             // chained slices: another one follows
 };
 
 static int finish_job(Job& j) {
@@ -351,6 +352,11 @@ static int finish_job(Job& j) {
     Lane& L = *j.lane;
     j.lane = nullptr;
     const SetOps* o = j.o;
+    if (j.op == kOpSign && j.pieces == 0) {
+        HIP_OK(hipStreamSynchronize(L.stream));
+        copy_rows(j.out, j.out_stride, L.hbuf, o->sig_bytes, o->sig_bytes, 0, j.num);
+        return kOk;
+    }
     if (j.op == kOpSign) {
         // each piece is copied out as soon as its event says its DMA is done,
         // while the later pieces are still in flight
@@ -403,6 +409,7 @@ static int run_slices(uint32_t num, int slices, Enq enq, bool chain = false) {
         const uint32_t a = c * per, b = a + per < num ? a + per : num;
         if (a >= b) break;
         if (chain && c > 0) jobs[c].after = D.lane[c - 1].kdone;
+        jobs[c].mark = chain && b < num;
         err = enq(D.lane[c], a, b - a, D.budget / slices, jobs[c]);
     }
     for (int c = 0; c < slices; c++) {
@@ -442,7 +449,8 @@ static int sign_enqueue(const SetOps* o, Lane& L, size_t budget, uint32_t num,
     p += al16(4ull * num);
     memcpy(p, optrand, (uint64_t)num * n);
     uint8_t* d = (uint8_t*)L.dbuf;
-    HIP_OK(hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, L.stream));
+    if (host_copy(d, h, in_bytes, hipMemcpyHostToDevice, L.stream))
+        return fail(kErrHip, "input copy failed%s");
     DevBatch b{};
     b.n = num;
     b.sk = d;
@@ -463,9 +471,14 @@ static int sign_enqueue(const SetOps* o, Lane& L, size_t budget, uint32_t num,
     if (job.after) HIP_OK(hipStreamWaitEvent(L.stream, job.after, 0));
     rc = o->sign(b, L.stream);
     if (rc) return fail(rc, "kernel launch failed%s");
-    HIP_OK(hipEventRecord(L.kdone, L.stream));
+    if (job.mark) HIP_OK(hipEventRecord(L.kdone, L.stream));
     const uint64_t sb = o->sig_bytes;
-    const auto pc = pieces(num, sb);
+    auto pc = pieces(num, sb);
+    if (out_bytes <= kKernelCopy) {
+        if (host_copy(h, dsig, out_bytes, hipMemcpyDeviceToHost, L.stream))
+            return fail(kErrHip, "output copy failed%s");
+        pc.first = 0;
+    }
     for (uint32_t c = 0; c < pc.first; c++) {
         const uint64_t a = (uint64_t)c * pc.second;
         const uint64_t cnt = a + pc.second < num ? pc.second : num - a;
@@ -521,11 +534,12 @@ static int verify_enqueue(const SetOps* o, Lane& L, size_t budget,
     // as soon as it is staged, while the pool stages the next ones
     const uint64_t sb = o->sig_bytes;
     const auto pc = pieces(num, sb);
+    const bool small = in_bytes <= kKernelCopy;  // all of it in one copy below
     std::atomic<int> err{kOk};
     HostPool::get().run(pc.first, [&](uint32_t c) {
         const uint32_t a = c * pc.second, e = a + pc.second < num ? a + pc.second : num;
         copy_rows(p, sb, sig, sig_stride, sb, a, e);
-        if (hipMemcpyAsync(d + pk_region + a * sb, p + a * sb, (uint64_t)(e - a) * sb,
+        if (!small && hipMemcpyAsync(d + pk_region + a * sb, p + a * sb, (uint64_t)(e - a) * sb,
                            hipMemcpyHostToDevice, L.stream) != hipSuccess)
             err = kErrHip;
     });
@@ -540,8 +554,11 @@ static int verify_enqueue(const SetOps* o, Lane& L, size_t budget,
     p += al16(8ull * num);
     memcpy(p, mlen, 4ull * num);
     const uint64_t tail = pk_region + sig_region;
-    HIP_OK(hipMemcpyAsync(d, h, pk_region, hipMemcpyHostToDevice, L.stream));
-    HIP_OK(hipMemcpyAsync(d + tail, h + tail, in_bytes - tail, hipMemcpyHostToDevice, L.stream));
+    const int cp = small ? host_copy(d, h, in_bytes, hipMemcpyHostToDevice, L.stream)
+                         : host_copy(d, h, pk_region, hipMemcpyHostToDevice, L.stream) |
+                               host_copy(d + tail, h + tail, in_bytes - tail,
+                                         hipMemcpyHostToDevice, L.stream);
+    if (cp) return fail(kErrHip, "input copy failed%s");
     DevBatch b{};
     b.n = num;
     b.pk = d;
@@ -561,7 +578,8 @@ static int verify_enqueue(const SetOps* o, Lane& L, size_t budget,
     b.ws = (uint8_t*)dst + out_bytes;
     rc = o->verify(b, L.stream);
     if (rc) return fail(rc, "kernel launch failed%s");
-    HIP_OK(hipMemcpyAsync(h, dst, 4ull * num, hipMemcpyDeviceToHost, L.stream));
+    if (host_copy(h, dst, out_bytes, hipMemcpyDeviceToHost, L.stream))
+        return fail(kErrHip, "output copy failed%s");
     job.lane = &L;
     job.o = o;
     job.op = kOpVerify;
@@ -602,7 +620,8 @@ static int keygen_enqueue(const SetOps* o, Lane& L, size_t budget,
     if (rc) return rc;
     for (uint32_t i = 0; i < num; i++) memcpy(L.hbuf + i * sb, seeds + i * seed_stride, sb);
     uint8_t* d = (uint8_t*)L.dbuf;
-    HIP_OK(hipMemcpyAsync(d, L.hbuf, num * sb, hipMemcpyHostToDevice, L.stream));
+    if (host_copy(d, L.hbuf, in_bytes, hipMemcpyHostToDevice, L.stream))
+        return fail(kErrHip, "input copy failed%s");
     DevBatch b{};
     b.n = num;
     b.seed = d;
@@ -612,7 +631,8 @@ static int keygen_enqueue(const SetOps* o, Lane& L, size_t budget,
     b.ws = d + in_bytes + out_bytes;
     rc = o->keygen(b, L.stream);
     if (rc) return fail(rc, "kernel launch failed%s");
-    HIP_OK(hipMemcpyAsync(L.hbuf, b.pk_out, out_bytes, hipMemcpyDeviceToHost, L.stream));
+    if (host_copy(L.hbuf, b.pk_out, out_bytes, hipMemcpyDeviceToHost, L.stream))
+        return fail(kErrHip, "output copy failed%s");
     job.lane = &L;
     job.o = o;
     job.op = kOpKeygen;

@@ -83,4 +83,8 @@ int set_error(int code, const char* msg);
 int tuned_split(int pid, int op, uint32_t trees);
 int num_sets();
 
+// copies between pinned host memory and the device (hostcopy.hip)
+static constexpr uint64_t kKernelCopy = 2048 << 10;
+int host_copy(void* dst, const void* src, uint64_t bytes, hipMemcpyKind kind, hipStream_t s);
+
 }  // namespace spx
