@@ -202,6 +202,9 @@ struct SetImpl {
             hipLaunchKernelGGL((k_ht<P, MODE, 16>), dim3(Lay::template ht_blocks<16>(trees)),
                                dim3(256), 0, s, A);
     }
+    // a launch of so many waves leaves each of them a SIMD (HashPh)
+    static constexpr bool kSha = P::hash == kSha2;
+    static bool alone(uint32_t waves) { return kSha && waves <= kAloneWaves; }
     // FORS leaves per lane in a fused launch of few waves: 2, or as many as 256
     // lanes per tree leave
     static constexpr int JF = P::a - 8 > 1 ? P::a - 8 : 1;
@@ -252,18 +255,23 @@ struct SetImpl {
         if (nwaves <= kFuseWaves) {
             if (nwaves <= kShortForsWaves) {
                 const uint32_t nf = fors_tiles<JF>(n);
-                hipLaunchKernelGGL((k_sign_fused<P, JF>), dim3(nf + cdiv(nwaves, 4)), dim3(256),
-                                   0, s, A, nf, nwaves);
+                const uint32_t wgs = nf + cdiv(nwaves, 4);
+                if (alone(4 * wgs))
+                    hipLaunchKernelGGL((k_sign_fused<P, JF, !kSha>), dim3(wgs), dim3(256), 0, s, A,
+                                       nf, nwaves);
+                else
+                    hipLaunchKernelGGL((k_sign_fused<P, JF, true>), dim3(wgs), dim3(256), 0, s, A,
+                                       nf, nwaves);
             } else {
                 const uint32_t nf = fors_tiles<J>(n);
-                hipLaunchKernelGGL((k_sign_fused<P, J>), dim3(nf + cdiv(nwaves, 4)), dim3(256),
-                                   0, s, A, nf, nwaves);
+                hipLaunchKernelGGL((k_sign_fused<P, J, true>), dim3(nf + cdiv(nwaves, 4)),
+                                   dim3(256), 0, s, A, nf, nwaves);
             }
             prof_mark(s, "k_sign_fused");
         } else {
             launch_fors<P, J>(A, n, s);
             prof_mark(s, "k_fors");
-            hipLaunchKernelGGL((k_chains<P, 0>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
+            hipLaunchKernelGGL((k_chains<P, 0, true>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
                                nwaves);
             prof_mark(s, "k_chains");
         }
@@ -302,14 +310,20 @@ struct SetImpl {
         prof_mark(s, "k_vprep");
         if (G == 1) {
             const uint32_t nf = cdiv((uint64_t)n * P::k, 256);
-            hipLaunchKernelGGL((k_vspec<P>), dim3(nf + cdiv((uint64_t)n * P::d * P::len * 8, 256)),
-                               dim3(256), 0, s, A, nf);
+            const uint32_t wgs = nf + cdiv((uint64_t)n * P::d * P::len * 8, 256);
+            if (alone(4 * wgs))
+                hipLaunchKernelGGL((k_vspec<P, !kSha>), dim3(wgs), dim3(256), 0, s, A, nf);
+            else
+                hipLaunchKernelGGL((k_vspec<P, true>), dim3(wgs), dim3(256), 0, s, A, nf);
             prof_mark(s, "k_vspec");
             hipLaunchKernelGGL((k_vht_spec<P>), dim3(n), dim3(64), 0, s, A);
             prof_mark(s, "k_vht");
             return hipGetLastError() == hipSuccess ? 0 : kErrHip;
         }
-        hipLaunchKernelGGL((k_vfors<P>), dim3(cdiv((uint64_t)n * P::k, 64)), dim3(64), 0, s, A);
+        const uint32_t fw = cdiv((uint64_t)n * P::k, 64);
+        // (of one-wave workgroups two can meet on a SIMD well before all have one)
+        if (alone(2 * fw)) hipLaunchKernelGGL((k_vfors<P, !kSha>), dim3(fw), dim3(64), 0, s, A);
+        else hipLaunchKernelGGL((k_vfors<P, true>), dim3(fw), dim3(64), 0, s, A);
         prof_mark(s, "k_vfors");
         launch_fors_pk<P>(A, n, s);
         prof_mark(s, "k_fors_pk");
@@ -336,7 +350,12 @@ struct SetImpl {
         hipLaunchKernelGGL((k_kprep<P>), dim3(cdiv(n, 64)), dim3(64), 0, s, A);
         prof_mark(s, "k_kprep");
         const uint32_t nwaves = chain_waves<P>(n);
-        hipLaunchKernelGGL((k_chains<P, 1>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A, nwaves);
+        if (alone(nwaves))
+            hipLaunchKernelGGL((k_chains<P, 1, !kSha>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
+                               nwaves);
+        else
+            hipLaunchKernelGGL((k_chains<P, 1, true>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
+                               nwaves);
         prof_mark(s, "k_chains_keygen");
         launch_ht<1>(A, n, S, s);
         prof_mark(s, "k_ht_keygen");

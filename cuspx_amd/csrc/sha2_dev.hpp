@@ -569,7 +569,9 @@ constexpr uint32_t sha2_known_words(int blk) {
     return m;
 }
 
-template <int N>
+// PH: F, H and PRF in two-phase rounds, which issue best from several waves
+// per SIMD; a wave alone on its SIMD runs the compiler's order sooner
+template <int N, bool PH = true>
 struct Sha2 {
     static constexpr int hash = kSha2;
     static constexpr int NW = N / 4;
@@ -604,6 +606,12 @@ struct Sha2 {
         return 0;
     }
 
+    template <uint32_t KNOWN>
+    __device__ static __forceinline__ void compress(uint32_t st[8], uint32_t w[16]) {
+        if constexpr (PH) sha256_compress_ph<KNOWN>(st, w);
+        else sha256_compress(st, w);
+    }
+
     // T over M payload words after the 22-byte address, all block indices
     // known at compile time (used for F, H and short T_l).
     template <int M>
@@ -616,11 +624,11 @@ struct Sha2 {
         for (int i = 0; i < 8; i++) st[i] = k.mid[i];
 #pragma unroll
         for (int i = 0; i < 16; i++) w[i] = block_word<M>(a, d, 0, i);
-        sha256_compress_ph<sha2_known_words<M>(0)>(st, w);
+        compress<sha2_known_words<M>(0)>(st, w);
         if constexpr (B == 2) {
 #pragma unroll
             for (int i = 0; i < 16; i++) w[i] = block_word<M>(a, d, 1, i);
-            sha256_compress_ph<sha2_known_words<M>(1)>(st, w);
+            compress<sha2_known_words<M>(1)>(st, w);
         }
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = st[i];
@@ -703,11 +711,26 @@ struct Sha2 {
     // W[32..35]: all made once per chain (chain_begin).
     static constexpr uint32_t kFKnown = sha2_known_words<NW>(0);
     static constexpr int kFix = 20;  // W[16 .. 35]
-    struct Chain {
+    struct ChainPh {
         uint32_t st[8];      // working variables after round 4
         uint32_t fix[kFix];  // parts of W[16 + i] fixed along the chain
     };
-    __device__ static __forceinline__ void chain_begin(const Key& k, const Adr& a, Chain& c) {
+    struct ChainPlain {  // F_prefix, F_step
+        uint32_t st[8];
+        Adr a;
+    };
+    using Chain = typename std::conditional<PH, ChainPh, ChainPlain>::type;
+    __device__ static __forceinline__ void chain_begin(const Key& k, const Adr& a, ChainPlain& c) {
+        c.a = a;
+        F_prefix(k, a, c.st);
+    }
+    __device__ static __forceinline__ void chain_step(const Key& k, const ChainPlain& c, uint32_t s,
+                                                      const uint32_t in[NW], uint32_t out[NW]) {
+        Adr a = c.a;
+        adr_hash(a, s);
+        F_step(k, c.st, a, in, out);
+    }
+    __device__ static __forceinline__ void chain_begin(const Key& k, const Adr& a, ChainPh& c) {
         constexpr Sha2Kinds kd(kFKnown, 0x1Fu);
         uint32_t w[16];
 #pragma unroll
@@ -731,7 +754,7 @@ struct Sha2 {
         sha256_rounds<0, 5>(c.st, w);
     }
     // one step at hash address s; in and out may be the same array
-    __device__ static __forceinline__ void chain_step(const Key& k, const Chain& c, uint32_t s,
+    __device__ static __forceinline__ void chain_step(const Key& k, const ChainPh& c, uint32_t s,
                                                       const uint32_t in[NW], uint32_t out[NW]) {
         static_assert((6 + NW + 2 + 15) / 16 == 1, "F is one block");
         Adr a{};
@@ -774,7 +797,7 @@ struct Sha2 {
         }
 #pragma unroll
         for (int i = 0; i < 8; i++) st[i] = kSha256IV[i];
-        sha256_compress_ph<sha2_known_words<NW>(0)>(st, w);  // sk_seed in the place of a value
+        compress<sha2_known_words<NW>(0)>(st, w);  // sk_seed in the place of a value
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = st[i];
     }

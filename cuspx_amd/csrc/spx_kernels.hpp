@@ -36,6 +36,16 @@ __host__ __device__ constexpr int max_int(int a, int b) { return a > b ? a : b; 
 
 template <class P>
 using HashT = typename std::conditional<P::hash == kSha2, Sha2<P::n>, Shake<P::n>>::type;
+// PH = false: for launches of at most kAloneWaves waves (one per SIMD), where
+// SHA-256 does without two-phase rounds.  With -> without them, us: k_chains of
+// SHA2-128f key generation, 1 key 48 -> 39, 200 (875 waves) 53 -> 44; k_vspec
+// SHA2-128f 1 request 46 -> 40, SHA2-256s 3 92 -> 75; k_sign_fused SHA2-128f 1
+// 51 -> 48, SHA2-192f 3 88 -> 81; k_vfors SHA2-192f 300 (155 waves) 55 -> 45,
+// but SHA2-128f 1900 (980 waves) 32 -> 38.
+template <class P, bool PH>
+using HashPh =
+    typename std::conditional<P::hash == kSha2, Sha2<P::n, PH>, Shake<P::n>>::type;
+constexpr uint32_t kAloneWaves = 1024;
 
 // ------------------------------------------------------------- arguments
 
@@ -396,9 +406,9 @@ constexpr int fors_lds_words() {
 // is the workgroup's tile (TPW trees), so the same body serves the fused
 // signing kernels.  smem: fors_lds_words<P>() words of LDS owned by the kernel
 // PK: count the roots and run T_k here (fors_count set)
-template <class P, int J, bool PK>
+template <class P, int J, bool PK, bool PH = true>
 __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint32_t* smem) {
-    using Hh = HashT<P>;
+    using Hh = HashPh<P, PH>;
     using Key = typename Hh::Key;
     constexpr int NW = P::nw;
     constexpr int LOGL = P::a - J;
@@ -1038,9 +1048,9 @@ inline void launch_fors_pk(const BatchArgs& A, uint32_t n, hipStream_t s) {
 
 // verify: one FORS tree per lane: leaf from the revealed sk, climb with the
 // auth path (fors_pk_from_sig, fors.cu:596-633; compute_root utils.cu:94-135)
-template <class P>
+template <class P, bool PH>
 __device__ __forceinline__ void vfors_lane(const BatchArgs& A, uint32_t g0) {
-    using Hh = HashT<P>;
+    using Hh = HashPh<P, PH>;
     using Key = typename Hh::Key;
     constexpr int NW = P::nw;
     const uint32_t g = g0 < A.n_req * P::k ? g0 : A.n_req * P::k - 1;  // repeated past the end
@@ -1075,9 +1085,9 @@ __device__ __forceinline__ void vfors_lane(const BatchArgs& A, uint32_t g0) {
     }
     store_val<P::hash, NW>(A.fors_roots + (size_t)g * P::n, node);
 }
-template <class P>
+template <class P, bool PH>
 __global__ void __launch_bounds__(64) k_vfors(BatchArgs A) {
-    vfors_lane<P>(A, blockIdx.x * 64 + threadIdx.x);
+    vfors_lane<P, PH>(A, blockIdx.x * 64 + threadIdx.x);
 }
 
 // ------------------------------------------------------------- hypertree
@@ -1188,9 +1198,9 @@ __host__ __device__ constexpr uint32_t chain_waves(uint32_t trees) {
     return (leaf_count<P>(trees) + 63) / 64 * P::len;
 }
 
-template <class P, int MODE>
+template <class P, int MODE, bool PH = true>
 __device__ __forceinline__ void chain_wave(const BatchArgs& A, uint32_t wave) {
-    using Hh = HashT<P>;
+    using Hh = HashPh<P, PH>;
     constexpr int NW = P::nw;
     constexpr int L = 1 << P::th;
     const uint32_t ntrees = MODE == 0 ? A.n_req * P::d : A.n_req;
@@ -1241,25 +1251,25 @@ __device__ __forceinline__ void chain_wave(const BatchArgs& A, uint32_t wave) {
     }
 }
 
-template <class P, int MODE>
+template <class P, int MODE, bool PH>
 __global__ void __launch_bounds__(256) k_chains(BatchArgs A, uint32_t nwaves) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + threadIdx.x / 64);
-    if (wave < nwaves) chain_wave<P, MODE>(A, wave);
+    if (wave < nwaves) chain_wave<P, MODE, PH>(A, wave);
 }
 
 // Signing: the FORS tiles of a batch (n_fors workgroups, first: a tile is
 // longer than a chain) and its WOTS chains in one launch, so that small
 // batches have both in flight together
-template <class P, int J>
+template <class P, int J, bool PH>
 __global__ void __launch_bounds__(256) k_sign_fused(BatchArgs A, uint32_t n_fors, uint32_t nwaves) {
     __shared__ __align__(16) uint32_t smem[fors_lds_words<P>()];
     if (blockIdx.x < n_fors) {
-        fors_tile<P, J, true>(A, blockIdx.x, smem);
+        fors_tile<P, J, true, PH>(A, blockIdx.x, smem);
         return;
     }
     const uint32_t wave =
         __builtin_amdgcn_readfirstlane((blockIdx.x - n_fors) * 4 + threadIdx.x / 64);
-    if (wave < nwaves) chain_wave<P, 0>(A, wave);
+    if (wave < nwaves) chain_wave<P, 0, PH>(A, wave);
 }
 
 // Hypertree subtrees from the parked chain ends: T_len of every leaf, then
@@ -2027,13 +2037,13 @@ __global__ void __launch_bounds__(256) k_vht(BatchArgs A) {
 // The first n_fors workgroups are the batch's FORS trees: neither waits for
 // the other, and both are serial runs that leave most of the chip idle (one
 // SHAKE256-256f signature: 95 us of trees, 123 us of chains).
-template <class P>
+template <class P, bool PH>
 __global__ void __launch_bounds__(256) k_vspec(BatchArgs A, uint32_t n_fors) {
     if (blockIdx.x < n_fors) {
-        vfors_lane<P>(A, blockIdx.x * 256 + threadIdx.x);
+        vfors_lane<P, PH>(A, blockIdx.x * 256 + threadIdx.x);
         return;
     }
-    using Hh = HashT<P>;
+    using Hh = HashPh<P, PH>;
     using Key = typename Hh::Key;
     constexpr bool SHA2 = P::hash == kSha2;
     constexpr int NW = P::nw;
