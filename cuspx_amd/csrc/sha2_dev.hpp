@@ -546,19 +546,6 @@ __device__ __forceinline__ void sha256_kw_msg_block(const uint32_t* src, lds_u32
     }
 }
 
-// one compression: on one lane, or on a lane pair holding identical inputs
-template <bool PAIR>
-__device__ __forceinline__ void sha256_compress_by(uint32_t st[8], uint32_t w[16]) {
-    if constexpr (PAIR) sha256_compress_dup(st, w);
-    else sha256_compress(st, w);
-}
-
-// write x into b[q] for a wave-uniform runtime q (v_cndmask per slot)
-__device__ __forceinline__ void put16(uint32_t b[16], int q, uint32_t x) {
-#pragma unroll
-    for (int i = 0; i < 16; i++) b[i] = (q == i) ? x : b[i];
-}
-
 // words of block blk of T over M payload words that are known: the zeros
 // after the 0x80 byte and the length
 template <int M>
@@ -805,20 +792,37 @@ struct Sha2 {
     // ------------------------------------------------ per-request hashing
 
     // midstate: compress(IV, pub_seed || 0^(64-n)) (seed_state, sha256.cu:391)
-    // PAIR: run by a lane pair holding identical inputs (the prep kernels)
-    template <bool PAIR = false>
     __device__ static __forceinline__ void midstate(const uint32_t pub[NW], uint32_t mid[8]) {
         uint32_t w[16];
 #pragma unroll
         for (int i = 0; i < 16; i++) w[i] = i < NW ? pub[i] : 0u;
 #pragma unroll
         for (int i = 0; i < 8; i++) mid[i] = kSha256IV[i];
-        sha256_compress_by<PAIR>(mid, w);
+        sha256_compress(mid, w);
     }
 
-    // The message hashes run on a lane pair holding identical inputs (the
-    // prep kernels give every request two lanes; sha256_compress_dup).
-    //
+    // The message hashes run on a group of 8 lanes holding identical inputs:
+    // blocks of the message on each of its lane pairs alike
+    // (sha256_compress_dup), independent blocks on a pair each (group_block:
+    // pair g of the group compresses the block that blk(g, w) forms from the
+    // IV; group_take then fetches pair g's result).
+    static constexpr int kGroup = 8;
+    template <class Blk>
+    __device__ static __forceinline__ void group_block(const Blk& blk, uint32_t st[8]) {
+        uint32_t w[16];
+        blk((threadIdx.x >> 1) & 3u, w);
+#pragma unroll
+        for (int i = 0; i < 8; i++) st[i] = kSha256IV[i];
+        sha256_compress_dup(st, w);
+    }
+    __device__ static __forceinline__ void group_take(const uint32_t st[8], uint32_t g,
+                                                      uint32_t out[8]) {
+        const int at = 4 * ((threadIdx.x & 56u) + 2 * g);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            out[i] = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)st[i]);
+    }
+
     // SHA-256 continuing from st over (pre[0..NPRE) || m[0..mlen)), where
     // `before` bytes were already absorbed.  m is 4-byte aligned; bytes past
     // mlen are never read beyond the word holding the last byte.  Blocks made
@@ -988,21 +992,18 @@ struct Sha2 {
     __device__ static void prf_msg(const uint32_t skprf[NW], const uint32_t opt[NW],
                                    const uint8_t* m, uint32_t mlen, uint32_t R[NW],
                                    lds_u32* kw_s = nullptr, bool prod = false) {
-        uint32_t st[8], w[16], inner[8];
+        uint32_t st[8], w[16], inner[8], keys[8];
+        group_block([&](uint32_t g, uint32_t b[16]) {  // the inner and the outer key's block
 #pragma unroll
-        for (int i = 0; i < 8; i++) st[i] = kSha256IV[i];
-#pragma unroll
-        for (int i = 0; i < 16; i++) w[i] = (i < NW ? skprf[i] : 0u) ^ 0x36363636u;
-        sha256_compress_dup(st, w);
+            for (int i = 0; i < 16; i++)
+                b[i] = (i < NW ? skprf[i] : 0u) ^ (g == 0 ? 0x36363636u : 0x5c5c5c5cu);
+        }, keys);
+        group_take(keys, 0, st);
         if constexpr (LONG) stream_msg_long<NW>(st, opt, m, mlen, 64, kw_s, prod);
         else stream_msg<NW>(st, opt, m, mlen, 64);
 #pragma unroll
         for (int i = 0; i < 8; i++) inner[i] = st[i];
-#pragma unroll
-        for (int i = 0; i < 8; i++) st[i] = kSha256IV[i];
-#pragma unroll
-        for (int i = 0; i < 16; i++) w[i] = (i < NW ? skprf[i] : 0u) ^ 0x5c5c5c5cu;
-        sha256_compress_dup(st, w);
+        group_take(keys, 1, st);
 #pragma unroll
         for (int i = 0; i < 16; i++)
             w[i] = i < 8 ? inner[i] : (i == 8 ? 0x80000000u : (i == 15 ? 768u : 0u));
@@ -1011,12 +1012,14 @@ struct Sha2 {
         for (int i = 0; i < NW; i++) R[i] = st[i];
     }
 
-    // digest bytes = MGF1(SHA256(R || pk || m), DG)  (hash_sha256.cu:200-247)
+    // digest bytes = MGF1(SHA256(R || pk || m), DG)  (hash_sha256.cu:200-247),
+    // and beside its two blocks the key's midstate
     template <int DG, bool LONG = false>
     __device__ static void h_msg(const uint32_t R[NW], const uint32_t pk[2 * NW],
                                  const uint8_t* m, uint32_t mlen, uint8_t dg[DG],
-                                 lds_u32* kw_s = nullptr, bool prod = false) {
-        uint32_t pre[3 * NW], st[8], seed[8], w[16];
+                                 uint32_t mid[8], lds_u32* kw_s = nullptr, bool prod = false) {
+        static_assert(DG <= 64, "two MGF1 blocks");
+        uint32_t pre[3 * NW], st[8], seed[8];
 #pragma unroll
         for (int i = 0; i < NW; i++) pre[i] = R[i];
 #pragma unroll
@@ -1027,19 +1030,22 @@ struct Sha2 {
         else stream_msg<3 * NW>(st, pre, m, mlen, 0);
 #pragma unroll
         for (int i = 0; i < 8; i++) seed[i] = st[i];
+        uint32_t out[8];
+        group_block([&](uint32_t g, uint32_t b[16]) {  // mgf1 (sha256.cu:362-383), midstate
 #pragma unroll
-        for (int c = 0; c < (DG + 31) / 32; c++) {  // mgf1, sha256.cu:362-383
+            for (int i = 0; i < 16; i++) {
+                const uint32_t x = i < 8 ? seed[i] : i == 8 ? g : i == 9 ? 0x80000000u
+                                                                : i == 15 ? 288u : 0u;
+                b[i] = g < 2 ? x : i < NW ? pk[i < NW ? i : 0] : 0u;
+            }
+        }, st);
+        group_take(st, 2, mid);
 #pragma unroll
-            for (int i = 0; i < 16; i++)
-                w[i] = i < 8 ? seed[i]
-                             : (i == 8 ? (uint32_t)c
-                                       : (i == 9 ? 0x80000000u : (i == 15 ? 288u : 0u)));
-#pragma unroll
-            for (int i = 0; i < 8; i++) st[i] = kSha256IV[i];
-            sha256_compress_dup(st, w);
+        for (int c = 0; c < (DG + 31) / 32; c++) {
+            group_take(st, c, out);
 #pragma unroll
             for (int i = 0; i < 32; i++)
-                if (32 * c + i < DG) dg[32 * c + i] = (uint8_t)(st[i >> 2] >> (24 - 8 * (i & 3)));
+                if (32 * c + i < DG) dg[32 * c + i] = (uint8_t)(out[i >> 2] >> (24 - 8 * (i & 3)));
         }
     }
 };

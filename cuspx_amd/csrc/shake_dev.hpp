@@ -1034,8 +1034,7 @@ struct Shake {
         stream_msg<3 * NW, DG>(k, pre, m, mlen, dg);
     }
 
-    // no midstate for SHAKE256 (zeros); PAIR as for Sha2::midstate
-    template <bool PAIR = false>
+    // no midstate for SHAKE256 (zeros)
     __device__ static __forceinline__ void midstate(const uint32_t*, uint32_t mid[8]) {
 #pragma unroll
         for (int i = 0; i < 8; i++) mid[i] = 0;
