@@ -35,8 +35,8 @@ PEAK_VALU_T = SIMDS * 32 * CLK_HZ / 1e12    # 78.64 T lane-instr/s (fast class)
 PEAK_VOP3_T = SIMDS * 16 * CLK_HZ / 1e12    # 39.32 T lane-instr/s (4-cycle class)
 # VALU lane-instructions per unit when profiles/pmc_counters.json has no
 # SQ_INSTS_VALU count for the kernel and batch (that count takes precedence)
-SHA256_OPS = 1237
-KECCAK_OPS = 4163
+SHA256_OPS = 1389
+KECCAK_OPS = 4056
 # a generic SHA-256 compression priced at 1450 VALU ops (F needs fewer); the
 # compression rate against 39.32 T / 1450 is reported as frac_at_1450_ops
 SHA256_OPS_UNFUSED = 1450
@@ -437,9 +437,9 @@ def mixed_phase(C, n, reps=3, seed=3):
     return {"sets": ["shake256-128f", "shake256-192f"], "requests": len(items),
             "message_bytes": "log-uniform 1..4096", "ms_per_batch": round(ms, 3),
             "signs_per_s": round(len(items) / ms * 1e3, 1), "spot_check_invalid": bad,
-            "launch": ("one hipGraph per replay: both sets' prep kernels, one persistent "
-                       "family kernel over every set's tiles, then T_k and the WOTS gather "
-                       "per set") if fused else
+            "launch": ("one hipGraph per replay: both sets' prep and FORS kernels, the chains "
+                       "of both in one launch, then subtrees, T_k and the WOTS gather per "
+                       "set") if fused else
                       ("one hipGraph per replay: each set's pipeline on its own forked "
                        "stream")}
 

@@ -151,7 +151,8 @@ def set_default_param(pid):
 
 def set_split(pid, op, lanes_per_leaf):
     """Force a work split (0 = automatic / tuned): lanes per WOTS leaf of the
-    hypertree kernel for OP_SIGN / OP_KEYGEN (1, 2, 4, 8, 16); mean lanes per
+    hypertree kernel for OP_SIGN / OP_KEYGEN (1, 2, 4, 8, 16; 4 runs as 2, 8
+    as 16); mean lanes per
     request of the verify kernel for OP_VERIFY (16, 32, 64; 128 when len = 67),
     which runs 256 / lanes requests per workgroup, or 1 for speculative
     verification (batches up to 256 requests)."""
@@ -640,9 +641,9 @@ def graph_sign_mixed(groups):
 
 
 def sign_mixed_device(groups, stream=None):
-    """Launch a mixed batch (list of SignGroup) directly on `stream`: one
-    persistent kernel when the groups are distinct fast sets of one hash
-    family, else the groups one after another."""
+    """Launch a mixed batch (list of SignGroup) directly on `stream`: the
+    chains of all groups in one launch when they are distinct fast sets of one
+    hash family, else the groups one after another."""
     L = lib()
     L.cuspx_sign_mixed_device.argtypes = [ctypes.POINTER(SignGroup), ctypes.c_int,
                                           ctypes.c_void_p]
@@ -655,8 +656,8 @@ class MixedSignBatch:
     """A resident mixed-parameter-set signing batch: requests are grouped by
     set, each group gets device buffers and a workspace, and the whole batch
     is one hipGraph (one launch per replay).  Distinct fast sets of one hash
-    family, each large enough for one or two lanes per WOTS leaf, run as one
-    persistent kernel; other mixes run each set's pipeline on its own forked
+    family, each large enough for one or two lanes per WOTS leaf, share one
+    launch of their chains; other mixes run each set's pipeline on its own forked
     stream.  launch(eager=True) launches the same batch
     without the graph.
 

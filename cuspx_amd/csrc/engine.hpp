@@ -67,7 +67,7 @@ const SetOps* get_set(int pid);
 constexpr int kNotFused = 1;
 
 // The fast sets of one hash family (128f, 192f, 256f) signed as one mixed
-// batch by one persistent kernel (family_impl.hpp).
+// batch, their chains in one launch (family_impl.hpp).
 struct FamilyOps {
     int pid[3];
     // Signs b[0..2] (one batch per set, in the order of pid; n may be 0).

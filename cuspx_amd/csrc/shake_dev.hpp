@@ -215,10 +215,9 @@ __device__ __forceinline__ void keccak_round_ph(uint32_t s[50], uint32_t rc_lo, 
     keccak_chi(s, B, rc_lo, rc_hi);
 }
 
-// Keccak-f[1600].  HEAD: only the first words of the result are used, so the
-// last round is left to the compiler, which drops what those do not need
-// (about 50 of its 180 instructions stay for a 16-byte output)
-template <bool HEAD>
+// Keccak-f[1600] of which only the first words are used: the last round is left
+// to the compiler, which drops what those do not need (about 50 of its 180
+// instructions stay for a 16-byte output)
 __device__ __forceinline__ void keccak_f(uint32_t s[50]) {
     keccak_round_ph(s, 0x00000001u, 0x00000000u);
 #pragma unroll 1
@@ -226,8 +225,7 @@ __device__ __forceinline__ void keccak_f(uint32_t s[50]) {
         keccak_round_ph(s, kKeccakRC[2 * r], kKeccakRC[2 * r + 1]);
         keccak_round_ph(s, kKeccakRC[2 * r + 2], kKeccakRC[2 * r + 3]);
     }
-    if constexpr (HEAD) keccak_round(s, 0x80008008u, 0x80000000u);
-    else keccak_round_ph(s, 0x80008008u, 0x80000000u);
+    keccak_round(s, 0x80008008u, 0x80000000u);
 }
 
 // ---------------------------------------------------- bit-interleaved form
@@ -822,7 +820,7 @@ struct Shake {
             if (i == 33) x ^= 0x80000000u;
             s[i] = x;
         }
-        keccak_f<true>(s);
+        keccak_f(s);
 #pragma unroll
         for (int i = 0; i < NW; i++) out[i] = s[i];
     }

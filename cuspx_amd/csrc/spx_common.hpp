@@ -172,13 +172,4 @@ __device__ __forceinline__ uint32_t val_byte(const uint32_t* v, int i) {
     return (w >> sh) & 0xFF;
 }
 
-// select v[i] for a wave-uniform runtime i without local-memory indexing
-template <int NW>
-__device__ __forceinline__ uint32_t pick(const uint32_t v[NW], int i) {
-    uint32_t r = v[0];
-#pragma unroll
-    for (int j = 1; j < NW; j++) r = (i == j) ? v[j] : r;
-    return r;
-}
-
 }  // namespace spx

@@ -17,8 +17,8 @@
 //                        captured chain value for the layer's message
 //   verify: k_vprep, k_vfors, k_fors_pk, k_vht (the chains of a workgroup's
 //           requests dealt over its lanes, layers in sequence); small
-//           batches: k_vspec (every chain from every start) + k_vht_spec
-//           (T_len and the climb per layer)
+//           batches: k_vspec (FORS trees, every chain from every start) +
+//           k_vht_spec (T_k, then T_len and the climb per layer)
 //   keygen: k_kprep, k_chains and k_ht in keygen mode (top layer only)
 //
 // Semantics follow sign.cu:1924-1994 (sign), sign.cu:3048-3121 (verify),
@@ -384,8 +384,8 @@ __device__ __forceinline__ void fors_pk_wave(const BatchArgs& A, uint32_t i, lds
 template <class P>
 __host__ __device__ constexpr int fors_pk_wave_words();
 
-// a FORS root of request req is stored: count it; true for the request's last root.  The wave that stored it
-// then computes the FORS public key (fors_pk_wave), so T_k overlaps the
+// a FORS root of request req is stored: count it; true for the request's last
+// root.  The wave that stored it then computes the FORS public key (fors_pk_wave), so T_k overlaps the
 // hypertree chains instead of taking a launch of its own (the k roots of one
 // request come from several workgroups; every counter was zeroed by the prep
 // kernel).  Large batches launch k_fors_pk instead: there the per-tile
@@ -727,10 +727,8 @@ __device__ __forceinline__ void sha2_kw_block(const Adr& a, const Rd& rd, int b,
 
 // SHAKE256 thash over M payload words (thash_shake256.cu:15-25: pub_seed ||
 // addr32 || payload), 136 bytes per permutation; rd(i) returns payload word
-// i, read a block at a time.  IL: the payload words are bit-interleaved and
-// the sponge runs in the interleaved domain (keccak_f_il); else plain.  The
-// output is a plain value either way.
-template <class P, int M, bool IL, class Rd>
+// i, bit-interleaved, read a block at a time.  The output is a plain value.
+template <class P, int M, class Rd>
 __device__ __forceinline__ void thash_shake_rd(const typename Shake<P::n>::Key& key, const Adr& a,
                                                const Rd& rd, uint32_t out[P::nw]) {
     using Hh = Shake<P::n>;
@@ -739,16 +737,8 @@ __device__ __forceinline__ void thash_shake_rd(const typename Shake<P::n>::Key& 
     constexpr int NB = T / 34 + 1;            // permutations (the pad always fits)
     constexpr int TAIL = T - 34 * (NB - 1);   // words in the last block: the 0x1F byte follows
     static_assert(NB >= 2, "at least two blocks");
-    uint32_t pre[NW + 8];                     // pub_seed || address
-    if constexpr (IL) {
-        typename Hh::ChainIl c;
-        Hh::chain_il_begin(key, a, c);
-#pragma unroll
-        for (int i = 0; i < NW + 8; i++) pre[i] = c.w[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < NW + 8; i++) pre[i] = i < NW ? key.pub[i < NW ? i : 0] : Hh::aw(a, i - NW);
-    }
+    typename Hh::ChainIl c;  // pub_seed || address
+    Hh::chain_il_begin(key, a, c);
     uint32_t s[50];
 #pragma unroll
     for (int i = 0; i < 50; i++) s[i] = 0;
@@ -759,7 +749,7 @@ __device__ __forceinline__ void thash_shake_rd(const typename Shake<P::n>::Key& 
 #pragma unroll
             for (int j = 0; j < 34 - NW - 8; j++) x[j] = rd(j);
 #pragma unroll
-            for (int i = 0; i < 34; i++) s[i] ^= i < NW + 8 ? pre[i < NW + 8 ? i : 0] : x[i - NW - 8];
+            for (int i = 0; i < 34; i++) s[i] ^= i < NW + 8 ? c.w[i < NW + 8 ? i : 0] : x[i - NW - 8];
         } else if (blk < NB - 1) {
             const int base = 34 * blk - NW - 8;
             uint32_t x[34];
@@ -774,9 +764,7 @@ __device__ __forceinline__ void thash_shake_rd(const typename Shake<P::n>::Key& 
             for (int j = 0; j < TAIL; j++) x[j] = rd(base + j);
 #pragma unroll
             for (int i = 0; i < TAIL; i++) s[i] ^= x[i];
-            if constexpr (!IL) {
-                s[TAIL] ^= 0x1Fu;
-            } else if constexpr ((TAIL & 1) == 0) {  // 0x1F at bit 0 of lane TAIL / 2
+            if constexpr ((TAIL & 1) == 0) {  // 0x1F at bit 0 of lane TAIL / 2
                 s[TAIL] ^= 7u;
                 s[TAIL + 1] ^= 3u;
             } else {                                  // 0x1F at bit 32 of lane TAIL / 2
@@ -785,14 +773,9 @@ __device__ __forceinline__ void thash_shake_rd(const typename Shake<P::n>::Key& 
             }
             s[33] ^= 0x80000000u;  // 0x80 at byte 135 (lane 16, bit 63: odd, so the same word)
         }
-        if constexpr (IL) keccak_f_il<false>(s);
-        else keccak_f<false>(s);
+        keccak_f_il<false>(s);
     }
-    if constexpr (IL) Hh::from_il(s, out);
-    else {
-#pragma unroll
-        for (int i = 0; i < NW; i++) out[i] = s[i];
-    }
+    Hh::from_il(s, out);
 }
 
 // SHAKE256 thash on a lane pair in the interleaved domain (both lanes
@@ -868,8 +851,8 @@ __device__ __forceinline__ void thash_shake_pair(const typename Shake<P::n>::Key
     Hh::from_il(il, out);
 }
 
-// SHAKE256 thash on a row of lanes (K: Keccak16, Keccak32) over a stream held in LDS as
-// interleaved words: pub_seed || address (PRE words) || M payload words ||
+// SHAKE256 thash on a row of lanes (K: Keccak16, Keccak32) over a stream held
+// in LDS as interleaved words: pub_seed || address (PRE words) || M payload words ||
 // pad, in whole rate blocks.  The caller fills the payload; every lane of the
 // row calls these.
 template <class P, int M>
@@ -1394,7 +1377,7 @@ __global__ void __launch_bounds__((HtShape<P, S>::WG)) k_ht(BatchArgs A) {
             else thash_sha2_rd<NW, TLW>(key.mid, pa, parked, node);
         } else {
             if constexpr (S == 2) thash_shake_pair<P, TLW>(key, pa, parked2, node);
-            else thash_shake_rd<P, TLW, true>(key, pa, parked, node);
+            else thash_shake_rd<P, TLW>(key, pa, parked, node);
         }
         if (q == 0) {
             uint8_t* auth = A.sig + (size_t)req * A.sig_stride + P::n + P::fors_bytes +
@@ -1585,8 +1568,8 @@ __device__ __forceinline__ void tlen_climb_pair(const typename HashT<P>::Key& ke
     climb_pair<P>(key, layer, tree, leaf, auth, nd, node);
 }
 
-// The same for SHAKE256 on a row of lanes (K: Keccak16, Keccak32), one loop over T_len
-// and the th nodes.  pk: the T_len stream (ThashRow<P, len * nw>) with the
+// The same for SHAKE256 on a row of lanes (K: Keccak16, Keccak32), one loop
+// over T_len and the th nodes.  pk: the T_len stream (ThashRow<P, len * nw>) with the
 // chain ends as payload; nd: the stream of one node; begin() of both has run.
 // auth: the auth path, interleaved words.  node is the layer root, plain, in
 // every lane.
@@ -1636,9 +1619,10 @@ struct LayerRow {
 // SHAKE256 chains run bit-interleaved).  The lane pair 2r, 2r + 1 then
 // computes T_len of request r block by block from LDS and climbs its subtree
 // (compute_root, utils.cu:94-135; tlen_climb_pair, or for SHA-256 with n <=
-// 24 the rounds of T_len's blocks on K + W that all waves computed before); SHAKE256 does so on 16 lanes per request (LayerRow).  The next layer's WOTS signature words and this
-// layer's auth path are fetched into registers while the chains run, so the
-// layer loop waits on no global load.
+// 24 the rounds of T_len's blocks on K + W that all waves computed before);
+// SHAKE256 does so on 16 lanes per request (LayerRow).  The next layer's WOTS
+// signature words and this layer's auth path are fetched into registers while
+// the chains run, so the layer loop waits on no global load.
 // CH: how a chain step runs.
 //  kVhtLane: on one lane.
 //  kVhtPhased (SHA-256): in two-phase rounds, for launches that put two or
@@ -2105,13 +2089,13 @@ __global__ void __launch_bounds__(256) k_vspec(BatchArgs A, uint32_t n_fors) {
 }
 
 // Speculative verify, part 2: one wave per request computes T_k and walks the
-// d layers (sign.cu:3077-3113): lanes pick each chain's end for the layer's message
-// from the candidates of k_vspec and load the auth path, then run T_len and
-// compute_root (utils.cu:94-135): SHA-256 on lane pairs with the message
-// schedules of T_len's blocks from one lane each, SHAKE256 on rows of 32
-// lanes (LayerRow).  The serial
-// work per layer is T_len + h' nodes instead of the longest chain + T_len +
-// h' nodes.
+// d layers (sign.cu:3077-3113): lanes pick each chain's end for the layer's
+// message from the candidates of k_vspec and load the auth path, then run
+// T_len and compute_root (utils.cu:94-135): SHA-256 on lane pairs with the
+// message schedules of T_len's blocks from one lane each, SHAKE256 on rows of
+// 32 lanes (LayerRow).  The serial work per layer is T_len + h' nodes instead
+// of the longest chain + T_len + h' nodes.  One SHAKE256-256f signature: 958 ->
+// 854 us against rows of 16 lanes.
 template <class P>
 __global__ void __launch_bounds__(64) k_vht_spec(BatchArgs A) {
     using Hh = HashT<P>;

@@ -52,7 +52,7 @@ int cuspx_param_id(const char *name);            /* "sha2-128f", ... ; -2 if unk
 int cuspx_get_param_info(int pid, cuspx_param_info *out);
 int cuspx_set_default_param(int pid);
 /* Work split of set pid at every batch size.  op 0 (sign) / 2 (keygen): lanes
- * per WOTS leaf of the hypertree kernel (1, 2, 4, 8, 16).  op 1 (verify): mean
+ * per WOTS leaf of the hypertree kernel (1, 2, 4, 8, 16; 4 runs as 2, 8 as 16).  op 1 (verify): mean
  * lanes per request of the verify kernel, which runs 256 / lanes requests per
  * workgroup (16, 32, 64; also 128 when len = 67), or 1 for speculative
  * verification (every WOTS chain from every start computed up front, then
@@ -201,8 +201,9 @@ int cuspx_graph_verify(int pid, uint32_t num, const uint8_t *pk, uint32_t pk_str
  * cuspx_sign_device; each with its own workspace).  When the non-empty
  * groups are distinct fast sets of one hash family (sha2-128f/192f/256f or
  * shake256-128f/192f/256f) and each is large enough to run at one or two
- * lanes per WOTS leaf, they are signed by ONE persistent kernel whose tile queue spans every set
- * (after each set's prep kernel; T_k and the WOTS gather per set after it).
+ * lanes per WOTS leaf, the chains of all sets run in one launch (after each
+ * set's prep and FORS kernels; subtrees, T_k and the WOTS gather per set after
+ * it).
  * Other mixes run each group's own pipeline on a forked stream.  Not in the
  * reference (its batches are single-set, sign.cu:5098). */
 typedef struct {
@@ -219,7 +220,7 @@ typedef struct {
     void *ws;
 } cuspx_sign_group;
 int cuspx_graph_sign_mixed(const cuspx_sign_group *groups, int ngroups, cuspx_graph **out);
-/* the same mixed batch launched directly on `stream` (the persistent kernel
+/* the same mixed batch launched directly on `stream` (the shared launch
  * when it applies, else the groups one after another) */
 int cuspx_sign_mixed_device(const cuspx_sign_group *groups, int ngroups, void *stream);
 int cuspx_graph_launch(cuspx_graph *g, void *stream);
