@@ -655,11 +655,10 @@ def sign_mixed_device(groups, stream=None):
 class MixedSignBatch:
     """A resident mixed-parameter-set signing batch: requests are grouped by
     set, each group gets device buffers and a workspace, and the whole batch
-    is one hipGraph (one launch per replay).  Distinct fast sets of one hash
-    family, each large enough for one or two lanes per WOTS leaf, share one
-    launch of their chains; other mixes run each set's pipeline on its own forked
-    stream.  launch(eager=True) launches the same batch
-    without the graph.
+    is one hipGraph (one launch per replay), each set's pipeline on its own
+    forked stream.  launch(eager=True) launches the same batch without the
+    graph: distinct fast sets of one hash family, each large enough for one or
+    two lanes per WOTS leaf, then share one launch of their chains.
 
     items: list of (pid, sk bytes, message bytes, optrand bytes)."""
 
