@@ -1,5 +1,5 @@
 """Verification's hypertree kernel in each of its forms: chain steps on a lane,
-on a lane pair (a workgroup per CU, groups of 64 lanes or more) and in
+on a lane pair (groups of 64 lanes or more) and in
 two-phase rounds (SHA-256, more workgroups than CUs), with a last workgroup
 that is not full.  Every request's verdict is known: signatures are the
 oracle's (the first of each set is compared with it), some with one bit
