@@ -62,8 +62,7 @@ struct FamilyImpl {
     template <class P>
     static void tail(const BatchArgs& A, uint32_t n, hipStream_t s) {
         if (!n) return;
-        hipLaunchKernelGGL((k_ht<P, 0, 1>), dim3(Layout<P>::template ht_blocks<1>(n * P::d)),
-                           dim3(HtShape<P, 1>::WG), 0, s, A);
+        launch_ht<P, 0, 1>(A, s);
         prof_mark(s, "k_ht");
         if (!A.fors_count) {
             launch_fors_pk<P>(A, n, s);
@@ -85,8 +84,6 @@ struct FamilyImpl {
         args<P0>(b[0], A0, pid_[0]);
         args<P1>(b[1], A1, pid_[1]);
         args<P2>(b[2], A2, pid_[2]);
-        FamilyWaves W{{chain_waves<P0>(n0 * P0::d), chain_waves<P1>(n1 * P1::d),
-                       chain_waves<P2>(n2 * P2::d)}};
         (void)hipGetLastError();  // report only errors of these launches
         prof_begin(s, "family");
         // prep_grid sets fields of the BatchArgs: call it before the launch
@@ -102,8 +99,21 @@ struct FamilyImpl {
         fors<P1, J1>(A1, n1, s);
         fors<P2, J2>(A2, n2, s);
         prof_mark(s, "k_fors");
-        const uint32_t grid = cdiv((uint64_t)W.n[0] + W.n[1] + W.n[2], 4);
-        hipLaunchKernelGGL((k_sign_family<P0, P1, P2>), dim3(grid), dim3(256), 0, s, A0, A1, A2, W);
+        // slices of the same share of every set (slices.hpp)
+        const uint64_t waves = (uint64_t)chain_waves<P0>(n0 * P0::d) + chain_waves<P1>(n1 * P1::d) +
+                               chain_waves<P2>(n2 * P2::d);
+        const uint64_t c = 64 * waves / kSliceLanes + 1;
+        for (uint64_t i = 0; i < c; i++) {
+            const uint32_t a0 = n0 * i / c, a1 = n1 * i / c, a2 = n2 * i / c;
+            const BatchArgs B0 = batch_rows<P0, 0>(A0, a0, n0 * (i + 1) / c - a0),
+                            B1 = batch_rows<P1, 0>(A1, a1, n1 * (i + 1) / c - a1),
+                            B2 = batch_rows<P2, 0>(A2, a2, n2 * (i + 1) / c - a2);
+            FamilyWaves W{{chain_waves<P0>(B0.n_req * P0::d), chain_waves<P1>(B1.n_req * P1::d),
+                           chain_waves<P2>(B2.n_req * P2::d)}};
+            const uint32_t grid = cdiv((uint64_t)W.n[0] + W.n[1] + W.n[2], 4);
+            hipLaunchKernelGGL((k_sign_family<P0, P1, P2>), dim3(grid), dim3(256), 0, s, B0, B1, B2,
+                               W);
+        }
         prof_mark(s, "k_sign_family");
         tail<P0>(A0, n0, s);
         tail<P1>(A1, n1, s);

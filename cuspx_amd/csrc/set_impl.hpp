@@ -3,6 +3,7 @@
 #pragma once
 #include "engine.hpp"
 #include "profile.hpp"
+#include "slices.hpp"
 #include "spx_kernels.hpp"
 
 namespace spx {
@@ -182,6 +183,50 @@ inline void launch_fors(const BatchArgs& A, uint32_t n, hipStream_t s) {
         hipLaunchKernelGGL((k_fors<P, J, false>), dim3(tiles), dim3(256), 0, s, A);
 }
 
+// A's requests [a, a + n) as a batch of their own for the chains' and the
+// subtrees' kernels, in A's workspace and outputs (MODE as for those kernels)
+template <class P, int MODE>
+inline BatchArgs batch_rows(const BatchArgs& A, uint32_t a, uint32_t n) {
+    BatchArgs B = A;
+    const size_t trees = (size_t)a * (MODE == 0 ? P::d : 1);
+    B.n_req = n;
+    B.plan += a;
+    B.tl_buf += trees << P::th;  // columns; tl_lanes stays the whole batch's
+    if (B.ht_parts) {
+        B.ht_parts += trees * (Layout<P>::max_parts() * P::nw);
+        B.ht_count += trees;
+    }
+    if (MODE == 0) {
+        B.sig += a * B.sig_stride;
+        B.roots += trees * P::n;
+        B.cap += trees * (P::len * 16 * P::n);
+    } else {
+        B.pk_out += (size_t)a * P::pk_bytes;
+        B.sk_out += (size_t)a * P::sk_bytes;
+    }
+    return B;
+}
+
+template <class P, int MODE, bool PH>
+inline void launch_chains(const BatchArgs& A, hipStream_t s) {
+    constexpr uint32_t trees = MODE == 0 ? P::d : 1;
+    for_slices(A.n_req, 64ull * chain_waves<P>(A.n_req * trees), [&](uint32_t a, uint32_t n) {
+        const uint32_t nwaves = chain_waves<P>(n * trees);
+        hipLaunchKernelGGL((k_chains<P, MODE, PH>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s,
+                           batch_rows<P, MODE>(A, a, n), nwaves);
+    });
+}
+template <class P, int MODE, int S>
+inline void launch_ht(const BatchArgs& A, hipStream_t s) {
+    constexpr uint32_t trees = MODE == 0 ? P::d : 1, WG = HtShape<P, S>::WG;
+    for_slices(A.n_req, (uint64_t)WG * Layout<P>::template ht_blocks<S>(A.n_req * trees),
+               [&](uint32_t a, uint32_t n) {
+                   hipLaunchKernelGGL((k_ht<P, MODE, S>),
+                                      dim3(Layout<P>::template ht_blocks<S>(n * trees)), dim3(WG),
+                                      0, s, batch_rows<P, MODE>(A, a, n));
+               });
+}
+
 template <class P, int J>
 struct SetImpl {
     using Lay = Layout<P>;
@@ -191,16 +236,10 @@ struct SetImpl {
     static size_t workspace(uint32_t n, int op) { return (size_t)Lay::bytes(pid_, n, op); }
 
     template <int MODE>
-    static void launch_ht(const BatchArgs& A, uint32_t trees, int S, hipStream_t s) {
-        if (S == 1)
-            hipLaunchKernelGGL((k_ht<P, MODE, 1>), dim3(Lay::template ht_blocks<1>(trees)),
-                               dim3(HtShape<P, 1>::WG), 0, s, A);
-        else if (S <= 4)
-            hipLaunchKernelGGL((k_ht<P, MODE, 2>), dim3(Lay::template ht_blocks<2>(trees)),
-                               dim3(256), 0, s, A);
-        else
-            hipLaunchKernelGGL((k_ht<P, MODE, 16>), dim3(Lay::template ht_blocks<16>(trees)),
-                               dim3(256), 0, s, A);
+    static void launch_ht(const BatchArgs& A, int S, hipStream_t s) {
+        if (S == 1) spx::launch_ht<P, MODE, 1>(A, s);
+        else if (S <= 4) spx::launch_ht<P, MODE, 2>(A, s);
+        else spx::launch_ht<P, MODE, 16>(A, s);
     }
     // a launch of so many waves leaves each of them a SIMD (HashPh)
     static constexpr bool kSha = P::hash == kSha2;
@@ -271,15 +310,14 @@ struct SetImpl {
         } else {
             launch_fors<P, J>(A, n, s);
             prof_mark(s, "k_fors");
-            hipLaunchKernelGGL((k_chains<P, 0, true>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
-                               nwaves);
+            launch_chains<P, 0, true>(A, s);
             prof_mark(s, "k_chains");
         }
         if (!A.fors_count) {
             launch_fors_pk<P>(A, n, s);
             prof_mark(s, "k_fors_pk");
         }
-        launch_ht<0>(A, n * P::d, S, s);
+        launch_ht<0>(A, S, s);
         prof_mark(s, "k_ht");
         hipLaunchKernelGGL((k_wots_gather<P>), dim3(cdiv((uint64_t)n * P::d * P::len, 256)),
                            dim3(256), 0, s, A);
@@ -349,15 +387,10 @@ struct SetImpl {
         prof_begin(s, set_name_);
         hipLaunchKernelGGL((k_kprep<P>), dim3(cdiv(n, 64)), dim3(64), 0, s, A);
         prof_mark(s, "k_kprep");
-        const uint32_t nwaves = chain_waves<P>(n);
-        if (alone(nwaves))
-            hipLaunchKernelGGL((k_chains<P, 1, !kSha>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
-                               nwaves);
-        else
-            hipLaunchKernelGGL((k_chains<P, 1, true>), dim3(cdiv(nwaves, 4)), dim3(256), 0, s, A,
-                               nwaves);
+        if (alone(chain_waves<P>(n))) launch_chains<P, 1, !kSha>(A, s);
+        else launch_chains<P, 1, true>(A, s);
         prof_mark(s, "k_chains_keygen");
-        launch_ht<1>(A, n, S, s);
+        launch_ht<1>(A, S, s);
         prof_mark(s, "k_ht_keygen");
         return hipGetLastError() == hipSuccess ? 0 : kErrHip;
     }
