@@ -81,9 +81,9 @@ struct BatchArgs {
     uint32_t* ht_count;       // split subtrees: parts finished per tree (zeroed by the prep kernel)
     uint32_t* fors_count;     // FORS roots finished per request (zeroed by the prep kernels)
     uint32_t n_req;
-    // prep kernels: workgroups of the lane-pair part; messages of long_min
-    // bytes or more (0: none) are hashed by the two-wave part after them
-    uint32_t prep_wgs;
+    // prep kernels: messages of long_min bytes or more (0: none) are hashed by
+    // the first long_wgs workgroups, in their two-wave form
+    uint32_t long_wgs;
     uint32_t long_min;
 };
 
@@ -117,7 +117,7 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
     pl.leaf = leaf;
 }
 
-// The prep kernels (128-lane workgroups).  Workgroups [0, prep_wgs): every
+// The prep kernels (128-lane workgroups).  Workgroups from long_wgs on: every
 // request hashes its message on a lane group; all its lanes compute
 // everything, the first one stores.  SHA-256: 8 lanes, 16 requests per
 // workgroup; the message's blocks run on each pair alike, the HMAC keys, the
@@ -125,9 +125,12 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
 // dependent blocks are 6 (SHA2-128f, 32 bytes: 30.4 -> 25.0 us at 1 request,
 // 45 -> 37 at 4096; k_vprep 19.8 -> 15.5).  SHAKE256: 32 lanes, Keccak32, 4
 // requests.  SHA-256 messages of at least long_min bytes are left to the
-// workgroups after those: each takes long requests in turn and runs one with
+// workgroups before those: each takes long requests in turn and runs one with
 // both waves (Sha2::stream_msg_long), the schedules of its message-only blocks
-// computed by wave 1 ahead of wave 0's rounds.
+// computed by wave 1 ahead of wave 0's rounds.  They come first so that the
+// dispatcher spreads them evenly: placed among thousands of short workgroups
+// that end at once, some CUs held several of them to the end (65536 SHA2-128f
+// requests of 4 KiB, k_vprep 28-38 ms; 12.5 ms first).
 //
 // Lanes past the last request repeat it and store nothing, here and in the
 // other kernels whose time is one wave's: a wave with less than all its
@@ -214,20 +217,21 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
     // one serial hash chain per request over the whole message: ask the SIMD
     // arbiter to favour these waves over concurrent bulk hypertree waves
     __builtin_amdgcn_s_setprio(3);
-    if (blockIdx.x >= A.prep_wgs) {
+    if (blockIdx.x < A.long_wgs) {
         if constexpr (prep_has_long<P>()) {
             __shared__ __align__(16) uint32_t kw_s[HashT<P>::kLongLdsWords];
             const bool prod = threadIdx.x >= 64;
 #pragma unroll 1
-            for (uint32_t i = blockIdx.x - A.prep_wgs; i < A.n_req; i += gridDim.x - A.prep_wgs)
+            for (uint32_t i = blockIdx.x; i < A.n_req; i += A.long_wgs)
                 if (prep_is_long(A, i))
                     prep_sign_one<P, true>(A, i, threadIdx.x == 0, (lds_u32*)kw_s, prod, nullptr);
         }
         return;
     }
     constexpr uint32_t PL = prep_lanes<P>();
-    const uint32_t i0 = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
-    if ((blockIdx.x * kPrepWg + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
+    const uint32_t lane0 = (blockIdx.x - A.long_wgs) * kPrepWg;
+    const uint32_t i0 = (lane0 + threadIdx.x) / PL;
+    if ((lane0 + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
     const uint32_t i = i0 < A.n_req ? i0 : A.n_req - 1;
     const bool first = i0 < A.n_req && threadIdx.x % PL == 0;
     if (A.ht_count && first) {
@@ -292,20 +296,21 @@ __device__ __forceinline__ void prep_verify_one(const BatchArgs& A, uint32_t i, 
 template <class P>
 __global__ void __launch_bounds__(kPrepWg) k_vprep(BatchArgs A) {
     __builtin_amdgcn_s_setprio(3);  // serial message hash per request, as in k_prep
-    if (blockIdx.x >= A.prep_wgs) {
+    if (blockIdx.x < A.long_wgs) {
         if constexpr (prep_has_long<P>()) {
             __shared__ __align__(16) uint32_t kw_s[HashT<P>::kLongLdsWords];
             const bool prod = threadIdx.x >= 64;
 #pragma unroll 1
-            for (uint32_t i = blockIdx.x - A.prep_wgs; i < A.n_req; i += gridDim.x - A.prep_wgs)
+            for (uint32_t i = blockIdx.x; i < A.n_req; i += A.long_wgs)
                 if (prep_is_long(A, i))
                     prep_verify_one<P, true>(A, i, threadIdx.x == 0, (lds_u32*)kw_s, prod, nullptr);
         }
         return;
     }
     constexpr uint32_t PL = prep_lanes<P>();
-    const uint32_t i0 = (blockIdx.x * kPrepWg + threadIdx.x) / PL;
-    if ((blockIdx.x * kPrepWg + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
+    const uint32_t lane0 = (blockIdx.x - A.long_wgs) * kPrepWg;
+    const uint32_t i0 = (lane0 + threadIdx.x) / PL;
+    if ((lane0 + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
     const uint32_t i = i0 < A.n_req ? i0 : A.n_req - 1;
     const bool first = i0 < A.n_req && threadIdx.x % PL == 0;
     if (prep_is_long(A, i)) return;
@@ -321,13 +326,13 @@ __global__ void __launch_bounds__(kPrepWg) k_vprep(BatchArgs A) {
 }
 
 // grid of the prep kernels for n requests whose messages are at most
-// mlen_bound bytes (0: not known); sets A.prep_wgs / A.long_min
+// mlen_bound bytes (0: not known); sets A.long_wgs / A.long_min
 template <class P>
 inline uint32_t prep_grid(BatchArgs& A, uint32_t n, uint32_t mlen_bound) {
-    A.prep_wgs = (uint32_t)(((uint64_t)n * prep_lanes<P>() + kPrepWg - 1) / kPrepWg);
     const bool lng = prep_has_long<P>() && (mlen_bound == 0 || mlen_bound >= kLongMsgBytes);
     A.long_min = lng ? kLongMsgBytes : 0;
-    return A.prep_wgs + (lng ? (n < kLongWgs ? n : kLongWgs) : 0);
+    A.long_wgs = !lng ? 0 : n < kLongWgs ? n : kLongWgs;
+    return A.long_wgs + (uint32_t)(((uint64_t)n * prep_lanes<P>() + kPrepWg - 1) / kPrepWg);
 }
 
 // resident-key midstates: mid[i] = state after pub_seed || 0^(64-n) for the
