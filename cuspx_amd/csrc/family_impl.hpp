@@ -86,14 +86,9 @@ struct FamilyImpl {
         args<P2>(b[2], A2, pid_[2]);
         (void)hipGetLastError();  // report only errors of these launches
         prof_begin(s, "family");
-        // prep_grid sets fields of the BatchArgs: call it before the launch
-        // that copies them
-        const uint32_t g0 = n0 ? prep_grid<P0>(A0, n0, b[0].mlen_bound) : 0;
-        const uint32_t g1 = n1 ? prep_grid<P1>(A1, n1, b[1].mlen_bound) : 0;
-        const uint32_t g2 = n2 ? prep_grid<P2>(A2, n2, b[2].mlen_bound) : 0;
-        if (n0) hipLaunchKernelGGL((k_prep<P0>), dim3(g0), dim3(kPrepWg), 0, s, A0);
-        if (n1) hipLaunchKernelGGL((k_prep<P1>), dim3(g1), dim3(kPrepWg), 0, s, A1);
-        if (n2) hipLaunchKernelGGL((k_prep<P2>), dim3(g2), dim3(kPrepWg), 0, s, A2);
+        if (n0) launch_prep<P0, false>(A0, n0, b[0].mlen_bound, s);
+        if (n1) launch_prep<P1, false>(A1, n1, b[1].mlen_bound, s);
+        if (n2) launch_prep<P2, false>(A2, n2, b[2].mlen_bound, s);
         prof_mark(s, "k_prep");
         fors<P0, J0>(A0, n0, s);
         fors<P1, J1>(A1, n1, s);

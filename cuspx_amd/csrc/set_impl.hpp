@@ -285,8 +285,7 @@ struct SetImpl {
         Lay::carve(pid_, A, (uint8_t*)b.ws, b.n, kOpSign);
         (void)hipGetLastError();  // report only errors of these launches
         prof_begin(s, set_name_);
-        const uint32_t prep_grid_wgs = prep_grid<P>(A, n, b.mlen_bound);  // sets fields of A
-        hipLaunchKernelGGL((k_prep<P>), dim3(prep_grid_wgs), dim3(kPrepWg), 0, s, A);
+        launch_prep<P, false>(A, n, b.mlen_bound, s);
         prof_mark(s, "k_prep");
         // (up to kForsPkInline requests T_k runs on the lane that stores a
         // request's last FORS root, inside the FORS tiles)
@@ -343,8 +342,7 @@ struct SetImpl {
         const int G = Lay::vsplit(pid_, n);
         (void)hipGetLastError();  // report only errors of these launches
         prof_begin(s, set_name_);
-        const uint32_t prep_grid_wgs = prep_grid<P>(A, n, b.mlen_bound);  // sets fields of A
-        hipLaunchKernelGGL((k_vprep<P>), dim3(prep_grid_wgs), dim3(kPrepWg), 0, s, A);
+        launch_prep<P, true>(A, n, b.mlen_bound, s);
         prof_mark(s, "k_vprep");
         if (G == 1) {
             const uint32_t nf = cdiv((uint64_t)n * P::k, 256);

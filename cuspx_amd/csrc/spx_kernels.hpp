@@ -124,7 +124,7 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
 // MGF1 blocks and the midstate on a pair each, so that a short message's 9
 // dependent blocks are 6 (SHA2-128f, 32 bytes: 30.4 -> 25.0 us at 1 request,
 // 45 -> 37 at 4096; k_vprep 19.8 -> 15.5).  SHAKE256: 32 lanes, Keccak32, 4
-// requests.  SHA-256 messages of at least long_min bytes are left to the
+// requests, and a lane pair in large batches.  SHA-256 messages of at least long_min bytes are left to the
 // workgroups before those: each takes long requests in turn and runs one with
 // both waves (Sha2::stream_msg_long), the schedules of its message-only blocks
 // computed by wave 1 ahead of wave 0's rounds.  They come first so that the
@@ -138,7 +138,15 @@ __device__ __forceinline__ void plan_from_digest(Plan& pl, const uint8_t* dg) {
 // by up to 3.5 times, changing from launch to launch (T_len's rounds on a
 // pair: 2.9k cycles a block with all lanes active, 2.9-10k with two of 16).
 template <class P>
-__host__ __device__ constexpr uint32_t prep_lanes() { return P::hash == kSha2 ? 8 : 32; }
+__host__ __device__ constexpr uint32_t prep_lanes(bool pair) {
+    return pair ? 2 : P::hash == kSha2 ? 8 : 32;
+}
+// SHAKE256 requests up to which a row of 32 lanes hashes a message: beyond,
+// the rows' instructions (two requests a wave) last longer than a lane pair's
+// serial run.  k_vprep of SHAKE256-128f, rows / pairs, us: 6144 requests of
+// 1000 B 57 / 62, of 16 KiB 715 / 734; 8192 68 / 62 and 900 / 734; 16384 of 16
+// KiB 1672 / 736; 65536 of 4 KiB 1665 / 385.
+constexpr uint32_t kPrepRows = 7168;
 constexpr uint32_t kPrepWg = 128;
 // the two-wave path from this length: a single SHA2-128f / 256f request of
 // 512 B signs in 0.329 / 0.624 ms against 0.336 / 0.634 on the lane pair,
@@ -164,8 +172,8 @@ __device__ __forceinline__ void prep_midstate(const BatchArgs& A, uint32_t row,
 
 // sign, one request: midstate, R = PRF_msg, digest = H_msg, plan; LONG: the
 // two-wave form over kw_s (prod: wave 1), else a lane group (SHAKE256: with
-// its row's sponge k)
-template <class P, bool LONG>
+// its row's sponge k, or a lane pair)
+template <class P, bool LONG, bool PAIR = false>
 __device__ __forceinline__ void prep_sign_one(const BatchArgs& A, uint32_t i, bool store,
                                               lds_u32* kw_s, bool prod, Keccak32* k) {
     using Hh = HashT<P>;
@@ -193,8 +201,8 @@ __device__ __forceinline__ void prep_sign_one(const BatchArgs& A, uint32_t i, bo
         Hh::template prf_msg<true>(skprf, opt, m, ml, R, kw_s, prod);
         Hh::template h_msg<P::dgst_bytes, true>(R, pk, m, ml, dg, mid, kw_s, prod);
     } else if constexpr (P::hash == kShake) {
-        Hh::prf_msg(*k, skprf, opt, m, ml, R);
-        Hh::template h_msg<P::dgst_bytes>(*k, R, pk, m, ml, dg);
+        Hh::template prf_msg<PAIR>(k, skprf, opt, m, ml, R);
+        Hh::template h_msg<P::dgst_bytes, PAIR>(k, R, pk, m, ml, dg);
     } else {
         Hh::prf_msg(skprf, opt, m, ml, R);
         Hh::template h_msg<P::dgst_bytes>(R, pk, m, ml, dg, mid);
@@ -212,7 +220,7 @@ __device__ __forceinline__ void prep_sign_one(const BatchArgs& A, uint32_t i, bo
 }
 
 // sign: midstate, R = PRF_msg, digest = H_msg, plan
-template <class P>
+template <class P, bool PAIR>
 __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
     // one serial hash chain per request over the whole message: ask the SIMD
     // arbiter to favour these waves over concurrent bulk hypertree waves
@@ -228,7 +236,7 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
         }
         return;
     }
-    constexpr uint32_t PL = prep_lanes<P>();
+    constexpr uint32_t PL = prep_lanes<P>(PAIR);
     const uint32_t lane0 = (blockIdx.x - A.long_wgs) * kPrepWg;
     const uint32_t i0 = (lane0 + threadIdx.x) / PL;
     if ((lane0 + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
@@ -240,20 +248,20 @@ __global__ void __launch_bounds__(kPrepWg) k_prep(BatchArgs A) {
     }
     if (A.fors_count && first) A.fors_count[i] = 0;
     if (prep_is_long(A, i)) return;
-    if constexpr (P::hash == kShake) {
+    if constexpr (P::hash == kShake && !PAIR) {
         constexpr int RW = HashT<P>::kRowWords;
         __shared__ __align__(16) uint32_t row_s[kPrepWg / PL * RW];
         Keccak32 k;
         k.init((lds_u32*)row_s + threadIdx.x / PL * RW);
         prep_sign_one<P, false>(A, i, first, nullptr, false, &k);
     } else {
-        prep_sign_one<P, false>(A, i, first, nullptr, false, nullptr);
+        prep_sign_one<P, false, PAIR>(A, i, first, nullptr, false, nullptr);
     }
 }
 
 // verify, one request: midstate, digest = H_msg(R from the signature), plan
-// (LONG as for prep_sign_one)
-template <class P, bool LONG>
+// (LONG, PAIR as for prep_sign_one)
+template <class P, bool LONG, bool PAIR = false>
 __device__ __forceinline__ void prep_verify_one(const BatchArgs& A, uint32_t i, bool store,
                                                 lds_u32* kw_s, bool prod, Keccak32* k) {
     using Hh = HashT<P>;
@@ -278,7 +286,7 @@ __device__ __forceinline__ void prep_verify_one(const BatchArgs& A, uint32_t i, 
         Hh::template h_msg<P::dgst_bytes, true>(R, pk, A.msg + A.moff[i], A.mlen[i], dg, mid,
                                                 kw_s, prod);
     } else if constexpr (P::hash == kShake) {
-        Hh::template h_msg<P::dgst_bytes>(*k, R, pk, A.msg + A.moff[i], A.mlen[i], dg);
+        Hh::template h_msg<P::dgst_bytes, PAIR>(k, R, pk, A.msg + A.moff[i], A.mlen[i], dg);
     } else {
         Hh::template h_msg<P::dgst_bytes>(R, pk, A.msg + A.moff[i], A.mlen[i], dg, mid);
     }
@@ -293,7 +301,7 @@ __device__ __forceinline__ void prep_verify_one(const BatchArgs& A, uint32_t i, 
 }
 
 // verify: midstate, digest = H_msg(R from the signature), plan
-template <class P>
+template <class P, bool PAIR>
 __global__ void __launch_bounds__(kPrepWg) k_vprep(BatchArgs A) {
     __builtin_amdgcn_s_setprio(3);  // serial message hash per request, as in k_prep
     if (blockIdx.x < A.long_wgs) {
@@ -307,32 +315,50 @@ __global__ void __launch_bounds__(kPrepWg) k_vprep(BatchArgs A) {
         }
         return;
     }
-    constexpr uint32_t PL = prep_lanes<P>();
+    constexpr uint32_t PL = prep_lanes<P>(PAIR);
     const uint32_t lane0 = (blockIdx.x - A.long_wgs) * kPrepWg;
     const uint32_t i0 = (lane0 + threadIdx.x) / PL;
     if ((lane0 + (threadIdx.x & ~63u)) / PL >= A.n_req) return;  // an empty wave
     const uint32_t i = i0 < A.n_req ? i0 : A.n_req - 1;
     const bool first = i0 < A.n_req && threadIdx.x % PL == 0;
     if (prep_is_long(A, i)) return;
-    if constexpr (P::hash == kShake) {
+    if constexpr (P::hash == kShake && !PAIR) {
         constexpr int RW = HashT<P>::kRowWords;
         __shared__ __align__(16) uint32_t row_s[kPrepWg / PL * RW];
         Keccak32 k;
         k.init((lds_u32*)row_s + threadIdx.x / PL * RW);
         prep_verify_one<P, false>(A, i, first, nullptr, false, &k);
     } else {
-        prep_verify_one<P, false>(A, i, first, nullptr, false, nullptr);
+        prep_verify_one<P, false, PAIR>(A, i, first, nullptr, false, nullptr);
     }
 }
 
 // grid of the prep kernels for n requests whose messages are at most
 // mlen_bound bytes (0: not known); sets A.long_wgs / A.long_min
-template <class P>
+template <class P, bool PAIR>
 inline uint32_t prep_grid(BatchArgs& A, uint32_t n, uint32_t mlen_bound) {
     const bool lng = prep_has_long<P>() && (mlen_bound == 0 || mlen_bound >= kLongMsgBytes);
     A.long_min = lng ? kLongMsgBytes : 0;
     A.long_wgs = !lng ? 0 : n < kLongWgs ? n : kLongWgs;
-    return A.long_wgs + (uint32_t)(((uint64_t)n * prep_lanes<P>() + kPrepWg - 1) / kPrepWg);
+    return A.long_wgs + (uint32_t)(((uint64_t)n * prep_lanes<P>(PAIR) + kPrepWg - 1) / kPrepWg);
+}
+// sets fields of A, which later launches then carry along
+template <class P, bool VERIFY>
+inline void launch_prep(BatchArgs& A, uint32_t n, uint32_t mlen_bound, hipStream_t s) {
+    auto go = [&](auto pair) {
+        constexpr bool PAIR = decltype(pair)::value;
+        const uint32_t wgs = prep_grid<P, PAIR>(A, n, mlen_bound);
+        if constexpr (VERIFY)
+            hipLaunchKernelGGL((k_vprep<P, PAIR>), dim3(wgs), dim3(kPrepWg), 0, s, A);
+        else hipLaunchKernelGGL((k_prep<P, PAIR>), dim3(wgs), dim3(kPrepWg), 0, s, A);
+    };
+    if constexpr (P::hash == kShake) {
+        if (n > kPrepRows) {
+            go(std::true_type{});
+            return;
+        }
+    }
+    go(std::false_type{});
 }
 
 // resident-key midstates: mid[i] = state after pub_seed || 0^(64-n) for the
