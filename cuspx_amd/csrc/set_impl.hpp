@@ -167,6 +167,11 @@ static constexpr uint32_t kFuseWaves = 8192;
 // SHAKE256-256f 1 278 -> 138, 7 321 -> 245, 14 (3987) 399 -> 436;
 // SHA2-256f 14 201 -> 194, 28 315 -> 332.
 static constexpr uint32_t kShortForsWaves = 3584;
+// Waves of FORS tiles up to which a tree of 2^14 leaves (192s, 256s) is split
+// over 4 workgroups, whose last one climbs the top two levels: one workgroup
+// per tree is a serial run of 64 leaves and their nodes on every lane, about
+// 270 hashes, which nothing else in a small batch hides.  SPLITFIG
+static constexpr uint32_t kSplitForsWaves = 4096;
 
 // J: FORS leaves per lane, 2^J (2^(a-J) lanes per tree).  Short tiles at every
 // size: a tile is a serial run of 3-4 x 2^J hashes, and with the two-phase
@@ -245,10 +250,17 @@ struct SetImpl {
     static constexpr bool kSha = P::hash == kSha2;
     static bool alone(uint32_t waves) { return kSha && waves <= kAloneWaves; }
     // FORS leaves per lane in a fused launch of few waves: 2, or as many as 256
-    // lanes per tree leave
-    static constexpr int JF = P::a - 8 > 1 ? P::a - 8 : 1;
+    // lanes per tree leave; trees of 2^14 leaves (192s, 256s) are split over
+    // FP = 4 workgroups (kSplitForsWaves)
+    static constexpr int JF = P::a - 8 > 4 ? P::a - 10 : P::a - 8 > 1 ? P::a - 8 : 1;
+    static constexpr int FP = fors_parts<P, JF>();
+    static_assert(FP == 1 || P::k * FP <= P::d * Lay::max_parts(), "the parts' roots fit ht_parts");
     template <int FJ>
-    static uint32_t fors_tiles(uint32_t n) { return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ)); }
+    static uint32_t fors_tiles(uint32_t n) {
+        constexpr int parts = fors_parts<P, FJ>();
+        if constexpr (parts > 1) return n * (P::k * parts);
+        else return cdiv((uint64_t)n * P::k, 256u >> (P::a - FJ));
+    }
 
     // workgroups of k_vht up to which each has a CU to itself
     static constexpr uint32_t kVhtAlone = 256;
@@ -291,7 +303,7 @@ struct SetImpl {
         // request's last FORS root, inside the FORS tiles)
         const uint32_t nwaves = chain_waves<P>(n * P::d);
         if (nwaves <= kFuseWaves) {
-            if (nwaves <= kShortForsWaves) {
+            if (FP > 1 || nwaves <= kShortForsWaves) {
                 const uint32_t nf = fors_tiles<JF>(n);
                 const uint32_t wgs = nf + cdiv(nwaves, 4);
                 if (alone(4 * wgs))
@@ -300,14 +312,23 @@ struct SetImpl {
                 else
                     hipLaunchKernelGGL((k_sign_fused<P, JF, true>), dim3(wgs), dim3(256), 0, s, A,
                                        nf, nwaves);
-            } else {
+            } else if constexpr (FP == 1) {
                 const uint32_t nf = fors_tiles<J>(n);
                 hipLaunchKernelGGL((k_sign_fused<P, J, true>), dim3(nf + cdiv(nwaves, 4)),
                                    dim3(256), 0, s, A, nf, nwaves);
             }
             prof_mark(s, "k_sign_fused");
         } else {
-            launch_fors<P, J>(A, n, s);
+            if (FP > 1 && 4 * fors_tiles<JF>(n) <= kSplitForsWaves) {
+                if constexpr (FP > 1) {
+                    const uint32_t nf = fors_tiles<JF>(n);
+                    if (alone(4 * nf))
+                        hipLaunchKernelGGL((k_fors<P, JF, true, !kSha>), dim3(nf), dim3(256), 0, s, A);
+                    else hipLaunchKernelGGL((k_fors<P, JF, true>), dim3(nf), dim3(256), 0, s, A);
+                }
+            } else {
+                launch_fors<P, J>(A, n, s);
+            }
             prof_mark(s, "k_fors");
             launch_chains<P, 0, true>(A, s);
             prof_mark(s, "k_chains");

@@ -77,7 +77,8 @@ struct BatchArgs {
     uint8_t* cap;             // [N][d][len][16][n]
     uint32_t* tl_buf;         // chain ends: [len*nw][leaves]
     uint32_t tl_lanes;
-    uint32_t* ht_parts;       // split subtrees: part roots [tree][part][nw]
+    uint32_t* ht_parts;       // split subtrees (before them, split FORS trees): part roots
+                              // [tree][part][nw]
     uint32_t* ht_count;       // split subtrees: parts finished per tree (zeroed by the prep kernel)
     uint32_t* fors_count;     // FORS roots finished per request (zeroed by the prep kernels)
     uint32_t n_req;
@@ -421,12 +422,19 @@ __host__ __device__ constexpr int fors_pk_wave_words();
 // request come from several workgroups; every counter was zeroed by the prep
 // kernel).  Large batches launch k_fors_pk instead: there the per-tile
 // release fences (an L2 write-back each) cost more than the launch.
-template <class P>
+// (FP: parts of a tree, each counted)
+template <class P, int FP>
 __device__ __forceinline__ bool fors_root_done(const BatchArgs& A, uint32_t req) {
     __threadfence();  // release this root before counting it
-    const bool last = atomicAdd(&A.fors_count[req], 1u) == (uint32_t)P::k - 1;
+    const bool last = atomicAdd(&A.fors_count[req], 1u) == (uint32_t)(P::k * FP) - 1;
     if (last) __threadfence();  // acquire: every root of the request is visible
     return last;
+}
+
+// workgroups of 256 lanes that a FORS tree of 2^J leaves per lane is split over
+template <class P, int J>
+__host__ __device__ constexpr int fors_parts() {
+    return P::a - J > 8 ? 1 << (P::a - J - 8) : 1;
 }
 
 // LDS words a FORS tile of set P uses (two levels of 256 nodes)
@@ -435,25 +443,74 @@ constexpr int fors_lds_words() {
     return 2 * 256 * P::nw;
 }
 
+// The top of request req's split FORS trees (FP parts each, their roots in
+// ht_parts) on a whole wave, a lane per tree: node m of 1 .. 2 FP - 1 (1 the
+// root) is H(2 m, 2 m + 1).  smem: 2 FP values per lane.  The FORS roots are
+// visible to the wave's later loads.
+template <class P, int FP, class Hh>
+__device__ __forceinline__ void fors_top(const BatchArgs& A, uint32_t req, lds_u32* smem) {
+    constexpr int NW = P::nw;
+    static_assert(2 * FP * 64 * NW <= fors_lds_words<P>() && P::k <= 64, "");
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t t = lane < (uint32_t)P::k ? lane : P::k - 1;  // repeated past the last tree
+    const Plan& pl = A.plan[req];
+    typename Hh::Key key;
+    Hh::load_key(pl, key);
+    Adr a = adr_make(0, pl.tree, kForsTree);
+    adr_keypair<P::th>(a, pl.leaf);
+    const uint32_t tg = pl.fors_idx[t];
+    uint8_t* rec = A.sig + (size_t)req * A.sig_stride + P::n + (size_t)t * (P::a + 1) * P::n;
+    const uint32_t* parts = A.ht_parts + ((size_t)req * P::k + t) * (FP * NW);
+    lds_u32* val = smem + lane;  // word w of node m at val[64 (m NW + w)]
+#pragma unroll 1
+    for (int i = 0; i < FP * NW; i++)
+        val[64 * (FP * NW + i)] = __builtin_nontemporal_load(parts + i);
+#pragma unroll 1
+    for (int m = FP - 1; m >= 1; m--) {
+        const uint32_t up = 31 - __builtin_clz((uint32_t)m);  // levels below the root
+        const uint32_t hgt = P::a - up, x = m - (1u << up);
+        uint32_t l[NW], r[NW], out[NW];
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            l[w] = val[64 * (2 * m * NW + w)];
+            r[w] = val[64 * ((2 * m + 1) * NW + w)];
+        }
+        adr_node(a, hgt, ((t << P::a) >> hgt) + x);
+        Hh::H(key, a, l, r, out);
+#pragma unroll
+        for (int w = 0; w < NW; w++) val[64 * (m * NW + w)] = out[w];
+        if (lane == t) {
+            if (m == 1)
+                store_val<P::hash, NW>(A.fors_roots + ((size_t)req * P::k + t) * P::n, out);
+            else if (x == ((tg >> hgt) ^ 1u))
+                store_val<P::hash, NW>(rec + P::n + (size_t)hgt * P::n, out);
+        }
+    }
+    __threadfence();
+}
+
 // sign: FORS trees, L = 2^(a-J) lanes per tree, 2^J leaves per lane; `blk`
-// is the workgroup's tile (TPW trees), so the same body serves the fused
-// signing kernels.  smem: fors_lds_words<P>() words of LDS owned by the kernel
+// is the workgroup's tile (TPW trees, or one of FP parts of a tree wider than
+// a workgroup), so the same body serves the fused signing kernels.  smem: fors_lds_words<P>() words of LDS owned by the kernel
 // PK: count the roots and run T_k here (fors_count set)
 template <class P, int J, bool PK, bool PH = true>
 __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint32_t* smem) {
     using Hh = HashPh<P, PH>;
     using Key = typename Hh::Key;
     constexpr int NW = P::nw;
-    constexpr int LOGL = P::a - J;
-    constexpr int L = 1 << LOGL;
     constexpr int WG = 256;
-    static_assert(L <= WG, "tree wider than a workgroup");
+    constexpr int FP = fors_parts<P, J>();
+    static_assert(FP == 1 || PK, "the last part climbs from the others' roots");
+    constexpr int LOGL = P::a - J - ilog2(FP);  // levels reduced in the workgroup
+    constexpr int L = 1 << LOGL;                // lanes of a tree, or of its part, here
     constexpr int TPW = WG / L;
     auto& lds = *reinterpret_cast<uint32_t (*)[2][WG][NW]>(smem);
 
     const int tid = threadIdx.x;
+    const uint32_t part = FP > 1 ? blk % FP : 0;
+    if (FP > 1) blk /= FP;
     const uint32_t g = blk * TPW + tid / L;  // global tree id
-    const uint32_t u = tid % L;
+    const uint32_t u = part * L + tid % L;
     const bool active = g < A.n_req * P::k;
     const uint32_t req = active ? g / P::k : 0;
     const uint32_t t = active ? g % P::k : 0;
@@ -514,7 +571,7 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
         if (tid < max_int(WG >> l, 64)) {
             const int i = tid & ((WG >> l) - 1);
             const uint32_t tau = i >> (LOGL - l);
-            const uint32_t x = i & ((L >> l) - 1);
+            const uint32_t x = part * (L >> l) + (i & ((L >> l) - 1));
             const uint32_t g2 = blk * TPW + tau;
             bool last = false;  // this lane stored its request's last root
             const bool act2 = g2 < A.n_req * P::k;
@@ -541,27 +598,39 @@ __device__ __forceinline__ void fors_tile(const BatchArgs& A, uint32_t blk, uint
                 const uint32_t tg = p2.fors_idx[t2];
                 if (hgt < (uint32_t)P::a && x == ((tg >> hgt) ^ 1u))
                     store_val<P::hash, NW>(rec2 + P::n + (size_t)hgt * P::n, out);
-                if (hgt == (uint32_t)P::a) {
+                if constexpr (FP > 1) {
+                    if (l == LOGL) {
+                        uint32_t* pr = A.ht_parts + ((size_t)g2 * FP + part) * NW;
+#pragma unroll
+                        for (int w = 0; w < NW; w++) pr[w] = out[w];
+                        last = fors_root_done<P, FP>(A, req2);
+                    }
+                } else if (hgt == (uint32_t)P::a) {
                     store_val<P::hash, NW>(A.fors_roots + ((size_t)req2 * P::k + t2) * P::n, out);
-                    if constexpr (PK) last = fors_root_done<P>(A, req2);
+                    if constexpr (PK) last = fors_root_done<P, 1>(A, req2);
                 }
             }
             if (PK && l == LOGL) {
                 // wave 0 alone is here (TPW <= 64): the tile's LDS is free
                 static_assert(TPW <= 64 && fors_pk_wave_words<P>() <= fors_lds_words<P>(), "");
 #pragma unroll 1
-                for (uint64_t m = __ballot(last); m; m &= m - 1)
-                    fors_pk_wave<P>(A, __shfl((int)req2, __ffsll((unsigned long long)m) - 1),
-                                    (lds_u32*)smem);
+                for (uint64_t m = __ballot(last); m; m &= m - 1) {
+                    const uint32_t rq = __shfl((int)req2, __ffsll((unsigned long long)m) - 1);
+                    if constexpr (FP > 1) {
+                        fors_top<P, FP, Hh>(A, rq, (lds_u32*)smem);
+                        Keccak16::order();
+                    }
+                    fors_pk_wave<P>(A, rq, (lds_u32*)smem);
+                }
             }
         }
     }
 }
 
-template <class P, int J, bool PK>
+template <class P, int J, bool PK, bool PH = true>
 __global__ void __launch_bounds__(256) k_fors(BatchArgs A) {
     __shared__ __align__(16) uint32_t smem[fors_lds_words<P>()];
-    fors_tile<P, J, PK>(A, blockIdx.x, smem);
+    fors_tile<P, J, PK, PH>(A, blockIdx.x, smem);
 }
 
 // thash (SHA-256) over M payload words after the 22-byte address,
