@@ -9,7 +9,8 @@ narrower ones keep more requests busy per lane; G = 1 is speculative
 verification (every chain from every start first, batches up to 256). The
 crossovers depend on the set and on the batch, so they are measured: for every
 set, operation and batch size this times device-resident launches at each
-split the set allows and writes the winners as
+split the set allows, chooses for all batch sizes together (settle) and writes
+the choices as
 
     <set> <sign|keygen|verify> <min_units> <lanes>
 
@@ -33,6 +34,11 @@ OPS = {"sign": 0, "keygen": 2, "verify": 1}
 # 4x grid left e.g. 2048 requests on the split timed best at 1024
 BATCHES_FAST = tuple(1 << i for i in range(13))   # 1 .. 4096
 BATCHES_SMALL = tuple(1 << i for i in range(11))  # 1 .. 1024
+# a table's last line holds for every larger batch, so verification and key
+# generation are timed to where every split fills the chip: with 4096 as the
+# last size SHAKE256-128f verification stayed at 32 lanes, which at 16384
+# requests take 14.5 ms against 9.3 at 16
+BATCHES_MORE = tuple(1 << i for i in range(15))  # 1 .. 16384
 
 
 def _time(fn, stream, reps):
@@ -49,11 +55,26 @@ def _time(fn, stream, reps):
     return best
 
 
-def _winner(times):
-    """The narrowest split within half a percent of the fastest (repeats of one
-    launch differ by that much, and a table that alternates has no meaning)."""
-    best = min(times.values())
-    return min(S for S, t in times.items() if t <= 1.005 * best)
+def settle(times, order):
+    """The split of each batch size, from times[i] = {split: time} for batches in
+    ascending order: a larger batch never takes a split that comes earlier in
+    `order` (the widest first), and the sum of the times over each batch's best
+    is the least.  Differences below half a percent (repeats of one launch
+    differ by that much) count as none, and the later split is taken.  (Winners
+    taken batch by batch alternate where two splits are equal, and a line made
+    of noise then holds up to the next one.)"""
+    best = None  # split of the last batch -> (cost, choices so far)
+    for t in times:
+        low = min(t.values())
+        row, upto = {}, (0.0, ()) if best is None else None
+        for S in order:
+            if best and S in best and (upto is None or best[S][0] <= upto[0]):
+                upto = best[S]
+            if S in t and upto is not None:
+                row[S] = (upto[0] + max(t[S] / low - 1.005, 0.0), upto[1] + (S,))
+        best = row
+    low = min(cost for cost, _ in best.values())
+    return next(list(best[S][1]) for S in reversed(order) if S in best and best[S][0] == low)
 
 
 def tune_set(name, batches, reps, log):
@@ -70,29 +91,40 @@ def tune_set(name, batches, reps, log):
     d_moff = D.from_array(np.arange(B, dtype=np.uint64) * 32)
     d_mlen = D.from_array(np.full(B, 32, np.uint32))
     d_pk, d_sk, d_sig = D(B * p.pk_bytes), D(B * p.sk_bytes), D(B * p.sig_bytes)
-    d_st = D(4 * B)
-    ws = D(max(C.workspace_bytes(pid, B, op) for op in (0, 1, 2)))
+    V = max(BATCHES_MORE)
+    ws = D(max(C.workspace_bytes(pid, B if op == 0 else V, op) for op in (0, 1, 2)))
     C.keygen_device(pid, B, d_seed.ptr, 3 * p.n, d_pk.ptr, d_sk.ptr, ws.ptr, sh)
     C.sign_device(pid, B, d_sk.ptr, p.sk_bytes, d_msg.ptr, d_moff.ptr, d_mlen.ptr, d_opt.ptr,
                   d_sig.ptr, p.sig_bytes, ws.ptr, sh)
     stream.sync()
+
+    def rows_of(buf, item):  # verification's V requests repeat the signed ones
+        a = buf.download().reshape(B, -1)
+        return D.from_array(a[np.arange(V) % B, :item])
+
+    v_pk, v_sig, v_msg = rows_of(d_pk, p.pk_bytes), rows_of(d_sig, p.sig_bytes), rows_of(d_msg, 32)
+    v_moff = D.from_array(np.arange(V, dtype=np.uint64) * 32)
+    v_mlen, d_st = D.from_array(np.full(V, 32, np.uint32)), D(4 * V)
+    k_seed = D.from_array(rng.integers(0, 256, V * 3 * p.n, dtype=np.uint8))
+    k_pk, k_sk = D(V * p.pk_bytes), D(V * p.sk_bytes)
     hi = 128 if p.len > 64 else 64
-    widths = {0: (1, 4, 16), 2: (1, 4, 16),  # 2 and 8 run as 4 and 16
-              1: (1,) + tuple(G for G in (16, 32, 64, 128) if G <= hi)}
+    order = {0: (16, 4, 1), 2: (16, 4, 1),  # 2 and 8 run as 4 and 16
+             1: (1,) + tuple(G for G in (128, 64, 32, 16) if G <= hi)}
     rows = []
     for op_name, op in OPS.items():
-        for b in batches:
+        grid, timed = batches if op == 0 else BATCHES_MORE, []
+        for b in grid:
             def run():
                 if op == 0:
                     C.sign_device(pid, b, d_sk.ptr, p.sk_bytes, d_msg.ptr, d_moff.ptr,
                                   d_mlen.ptr, d_opt.ptr, d_sig.ptr, p.sig_bytes, ws.ptr, sh)
                 elif op == 1:
-                    C.verify_device(pid, b, d_pk.ptr, p.pk_bytes, d_sig.ptr, p.sig_bytes,
-                                    d_msg.ptr, d_moff.ptr, d_mlen.ptr, d_st.ptr, ws.ptr, sh)
+                    C.verify_device(pid, b, v_pk.ptr, p.pk_bytes, v_sig.ptr, p.sig_bytes,
+                                    v_msg.ptr, v_moff.ptr, v_mlen.ptr, d_st.ptr, ws.ptr, sh)
                 else:
-                    C.keygen_device(pid, b, d_seed.ptr, 3 * p.n, d_pk.ptr, d_sk.ptr, ws.ptr, sh)
+                    C.keygen_device(pid, b, k_seed.ptr, 3 * p.n, k_pk.ptr, k_sk.ptr, ws.ptr, sh)
             times, seen = {}, set()
-            for S in widths[op]:
+            for S in order[op]:
                 C.set_split(pid, op, S)
                 eff = C.get_split(pid, op, b)
                 if eff in seen:
@@ -100,18 +132,19 @@ def tune_set(name, batches, reps, log):
                 seen.add(eff)
                 times[eff] = _time(run, stream, reps)
             C.set_split(pid, op, 0)
-            default = C.get_split(pid, op, b)
-            win = _winner(times)
             if op == 1:
                 st = d_st.download(np.int32, b)
                 if np.count_nonzero(st):
                     raise RuntimeError("%s: verify rejected a valid signature" % name)
-            trees = b * p.d if op == 0 else b
-            rows.append((name, op_name, trees, win))
-            log("%-14s %-6s batch %5d  %s  -> S=%d (heuristic S=%d, %.3f vs %.3f ms)" % (
-                name, op_name, b, " ".join("S%d %.3f" % kv for kv in sorted(times.items())), win,
-                default, times[win], times.get(default, float("nan"))))
-    for buf in (d_seed, d_opt, d_msg, d_moff, d_mlen, d_pk, d_sk, d_sig, d_st, ws):
+            timed.append(times)
+        for b, times, S in zip(grid, timed, settle(timed, order[op])):
+            rows.append((name, op_name, b * p.d if op == 0 else b, S))
+            now = C.get_split(pid, op, b)
+            log("%-14s %-6s batch %5d  %s  -> S=%d (now S=%d, %.3f vs %.3f ms)" % (
+                name, op_name, b, " ".join("S%d %.3f" % kv for kv in sorted(times.items())), S,
+                now, times[S], times.get(now, float("nan"))))
+    for buf in (d_seed, d_opt, d_msg, d_moff, d_mlen, d_pk, d_sk, d_sig, d_st, ws, v_pk, v_sig,
+                v_msg, v_moff, v_mlen, k_seed, k_pk, k_sk):
         buf.free()
     return rows
 
