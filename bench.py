@@ -55,9 +55,9 @@ def mix_ceiling_units(rate, ops_per_unit):
 
 
 def kernel_work(p, batch):
-    """Compressions (SHA-2) or permutations (SHAKE) of the hypertree tiles of
-    one sign launch: every layer's WOTS leaves (PRF + 15 F per chain, T_len)
-    and subtree nodes."""
+    """Compressions (SHA-2) or permutations (SHAKE) of the hypertree of one
+    sign batch (k_chains and k_ht): every layer's WOTS leaves (PRF + 15 F per
+    chain, T_len) and subtree nodes."""
     th = p.full_h // p.d
     leaves = batch * p.d * (1 << th)
     nodes = batch * p.d * ((1 << th) - 1)
