@@ -43,10 +43,11 @@ SHA256_OPS_UNFUSED = 1450
 # Issue rate of independent instructions in the proportions and the two-phase
 # order of the unit's rounds (wave-instructions per SIMD per ns; rotates and
 # v_add3 at raised wave priority, the rest beside other waves' rotates):
-# SHA-256 10 : 18 at 8 waves per SIMD, a wave instruction every 2.22 cycles;
-# Keccak-f 48 : 120 at 5 waves, every 2.33 cycles.
-MIX_RATE_SHA256 = 1.079
-MIX_RATE_KECCAK = 1.030
+# SHA-256 12 : 14 (a quarter of the rounds 7 : 9, without a schedule word) at 8
+# waves per SIMD, a wave instruction every 2.237 cycles; Keccak-f 52 : 122 in
+# runs of 5 and 47 rotates at 5 waves, every 2.343 cycles.
+MIX_RATE_SHA256 = 1.073
+MIX_RATE_KECCAK = 1.024
 
 
 def mix_ceiling_units(rate, ops_per_unit):

@@ -654,14 +654,14 @@ static int keygen_host(const SetOps* o, uint32_t num, const uint8_t* seeds, uint
 }
 
 // slices of a multi-stream call: at most 2, of at least 2048 items (sign,
-// keygen) or 4096 (verify).  Measured on SHA2-128f host buffers, best of 3,
-// slices 1 / 2 / 3 / 4: chained signing slices at 4096 items 17.43 / 17.19 /
-// 17.17 / 17.09 ms and at 8192 33.80 / 32.23 / 32.98 / 32.84 ms (each slice's
-// output copy hides behind the next slice's kernels, smaller launches lose
-// at their tails); concurrent verify slices at 4096 3.60 / 5.02 / 5.39 /
-// 5.16 ms and at 8192 6.54 / 5.82 / 8.24 / 8.16 ms (a verify launch is bound
-// by its 22-layer dependent path, so it gains from sharing the CUs only when
-// each slice still fills them).
+// keygen) or 4096 (verify).  SHA2-128f host buffers, best of 7, slices 1 / 2 /
+// 3 / 4, ms: chained signing slices at 4096 items 12.82 / 11.83 / 11.38 / 11.17,
+// at 8192 24.73 / 22.59 / 21.96 / 21.90, at 16384 47.5 / 43.4 / 42.6 / 42.5 (each
+// slice's output copy hides behind the next slice's kernels; the third and
+// fourth gain 1-6% for as many more lanes' buffers); concurrent verify slices
+// at 4096 3.37 / 3.72 / 4.90 / 4.51, at 8192 5.49 / 5.18 / 5.73 / 6.04, at 16384
+// 10.63 / 8.42 / 9.10 / 8.46 (a verify launch is bound by its 22-layer dependent
+// path, so it gains from sharing the CUs only when each slice still fills them).
 static int ms_slices(int op, uint32_t num) {
     const uint32_t s = num / (op == kOpVerify ? 4096u : 2048u);
     return s < 1 ? 1 : s > 2 ? 2 : (int)s;

@@ -151,12 +151,16 @@ struct Layout {
     }
 };
 
-// Chain waves up to which FORS and chains share a launch (k_sign_fused): as
-// many as the chip holds at once, so the batch is a matter of latency and
-// FORS should not run before the chains.  Larger batches launch k_fors and
-// k_chains one after the other: the fused kernel takes the FORS tile's
-// registers (88-144 VGPRs) for the chains too, and k_chains alone needs 64
-// or fewer for SHA-256 and so issues from 8 waves per SIMD instead of 3-5.
+// Chain waves up to which FORS and chains share a launch (k_sign_fused), so
+// that FORS does not run before the chains; larger batches launch k_fors and
+// k_chains one after the other.  The fused kernel takes the FORS tile's
+// registers (103-152 VGPRs, 4 or 3 waves per SIMD) for the chains too, which
+// k_chains alone runs at 8 (SHA-256, 58-61 VGPRs) or 5; what it gains is the
+// overlap.  Whole call, separate / fused, us: SHA2-128f 1 request 171 / 105,
+// 61 320 / 258, 85 (8190 waves) 364 / 310, 130 487 / 420, 250 (24080) 768 /
+// 720; SHAKE256-256f 28 1013 / 867, 60 1773 / 1600; SHA2-128s 8 642 / 497.  So
+// the crossover lies beyond 24000 waves, and the line is short of it: 8 waves
+// per SIMD, the last size where the chains alone are one round of waves.
 static constexpr uint32_t kFuseWaves = 8192;
 // Chain waves of a fused launch up to which its FORS tiles are the narrowest
 // (JF leaves per lane): with 3.5 chain waves per SIMD or fewer there is room
@@ -170,7 +174,11 @@ static constexpr uint32_t kShortForsWaves = 3584;
 // Waves of FORS tiles up to which a tree of 2^14 leaves (192s, 256s) is split
 // over 4 workgroups, whose last one climbs the top two levels: one workgroup
 // per tree is a serial run of 64 leaves and their nodes on every lane, about
-// 270 hashes, which nothing else in a small batch hides.  SPLITFIG
+// 270 hashes, which nothing else in a small batch hides.  4096 waves are 4 per
+// SIMD, about what the kernels hold at once (117-152 VGPRs).  Whole -> split,
+// us: k_sign_fused of 1 SHA2-192s request 843 -> 297, of 1 SHAKE256-256s 1784 ->
+// 537; k_fors of SHA2-192s 3 requests 826 -> 232, 15 (4080 waves) 853 -> 547,
+// SHA2-256s 5 845 -> 316, 20 (7040 waves) 986 -> 877.
 static constexpr uint32_t kSplitForsWaves = 4096;
 
 // J: FORS leaves per lane, 2^J (2^(a-J) lanes per tree).  Short tiles at every

@@ -527,7 +527,7 @@ __device__ __forceinline__ void keccak_f_il_pair(uint32_t s[25]) {
 // rotated by one) are fixed DPP row moves; 7 and 15 idle.  After rho (a rotate
 // count per lane and row) every word goes through LDS to its place under pi,
 // and each lane reads its new column and the two after it, which chi needs.
-// About 34 instructions and one LDS round trip per round, against 128
+// 35 instructions (21 VALU, 11 LDS) and one LDS round trip per round, against 128
 // instructions on a lane pair.
 struct Keccak16Tab {
     uint8_t rot[16][5];   // v_alignbit count of row y
@@ -555,7 +555,8 @@ struct Keccak16 {
     static constexpr int kLanes = 16;
     // per row of 16 lanes, 16-byte aligned.  Columns are 8 words apart, the odd
     // halves 4 words further, and rows an odd multiple of 16 words, so that
-    // the four rows of a wave touch different banks.
+    // the four rows of a wave start in different banks (of 5.6 LDS cycles per
+    // access SQ_LDS_BANK_CONFLICT still counts 3.0).
     static constexpr int kLdsWords = 112;
     static constexpr int row_words(int w) { return ((w + 15) / 16 | 1) * 16; }
     typedef uint32_t __attribute__((address_space(3))) lds_word;
@@ -661,8 +662,8 @@ struct Keccak16 {
 
 // The same on two such rows, 32 lanes: the first holds rows y = 0, 1, 2 of the
 // columns in s, the second rows 3 and 4 (and a zero), and the column parities
-// are put together by swapping the rows (v_permlane16_swap).  About 26
-// instructions per round.  A permutation alone on its SIMD: 5.5 us on a lane
+// are put together by swapping the rows (v_permlane16_swap).  26 instructions
+// (17 VALU, 6 LDS) per round.  A permutation alone on its SIMD: 5.5 us on a lane
 // pair, 2.50 on 16 lanes, 2.12 on 32; four waves per CU 2.86 and 2.47.
 struct Keccak32Tab {
     uint8_t rot[32][3], wr[32][3], rd[32][3];  // as Keccak16Tab

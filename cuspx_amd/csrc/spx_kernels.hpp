@@ -149,10 +149,13 @@ __host__ __device__ constexpr uint32_t prep_lanes(bool pair) {
 // KiB 1672 / 736; 65536 of 4 KiB 1665 / 385.
 constexpr uint32_t kPrepRows = 7168;
 constexpr uint32_t kPrepWg = 128;
-// the two-wave path from this length: a single SHA2-128f / 256f request of
-// 512 B signs in 0.329 / 0.624 ms against 0.336 / 0.634 on the lane pair,
-// 2 KiB in 0.396 / 0.686 against 0.432 / 0.723, 64 KiB in 3.28 / 3.56
-// against 4.60 / 5.07 (below 512 B the two are equal)
+// the two-wave path from this length: signing one SHA2-128f / 256f request of
+// 512 B takes 129 / 233 us against 141 / 240 on the group of 8 lanes, of 2 KiB
+// 191 / 295 against 240 / 339, of 64 KiB 2.69 / 2.80 ms against 4.40 / 4.33; 300
+// requests of 512 B 0.895 / 2.898 ms against 0.903 / 2.924.  (In batches that
+// fill the SIMDs with groups the 512 workgroups are behind: 2000 requests of
+// 512 B 5.12 / 17.64 ms against 4.97 / 17.42, of 2 KiB 5.42 / 18.01 against
+// 5.10 / 17.59.)
 constexpr uint32_t kLongMsgBytes = 512;
 constexpr uint32_t kLongWgs = 512;         // at most this many two-wave workgroups
 
@@ -1367,8 +1370,9 @@ __global__ void __launch_bounds__(256) k_sign_fused(BatchArgs A, uint32_t n_fors
 //
 // At S = 1 a subtree is one workgroup's (512 lanes for 512 leaves).  With
 // more lanes per leaf, a subtree whose lanes exceed 256 is split over PARTS
-// workgroups, which costs each of them a device-scope fence: at S = 1 that
-// took longer than the hashes (SHA2-128s, 256 requests, 819 -> 378 us).  Each part reduces its leaves to a part root in LDS; the part
+// workgroups, which costs each of them a device-scope fence: at S = 1, two
+// workgroups per subtree took longer than one (SHA2-128s, 256 requests, 819 us
+// against 378).  Each part reduces its leaves to a part root in LDS; the part
 // that finishes last (device-scope counter, release/acquire fences, no
 // waiting) climbs the remaining log2(PARTS) levels from the part roots.
 template <class P, int S>
