@@ -1,6 +1,7 @@
 """Batches whose WOTS chains are 2^32 lanes and more, which one launch cannot
-hold (SHA2-128s: 34240 signatures, 239675 keys): every signature verifies and
-samples are the oracle's; the keys are those of the two halves."""
+hold (SHA2-128s: 34240 signatures, 239675 keys), and the subtrees' launch cut as
+well (16 lanes per leaf, split subtrees): every signature verifies and samples
+are the oracle's; the keys are those of the two halves."""
 import random
 
 import numpy as np
@@ -14,10 +15,11 @@ pytestmark = pytest.mark.gpu
 NAME = "sha2-128s"
 
 
-def test_signing_past_one_launch():
+@pytest.mark.parametrize("n,split", [(34261, 0), (39007, 16)])
+def test_signing_past_one_launch(n, split):
     pid = C.param_id(NAME)
     p = C.params(pid)
-    n, keys = 34261, 5
+    keys = 5
     rng = random.Random(n)
     pk, sk = C.batch_keygen(pid, np.frombuffer(rng.randbytes(3 * p.n * keys), np.uint8))
     at = np.arange(n) % keys
@@ -31,8 +33,12 @@ def test_signing_past_one_launch():
     ws = D(C.workspace_bytes(pid, n, C.OP_SIGN))
     st = C.Stream()
     print("%s: %d signatures, %.1f GB of workspace" % (NAME, n, ws.nbytes / 1e9), flush=True)
-    C.sign_device(pid, n, d_sk.ptr, p.sk_bytes, d_msg.ptr, d_moff.ptr, d_mlen.ptr, d_opt.ptr,
-                  d_sig.ptr, p.sig_bytes, ws.ptr, st.handle)
+    C.set_split(pid, C.OP_SIGN, split)
+    try:
+        C.sign_device(pid, n, d_sk.ptr, p.sk_bytes, d_msg.ptr, d_moff.ptr, d_mlen.ptr, d_opt.ptr,
+                      d_sig.ptr, p.sig_bytes, ws.ptr, st.handle)
+    finally:
+        C.set_split(pid, C.OP_SIGN, 0)
     C.verify_device(pid, n, d_pk.ptr, p.pk_bytes, d_sig.ptr, p.sig_bytes, d_msg.ptr, d_moff.ptr,
                     d_mlen.ptr, d_st.ptr, ws.ptr, st.handle)
     st.sync()
@@ -44,10 +50,10 @@ def test_signing_past_one_launch():
             opt[p.n * i:p.n * (i + 1)].tobytes()), i
 
 
-def test_keygen_past_one_launch():
+@pytest.mark.parametrize("n,split", [(239701, 0), (262147, 16)])
+def test_keygen_past_one_launch(n, split):
     pid = C.param_id(NAME)
     p = C.params(pid)
-    n = 239701
     seeds = np.frombuffer(random.Random(n).randbytes(3 * p.n * n), np.uint8)
     D = C.DeviceBuffer
     d_seed, ws = D.from_array(seeds), D(C.workspace_bytes(pid, n, C.OP_KEYGEN))
@@ -55,8 +61,12 @@ def test_keygen_past_one_launch():
 
     def keys(a, b):
         d_pk, d_sk = D((b - a) * p.pk_bytes), D((b - a) * p.sk_bytes)
-        C.keygen_device(pid, b - a, d_seed.ptr + 3 * p.n * a, 3 * p.n, d_pk.ptr, d_sk.ptr, ws.ptr,
-                        st.handle)
+        C.set_split(pid, C.OP_KEYGEN, split)
+        try:
+            C.keygen_device(pid, b - a, d_seed.ptr + 3 * p.n * a, 3 * p.n, d_pk.ptr, d_sk.ptr,
+                            ws.ptr, st.handle)
+        finally:
+            C.set_split(pid, C.OP_KEYGEN, 0)
         st.sync()
         return d_pk.download(), d_sk.download()
 
