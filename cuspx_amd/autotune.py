@@ -38,7 +38,16 @@ BATCHES_SMALL = tuple(1 << i for i in range(11))  # 1 .. 1024
 # generation are timed to where every split fills the chip: with 4096 as the
 # last size SHAKE256-128f verification stayed at 32 lanes, which at 16384
 # requests take 14.5 ms against 9.3 at 16
-BATCHES_MORE = tuple(1 << i for i in range(15))  # 1 .. 16384
+BATCHES_KEYGEN = tuple(1 << i for i in range(15))  # 1 .. 16384
+# k_vht's time is a staircase: 256 workgroups of 256 / G requests fill the CUs
+# once, so a stair of any G ends at a multiple of 512 requests, and the best G
+# changes from stair to stair (SHAKE256-256s, 16 / 64 lanes: 4096 requests 2.93 /
+# 3.58 ms, 5000 5.77 / 4.49).  A size stands for the requests down to the size
+# before it, and is timed half-way as well: a launch that ends with full CUs can
+# be ahead of every smaller one of its stair (SHA2-128f at 32 lanes, 6000 requests
+# 2.27 ms, 6144 1.85).  Speculative verification grows with every request.
+BATCHES_VERIFY = ((1, 2, 4, 8, 16, 32, 64, 96) + tuple(range(104, 257, 8)) + (384,) +
+                  tuple(512 * i for i in range(1, 33)) + (18432, 20480, 24576, 32768))
 
 
 def _time(fn, stream, reps):
@@ -55,26 +64,34 @@ def _time(fn, stream, reps):
     return best
 
 
-def settle(times, order):
+CHANGE = 0.005
+
+
+def settle(times, order, back=False):
     """The split of each batch size, from times[i] = {split: time} for batches in
-    ascending order: a larger batch never takes a split that comes earlier in
-    `order` (the widest first), and the sum of the times over each batch's best
-    is the least.  Differences below half a percent (repeats of one launch
-    differ by that much) count as none, and the later split is taken.  (Winners
-    taken batch by batch alternate where two splits are equal, and a line made
-    of noise then holds up to the next one.)"""
+    ascending order: the least sum of the times over each batch's best, counting
+    half a percent (repeats of one launch differ by that much) for each change
+    and differences below it as none.  Unless `back`, a larger batch never takes
+    a split that comes earlier in `order` (the widest first).  Of equal sums
+    later splits are taken.  (Winners taken batch by batch alternate where two
+    splits are equal, and a line made of noise then holds up to the next one.)"""
     best = None  # split of the last batch -> (cost, choices so far)
     for t in times:
         low = min(t.values())
-        row, upto = {}, (0.0, ()) if best is None else None
-        for S in order:
-            if best and S in best and (upto is None or best[S][0] <= upto[0]):
-                upto = best[S]
-            if S in t and upto is not None:
-                row[S] = (upto[0] + max(t[S] / low - 1.005, 0.0), upto[1] + (S,))
+        row = {}
+        for i, S in enumerate(order):
+            if S not in t:
+                continue
+            cost, path = 0.0, ()
+            if best is not None:
+                come = [(c + CHANGE * (Q != S), -order.index(Q), p) for Q, (c, p) in best.items()
+                        if back or order.index(Q) <= i]
+                if not come:
+                    continue
+                cost, _, path = min(come, key=lambda x: x[:2])
+            row[S] = (cost + max(t[S] / low - 1 - CHANGE, 0.0), path + (S,))
         best = row
-    low = min(cost for cost, _ in best.values())
-    return next(list(best[S][1]) for S in reversed(order) if S in best and best[S][0] == low)
+    return list(min(best.items(), key=lambda x: (x[1][0], -order.index(x[0])))[1][1])
 
 
 def tune_set(name, batches, reps, log):
@@ -91,7 +108,7 @@ def tune_set(name, batches, reps, log):
     d_moff = D.from_array(np.arange(B, dtype=np.uint64) * 32)
     d_mlen = D.from_array(np.full(B, 32, np.uint32))
     d_pk, d_sk, d_sig = D(B * p.pk_bytes), D(B * p.sk_bytes), D(B * p.sig_bytes)
-    V = max(BATCHES_MORE)
+    V = max(BATCHES_VERIFY + BATCHES_KEYGEN)
     ws = D(max(C.workspace_bytes(pid, B if op == 0 else V, op) for op in (0, 1, 2)))
     C.keygen_device(pid, B, d_seed.ptr, 3 * p.n, d_pk.ptr, d_sk.ptr, ws.ptr, sh)
     C.sign_device(pid, B, d_sk.ptr, p.sk_bytes, d_msg.ptr, d_moff.ptr, d_mlen.ptr, d_opt.ptr,
@@ -112,9 +129,12 @@ def tune_set(name, batches, reps, log):
              1: (1,) + tuple(G for G in (128, 64, 32, 16) if G <= hi)}
     rows = []
     for op_name, op in OPS.items():
-        grid, timed = batches if op == 0 else BATCHES_MORE, []
+        grid, timed, first = (batches, BATCHES_VERIFY, BATCHES_KEYGEN)[op], [], 0
         for b in grid:
-            def run():
+            sizes = {b, (first + b) // 2 or b} if op == 1 else {b}
+            first = b + 1
+
+            def run(b):
                 if op == 0:
                     C.sign_device(pid, b, d_sk.ptr, p.sk_bytes, d_msg.ptr, d_moff.ptr,
                                   d_mlen.ptr, d_opt.ptr, d_sig.ptr, p.sig_bytes, ws.ptr, sh)
@@ -130,15 +150,17 @@ def tune_set(name, batches, reps, log):
                 if eff in seen:
                     continue
                 seen.add(eff)
-                times[eff] = _time(run, stream, reps)
+                times[eff] = sum(_time(lambda: run(n), stream, reps) for n in sizes) / len(sizes)
             C.set_split(pid, op, 0)
             if op == 1:
                 st = d_st.download(np.int32, b)
                 if np.count_nonzero(st):
                     raise RuntimeError("%s: verify rejected a valid signature" % name)
             timed.append(times)
-        for b, times, S in zip(grid, timed, settle(timed, order[op])):
-            rows.append((name, op_name, b * p.d if op == 0 else b, S))
+        first = 0
+        for b, times, S in zip(grid, timed, settle(timed, order[op], back=op == 1)):
+            rows.append((name, op_name, first if op == 1 else b * p.d if op == 0 else b, S))
+            first = b + 1
             now = C.get_split(pid, op, b)
             log("%-14s %-6s batch %5d  %s  -> S=%d (now S=%d, %.3f vs %.3f ms)" % (
                 name, op_name, b, " ".join("S%d %.3f" % kv for kv in sorted(times.items())), S,
